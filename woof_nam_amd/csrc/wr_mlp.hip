@@ -294,14 +294,42 @@ __global__ void k_splitk_reduce(const float *__restrict__ part, int splits, long
     out[i] = s;
 }
 
-// column sums db[n] = sum_m X[m * ld + n] (fixed order; one thread per column)
-__global__ void k_colsum(const float *__restrict__ X, int M, int N, long long ld, float *__restrict__ out)
+// Column sums db[n] = sum_m X[m * ld + n], in a fixed order.  A workgroup owns CS_N columns (64-byte row
+// segments) and its CS_R row groups walk every CS_R-th row with CS_U loads in flight, each into its own
+// sum; the sums of a column then meet in a tree through LDS.  One thread per column, as this ran
+// before, is one chain of M dependent loads on N / 64 waves: 3 ms for the 16,384 x 504 error of a
+// training step, against 20 us here (bound by the few workgroups that N / CS_N gives).
+constexpr int CS_N = 16, CS_R = 64, CS_U = 8;
+__global__ void __launch_bounds__(CS_N * CS_R) k_colsum(const float *__restrict__ X, int M, int N, long long ld,
+                                                        float *__restrict__ out)
 {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    float s = 0.f;
-    for (int m = 0; m < M; ++m) s += X[(size_t)m * ld + n];
-    out[n] = s;
+    __shared__ float red[CS_R][CS_N + 1];
+    const int c = threadIdx.x % CS_N, r = threadIdx.x / CS_N;
+    const int n = blockIdx.x * CS_N + c;
+    float s[CS_U];
+#pragma unroll
+    for (int u = 0; u < CS_U; ++u) s[u] = 0.f;
+    if (n < N) {
+        int m = r;
+        for (; m + (CS_U - 1) * CS_R < M; m += CS_U * CS_R)
+#pragma unroll
+            for (int u = 0; u < CS_U; ++u) s[u] += X[(size_t)(m + u * CS_R) * ld + n];
+#pragma unroll
+        for (int u = 0; u < CS_U; ++u)
+            if (m + u * CS_R < M) s[u] += X[(size_t)(m + u * CS_R) * ld + n];
+    }
+#pragma unroll
+    for (int o = CS_U / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int u = 0; u < o; ++u) s[u] += s[u + o];
+    red[r][c] = s[0];
+    __syncthreads();
+#pragma unroll
+    for (int o = CS_R / 2; o > 0; o >>= 1) {
+        if (r < o) red[r][c] += red[r + o][c];
+        __syncthreads();
+    }
+    if (r == 0 && n < N) out[n] = red[0][c];
 }
 
 // dY = 2 (Y - T) * scale; per-block partial sum of squared error
@@ -488,7 +516,7 @@ int wr_mlp_colsum(const float *X, int32_t M, int32_t N, int64_t ld, float *out, 
 {
     if (!X || !out || M < 0 || N < 0) return WR_ERR_ARG;
     if (N == 0) return WR_OK;
-    hipLaunchKernelGGL(k_colsum, dim3((N + 255) / 256), dim3(256), 0, (hipStream_t)stream, X, M, N, (long long)ld, out);
+    hipLaunchKernelGGL(k_colsum, dim3((N - 1) / CS_N + 1), dim3(CS_N * CS_R), 0, (hipStream_t)stream, X, M, N, (long long)ld, out);
     return hipGetLastError() == hipSuccess ? WR_OK : WR_ERR_HIP;
 }
 
