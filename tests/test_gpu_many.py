@@ -1,0 +1,50 @@
+"""Small tiles: every band of a tile in one launch against the per-band launches.
+
+WR_MANY_COLS=0 (read when a context is created) keeps the per-band kernels; both run the same column
+functions, so every output is the same bits, at the edges of a 64-column block, for both precisions and
+routes, with and without the optional column inputs."""
+import numpy as np
+import pytest
+import torch
+
+from woof_nam_amd import abi, gen
+from woof_nam_amd.radiation import Radiation
+
+pytestmark = pytest.mark.gpu
+
+
+def columns(n, seed, ext, device):
+    c = gen.columns(n, seed=seed)
+    if ext:
+        rng = np.random.default_rng(seed)
+        dp = np.diff(c["p_lev"], axis=0) * (1000.0 / 9.80665)
+        c["cwp"], c["cip"], c["crp"] = c["qc"] * dp, c["qi"] * dp, 0.1 * c["qc"] * dp
+        c["rew"] = rng.uniform(5.0, 14.0, size=c["t_lay"].shape)
+        c["rei"] = rng.uniform(20.0, 100.0, size=c["t_lay"].shape)
+        c["o3_top"] = 0.5 * c["o3_lay"][0]
+        for k, nb in abi.AER_BANDS.items():
+            a = np.empty((3, nb, c["t_lay"].shape[0] + 1, n), dtype=np.float32)
+            a[0], a[1], a[2] = rng.uniform(0.0, 0.02, size=a[0].shape), 0.9, 0.65
+            c[k] = a
+    return {k: torch.from_numpy(np.ascontiguousarray(v)).to(device) for k, v in c.items()}
+
+
+@pytest.mark.parametrize("mcica,ext", [(1, False), (0, False), (1, True), (0, True)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_one_launch_equals_per_band_launches(gpu_device, monkeypatch, precision, mcica, ext):
+    p = Radiation.default_params(mcica=mcica, seed=11)
+    rads = []
+    for env in ("0", None):
+        monkeypatch.setenv("WR_MANY_COLS", env) if env else monkeypatch.delenv("WR_MANY_COLS")
+        rads.append(Radiation(0, max_cols=700))
+    try:
+        for n in (1, 63, 64, 65, 701):              # 701: a full tile and a one-column tile
+            print(f"case one launch {precision} mcica={mcica} ext={ext} ncol={n}", flush=True)
+            cols = columns(n, 50 + n, ext, gpu_device)
+            a, b = (r.run(cols, params=p, precision=precision)[0] for r in rads)
+            torch.cuda.synchronize()
+            for k in abi.OUTPUT_FIELDS:
+                assert torch.equal(a[k].view(torch.int64), b[k].view(torch.int64)), (k, n)
+    finally:
+        for r in rads:
+            r.close()

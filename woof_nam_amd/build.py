@@ -35,6 +35,7 @@ OBJ = PKG / "_build"
 ARCH = os.environ.get("WR_OFFLOAD_ARCH", "gfx950")
 
 UNITS = ["wr_host.hip", "wr_fp64.hip", "wr_fp64_ext.hip", "wr_mixed.hip", "wr_mixed_ext.hip", "wr_mlp.hip", "wr_surr.hip",
+         "wr_many_fp64.hip", "wr_many_fp64_nam.hip", "wr_many_mixed.hip", "wr_many_mixed_nam.hip", "wr_many_surr.hip",
          "wr_nmmb.hip", "wr_solar.hip", "wr_aer.hip", "wr_serve.hip"]
 CFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -55,11 +56,14 @@ def hipcc() -> str:
 # per SIMD of every band kernel come from per-band tables in the sources (wr_kernels.h, wr_nam.h).
 # WR_LW_GSPLIT=2 (two lanes per column in LW, half of the g-points each) halves the LW registers but
 # measured 9 % slower: the per-layer column work then runs twice.
-_FP32_UNIT = ["-ffp-contract=fast", "-fno-hip-fp32-correctly-rounded-divide-sqrt"]
+_FP32_UNIT = ["-ffp-contract=on", "-fno-hip-fp32-correctly-rounded-divide-sqrt"]
 UNIT_FLAGS = {
     "wr_mixed.hip": _FP32_UNIT,
     "wr_mixed_ext.hip": _FP32_UNIT,
     "wr_surr.hip": _FP32_UNIT,
+    "wr_many_mixed.hip": _FP32_UNIT,
+    "wr_many_mixed_nam.hip": _FP32_UNIT,
+    "wr_many_surr.hip": _FP32_UNIT,
 }
 
 

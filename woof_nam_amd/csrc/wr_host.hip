@@ -17,6 +17,7 @@
 
 #include "wr_glw.h"
 #include "wr_internal.h"
+#include "wr_many.h"
 
 using namespace wr;
 
@@ -523,13 +524,23 @@ uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_
     return m & ((1u << nb) - 1u);
 }
 
+// Tiles of up to this many columns run every band in one launch (wr_many.h); WR_MANY_COLS overrides it
+// at context creation (0: never).
+constexpr int MANY_COLS_DEFAULT = 8192;
+int many_cols_env()
+{
+    const char *e = getenv("WR_MANY_COLS");
+    return e ? std::max(0, atoi(e)) : MANY_COLS_DEFAULT;
+}
+constexpr size_t MANY_BLOCK = std::max(many_block_bytes<double, false>(64 + 1), many_block_bytes<float, false>(64 + 1));
+
 // Device bytes of a context's tile work space for tiles of m columns, and the band-stream count.
 struct Sizes {
-    size_t acc, iws, dws, rtr, sflux_d, sflux_f, lwrec, pool;
+    size_t acc, iws, dws, rtr, sflux_d, sflux_f, lwrec, pool, pool_all;
     int naux;
     size_t total() const
     {
-        return acc + iws + dws + rtr + sflux_d + sflux_f + lwrec + pool * (size_t)(naux > 1 ? naux : 1);
+        return acc + iws + dws + rtr + sflux_d + sflux_f + lwrec + pool_all;
     }
 };
 Sizes sizes(int32_t max_cols)
@@ -558,6 +569,10 @@ Sizes sizes(int32_t max_cols)
     const char *e = getenv("WR_BAND_STREAMS");
     const int na = e ? atoi(e) : WR_NAUX;
     z.naux = na < 0 ? 0 : (na > WR_NAUX ? WR_NAUX : na);
+    // the streams' pools lie one after another; together they also hold every band's slots of the tiles
+    // that run their bands in one launch
+    const size_t many = (size_t)((std::min(max_cols, many_cols_env()) + 63) / 64) * MANY_BLOCK;
+    z.pool_all = std::max(z.pool * (size_t)(z.naux > 1 ? z.naux : 1), many);
     return z;
 }
 
@@ -565,13 +580,14 @@ Sizes sizes(int32_t max_cols)
 // The mixed-precision tile work space for up to WR_NOALLOC_MAX_COLS columns of up to 64 radiation
 // layers, in one static device array (every device the library runs on holds its own copy until the
 // process ends).  Layout (256-byte aligned parts): FP32 band flux planes, column words, layer logs and
-// level temperatures, NAM-route overlap factors, FP32 solar source, and one band stream's level pool
-// with a slot for every 64-column block.  The kernels write every word of it that they read, so
+// level temperatures, NAM-route overlap factors, FP32 solar source, and a level pool with the slots of
+// all bands for NA_BLOCKS 64-column blocks.  The kernels write every word of it that they read, so
 // nothing needs clearing between calls; calls that overlap on one device race on it.
 struct NaLayout {
     size_t acc, iws, dws, rtr, sflux, pool, total;
 };
 constexpr size_t na_al(size_t x) { return (x + 255) & ~(size_t)255; }
+constexpr int NA_BLOCKS = 16;  // 64-column blocks whose bands run at once
 constexpr NaLayout na_layout()
 {
     const size_t m = WR_NOALLOC_MAX_COLS;
@@ -582,14 +598,12 @@ constexpr NaLayout na_layout()
     z.dws = off, off += na_al(sizeof(double) * (4 + 2 * (size_t)NL) * m);
     z.rtr = off, off += na_al((sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m);
     z.sflux = off, off += na_al(sizeof(float) * 112 * m);
-    const size_t lane_max = std::max(cache_slot_bytes(sw_nv_mc<float>(), 16, 64 + 1, (int)sizeof(float)),
-                                     cache_slot_bytes(LW_NV_F32, 16, 64 + 1, (int)sizeof(float)));
-    z.pool = off, off += (m + 63) / 64 * lane_max;
+    z.pool = off, off += NA_BLOCKS * many_block_bytes<float, false>(64 + 1);
     z.total = off;
     return z;
 }
 constexpr NaLayout NA = na_layout();
-static_assert(NA.total <= ((size_t)256 << 20), "the no-alloc work space stays under 256 MiB");
+static_assert(NA.total <= ((size_t)384 << 20), "the no-alloc work space stays under 384 MiB");
 
 static __device__ __align__(256) char scratch[NA.total];
 
@@ -672,7 +686,9 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
     }
     if (rc == WR_OK) {
         c->pool_bytes = z.pool;
-        if (hipMalloc((void **)&c->pool[0], c->pool_bytes) != hipSuccess) rc = WR_ERR_NOMEM;
+        c->pool_all = z.pool_all;
+        c->many_cols = many_cols_env();
+        if (hipMalloc((void **)&c->pool[0], c->pool_all) != hipSuccess) rc = WR_ERR_NOMEM;
     }
     if (rc == WR_OK) {
         // WR_BAND_STREAMS=0 keeps the band kernels on the caller's stream
@@ -683,8 +699,7 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
                 rc = WR_ERR_HIP;
         // one level pool per band stream (stream 0 shares the caller's), all allocated here: no later
         // call allocates
-        for (int q = 1; q < c->naux && rc == WR_OK; ++q)
-            if (hipMalloc((void **)&c->pool[q], c->pool_bytes) != hipSuccess) rc = WR_ERR_NOMEM;
+        for (int q = 1; q < c->naux && rc == WR_OK; ++q) c->pool[q] = c->pool[0] + (size_t)q * c->pool_bytes;
         if (rc == WR_OK && c->naux > 0 && hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess)
             rc = WR_ERR_HIP;
     }
@@ -741,7 +756,8 @@ int wr_run_mixed_noalloc(wr_ctx *ctx, const wr_columns *in, const wr_params *par
     t.lw_glane = 0;
     for (int q = 0; q < WR_NAUX; ++q) t.pool[q] = nullptr;
     t.pool[0] = base + NA.pool;
-    t.pool_bytes = NA.total - NA.pool;
+    t.pool_bytes = t.pool_all = NA.total - NA.pool;
+    t.many_cols = WR_NOALLOC_MAX_COLS;
     t.naux = 0;
     rc = run(&t, in, par, out, nullptr, stream, MODE_MIXED);
     ctx->ev_n = t.ev_n;
@@ -856,6 +872,7 @@ const char *wr_kernel_name(int32_t kid)
     if (kid == KID_MLP) return "mlp_gemm";
     if (kid == KID_RTRFAC) return "k_rtr_fac";
     if (kid == KID_LWREC) return "k_lwrec";
+    if (kid == KID_MANY) return "k_many";
     return "?";
 }
 
@@ -906,8 +923,8 @@ void wr_destroy(wr_ctx *c)
     (void)hipFree(c->sx);
     (void)hipFree(c->sy);
     (void)hipFree(c->sflag);
+    (void)hipFree(c->pool[0]);
     for (int q = 0; q < WR_NAUX; ++q) {
-        (void)hipFree(c->pool[q]);
         if (c->aux[q]) (void)hipStreamDestroy(c->aux[q]);
         if (c->join[q]) (void)hipEventDestroy(c->join[q]);
     }

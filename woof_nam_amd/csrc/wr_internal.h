@@ -44,6 +44,8 @@ struct wr_ctx {
     // pool[q]: aux stream q), pool_bytes each, all allocated by wr_create
     char *pool[WR_NAUX];
     size_t pool_bytes;
+    size_t pool_all;                 // bytes from pool[0] on, pool[1..] among them: one launch may use them all
+    int many_cols;                   // tiles of up to this many columns run every band in one launch
     // band-kernel streams (default priority, non-blocking) and their fork/join events
     int naux;
     hipStream_t aux[WR_NAUX];
@@ -56,7 +58,7 @@ struct wr_ctx {
 
 // kernel ids reported by wr_timing_read
 enum { KID_ZERO = 0, KID_COLPREP = 1, KID_DAYLIST = 2, KID_LW0 = 3, KID_SW0 = 19, KID_POST = 33, KID_DIAG = 34,
-       KID_FEAT = 35, KID_MLP = 36, KID_RTRFAC = 37, KID_LWREC = 38, KID_COUNT = 39 };
+       KID_FEAT = 35, KID_MLP = 36, KID_RTRFAC = 37, KID_LWREC = 38, KID_MANY = 39, KID_COUNT = 40 };
 
 inline void tbeg(wr_ctx *c, int kid, hipStream_t s)
 {
@@ -121,6 +123,11 @@ int wr_launch_fp64_ext(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, co
                        int band, hipStream_t s);
 int wr_launch_mixed_ext(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, const wr::OutPtrs &out, int col0, int n,
                         int band, hipStream_t s);
+// every band of a small tile in one launch (wr_many.h), on the tile that launch_tile / launch_tile_nam set up
+namespace wr {
+template <typename R> struct BandJob;
+template <typename R, bool NAM, bool SURR> int launch_many(const BandJob<R> &j, hipStream_t s);
+}  // namespace wr
 int wr_launch_diag_fp64(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, const wr_diag *dg, int col0, int n,
                         hipStream_t s);
 int wr_launch_diag_mixed(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, const wr_diag *dg, int col0, int n,

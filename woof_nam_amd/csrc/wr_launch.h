@@ -326,6 +326,9 @@ int run_bands(wr_ctx *c, int band, hipStream_t s, F &&one)
     return WR_OK;
 }
 
+// Whether a tile of n columns runs all its bands in one launch (wr_many.h)
+inline bool use_many(const wr_ctx *c, int n, int band) { return band < 0 && n <= c->many_cols && !c->lw_glane; }
+
 // One tile of n columns from col0 (McICA route): column scalars, day list, band kernels, FP64 post.
 // No host synchronisation.  EXT selects the band kernels that read the optional column inputs (the
 // caller passes EXT = has_ext(in) or true).
@@ -347,7 +350,9 @@ int launch_tile(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, const
         hipLaunchKernelGGL((k_lwrec<R>), dim3((n + 63) / 64), dim3(64), 0, s, tabs, in, par, col0, n, j.cs, j.rec);
         tend(c, s);
     }
-    int rc = run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band<R, SURR, EXT>(j, id, q, pool); });
+    int rc = use_many(c, n, band)
+                 ? launch_many<R, false, SURR>(j, s)
+                 : run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band<R, SURR, EXT>(j, id, q, pool); });
     if (rc != WR_OK) return rc;
     tbeg(c, KID_POST, s);
     hipLaunchKernelGGL(k_post<R>, dim3((n + 255) / 256), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);
@@ -377,7 +382,9 @@ int launch_tile_nam(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, c
     tbeg(c, KID_RTRFAC, s);
     hipLaunchKernelGGL((k_rtr_fac<R>), dim3((n + 63) / 64), dim3(64), 0, s, in, col0, n, rt);
     tend(c, s);
-    int rc = run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band_nam<R, EXT>(j, id, q, pool); });
+    int rc = use_many(c, n, band)
+                 ? launch_many<R, true, false>(j, s)
+                 : run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band_nam<R, EXT>(j, id, q, pool); });
     if (rc != WR_OK) return rc;
     tbeg(c, KID_POST, s);
     hipLaunchKernelGGL(k_post<R>, dim3((n + 255) / 256), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);

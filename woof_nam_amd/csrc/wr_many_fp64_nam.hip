@@ -1,0 +1,6 @@
+// wr_many_fp64_nam.hip -- the one-launch band kernel of small tiles (FP64, NAM route).
+#include "wr_many.h"
+
+namespace wr {
+template int launch_many<double, true, false>(const BandJob<double> &, hipStream_t);
+}  // namespace wr

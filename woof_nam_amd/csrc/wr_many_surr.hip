@@ -1,0 +1,6 @@
+// wr_many_surr.hip -- the one-launch band kernel of small tiles (mixed precision, learned gas optics, McICA route).
+#include "wr_many.h"
+
+namespace wr {
+template int launch_many<float, false, true>(const BandJob<float> &, hipStream_t);
+}  // namespace wr
