@@ -122,6 +122,8 @@ template <typename R> struct Tabs {
     const WR_G R *totplnk, *delwave, *absliq1, *absice1;
     const WR_G int32_t *ipat, *layreffr, *ix1, *ix2, *ibx;
     const WR_G R *exp_tbl, *tfn_tbl, *tau_tbl, *sw_exp_tbl;
+    const WR_G R *chir;    // [6][59] reference ratios of the binary gas pairs (chi_row in wr_lw.h)
+    const WR_G R *lut4;    // FP64: [NTBL + 1]{exp, tfn, tau, 0}, the LW tables of one index side by side
     const WR_G double *sw_exp_tbl64;  // FP64 SW exp table (layers that take the FP64 R/T branch)
     const WR_G R *sf01, *sf02, *sf03, *sw_strrat, *sw_specwt;
     const WR_G R *extliq1, *ssaliq1, *asyliq1, *extice3, *ssaice3, *asyice3;

@@ -115,6 +115,13 @@ struct Blob {
         }
         return (const WR_G T *)(base + off);
     }
+    template <typename T> const WR_G T *put(const T *src, size_t n)
+    {
+        const size_t off = align();
+        bytes.resize(off + n * sizeof(T), 0);
+        memcpy(bytes.data() + off, src, n * sizeof(T));
+        return (const WR_G T *)(base + off);
+    }
     template <typename T> WR_G T *reserve(size_t n)
     {
         const size_t off = align();
@@ -203,6 +210,7 @@ template <typename R> int bind_tables(const TFile &f, Blob &b, Tabs<R> &T)
     T.tfn_tbl = b.reserve<R>(NTBL + 1);
     T.tau_tbl = b.reserve<R>(NTBL + 1);
     T.sw_exp_tbl = b.reserve<R>(NTBL + 1);
+    if (sizeof(R) == 8) T.lut4 = b.reserve<R>(4 * (NTBL + 1));
 
     for (int k = 0; k < 16; ++k) {
         LwBand<R> &B = T.lw[k];
@@ -266,6 +274,10 @@ template <typename R> int bind_tables(const TFile &f, Blob &b, Tabs<R> &T)
     auto rr = [&](int g1, int l1, int g2, int l2) {
         return (R)((double)cm[(l1 - 1) * 7 + (g1 - 1)] / (double)cm[(l2 - 1) * 7 + (g2 - 1)]);
     };
+    R chir[CHI_PAIRS * 59];  // the same ratios per reference level, for the key species of the lower and upper levels
+    for (int q = 0; q < CHI_PAIRS; ++q)
+        for (int l = 1; l <= 59; ++l) chir[q * 59 + l - 1] = rr(CHI_PAIR[q][0], l, CHI_PAIR[q][1], l);
+    T.chir = b.put<R>(chir, CHI_PAIRS * 59);
     T.lw[2].refrat_planck_a = rr(1, 9, 2, 9);
     T.lw[2].refrat_planck_b = rr(1, 13, 2, 13);
     T.lw[2].refrat_m_a = rr(1, 3, 2, 3);
@@ -536,11 +548,11 @@ constexpr size_t MANY_BLOCK = std::max(many_block_bytes<double, false>(64 + 1), 
 
 // Device bytes of a context's tile work space for tiles of m columns, and the band-stream count.
 struct Sizes {
-    size_t acc, iws, dws, rtr, sflux_d, sflux_f, lwrec, pool, pool_all;
+    size_t acc, iws, dws, rtr, sflux_d, sflux_f, rec, lwrec, pool, pool_all;
     int naux;
     size_t total() const
     {
-        return acc + iws + dws + rtr + sflux_d + sflux_f + lwrec + pool_all;
+        return acc + iws + dws + rtr + sflux_d + sflux_f + rec + lwrec + pool_all;
     }
 };
 Sizes sizes(int32_t max_cols)
@@ -553,6 +565,7 @@ Sizes sizes(int32_t max_cols)
     z.rtr = (sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m;      // NAM-route overlap factors
     z.sflux_d = sizeof(double) * 112 * m;
     z.sflux_f = sizeof(float) * 112 * m;
+    z.rec = rec_block_bytes((int)sizeof(double)) * 64 * ((m + 63) / 64);     // layer records, up to 64 layers
     z.lwrec = lw_glane_env() ? lwrec_bytes_per_col<double>(64 + 1) * m + 3 * 256 : 0;  // LW layer records
     // level pool: room for every 64-column block of a tile in the largest slot layout (FP64 SW:
     // 2 values, FP32 SW: 7 values, x 16 g x levels), at most WR_POOL_GB (default 6) GB per stream
@@ -580,11 +593,11 @@ Sizes sizes(int32_t max_cols)
 // The mixed-precision tile work space for up to WR_NOALLOC_MAX_COLS columns of up to 64 radiation
 // layers, in one static device array (every device the library runs on holds its own copy until the
 // process ends).  Layout (256-byte aligned parts): FP32 band flux planes, column words, layer logs and
-// level temperatures, NAM-route overlap factors, FP32 solar source, and a level pool with the slots of
+// level temperatures, NAM-route overlap factors, FP32 solar source, layer records, and a level pool with the slots of
 // all bands for NA_BLOCKS 64-column blocks.  The kernels write every word of it that they read, so
 // nothing needs clearing between calls; calls that overlap on one device race on it.
 struct NaLayout {
-    size_t acc, iws, dws, rtr, sflux, pool, total;
+    size_t acc, iws, dws, rtr, sflux, rec, pool, total;
 };
 constexpr size_t na_al(size_t x) { return (x + 255) & ~(size_t)255; }
 constexpr int NA_BLOCKS = 16;  // 64-column blocks whose bands run at once
@@ -598,12 +611,13 @@ constexpr NaLayout na_layout()
     z.dws = off, off += na_al(sizeof(double) * (4 + 2 * (size_t)NL) * m);
     z.rtr = off, off += na_al((sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m);
     z.sflux = off, off += na_al(sizeof(float) * 112 * m);
+    z.rec = off, off += na_al(rec_block_bytes((int)sizeof(float)) * 64 * ((m + 63) / 64));
     z.pool = off, off += NA_BLOCKS * many_block_bytes<float, false>(64 + 1);
     z.total = off;
     return z;
 }
 constexpr NaLayout NA = na_layout();
-static_assert(NA.total <= ((size_t)384 << 20), "the no-alloc work space stays under 384 MiB");
+static_assert(NA.total <= ((size_t)448 << 20), "the no-alloc work space stays under 448 MiB");
 
 static __device__ __align__(256) char scratch[NA.total];
 
@@ -669,7 +683,7 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
             hipMalloc((void **)&c->dws, z.dws) != hipSuccess || hipMalloc(&c->rtr, z.rtr) != hipSuccess ||
             hipMalloc((void **)&c->sflux_d, z.sflux_d) != hipSuccess ||
             hipMalloc((void **)&c->sflux_f, z.sflux_f) != hipSuccess ||
-            (z.lwrec && hipMalloc(&c->lwrec, z.lwrec) != hipSuccess))
+            hipMalloc((void **)&c->rec, z.rec) != hipSuccess || (z.lwrec && hipMalloc(&c->lwrec, z.lwrec) != hipSuccess))
             rc = WR_ERR_NOMEM;
         c->lw_glane = z.lwrec > 0;
         if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
@@ -752,6 +766,7 @@ int wr_run_mixed_noalloc(wr_ctx *ctx, const wr_columns *in, const wr_params *par
     t.rtr = base + NA.rtr;
     t.sflux_d = nullptr;
     t.sflux_f = (float *)(base + NA.sflux);
+    t.rec = base + NA.rec;
     t.lwrec = nullptr;  // lane-per-column LW kernels
     t.lw_glane = 0;
     for (int q = 0; q < WR_NAUX; ++q) t.pool[q] = nullptr;
@@ -873,6 +888,8 @@ const char *wr_kernel_name(int32_t kid)
     if (kid == KID_RTRFAC) return "k_rtr_fac";
     if (kid == KID_LWREC) return "k_lwrec";
     if (kid == KID_MANY) return "k_many";
+    if (kid == KID_SWPREP) return "k_swprep";
+    if (kid == KID_MCICA) return "k_mcica";
     return "?";
 }
 
@@ -919,6 +936,7 @@ void wr_destroy(wr_ctx *c)
     (void)hipFree(c->rtr);
     (void)hipFree(c->sflux_d);
     (void)hipFree(c->sflux_f);
+    (void)hipFree(c->rec);
     (void)hipFree(c->lwrec);
     (void)hipFree(c->sx);
     (void)hipFree(c->sy);

@@ -26,6 +26,7 @@ struct wr_ctx {
     void *rtr;                       // maximum-random overlap factors of the NAM LW route
     double *sflux_d;                 // [112][max_cols]
     float *sflux_f;
+    char *rec;                       // layer records and McICA words of a tile (wr_rec.h), sized for FP64
     void *lwrec;                     // LW layer records of a tile (g-lane LW kernels), sized for FP64
     int lw_glane;                    // 1: McICA LW bands as g-lane kernels over the layer records
     uint32_t lw_lds;                 // bit B: the FP32 McICA kernel of LW band B + 1 stages its tables in LDS
@@ -58,7 +59,8 @@ struct wr_ctx {
 
 // kernel ids reported by wr_timing_read
 enum { KID_ZERO = 0, KID_COLPREP = 1, KID_DAYLIST = 2, KID_LW0 = 3, KID_SW0 = 19, KID_POST = 33, KID_DIAG = 34,
-       KID_FEAT = 35, KID_MLP = 36, KID_RTRFAC = 37, KID_LWREC = 38, KID_MANY = 39, KID_COUNT = 40 };
+       KID_FEAT = 35, KID_MLP = 36, KID_RTRFAC = 37, KID_LWREC = 38, KID_MANY = 39, KID_SWPREP = 40, KID_MCICA = 41,
+       KID_COUNT = 42 };
 
 inline void tbeg(wr_ctx *c, int kid, hipStream_t s)
 {

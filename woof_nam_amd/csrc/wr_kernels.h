@@ -17,8 +17,7 @@
 #pragma once
 #include <type_traits>
 
-#include "wr_lw.h"
-#include "wr_sw.h"
+#include "wr_rec.h"
 
 // Default minimum waves per SIMD of the LW band kernels (register budget 512 / waves).  One
 // keeps everything in registers (AGPRs included), with no scratch (private segment) that the runtime
@@ -29,6 +28,11 @@
 #endif
 
 namespace wr {
+
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef double f64x2v __attribute__((ext_vector_type(2)));
+typedef double f64x4v __attribute__((ext_vector_type(4)));
 
 // Level fluxes of ONE band for one tile ([nrl+1][n] planes, written once per level; sw_clr0 [n]), in
 // the band kernel's precision P: FP64 planes for the FP64 kernels; FP32 planes for the FP32 kernels,
@@ -62,18 +66,9 @@ __host__ __device__ inline AccT<P> band_acc(const BandAcc &ba, int id)  // id 0.
     }
     return a;
 }
-struct ColScal {
-    WR_G int *lw_laytrop, *lcf1, *day, *sw_laytrop, *dlist, *nday;
-    WR_G double *pwv, *zcf1, *zcf0;
-    // per tile column, written by k_colprep: la[kin * n + t] = log of the layer pressure (layer kin,
-    // top-first); tz[L * n + t] = LW level temperature, L = 0 the top layer's temperature, L = kin + 1
-    // the interface below layer kin, L = nrl the skin temperature
-    WR_G double *la, *tz;
-};
 
-template <typename R>
-__global__ void __launch_bounds__(256) k_colprep(const Tabs<R> *__restrict__ T, ColIn in, RunPar par, int col0, int n,
-                                                 ColScal cs, R *__restrict__ sflux)
+// Column scalars of a tile, one thread per column; the layer logs come from k_layers.
+static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int n, ColScal cs)
 {
 #pragma clang fp contract(off)
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -89,10 +84,12 @@ __global__ void __launch_bounds__(256) k_colprep(const Tabs<R> *__restrict__ T, 
     const double tem2c = 1.0e-20 * 1.0e3 * CON_AVGD;
     double tem1 = 0.0, tem2 = 0.0, z0 = 1.0, z1 = 1.0;
     int lt = 0, lcf = 0, swlt = nrl;
-    int jpk[NL];
+    double pb = rc.plvl(nrl);
     for (int k = 0; k < nrl; ++k) {
         const int kin = nrl - 1 - k;
-        const double dlp = rc.plvl(kin + 1) - rc.plvl(kin);
+        const double pt = rc.plvl(kin);
+        const double dlp = pb - pt;
+        pb = pt;
         const double qv = rc.qlyr(kin);
         const double h2ovmr = fmax(0.0, qv * AMDW / (1.0 - qv));
         const double tem0 = (1.0 - h2ovmr) * CON_AMD + h2ovmr * CON_AMW;
@@ -100,15 +97,11 @@ __global__ void __launch_bounds__(256) k_colprep(const Tabs<R> *__restrict__ T, 
         const double ca0 = fmax(0.0, cdry * h2ovmr);
         tem1 = tem1 + cdry + ca0;
         tem2 = tem2 + ca0;
-        const double la = log_d(rc.plyr(kin));
-        cs.la[(size_t)kin * n + t] = la;
-        if (la > 4.56) {
+        if (cs.la[(size_t)kin * n + t] > 4.56) {
             lt += 1;
             swlt = k + 1;
         }
-        jpk[k] = imax(1, imin(58, (int)(36.0 - 5.0 * (la + 0.04))));
-        double ct, cwp, cip;
-        rc.cloud(kin, ct, cwp, cip);
+        const double ct = rc.cfrac(kin);
         if (ct > EPS) lcf = 1;
         if (ct > FTINY) {
             z1 = fmin(z1, 1.0 - ct);
@@ -119,16 +112,9 @@ __global__ void __launch_bounds__(256) k_colprep(const Tabs<R> *__restrict__ T, 
     }
     cs.lw_laytrop[t] = lt;
     cs.lcf1[t] = lcf;
-    // LW level temperatures, the operations the band kernels' sweeps used to repeat per band
-    cs.tz[t] = rc.tlyr(0);
-    for (int kin = 0; kin + 1 < nrl; ++kin)
-        cs.tz[(size_t)(kin + 1) * n + t] = tlvl_v(rc.tlyr(kin + 1), rc.tlyr(kin), log_d(rc.plvl(kin + 1)),
-                                                  cs.la[(size_t)(kin + 1) * n + t], cs.la[(size_t)kin * n + t]);
-    cs.tz[(size_t)nrl * n + t] = rc.tskn();
     const double tem0p = 10.0 * tem2 / (AMDW * tem1 * CON_G);
     cs.pwv[t] = tem0p * rc.plvl(nrl);
-    const double cz = in.cosz[i];
-    const int day = cz >= 1.0e-4;
+    const int day = in.cosz[i] >= 1.0e-4;
     cs.day[t] = day;
     if (!day) return;
     z0 = z0 * z1;
@@ -137,52 +123,62 @@ __global__ void __launch_bounds__(256) k_colprep(const Tabs<R> *__restrict__ T, 
     cs.zcf1[t] = 1.0 - z0;
     cs.zcf0[t] = z0;
     cs.sw_laytrop[t] = swlt;
-    // solar source per g-point (phys_rrtm_sw_taumol.cu:59-120)
-    for (int b = 0; b < 14; ++b) {
-        const int jb = b + 16, ibd = T->ibx[b], njb = SW_NG[b], ns = SW_NS[b], lr = T->layreffr[b];
-        if (jb == 16 || jb == 20 || jb == 23 || jb == 25 || jb == 26 || jb == 29) {
-            for (int j = 0; j < njb; ++j) sflux[(size_t)(ns + j) * n + t] = T->sf01[(ibd - 1) * 16 + j];
-        } else if (jb == 27) {
-            for (int j = 0; j < njb; ++j) sflux[(size_t)(ns + j) * n + t] = T->scalekur * T->sf01[(ibd - 1) * 16 + j];
-        } else {
-            int ks, mfs;
-            const WR_G R *tab;
-            if (jb == 17 || jb == 28) {
-                ks = nrl;
-                for (int k = swlt; k <= nrl - 1; ++k)
-                    if (jpk[k - 1] < lr && jpk[k] >= lr) {
-                        ks = k + 1;
-                        break;
-                    }
-                tab = T->sf02;
-                mfs = 5;
-            } else {
-                ks = swlt;
-                for (int k = 1; k <= swlt - 1; ++k)
-                    if (jpk[k - 1] < lr && jpk[k] >= lr) {
-                        ks = k + 1;
-                        break;
-                    }
-                tab = T->sf03;
-                mfs = 9;
-            }
-            SwLay<R> L;
-            const int kin = nrl - 1 - (ks - 1);
-            sw_layer<R>(T, rc, par, kin, log_d(rc.plyr(kin)), L);
-            const R colm1 = L.colamt[T->ix1[b] - 1];
-            const R colm2 = L.colamt[T->ix2[b] - 1];
-            const R speccomb = colm1 + T->sw_strrat[b] * colm2;
-            const R specmult = T->sw_specwt[b] * fmin((R)0.999999, colm1 / speccomb);
-            const int jsi = (int)specmult;
-            const int js = 1 + jsi;
-            const R fs = specmult - (R)jsi;
-            const int base = ((ibd - 1) * mfs) * 16;
-            for (int j = 0; j < njb; ++j) {
-                const R a = tab[base + (js - 1) * 16 + j];
-                const R c = tab[base + js * 16 + j];
-                sflux[(size_t)(ns + j) * n + t] = a + fs * (c - a);
-            }
+}
+
+// Solar source per g-point (phys_rrtm_sw_taumol.cu:59-120), one thread per (day-list entry, band).
+template <typename R>
+__global__ void __launch_bounds__(64) k_sflux(const Tabs<R> *__restrict__ T, ColIn in, RunPar par, int col0, int n, ColScal cs,
+                                              R *__restrict__ sflux)
+{
+    const int tt = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y;
+    if (tt >= *cs.nday) return;
+    const int t = cs.dlist[tt];
+    const RadCol rc{in, col0 + t, in.nlay + 1};
+    const int nrl = rc.nrl, swlt = cs.sw_laytrop[t];
+    const int jb = b + 16, ibd = T->ibx[b], njb = SW_NG[b], ns = SW_NS[b], lr = T->layreffr[b];
+    if (jb == 16 || jb == 20 || jb == 23 || jb == 25 || jb == 26 || jb == 29) {
+        for (int j = 0; j < njb; ++j) sflux[(size_t)(ns + j) * n + t] = T->sf01[(ibd - 1) * 16 + j];
+        return;
+    }
+    if (jb == 27) {
+        for (int j = 0; j < njb; ++j) sflux[(size_t)(ns + j) * n + t] = T->scalekur * T->sf01[(ibd - 1) * 16 + j];
+        return;
+    }
+    auto jp = [&](int k) {  // reference pressure index of surface-first layer k
+        return imax(1, imin(58, (int)(36.0 - 5.0 * (cs.la[(size_t)(nrl - 1 - k) * n + t] + 0.04))));
+    };
+    const bool upper = jb == 17 || jb == 28;
+    const WR_G R *tab = upper ? T->sf02 : T->sf03;
+    const int mfs = upper ? 5 : 9, k0 = upper ? swlt : 1, k1 = upper ? nrl - 1 : swlt - 1;
+    int ks = upper ? nrl : swlt;
+    for (int k = k0, prev = jp(k0 - 1); k <= k1; ++k) {
+        const int cur = jp(k);
+        if (prev < lr && cur >= lr) {
+            ks = k + 1;
+            break;
         }
+        prev = cur;
+    }
+    SwLay<R> L;
+    const int kin = nrl - 1 - (ks - 1);
+    sw_layer<R>(T, rc, par, kin, cs.la[(size_t)kin * n + t], L);
+    const int i1 = T->ix1[b] - 1, i2 = T->ix2[b] - 1;
+    R colm1 = (R)0, colm2 = (R)0;
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+        colm1 = m == i1 ? L.colamt[m] : colm1;
+        colm2 = m == i2 ? L.colamt[m] : colm2;
+    }
+    const R speccomb = colm1 + T->sw_strrat[b] * colm2;
+    const R specmult = T->sw_specwt[b] * fmin((R)0.999999, colm1 / speccomb);
+    const int jsi = (int)specmult;
+    const int js = 1 + jsi;
+    const R fs = specmult - (R)jsi;
+    const int base = ((ibd - 1) * mfs) * 16;
+    for (int j = 0; j < njb; ++j) {
+        const R a = tab[base + (js - 1) * 16 + j];
+        const R c = tab[base + js * 16 + j];
+        sflux[(size_t)(ns + j) * n + t] = a + fs * (c - a);
     }
 }
 
@@ -351,65 +347,16 @@ __device__ __forceinline__ void surr_lw(const Surr &sg, size_t s, R *tau, R *fr,
     }
 }
 
-// the layer quantities the LW transfer needs besides the gas optics
-template <typename R> __device__ __forceinline__ void lw_layer_cloud(const LayV &v, LwLay<R> &L)
-{
-    L.ct = v.ct;
-    L.clwp = v.cwp * 1.5;
-    L.ciwp = v.cip * 1.5;
-    L.tavel = v.t;
-    L.delp = v.pb - v.pt;
-}
-
-// ---- per-wave level cache of the band kernels -------------------------------------------------------
-// The SW adding method keeps two reflectances per g-point and level from the bottom-up sweep for the
-// top-down sweep (the FP32 kernels also keep each layer's R/T, and the FP32 LW kernel its upward
-// transmittance and source).  They live in a slot of the context's pool, not in per-lane private
-// arrays (which would need kilobytes of scratch per lane, backed by the runtime on every HIP queue):
-// one slot per resident 64-lane workgroup (the kernels loop over column blocks, so the slot count
-// bounds the memory), laid out [level][value][g][lane] so that every access is one coalesced 64-lane
-// row.  Level-major order makes the offset of every (value, g) row within a level a compile-time
-// constant; with the level innermost instead, the compiler kept one 64-bit address per row live
-// across the level loops, and the SW kernels spilled up to 150 registers more (8 % slower).
-// A slot holds nk = nlay + 2 levels (layers 0..nrl-1, or levels 0..nrl) of nv values per g-point.
-template <typename R> struct LaneCache {
-    WR_G R *p;  // this lane's element 0
-    int nv;
-    __device__ __forceinline__ R &at(int v, int ng, int g, int k) const
-    {
-        return p[(((size_t)k * nv + v) * ng + g) * 64];
-    }
-};
+// ---- per-wave level slots of the band kernels -------------------------------------------------------
+// What a column's second sweep takes over from its first lives in a slot of the context's pool, not in
+// per-lane private arrays (which would need kilobytes of scratch per lane, backed by the runtime on every
+// HIP queue): one slot per resident 64-lane wave (the kernels loop over column blocks, so the slot count
+// bounds the memory), laid out [level][g][lane][value], so that every access is one contiguous run of the
+// wave and the offset of a g-point within a level is a compile-time constant.  A slot holds nk = nlay + 2
+// levels of nv values per g-point.
 __host__ __device__ constexpr size_t cache_slot_bytes(int nv, int ng, int nk, int rbytes)
 {
     return (size_t)64 * nv * ng * nk * rbytes;
-}
-template <typename R>
-__device__ __forceinline__ LaneCache<R> lane_cache(char *pool, int nv, int ng, int nk)
-{
-    LaneCache<R> c;
-    c.p = (WR_G R *)(pool + (size_t)blockIdx.x * cache_slot_bytes(nv, ng, nk, (int)sizeof(R))) + threadIdx.x;
-    c.nv = nv;
-    return c;
-}
-constexpr int SW_NV = 2;  // per level and g: zrupb, zrupd (reflectances of the medium below)
-// The FP32 SW kernels also keep each layer's R/T (rb, rd, tb, td, ld) for the top-down sweep instead
-// of recomputing optics and two-stream there (3 % faster); in FP64 the extra HBM traffic outweighs it.
-template <typename R> constexpr int sw_nv_mc() { return sizeof(R) == 4 ? SW_NV + 5 : SW_NV; }
-
-// Lanes per column of the LW band kernels: one by default.  WR_LW_GSPLIT=2 gives the FP32
-// instantiations two (each lane takes half of the band's g-points, which halves the registers a lane
-// holds; the two partial g-sums meet through a lane swap), but the per-layer column work then runs
-// twice and it measured 9 % slower.  FP64 always uses one (sums over g in the reference's order).
-#ifndef WR_LW_GSPLIT
-#define WR_LW_GSPLIT 1
-#endif
-template <typename R> constexpr int lw_gsplit() { return sizeof(R) == 4 ? WR_LW_GSPLIT : 1; }
-
-template <int GS, typename R> __device__ __forceinline__ R gsum(R s)
-{
-    if constexpr (GS == 2) return s + __shfl_xor(s, 1);
-    return s;
 }
 
 // Optics chunks and wave bounds of the LW band kernels, per band.  These kernels wait on table gathers
@@ -432,10 +379,10 @@ template <int GS, typename R> __device__ __forceinline__ R gsum(R s)
 // gathers in flight, no second wave to cover the waits).
 // WR_LWC_WAVES / WR_LW64_WAVES > 0 or WR_LW_CHUNK / WR_LW64_CHUNK >= 0 override the tables for every
 // band (tuning builds).
-constexpr int LWC_WAVES[16] = {1, 1, 2, 2, 2, 1, 2, 1, 2, 1, 1, 1, 1, 1, 3, 3};
-constexpr int LWC_CHUNK[16] = {0, 0, 4, 4, 4, 4, 4, 4, 4, 0, 0, 4, 0, 0, 0, 0};
-constexpr int LW64_WAVES[16] = {2, 1, 1, 1, 1, 1, 1, 2, 1, 1, 1, 2, 1, 1, 1, 1};
-constexpr int LW64_CHUNK[16] = {2, 2, 0, 0, 0, 2, 0, 4, 0, 0, 2, 2, 0, 0, 0, 0};
+constexpr int LWC_WAVES[16] = {4, 4, 3, 3, 3, 4, 3, 4, 3, 4, 4, 4, 4, 4, 4, 4};
+constexpr int LWC_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
+constexpr int LW64_WAVES[16] = {2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2};
+constexpr int LW64_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
 #ifndef WR_LWC_WAVES
 #define WR_LWC_WAVES 0
 #endif
@@ -462,214 +409,248 @@ constexpr int chunk_of(int ngl, int want)
     return ngl;
 }
 template <int B> constexpr int lw_chunk() { return chunk_of(LW_NG[B], WR_LW_CHUNK >= 0 ? WR_LW_CHUNK : LWC_CHUNK[B]); }
-template <typename R, int B, int NGL> constexpr int lw_chunk_r()
+template <typename R, int B> constexpr int lw_chunk_r()
 {
-    return sizeof(R) == 8 ? chunk_of(NGL, WR_LW64_CHUNK >= 0 ? WR_LW64_CHUNK : LW64_CHUNK[B]) : NGL;
+    return sizeof(R) == 8 ? chunk_of(LW_NG[B], WR_LW64_CHUNK >= 0 ? WR_LW64_CHUNK : LW64_CHUNK[B]) : lw_chunk<B>();
 }
-// lw_optics of g-points g0 .. g0 + NGL - 1 in chunks of CH, from the band tables Bt
-template <typename R, int B, int NGL, int CH, typename BT>
-__device__ __forceinline__ void lw_optics_ch(const Tabs<R> *__restrict__ T, const BT &Bt, const LwLay<R> &L, R *tau, R *fr,
-                                             int g0)
+// ---- LW band kernels (rtrnmc, McICA) ------------------------------------------------------------
+// One lane per column, one wave per 64-column block; the layer's set-up comes from its record row
+// (wr_rec.h), the McICA bits of the band's g-points from one word per layer.  The g-points of a layer run
+// in chunks: a chunk's table gathers, its transmittances and its radiances are done before the next
+// chunk's gathers are issued (a scheduling barrier stands between), which bounds the registers.  Inside a chunk
+// nothing branches per g-point: both forms of the transmittance are evaluated and selected, so that the
+// chunk's chains (division, table gather or exponential) overlap; a form that no lane of the wave needs
+// is skipped as a whole.
+
+// Transmittance, source factor and optical depth of the LW tables at od (rtrnmc's tblind quantisation).
+// FP64 reads the table the oracle reproduces; FP32 evaluates the entry.  FP32: tblind of the largest
+// depths rounds to 1, where the table ends in (1e-20, 1, 1e10); the index stops just below it, which gives
+// those values to FP32 accuracy.  tau and 1 / tau share one reciprocal.
+template <typename R> __device__ __forceinline__ void lw_lut(const Tabs<R> *__restrict__ T, R od, R &e, R &tfn, R &tau)
 {
-    if constexpr (CH >= NGL) {
-        lw_optics_t<R, B, NGL>(T, Bt, L, tau, fr, g0);
+    if constexpr (sizeof(R) == 4) {
+        const R tb = od * __builtin_amdgcn_rcpf((R)(1.0 / 0.278) + od);
+        const R fi = fmin(floorf(__builtin_fmaf((R)NTBL, tb, (R)0.5)), (R)9999.999);
+        const R ci = (R)NTBL - fi;
+        const R r = __builtin_amdgcn_rcpf(fi * ci);
+        tau = ((R)(1.0 / 0.278) * fi) * (fi * r);
+        const R it = (ci * r) * (ci * (R)0.278);
+        e = fmax(M<R>::exp(-tau), (R)1.0e-20);
+        const R big = __builtin_fmaf((R)-2, it - e * __builtin_amdgcn_rcpf((R)1 - e), (R)1);
+        tfn = tau < (R)0.06 ? tau * (R)(1.0 / 6.0) : big;
     } else {
+        const R tb = od / ((R)(1.0 / 0.278) + od);
+        const f64x4v q = ((const WR_G f64x4v *)T->lut4)[imin(NTBL, (int)((R)NTBL * tb + (R)0.5))];
+        e = q.x, tfn = q.y, tau = q.z;
+    }
+}
+
+template <typename R, int CH> struct GasV {  // CH g-points: transmittance, absorptance, source factor, optical depth
+    R tr[CH], at[CH], gf[CH], od[CH];
+};
+template <typename R, int CH>
+__device__ __forceinline__ void lw_gas_v(const Tabs<R> *__restrict__ T, R sdif, R taer, const R *tau, GasV<R, CH> &q)
+{
+    bool any = false;
 #pragma unroll
-        for (int c = 0; c < NGL; c += CH) {
-            lw_optics_t<R, B, CH>(T, Bt, L, tau + c, fr + c, g0 + c);
-            __builtin_amdgcn_sched_barrier(0);
+    for (int j = 0; j < CH; ++j) {
+        const R od = fmax((R)0, sdif * (tau[j] + taer));
+        q.od[j] = od;
+        q.at[j] = od - (R)0.5 * od * od;
+        q.tr[j] = (R)1 - q.at[j];
+        q.gf[j] = (R)0.166667 * od;
+        any |= !(od <= (R)0.06);
+    }
+    if (__any(any)) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            R e, tfn, ta;
+            lw_lut<R>(T, q.od[j], e, tfn, ta);
+            const bool big = !(q.od[j] <= (R)0.06);
+            q.tr[j] = big ? e : q.tr[j];
+            q.at[j] = big ? (R)1 - e : q.at[j];
+            q.gf[j] = big ? tfn : q.gf[j];
+            q.od[j] = big ? ta : q.od[j];
         }
     }
 }
-template <typename R, int B, int NGL, int CH>
-__device__ __forceinline__ void lw_optics_ch(const Tabs<R> *__restrict__ T, const LwLay<R> &L, R *tau, R *fr, int g0)
+// the same for the total (gas plus cloud) optical depth: transmittance, absorptance, source factor
+template <typename R, int CH>
+__device__ __forceinline__ void lw_tot_v(const Tabs<R> *__restrict__ T, const R *od, R odcld, R *tr, R *at, R *gf)
 {
-    lw_optics_ch<R, B, NGL, CH>(T, T->lw[B], L, tau, fr, g0);
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const R x = od[j] + odcld;
+        at[j] = x - (R)0.5 * x * x;
+        tr[j] = (R)1 - at[j];
+        gf[j] = (R)0.166667 * x;
+        any |= !(x < (R)0.06);
+    }
+    if (__any(any)) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const R x = od[j] + odcld;
+            R e, tfn, ta;
+            lw_lut<R>(T, x, e, tfn, ta);
+            const bool big = !(x < (R)0.06);
+            tr[j] = big ? e : tr[j];
+            at[j] = big ? (R)1 - e : at[j];
+            gf[j] = big ? tfn : gf[j];
+        }
+    }
 }
 
-// One column of LW band B (GS lanes per column; gt = the lane's index over the tile), optics from the
-// band tables Bt: down sweep, surface, up sweep with the optics recomputed.
+// What the LW transfer of one column needs besides its layers.
+template <typename R> struct LwCol {
+    int i, t, nrl, lcf1, table;
+    R sdif, semis, reflct;
+};
+template <typename R, int B, bool SURR>
+__device__ __forceinline__ LwCol<R> lw_col(const ColIn &in, int col0, const ColScal &cs, const Surr &sg, int t)
+{
+    LwCol<R> c;
+    c.i = col0 + t, c.t = t, c.nrl = in.nlay + 1;
+    c.lcf1 = cs.lcf1[t];
+    c.table = SURR ? sg.table(t, B) : 1;
+    const double pwv = cs.pwv[t];
+    c.sdif = (R)((B == 0 || B == 3 || B == 9) ? 1.66 : fmin(1.80, fmax(1.50, LW_A0[B] + LW_A1[B] * exp_d(LW_A2[B] * pwv))));
+    const double sfe = in.emis[c.i];
+    c.semis = (R)((sfe > EPS && sfe <= 1.0) ? sfe : 1.0);
+    c.reflct = (R)1 - c.semis;
+    return c;
+}
+
+// A layer of a column as the sweeps use it: Planck sources of the layer and of the level below, cloud.
+template <typename R> struct LwLayer {
+    LwLay<R> L;
+    R blay, bbot;   // Planck function at the layer and at the level below it
+    R taer, odcld;  // aerosol absorption depth; cloud depth times the diffusivity secant
+    bool cloudy;    // this lane's layer holds cloud
+};
+template <typename R, int B>
+__device__ __forceinline__ void lw_get(const Tabs<R> *__restrict__ T, const ColIn &in, const RunPar &par, const RecPtrs &rp,
+                                       const LwCol<R> &c, int blk, int lane, int k, LwLayer<R> &y)
+{
+    const LRow<R> row = lrow<R>(rp, blk, k, lane);
+    const uint32_t w0 = row.w(0), w1 = row.w(1);
+    lrow_get<R>(row, w0, y.L);
+    y.blay = planck_of<R>(T, B, (int)(w0 >> 22), row.f(LF_PL));
+    y.bbot = planck_of<R>(T, B, (int)(w1 & 255u), row.f(LF_PB));
+    y.cloudy = (w1 & 256u) != 0;
+    const RadCol rc{in, c.i, c.nrl};
+    y.taer = (R)rc.aer_lw_tau(B, c.nrl - 1 - k);  // tautot = taug + tauaer
+    y.odcld = (R)0;
+    if (__any(y.cloudy)) {
+        double rl = par.re_liq, ri = par.re_ice, rain = 0.0;
+        if (y.cloudy) rc.props(c.nrl - 1 - k, par.re_liq, par.re_ice, rl, ri, rain);
+        const R tc = lw_taucld_r<R>(T, B, row.f(LF_LIQ), row.f(LF_ICE), rl, ri, rain);
+        y.odcld = c.sdif * (y.cloudy ? tc : (R)0);
+    }
+}
+// gas optical depth and Planck fraction of g-points g0 .. g0 + CH - 1 of a layer
+template <typename R, int B, bool SURR, int CH, typename BT>
+__device__ __forceinline__ void lw_taufr(const Tabs<R> *__restrict__ T, const BT &Bt, const Surr &sg, const LwCol<R> &c, int n,
+                                         int k, const LwLay<R> &L, int g0, R *tau, R *fr)
+{
+    if (SURR && !c.table)
+        surr_lw<R, B, CH>(sg, (size_t)k * n + c.t, tau, fr, g0);
+    else
+        lw_optics_t<R, B, CH>(T, Bt, L, tau, fr, g0);
+}
+
+// One column of LW band B in FP64, optics from the band tables Bt: down sweep, surface, up sweep with the
+// optics evaluated again.  Every sum and product in the reference's order.
 template <typename R, int B, bool SURR, typename BT>
 __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par,
-                                          int col0, int n, const ColScal &cs, const AccT<R> &acc, const Surr &sg, int gt)
+                                          int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
+                                          const Surr &sg, int blk, int lane)
 {
-    constexpr int GS = lw_gsplit<R>();
-    constexpr int NG = LW_NG[B];
-    constexpr int NGL = NG / GS;
-    static_assert(NG % GS == 0, "g-points split evenly over the lanes of a column");
-    constexpr int NS = LW_NS[B];
-    const int t = gt / GS;
-    const int g0 = (gt % GS) * NGL;
-    const bool lead = (gt % GS) == 0;  // writes the column's level fluxes
-    if (t >= valid_cols(in, col0, n)) return;  // both lanes of a column leave together
-    const int i = col0 + t;
-    const RadCol rc{in, i, in.nlay + 1};
-    const int nrl = rc.nrl;
-    const int lcf1 = cs.lcf1[t];
-    const int table = SURR ? sg.table(t, B) : 1;  // 0: learned gas optics for this column
-    const double pwv = cs.pwv[t];
-    const R sdif = (R)((B == 0 || B == 3 || B == 9) ? 1.66 : fmin(1.80, fmax(1.50, LW_A0[B] + LW_A1[B] * exp_d(LW_A2[B] * pwv))));
-    const double sfe = in.emis[i];
-    const R semis = (R)((sfe > EPS && sfe <= 1.0) ? sfe : 1.0);
-    const uint64_t col = in.col_id ? in.col_id[i] : (uint64_t)i;
-    const uint64_t seed = in.seed_dev ? *in.seed_dev : par.seed;
-    uint64_t mb[NGL];
-    for (int jj = 0; jj < NGL; ++jj)
-        mb[jj] = mcica_g(col, seed, 0, NS + g0 + jj, nrl, par.iovr, [&](int k) { return lcf1 ? rc.cfrac(nrl - 1 - k) : 0.0; });
-
-    if (lead) acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
-    // ---- down sweep, top to surface ----
-    R rad[NGL];
+    constexpr int NG = LW_NG[B], CH = lw_chunk_r<R, B>();
+    const int t = blk * 64 + lane;
+    if (t >= valid_cols(in, col0, n)) return;
+    const LwCol<R> c = lw_col<R, B, SURR>(in, col0, cs, sg, t);
+    const int nrl = c.nrl;
+    acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
+    R rad[NG];
 #pragma unroll
-    for (int jj = 0; jj < NGL; ++jj) rad[jj] = (R)0;
-    // layer inputs: cur = layer kin, nxt = kin + 1 (loaded an iteration ahead), nn = kin + 2
-    LayV cur = rc.lay(0), nxt = cur;
-    if (nrl > 1) nxt = rc.lay(1);
-    double tz_top = cs.tz[t], la_nx = cs.la[t], tz_nx = 0.0;
-    if constexpr (sizeof(R) != 8) tz_nx = cs.tz[(size_t)n + t];
-    for (int kin = 0; kin < nrl; ++kin) {
-        const int k = nrl - 1 - kin;
-        LayV nn = nxt;
-        if (kin + 2 < nrl) nn = rc.lay(kin + 2);
-        // this layer's log pressure and bottom level temperature: FP32 kernels load k_colprep's values an
-        // iteration ahead; FP64 kernels evaluate them here by the same operations (measured faster there)
-        double la_c, tz_bot;
-        if constexpr (sizeof(R) == 8) {
-            la_c = la_nx;
-            if (kin + 1 < nrl) {
-                la_nx = log_d(nxt.pl);
-                tz_bot = tlvl_v(nxt.t, cur.t, log_d(cur.pb), la_nx, la_c);
-            } else {
-                tz_bot = rc.tskn();
-            }
-        } else {
-            la_c = la_nx, tz_bot = tz_nx;
-            if (kin + 1 < nrl) la_nx = cs.la[(size_t)(kin + 1) * n + t], tz_nx = cs.tz[(size_t)(kin + 2) * n + t];
-        }
-        LwLay<R> L;
-        R tau[NGL], fr[NGL];
-        if (SURR && !table) {
-            lw_layer_cloud<R>(cur, L);
-            surr_lw<R, B, NGL>(sg, (size_t)k * n + t, tau, fr, g0);
-        } else {
-            lw_layer<R>(T, cur, par, la_c, L);
-            lw_optics_ch<R, B, NGL, lw_chunk_r<R, B, NGL>()>(T, Bt, L, tau, fr, g0);
-        }
-        const R blay = planck<R>(T, B, L.tavel);
-        const R dplnkd = planck<R>(T, B, tz_bot) - blay;
-        const R taucld = lw_taucld_l<R>(T, B, lcf1, L, rc, kin, par);
-        const R taer = (R)rc.aer_lw_tau(B, kin);  // tautot = taug + tauaer
-        R s = (R)0;
+    for (int g = 0; g < NG; ++g) rad[g] = (R)0;
+    // one layer of a sweep: dir 0 down (source between the layer and the level below), 1 up
+    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, uint32_t bits, bool sfc, R pk0, R &s, R &s0) {
+        s = (R)0, s0 = (R)0;
+        R ecld = (R)1;
+        if (__any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
 #pragma unroll
-        for (int jj = 0; jj < NGL; ++jj) {
-            const GasT<R> q = lw_gas<R>(T, sdif, tau[jj] + taer);
-            const R plfrac = fr[jj];
-            const R bbdgas = plfrac * (blay + dplnkd * q.gasfac);
-            const R gassrcd = bbdgas * q.atrgas;
-            const R clfm = ((mb[jj] >> k) & 1) ? (R)1 : (R)0;
-            if (clfm >= (R)EPS) {
-                const R odcld = sdif * taucld;
-                const R efclrfr = (R)1 - ((R)1 - M<R>::exp(-odcld)) * clfm;
-                R totfac, atrtot;
-                lw_tot<R>(T, q.odepth + odcld, totfac, atrtot);
-                const R bbdtot = plfrac * (blay + dplnkd * totfac);
-                const R totsrcd = bbdtot * atrtot;
-                rad[jj] = rad[jj] * q.trng * efclrfr + gassrcd + clfm * (totsrcd - gassrcd);
-            } else {
-                rad[jj] = rad[jj] * q.trng + gassrcd;
+        for (int g0 = 0; g0 < NG; g0 += CH) {
+            R tau[CH], fr[CH];
+            lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
+            GasV<R, CH> q;
+            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
+            if (sfc) {  // surface emission and reflection
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const R rad0 = c.semis * fr[j] * pk0;
+                    rad[g0 + j] = rad0 + c.reflct * rad[g0 + j];
+                    s0 = s0 + rad[g0 + j];
+                }
             }
-            s = s + rad[jj];
+            R nr[CH], gas[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const R bb = fr[j] * (y.blay + dplnk * q.gf[j]);
+                gas[j] = bb * q.at[j];
+                nr[j] = rad[g0 + j] * q.tr[j] + gas[j];
+            }
+            if (__any((bits >> g0) & ((1u << CH) - 1u))) {
+                R tr[CH], at[CH], gf[CH];
+                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+                const R efclrfr = (R)1 - ((R)1 - ecld);
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const R bbt = fr[j] * (y.blay + dplnk * gf[j]);
+                    const R tot = bbt * at[j];
+                    const R rc = rad[g0 + j] * q.tr[j] * efclrfr + gas[j] + (tot - gas[j]);
+                    nr[j] = (bits >> (g0 + j)) & 1u ? rc : nr[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                rad[g0 + j] = nr[j];
+                s = s + nr[j];
+            }
+            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
         }
-        s = gsum<GS>(s);
-        if (lead) acc.lw_dn[(size_t)k * n + t] = s;
-        tz_top = tz_bot;
-        cur = nxt, nxt = nn;
+    };
+    R s, s0;
+    for (int k = nrl - 1; k >= 0; --k) {  // down sweep, top to surface
+        LwLayer<R> y;
+        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
+        sweep(k, y, y.bbot - y.blay, bits, false, (R)0, s, s0);
+        acc.lw_dn[(size_t)k * n + t] = s;
     }
-    // ---- up sweep, surface to top ----
-    const R reflct = (R)1 - semis;
-    double tz_bot = cs.tz[(size_t)nrl * n + t];
-    // layer inputs: cur = layer kin, nxt = kin - 1 (loaded an iteration ahead), nn = kin - 2
-    cur = rc.lay(nrl - 1), nxt = cur;
-    if (nrl > 1) nxt = rc.lay(nrl - 2);
-    if constexpr (sizeof(R) == 8)
-        la_nx = log_d(cur.pl);
-    else
-        la_nx = cs.la[(size_t)(nrl - 1) * n + t], tz_nx = cs.tz[(size_t)(nrl - 1) * n + t];
-    for (int kin = nrl - 1; kin >= 0; --kin) {
-        const int k = nrl - 1 - kin;
-        LayV nn = nxt;
-        if (kin >= 2) nn = rc.lay(kin - 2);
-        const double la_c = la_nx;
-        if constexpr (sizeof(R) == 8) {
-            if (kin > 0) {
-                la_nx = log_d(nxt.pl);
-                tz_top = tlvl_v(cur.t, nxt.t, log_d(cur.pt), la_c, la_nx);
-            } else {
-                tz_top = cur.t;
-            }
-        } else {
-            tz_top = tz_nx;
-            if (kin > 0) la_nx = cs.la[(size_t)(kin - 1) * n + t], tz_nx = cs.tz[(size_t)(kin - 1) * n + t];
+    for (int k = 0; k < nrl; ++k) {  // up sweep, surface to top
+        LwLayer<R> y;
+        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
+        // the level above is the next layer's lower level; above the top layer, its own temperature
+        R btop = y.blay;
+        if (k + 1 < nrl) {
+            const LRow<R> up = lrow<R>(rp, blk, k + 1, lane);
+            btop = planck_of<R>(T, B, (int)(up.w(1) & 255u), up.f(LF_PB));
         }
-        LwLay<R> L;
-        R tau[NGL], fr[NGL];
-        if (SURR && !table) {
-            lw_layer_cloud<R>(cur, L);
-            surr_lw<R, B, NGL>(sg, (size_t)k * n + t, tau, fr, g0);
-        } else {
-            lw_layer<R>(T, cur, par, la_c, L);
-            lw_optics_ch<R, B, NGL, lw_chunk_r<R, B, NGL>()>(T, Bt, L, tau, fr, g0);
-        }
-        const R blay = planck<R>(T, B, L.tavel);
-        const R dplnku = planck<R>(T, B, tz_top) - blay;
-        if (k == 0) {  // surface emission and reflection
-            const R pk0 = planck<R>(T, B, rc.tskn());
-            R s0 = (R)0;
-#pragma unroll
-            for (int jj = 0; jj < NGL; ++jj) {
-                const R rad0 = semis * fr[jj] * pk0;
-                rad[jj] = rad0 + reflct * rad[jj];
-                s0 = s0 + rad[jj];
-            }
-            s0 = gsum<GS>(s0);
-            if (lead) acc.lw_up[t] = s0;
-        }
-        const R taucld = lw_taucld_l<R>(T, B, lcf1, L, rc, kin, par);
-        const R taer = (R)rc.aer_lw_tau(B, kin);  // tautot = taug + tauaer
-        R s = (R)0;
-#pragma unroll
-        for (int jj = 0; jj < NGL; ++jj) {
-            const GasT<R> q = lw_gas<R>(T, sdif, tau[jj] + taer);
-            const R plfrac = fr[jj];
-            const R bbugas = plfrac * (blay + dplnku * q.gasfac);
-            const R gassrcu = bbugas * q.atrgas;
-            const R clfm = ((mb[jj] >> k) & 1) ? (R)1 : (R)0;
-            if (clfm > (R)EPS) {
-                const R odcld = sdif * taucld;
-                const R efclrfr = (R)1 - ((R)1 - M<R>::exp(-odcld)) * clfm;
-                R totfac, atrtot;
-                lw_tot<R>(T, q.odepth + odcld, totfac, atrtot);
-                const R bbutot = plfrac * (blay + dplnku * totfac);
-                const R totsrcu = bbutot * atrtot;
-                rad[jj] = rad[jj] * q.trng * efclrfr + gassrcu + clfm * (totsrcu - gassrcu);
-            } else {
-                rad[jj] = rad[jj] * q.trng + gassrcu;
-            }
-            s = s + rad[jj];
-        }
-        s = gsum<GS>(s);
-        if (lead) acc.lw_up[(size_t)(k + 1) * n + t] = s;
-        tz_bot = tz_top;
-        cur = nxt, nxt = nn;
+        sweep(k, y, btop - y.blay, bits, k == 0, y.bbot, s, s0);  // the level below the lowest layer is the skin
+        if (k == 0) acc.lw_up[t] = s0;
+        acc.lw_up[(size_t)(k + 1) * n + t] = s;
     }
 }
 
 template <typename R, int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__(64, (lw_waves<R, B>())) k_lw(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
-                                           int n, ColScal cs, AccT<R> acc, Surr sg)
+                                           int n, ColScal cs, RecPtrs rp, AccT<R> acc, Surr sg)
 {
     const ColIn in = band_in<EXT>(in_);
-    lw_column<R, B, SURR>(T, T->lw[B], in, par, col0, n, cs, acc, sg, blockIdx.x * blockDim.x + threadIdx.x);
+    lw_column<R, B, SURR>(T, T->lw[B], in, par, col0, n, cs, rp, acc, sg, (int)blockIdx.x, (int)threadIdx.x);
 }
 
 // The band tables of an LDS image (the LwImg order), absb from PB: the image's when the image holds it,
@@ -690,6 +671,9 @@ __device__ __forceinline__ LwBandT<R, const WR_L R *, PB> lds_band(const WR_L R 
     Bl.refrat_m_a = G.refrat_m_a, Bl.refrat_m_b = G.refrat_m_b, Bl.refrat_m_a3 = G.refrat_m_a3;
     return Bl;
 }
+// the wave's index in its workgroup, as the wave-uniform value it is
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64)); }
+
 // copies the image into the workgroup's LDS (16-byte words) and waits for the whole workgroup
 template <typename R, typename I> __device__ __forceinline__ void lds_fill(float4 *dst, const I &im)
 {
@@ -706,9 +690,9 @@ template <typename R, typename I> __device__ __forceinline__ void lds_fill(float
 template <typename R, int B> constexpr int lwl64_wpg() { return 4 * lw_waves<R, B>(); }
 template <int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<double, B>()))
-    k_lwl64(const Tabs<double> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, AccT<double> acc, Surr sg)
+    k_lwl64(const Tabs<double> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp,
+            AccT<double> acc, Surr sg)
 {
-    static_assert(lw_gsplit<double>() == 1, "one lane per column");
     extern __shared__ float4 lwl64_tab[];
     const ColIn in = band_in<EXT>(in_);
     const LwImg<double> &im = T->lw_img[B];
@@ -716,112 +700,95 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
     const auto Bl = lds_band<double>((const WR_L double *)lwl64_tab, im, T->lw[B], T->lw[B].absb);
     constexpr int WPG = lwl64_wpg<double, B>();
     const int lane = threadIdx.x % 64;
-    for (int blk = blockIdx.x * WPG + threadIdx.x / 64; blk * 64 < n; blk += gridDim.x * WPG)
-        lw_column<double, B, SURR>(T, Bl, in, par, col0, n, cs, acc, sg, blk * 64 + lane);
+    for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
+        lw_column<double, B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane);
 }
 
 // FP32 LW band kernel with a cached upward sweep.  The down sweep also forms, per layer and g-point,
 // the upward transmittance a = trng * efclrfr and source b (gas plus cloud term) and keeps them in the
-// lane's pool slot (8 bytes per layer and g-point); the up sweep is then rad = rad * a + b, with no
-// optics.  The FP64 kernels recompute the upward optics instead: their sums follow the reference's
+// lane's pool slot (8 bytes per layer and g-point, one store); the up sweep is then rad = rad * a + b,
+// with no optics.  The FP64 kernels recompute the upward optics instead: their sums follow the reference's
 // operation order, and twice the bytes would not pay.
 constexpr int LW_NV_F32 = 2;
-// the smallest divisor of the band's g-point count that is >= the chunk asked for
 template <int B, bool SURR, typename BT>
 __device__ __forceinline__ void lw_column_f32c(const Tabs<float> *__restrict__ T, const BT &Bt, const ColIn &in,
-                                               const RunPar &par, int col0, int n, const ColScal &cs, const AccT<float> &acc,
-                                               const Surr &sg, int t, const LaneCache<float> &cc)
+                                               const RunPar &par, int col0, int n, const ColScal &cs, const RecPtrs &rp,
+                                               const AccT<float> &acc, const Surr &sg, int blk, int lane, WR_G char *slot)
 {
     using R = float;
-    constexpr int NG = LW_NG[B];
-    constexpr int NS = LW_NS[B];
-    const int i = col0 + t;
-    const RadCol rc{in, i, in.nlay + 1};
-    const int nrl = rc.nrl;
-    const int lcf1 = cs.lcf1[t];
-    const int table = SURR ? sg.table(t, B) : 1;
-    const double pwv = cs.pwv[t];
-    const R sdif = (R)((B == 0 || B == 3 || B == 9) ? 1.66 : fmin(1.80, fmax(1.50, LW_A0[B] + LW_A1[B] * exp_d(LW_A2[B] * pwv))));
-    const double sfe = in.emis[i];
-    const R semis = (R)((sfe > EPS && sfe <= 1.0) ? sfe : 1.0);
-    const R reflct = (R)1 - semis;
-    const uint64_t col = in.col_id ? in.col_id[i] : (uint64_t)i;
-    const uint64_t seed = in.seed_dev ? *in.seed_dev : par.seed;
-    uint64_t mb[NG];
-    for (int g = 0; g < NG; ++g)
-        mb[g] = mcica_g(col, seed, 0, NS + g, nrl, par.iovr, [&](int k) { return lcf1 ? rc.cfrac(nrl - 1 - k) : 0.0; });
-
+    constexpr int NG = LW_NG[B], CH = lw_chunk<B>();
+    const int t = blk * 64 + lane;
+    if (t >= valid_cols(in, col0, n)) return;
+    const LwCol<R> c = lw_col<R, B, SURR>(in, col0, cs, sg, t);
+    const int nrl = c.nrl;
+    WR_G f32x2v *ab = (WR_G f32x2v *)slot + lane;  // [layer][g][lane]
     acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
     R rad[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) rad[g] = (R)0;
-    LayV cur = rc.lay(0);  // layer kin; the next one is loaded an iteration ahead
-    double tz_top = cs.tz[t], la_nx = cs.la[t], tz_nx = cs.tz[(size_t)n + t];
-    for (int kin = 0; kin < nrl; ++kin) {
-        const int k = nrl - 1 - kin;
-        const LayV nxt = (kin + 1 < nrl) ? rc.lay(kin + 1) : cur;
-        // this layer's log pressure and bottom level temperature, loaded an iteration ahead
-        const double la_c = la_nx, tz_bot = tz_nx;
-        if (kin + 1 < nrl) la_nx = cs.la[(size_t)(kin + 1) * n + t], tz_nx = cs.tz[(size_t)(kin + 2) * n + t];
-        LwLay<R> L;
-        R tau[NG], fr[NG];
-        if (SURR && !table) {
-            lw_layer_cloud<R>(cur, L);
-            surr_lw<R, B>(sg, (size_t)k * n + t, tau, fr);
-        } else {
-            lw_layer<R>(T, cur, par, la_c, L);
-            lw_optics_ch<R, B, NG, lw_chunk<B>()>(T, Bt, L, tau, fr, 0);
-        }
-        const R blay = planck<R>(T, B, L.tavel);
-        const R dplnkd = planck<R>(T, B, tz_bot) - blay;
-        const R dplnku = planck<R>(T, B, tz_top) - blay;
-        const R taucld = lw_taucld_l<R>(T, B, lcf1, L, rc, kin, par);
-        const R taer = (R)rc.aer_lw_tau(B, kin);  // tautot = taug + tauaer
-        R s = (R)0;
+    R btop = (R)0;  // Planck function at the level above the layer
+    for (int k = nrl - 1; k >= 0; --k) {
+        LwLayer<R> y;
+        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
+        if (k == nrl - 1) btop = y.blay;
+        const R dd = y.bbot - y.blay, du = btop - y.blay;
+        R ecld = (R)1;
+        if (__any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
+        R s = (R)0, s0 = (R)0;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const GasT<R> q = lw_gas<R>(T, sdif, tau[g] + taer);
-            const R plfrac = fr[g];
-            const R gassrcd = plfrac * (blay + dplnkd * q.gasfac) * q.atrgas;
-            const R gassrcu = plfrac * (blay + dplnku * q.gasfac) * q.atrgas;
-            const R clfm = ((mb[g] >> k) & 1) ? (R)1 : (R)0;
-            R a = q.trng, b = gassrcu;
-            if (clfm >= (R)EPS) {
-                const R odcld = sdif * taucld;
-                const R efclrfr = (R)1 - ((R)1 - M<R>::exp(-odcld)) * clfm;
-                R totfac, atrtot;
-                lw_tot<R>(T, q.odepth + odcld, totfac, atrtot);
-                const R totsrcd = plfrac * (blay + dplnkd * totfac) * atrtot;
-                const R totsrcu = plfrac * (blay + dplnku * totfac) * atrtot;
-                rad[g] = rad[g] * q.trng * efclrfr + gassrcd + clfm * (totsrcd - gassrcd);
-                a = q.trng * efclrfr;
-                b = gassrcu + clfm * (totsrcu - gassrcu);
-            } else {
-                rad[g] = rad[g] * q.trng + gassrcd;
+        for (int g0 = 0; g0 < NG; g0 += CH) {
+            R tau[CH], fr[CH];
+            lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
+            GasV<R, CH> q;
+            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
+            R a[CH], bd[CH], bu[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const R fa = fr[j] * q.at[j];
+                bd[j] = fa * (y.blay + dd * q.gf[j]);
+                bu[j] = fa * (y.blay + du * q.gf[j]);
+                a[j] = q.tr[j];
             }
-            s = s + rad[g];
-            cc.at(0, NG, g, k) = a;
-            cc.at(1, NG, g, k) = b;
+            if (__any((bits >> g0) & ((1u << CH) - 1u))) {
+                R tr[CH], at[CH], gf[CH];
+                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const bool cl = (bits >> (g0 + j)) & 1u;
+                    const R fa = fr[j] * at[j];
+                    const R td = fa * (y.blay + dd * gf[j]), tu = fa * (y.blay + du * gf[j]);
+                    a[j] = cl ? q.tr[j] * ecld : a[j];
+                    bd[j] = cl ? td : bd[j];
+                    bu[j] = cl ? tu : bu[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const R r = rad[g0 + j] * a[j] + bd[j];
+                rad[g0 + j] = r;
+                s = s + r;
+                ab[((size_t)k * NG + g0 + j) * 64] = (f32x2v){a[j], bu[j]};
+            }
+            if (k == 0) {  // surface emission and reflection start the upward sweep
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    rad[g0 + j] = c.semis * fr[j] * y.bbot + c.reflct * rad[g0 + j];
+                    s0 = s0 + rad[g0 + j];
+                }
+            }
+            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
         }
         acc.lw_dn[(size_t)k * n + t] = s;
-        if (k == 0) {  // surface emission and reflection start the upward sweep
-            const R pk0 = planck<R>(T, B, rc.tskn());
-            R s0 = (R)0;
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                rad[g] = semis * fr[g] * pk0 + reflct * rad[g];
-                s0 = s0 + rad[g];
-            }
-            acc.lw_up[t] = s0;
-        }
-        tz_top = tz_bot;
-        cur = nxt;
+        if (k == 0) acc.lw_up[t] = s0;
+        btop = y.bbot;
     }
     for (int k = 0; k < nrl; ++k) {  // up sweep over the cached layers
         R s = (R)0;
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            rad[g] = rad[g] * cc.at(0, NG, g, k) + cc.at(1, NG, g, k);
+            const f32x2v v = ab[((size_t)k * NG + g) * 64];
+            rad[g] = rad[g] * v.x + v.y;
             s = s + rad[g];
         }
         acc.lw_up[(size_t)(k + 1) * n + t] = s;
@@ -830,15 +797,13 @@ __device__ __forceinline__ void lw_column_f32c(const Tabs<float> *__restrict__ T
 
 template <int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__(64, lwc_waves<B>()) k_lwc(const Tabs<float> *__restrict__ T, ColIn in_, RunPar par,
-                                                         int col0, int n, ColScal cs, AccT<float> acc, Surr sg,
+                                                         int col0, int n, ColScal cs, RecPtrs rp, AccT<float> acc, Surr sg,
                                                          char *__restrict__ pool)
 {
     const ColIn in = band_in<EXT>(in_);
-    const LaneCache<float> cc = lane_cache<float>(pool, LW_NV_F32, LW_NG[B], in.nlay + 2);
-    for (int blk = blockIdx.x; blk * 64 < n; blk += gridDim.x) {
-        const int t = blk * 64 + threadIdx.x;
-        if (t < valid_cols(in, col0, n)) lw_column_f32c<B, SURR>(T, T->lw[B], in, par, col0, n, cs, acc, sg, t, cc);
-    }
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(LW_NV_F32, LW_NG[B], in.nlay + 2, 4));
+    for (int blk = blockIdx.x; blk * 64 < n; blk += gridDim.x)
+        lw_column_f32c<B, SURR>(T, T->lw[B], in, par, col0, n, cs, rp, acc, sg, blk, (int)threadIdx.x, slot);
 }
 
 // k_lwc with the band's tables in LDS.  Persistent workgroups of one wave per SIMD times the band's
@@ -849,8 +814,8 @@ __global__ void __launch_bounds__(64, lwc_waves<B>()) k_lwc(const Tabs<float> *_
 template <int B> constexpr int lwl_wpg() { return 4 * lwc_waves<B>(); }
 template <int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__(64 * lwl_wpg<B>(), lwc_waves<B>())
-    k_lwl(const Tabs<float> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, AccT<float> acc, Surr sg,
-          char *__restrict__ pool)
+    k_lwl(const Tabs<float> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp, AccT<float> acc,
+          Surr sg, char *__restrict__ pool)
 {
     extern __shared__ float4 lwl_tab[];
     const ColIn in = band_in<EXT>(in_);
@@ -859,206 +824,10 @@ __global__ void __launch_bounds__(64 * lwl_wpg<B>(), lwc_waves<B>())
     const WR_L float *lt = (const WR_L float *)lwl_tab;
     const auto Bl = lds_band<float>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
     constexpr int WPG = lwl_wpg<B>();
-    const int lane = threadIdx.x % 64, slot = blockIdx.x * WPG + threadIdx.x / 64;
-    LaneCache<float> cc;
-    cc.p = (WR_G float *)(pool + (size_t)slot * cache_slot_bytes(LW_NV_F32, LW_NG[B], in.nlay + 2, 4)) + lane;
-    cc.nv = LW_NV_F32;
-    for (int blk = slot; blk * 64 < n; blk += gridDim.x * WPG) {
-        const int t = blk * 64 + lane;
-        if (t < valid_cols(in, col0, n)) lw_column_f32c<B, SURR>(T, Bl, in, par, col0, n, cs, acc, sg, t, cc);
-    }
-}
-
-// ---- SW band kernel (McICA two-stream) -------------------------------------------------------------
-// single-scattering albedo above which the mixed path evaluates the SW layer R/T in FP64
-constexpr double W0_FP64 = 0.999999;
-
-template <typename R, int B> struct SwLayerRT {
-    R rb[SW_NG[B]], rd[SW_NG[B]], tb[SW_NG[B]], td[SW_NG[B]], ld[SW_NG[B]];
-};
-
-// Layer R/T of one g-point from its gas (tg) and Rayleigh (tr) optical depths with the aerosol's
-// optical depth, single-scattering albedo and asymmetry (ta, sa, ya), plus the cloud
-// (tau, tau*w, tau*w*g) when cld.  FP32 evaluates in FP64 where FP32 loses the answer:
-// near-conservative scattering (w0 > 1 - 1e-6: 1 - w0 and gamma1 - gamma2 cancel; an FP32 pre-test
-// with a 10x wider margin skips the FP64 test for most layers) and near the two-stream singularity
-// k mu = 1 (flagged by the FP32 evaluation); the optical properties are then summed in FP64.
-template <typename R>
-__device__ __forceinline__ void layer_rt_eval(const Tabs<R> *__restrict__ T, R tr, R tg, R ta, R sa, R ya, bool cld, R ctau,
-                                              R cssa, R casy, R cz, R snt, R &rb, R &rd, R &tb, R &td, R &ld)
-{
-    // clear-sky optical parameters with the aerosol (phys_rrtm_sw_spcvrtc.cu:323-329)
-    R ztau0 = fmax((R)FTINY, tr + tg + ta);
-    R zssa0 = tr + ta * sa;
-    R zasy0 = ya * sa * ta;
-    if (cld) {
-        ztau0 = ztau0 + ctau;
-        zssa0 = zssa0 + cssa;
-        zasy0 = zasy0 + casy;
-    }
-    if constexpr (sizeof(R) < sizeof(double)) {
-        const double ta0 = (double)ta, sa0 = (double)sa, ya0 = (double)ya;
-        const double t0 = fmax(FTINY, (double)tr + (double)tg + ta0) + (cld ? (double)ctau : 0.0);
-        const double s0 = (double)tr + ta0 * sa0 + (cld ? (double)cssa : 0.0);
-        const double g0 = ya0 * sa0 * ta0 + (cld ? (double)casy : 0.0);
-        bool fp64 = zssa0 > (R)0.99999 * ztau0 && s0 > W0_FP64 * t0;
-        if (!fp64) layer_rt<R>(ztau0, zssa0, zasy0, cz, snt, T->sw_exp_tbl, rb, rd, tb, td, ld, &fp64);
-        if (fp64) {
-            double b, d, e, f, h;
-            layer_rt<double>(t0, s0, g0, (double)cz, (double)snt, T->sw_exp_tbl64, b, d, e, f, h);
-            rb = (R)b, rd = (R)d, tb = (R)e, td = (R)f, ld = (R)h;
-        }
-    } else {
-        layer_rt<R>(ztau0, zssa0, zasy0, cz, snt, T->sw_exp_tbl, rb, rd, tb, td, ld);
-    }
-}
-
-template <typename R, int B, bool SURR, typename BT>
-__device__ __forceinline__ void sw_layer_rt(const Tabs<R> *__restrict__ T, const BT &Bt, const RadCol &rc, const RunPar &par, int k,
-                                            int lt, double cf1, const uint64_t *mb, R cz, R snt, SwLayerRT<R, B> &o,
-                                            const Surr &sg, size_t s, int table, double la)
-{
-    constexpr int NG = SW_NG[B];
-    const int nrl = rc.nrl;
-    const int kin = nrl - 1 - k;
-    SwLay<R> L;
-    R tg[NG], tr[NG];
-    if (SURR && !table) {
-        rc.cloud(kin, L.ct, L.cwp, L.cip);
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const R tau = (R)__expf(surr_out(sg, 280 + SW_NS[B] + g, s));
-            const R ssa = (R)fminf(1.0f, fmaxf(0.0f, surr_out(sg, 392 + SW_NS[B] + g, s)));
-            tr[g] = tau * ssa;
-            tg[g] = tau - tr[g];
-        }
-    } else {
-        sw_layer<R>(T, rc, par, kin, la, L);
-        sw_optics_t<R, B>(T, Bt, L, k + 1, lt, tg, tr);
-    }
-    double ta, sa, ya;
-    rc.aer_sw3(B, kin, ta, sa, ya);
-    R ctau = (R)0, cssa = (R)1, casy = (R)0;
-    if (cf1 > 0.0 && L.ct > FTINY) sw_cloud_l<R>(T, B, L, rc, kin, par, ctau, cssa, casy);
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-        layer_rt_eval<R>(T, tr[g], tg[g], (R)ta, (R)sa, (R)ya, (mb[g] >> k) & 1, ctau, cssa, casy, cz, snt, o.rb[g],
-                         o.rd[g], o.tb[g],
-                         o.td[g], o.ld[g]);
-}
-
-// One day column of one SW band (spcvrtc, McICA): bottom-up adding pass (reflectances of each level
-// to the lane cache), then the top-down pass with the layer R/T recomputed and the level fluxes.
-template <typename R, int B, bool SURR, typename BT>
-__device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par, int col0,
-                                          int n, const ColScal &cs, const R *__restrict__ sflux, const AccT<R> &acc,
-                                          const Surr &sg, int t, const LaneCache<R> &cc)
-{
-    constexpr bool CACHE_RT = sw_nv_mc<R>() > SW_NV;
-    constexpr int NG = SW_NG[B];
-    constexpr int NS = SW_NS[B];
-    const int i = col0 + t;
-    const RadCol rc{in, i, in.nlay + 1};
-    const int nrl = rc.nrl, nlp1 = nrl + 1;
-    const double czd = in.cosz[i];
-    const R cz = (R)czd, snt = (R)(1.0 / czd);
-    const double ssolar = (par.solcon / S0) * czd;
-    const double alb = in.alb[i];
-    const R asfc = (R)((SW_IDXSFC[B] != 0) ? alb : 0.5 * (alb + alb));
-    const double cf1 = cs.zcf1[t];
-    const int lt = cs.sw_laytrop[t];
-    const int table = SURR ? sg.table(t, 16 + B) : 1;
-    const uint64_t col = in.col_id ? in.col_id[i] : (uint64_t)i;
-    const uint64_t seed = in.seed_dev ? *in.seed_dev : par.seed;
-    uint64_t mb[NG];
-    for (int g = 0; g < NG; ++g) {
-        mb[g] = mcica_g(col, seed, 1, NS + g, nrl, par.iovr, [&](int k) {
-            const double ct = rc.cfrac(nrl - 1 - k);
-            return (cf1 > 0.0) ? ((ct < FTINY) ? 0.0 : ct) : 0.0;
-        });
-    }
-    // bottom-up: reflectance of the medium below each level (swflux sweep 1); zrupb/zrupd of level
-    // L (1-based, surface L = 1) sit at cache entry L - 1, the latest level also in pb/pd
-    R pb[NG], pd[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        pb[g] = asfc, pd[g] = asfc;
-        cc.at(0, NG, g, 0) = asfc;
-        cc.at(1, NG, g, 0) = asfc;
-    }
-    for (int k = 0; k < nrl; ++k) {
-        SwLayerRT<R, B> o;
-        sw_layer_rt<R, B, SURR>(T, Bt, rc, par, k, lt, cf1, mb, cz, snt, o, sg, (size_t)k * n + t, table,
-                                cs.la[(size_t)(nrl - 1 - k) * n + t]);
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const R zden1 = (R)1 / ((R)1 - pd[g] * o.rd[g]);
-            const R nb = o.rb[g] + (o.td[g] * ((o.tb[g] - o.ld[g]) * pd[g] + o.ld[g] * pb[g])) * zden1;
-            const R nd = o.rd[g] + o.td[g] * o.td[g] * pd[g] * zden1;
-            pb[g] = nb, pd[g] = nd;
-            cc.at(0, NG, g, k + 1) = nb;
-            cc.at(1, NG, g, k + 1) = nd;
-            if constexpr (CACHE_RT) {
-                cc.at(2, NG, g, k) = o.rb[g];
-                cc.at(3, NG, g, k) = o.rd[g];
-                cc.at(4, NG, g, k) = o.tb[g];
-                cc.at(5, NG, g, k) = o.td[g];
-                cc.at(6, NG, g, k) = o.ld[g];
-            }
-        }
-    }
-    // top-down: direct beam, diffuse transmission and reflection from above, level fluxes
-    R tdbt[NG], tdn[NG], rdnd[NG], zsolar[NG];
-    R su = (R)0, sd = (R)0;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        zsolar[g] = (R)ssolar * sflux[(size_t)(NS + g) * n + t];
-        tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0;
-        const R zden1 = (R)1 / ((R)1 - rdnd[g] * pd[g]);
-        const R zfu = (tdbt[g] * pb[g] + (tdn[g] - tdbt[g]) * pd[g]) * zden1;
-        const R zfd = tdbt[g] + (tdn[g] - tdbt[g] + tdbt[g] * pb[g] * rdnd[g]) * zden1;
-        su = su + zsolar[g] * zfu;
-        sd = sd + zsolar[g] * zfd;
-    }
-    acc.sw_up[(size_t)nrl * n + t] = su;
-    acc.sw_dn[(size_t)nrl * n + t] = sd;
-    acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
-    for (int s = nrl; s >= 1; --s) {
-        SwLayerRT<R, B> o;
-        if constexpr (CACHE_RT) {
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                o.rb[g] = cc.at(2, NG, g, s - 1), o.rd[g] = cc.at(3, NG, g, s - 1), o.tb[g] = cc.at(4, NG, g, s - 1);
-                o.td[g] = cc.at(5, NG, g, s - 1), o.ld[g] = cc.at(6, NG, g, s - 1);
-            }
-        } else {
-            sw_layer_rt<R, B, SURR>(T, Bt, rc, par, s - 1, lt, cf1, mb, cz, snt, o, sg, (size_t)(s - 1) * n + t, table,
-                                    cs.la[(size_t)(nrl - s) * n + t]);
-        }
-        su = (R)0, sd = (R)0;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const R tdbt_s = o.ld[g] * tdbt[g];
-            R tdn_s, rdnd_s;
-            if (s == nrl) {
-                tdn_s = o.tb[g];
-                rdnd_s = o.rd[g];
-            } else {
-                const R zden1 = (R)1 / ((R)1 - o.rd[g] * rdnd[g]);
-                tdn_s = tdbt[g] * o.tb[g] + (o.td[g] * ((tdn[g] - tdbt[g]) + tdbt[g] * o.rb[g] * rdnd[g])) * zden1;
-                rdnd_s = o.rd[g] + o.td[g] * o.td[g] * rdnd[g] * zden1;
-            }
-            tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
-            const R zb = cc.at(0, NG, g, s - 1), zd = cc.at(1, NG, g, s - 1);  // level s
-            const R zden1 = (R)1 / ((R)1 - rdnd_s * zd);
-            const R zfu = (tdbt_s * zb + (tdn_s - tdbt_s) * zd) * zden1;
-            const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * zb * rdnd_s) * zden1;
-            su = su + zsolar[g] * zfu;
-            sd = sd + zsolar[g] * zfd;
-        }
-        acc.sw_up[(size_t)(s - 1) * n + t] = su;
-        acc.sw_dn[(size_t)(s - 1) * n + t] = sd;
-    }
+    const int lane = threadIdx.x % 64, w = blockIdx.x * WPG + wave_id();
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(LW_NV_F32, LW_NG[B], in.nlay + 2, 4));
+    for (int blk = w; blk * 64 < n; blk += gridDim.x * WPG)
+        lw_column_f32c<B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane, slot);
 }
 
 // Waves per SIMD the SW kernels are compiled for, per band, measured serialised on the 954x835x60
@@ -1068,9 +837,15 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
 //   two waves by their register count, and the bound only slowed their schedule (8-14 %);
 // * FP32 NAM route: two waves for every band but 22 (one wave 25-45 % slower).
 // WR_SW64_WAVES / WR_SW32_WAVES > 0 override the tables for every band (tuning builds).
-constexpr int SW64_WAVES[14] = {2, 1, 1, 1, 1, 1, 1, 1, 1, 2, 2, 1, 2, 1};
-constexpr int SW32_WAVES[14] = {1, 2, 1, 1, 2, 2, 1, 2, 1, 1, 1, 2, 2, 2};
-constexpr int SWR32_WAVES[14] = {2, 2, 2, 2, 2, 2, 1, 2, 2, 2, 2, 2, 2, 2};
+constexpr int SW64_WAVES[14] = {2, 1, 1, 1, 1, 1, 2, 1, 1, 2, 2, 1, 2, 1};
+constexpr int SW32_WAVES[14] = {3, 2, 2, 2, 2, 2, 4, 2, 2, 3, 3, 2, 3, 2};
+constexpr int SWR32_WAVES[14] = {3, 2, 2, 2, 2, 2, 4, 2, 2, 3, 3, 2, 3, 2};
+// g-points per chunk of the layer R/T (0: the whole band), by precision and route
+constexpr int SW_CHUNK64 = 2, SW_CHUNK32 = 2, SWR_CHUNK64 = 2, SWR_CHUNK32 = 2;
+template <typename R, int B, bool NAM = false> constexpr int sw_chunk()
+{
+    return chunk_of(SW_NG[B], sizeof(R) == 8 ? (NAM ? SWR_CHUNK64 : SW_CHUNK64) : (NAM ? SWR_CHUNK32 : SW_CHUNK32));
+}
 #ifndef WR_SW64_WAVES
 #define WR_SW64_WAVES 0
 #endif
@@ -1083,19 +858,460 @@ template <typename R, int B, bool NAM = false> constexpr int sw_waves()
     return WR_SW32_WAVES > 0 ? WR_SW32_WAVES : (NAM ? SWR32_WAVES[B] : SW32_WAVES[B]);
 }
 
+// ---- SW band kernels (McICA two-stream) ------------------------------------------------------------
+// One lane per day column, one wave per block of 64 day-list entries, layer set-up and McICA words from the
+// records.  Per layer the g-points run in chunks as in the LW kernels: layer R/T of a chunk without
+// per-g-point branches, so that its chains of divisions, square roots and exponentials overlap.
+
+// single-scattering albedo above which the mixed path evaluates the SW layer R/T in FP64
+constexpr double W0_FP64 = 0.999999;
+
+
+template <typename R, int CH> struct RtV {  // layer reflectances, transmittances and direct transmission of CH g-points
+    R rb[CH], rd[CH], tb[CH], td[CH], ld[CH];
+};
+
+// exp(-z) of the SW table for CH arguments: the series below 0.06, the table entry above
+template <typename R, int CH>
+__device__ __forceinline__ void expm_v(const R *z, const WR_G R *__restrict__ tbl, R *e)
+{
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        e[j] = (R)1 - z[j] + (R)0.5 * z[j] * z[j];
+        any |= !(z[j] <= (R)0.06);
+    }
+    if (__any(any)) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            R v;
+            if constexpr (sizeof(R) == 4) {
+                const R tb = z[j] * __builtin_amdgcn_rcpf((R)(1.0 / 0.278) + z[j]);
+                const R fi = fmin(floorf(__builtin_fmaf((R)NTBL, tb, (R)0.5)), (R)9999.999);
+                v = M<R>::exp(-(((R)(1.0 / 0.278) * fi) * __builtin_amdgcn_rcpf((R)NTBL - fi)));
+            } else {
+                const R ft = z[j] / ((R)(1.0 / 0.278) + z[j]);
+                v = tbl[imax(0, imin(10000, (int)((R)0.5 + (R)10000 * ft)))];
+            }
+            e[j] = !(z[j] <= (R)0.06) ? v : e[j];
+        }
+    }
+}
+
+template <typename R> __device__ __forceinline__ R rdiv(R a, R b)
+{
+    if constexpr (sizeof(R) == 4) return a * __builtin_amdgcn_rcpf(b);
+    return a / b;
+}
+
+// layer_rt (delta scaling, PIFM, layer R/T) for CH g-points; FP32 flags a g-point near the two-stream
+// singularity k mu = 1, where numerator and denominator of the direct-beam terms both vanish
+template <typename R, int CH>
+__device__ __forceinline__ void layer_rt_v(const R *ztau0, const R *zssa0, const R *zasy0, R cz, R snt,
+                                           const WR_G R *__restrict__ tbl, RtV<R, CH> &o, bool *ill)
+{
+    R zb1[CH], zb2[CH], zb3[CH], e1[CH], e2[CH];
+    R g1[CH], g2[CH], g3[CH], rk[CH], w1[CH];
+    bool far = false;
+    // FP32: cap the exponents at 80 so exp(-zb) stays a normal number and 1/exp(-zb) finite (the R/T
+    // expressions depend on the capped terms only through factors below exp(-160))
+    const R zcap = (sizeof(R) < sizeof(double)) ? (R)80 : (R)500;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const R zssaw = fmin((R)ONEMINUS, rdiv<R>(zssa0[j], ztau0[j]));
+        const R zasyw = rdiv<R>(zasy0[j], fmax((R)FTINY, zssa0[j]));
+        const R za1s = zasyw * zasyw;
+        const R za2s = zssaw * za1s;
+        const R ztau1 = ((R)1 - za2s) * ztau0[j];
+        w1[j] = rdiv<R>(zssaw - za2s, (R)1 - za2s);
+        const R zasy1 = rdiv<R>(zasyw, (R)1 + zasyw);
+        const R zasy3 = (R)0.75 * zasy1;
+        g1[j] = (R)2 - w1[j] * ((R)1.25 + zasy3);
+        g2[j] = (R)0.75 * w1[j] * ((R)1 - zasy1);
+        g3[j] = (R)0.5 - zasy3 * cz;
+        rk[j] = sqrt((g1[j] - g2[j]) * (g1[j] + g2[j]));
+        zb1[j] = fmin(rk[j] * ztau1, zcap);
+        zb3[j] = ztau1 * snt;
+        zb2[j] = fmin(zb3[j], zcap);
+        far |= zb3[j] > zcap;
+    }
+    expm_v<R, CH>(zb1, tbl, e1);
+    expm_v<R, CH>(zb2, tbl, e2);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) o.ld[j] = e2[j];
+    if (__any(far)) {
+        R e3[CH];
+        expm_v<R, CH>(zb3, tbl, e3);
+#pragma unroll
+        for (int j = 0; j < CH; ++j) o.ld[j] = zb3[j] > zcap ? e3[j] : o.ld[j];
+    }
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const R zgam1 = g1[j], zgam2 = g2[j], zgam3 = g3[j], zrk = rk[j];
+        const R zgam4 = (R)1 - zgam3;
+        const R eps1 = (R)1.0e-8;
+        const R za1 = zgam1 * zgam4 + zgam2 * zgam3;
+        const R za2 = zgam1 * zgam3 + zgam2 * zgam4;
+        const R zrk2 = (R)2 * zrk;
+        const R zrp = zrk * cz;
+        const R zrp1 = (R)1 + zrp;
+        const R zrm1 = (R)1 - zrp;
+        R zrpp = (R)1 - zrp * zrp;
+        if constexpr (sizeof(R) == 4) ill[j] = fabs(zrpp) < (R)1.0e-2;
+        if (fabs(zrpp) < eps1) zrpp = (zrpp < (R)0) ? -eps1 : eps1;
+        const R zrkg1 = zrk + zgam1;
+        const R zrkg3 = zrk * zgam3;
+        const R zrkg4 = zrk * zgam4;
+        const R zr1 = zrm1 * (za2 + zrkg3);
+        const R zr2 = zrp1 * (za2 - zrkg3);
+        const R zr3 = zrk2 * (zgam3 - za2 * cz);
+        const R zr4 = zrpp * zrkg1;
+        const R zr5 = zrpp * (zrk - zgam1);
+        const R zt1 = zrp1 * (za1 + zrkg4);
+        const R zt2 = zrm1 * (za1 - zrkg4);
+        const R zt3 = zrk2 * (zgam4 + za1 * cz);
+        const R zexm1 = e1[j], zexm2 = e2[j];
+        const R zexp1 = rdiv<R>((R)1, zexm1);
+        const R zexp2 = rdiv<R>((R)1, zexm2);
+        const R ze1r45 = zr4 * zexp1 + zr5 * zexm1;
+        const R zden1 = rdiv<R>(w1[j], ze1r45);
+        const R rb = fmax((R)0, fmin((R)1, (zr1 * zexp1 - zr2 * zexm1 - zr3 * zexm2) * zden1));
+        const R tb = fmax((R)0, fmin((R)1, zexm2 * ((R)1 - (zt1 * zexp1 - zt2 * zexm1 - zt3 * zexp2) * zden1)));
+        const bool tiny = ze1r45 >= -eps1 && ze1r45 <= eps1;
+        o.rb[j] = tiny ? eps1 : rb;
+        o.tb[j] = tiny ? zexm2 : tb;
+        const R zden1d = rdiv<R>(zr4, ze1r45 * zrkg1);
+        o.rd[j] = fmax((R)0, fmin((R)1, zgam2 * (zexp1 - zexm1) * zden1d));
+        o.td[j] = fmax((R)0, fmin((R)1, zrk2 * zden1d));
+    }
+}
+
+// What a layer's two-stream solution of one column needs besides the g-point optics.
+template <typename R> struct SwSky {
+    R ta, sa, ya;         // aerosol optical depth, single-scattering albedo, asymmetry
+    R ctau, cssa, casy;   // cloud tau, tau w, tau w g
+    R cz, snt;
+};
+
+// LDS of one wave for the FP64 evaluations of the FP32 kernels
+struct alignas(16) Fix64 {
+    double t0[64], s0[64], g0[64];
+    float cz[64], snt[64];
+};
+
+// Layer R/T of CH g-points from their gas (tg) and Rayleigh (tr) optical depths, the aerosol and, where
+// bit j of cld is set, the cloud.  FP32 evaluates in FP64 where FP32 loses the answer: near-conservative
+// scattering (w0 > 1 - 1e-6: 1 - w0 and gamma1 - gamma2 cancel; an FP32 pre-test with a 10x wider
+// margin skips the FP64 test for most layers) and near the two-stream singularity.  About one g-point
+// and layer in a hundred is of that kind, so nearly every wave has some in every chunk: the (lane,
+// g-point) pairs of the chunk are gathered through LDS and evaluated together, one per lane, where a
+// branch per g-point took the FP64 evaluation (about 200 operations) once for each g-point with any.
+template <typename R, int CH>
+__device__ __forceinline__ void layer_rt_sky(const Tabs<R> *__restrict__ T, const R *tr, const R *tg, const SwSky<R> &y,
+                                             uint32_t cld, RtV<R, CH> &o, Fix64 *fx)
+{
+    R t0[CH], s0[CH], a0[CH];
+    bool ill[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        // clear-sky optical parameters with the aerosol (phys_rrtm_sw_spcvrtc.cu:323-329)
+        t0[j] = fmax((R)FTINY, tr[j] + tg[j] + y.ta);
+        s0[j] = tr[j] + y.ta * y.sa;
+        a0[j] = y.ya * y.sa * y.ta;
+        const bool c = (cld >> j) & 1u;
+        t0[j] = c ? t0[j] + y.ctau : t0[j];
+        s0[j] = c ? s0[j] + y.cssa : s0[j];
+        a0[j] = c ? a0[j] + y.casy : a0[j];
+    }
+    layer_rt_v<R, CH>(t0, s0, a0, y.cz, y.snt, T->sw_exp_tbl, o, ill);
+    if constexpr (sizeof(R) == 4) {
+        auto wide = [&](int j, double &t, double &s, double &a) {  // the optical parameters summed in FP64
+            const double ta = (double)y.ta, sa = (double)y.sa, ya = (double)y.ya;
+            const bool c = (cld >> j) & 1u;
+            t = fmax(FTINY, (double)tr[j] + (double)tg[j] + ta) + (c ? (double)y.ctau : 0.0);
+            s = (double)tr[j] + ta * sa + (c ? (double)y.cssa : 0.0);
+            a = ya * sa * ta + (c ? (double)y.casy : 0.0);
+        };
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool pre = s0[j] > (R)0.99999 * t0[j];
+            if (__any(pre)) {
+                double t, s, a;
+                wide(j, t, s, a);
+                ill[j] |= pre && s > W0_FP64 * t;
+            }
+            any |= ill[j];
+        }
+        if (__any(any)) {
+            const uint64_t active = __ballot(1);
+            const uint64_t below = ((uint64_t)1 << (threadIdx.x & 63)) - 1;
+            int total = 0, pos[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const uint64_t m = __ballot(ill[j]);
+                pos[j] = total + __popcll(m & below);
+                total += __popcll(m);
+            }
+            const int rank = __popcll(active & below);
+            const int lanes = __popcll(active);
+            for (int first = 0; first < total; first += lanes) {  // one round, unless most of the chunk is of that kind
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int p = pos[j] - first;
+                    if (ill[j] && p >= 0 && p < lanes) {
+                        double t, s, a;
+                        wide(j, t, s, a);
+                        fx->t0[p] = t, fx->s0[p] = s, fx->g0[p] = a, fx->cz[p] = y.cz, fx->snt[p] = y.snt;
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (first + rank < total) {
+                    const double t = fx->t0[rank], s = fx->s0[rank], a = fx->g0[rank];
+                    RtV<double, 1> d;
+                    layer_rt_v<double, 1>(&t, &s, &a, (double)fx->cz[rank], (double)fx->snt[rank], T->sw_exp_tbl64, d, nullptr);
+                    float *q0 = (float *)&fx->t0[rank], *q1 = (float *)&fx->s0[rank], *q2 = (float *)&fx->g0[rank];
+                    q0[0] = (R)d.rb[0], q0[1] = (R)d.rd[0], q1[0] = (R)d.tb[0], q1[1] = (R)d.td[0], q2[0] = (R)d.ld[0];
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int p = pos[j] - first;
+                    if (ill[j] && p >= 0 && p < lanes) {
+                        const float *q0 = (const float *)&fx->t0[p], *q1 = (const float *)&fx->s0[p], *q2 = (const float *)&fx->g0[p];
+                        o.rb[j] = q0[0], o.rd[j] = q0[1], o.tb[j] = q1[0], o.td[j] = q1[1], o.ld[j] = q2[0];
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+}
+
+// One layer of a day column: optics record and sky.
+template <typename R> struct SwLayer {
+    SwLay<R> L;
+    SwSky<R> y;
+    bool cloudy;
+};
+template <typename R, int B>
+__device__ __forceinline__ void sw_get(const Tabs<R> *__restrict__ T, const ColIn &in, const RunPar &par, const RecPtrs &rp,
+                                       int i, R cz, R snt, int blk, int lane, int k, SwLayer<R> &a)
+{
+    const LRow<R> row = srow<R>(rp, blk, k, lane);
+    srow_get<R>(row, row.w(0), a.L);
+    a.cloudy = row.w(1) != 0;
+    const RadCol rc{in, i, rp.nrl};
+    double ta, sa, ya;
+    rc.aer_sw3(B, rp.nrl - 1 - k, ta, sa, ya);
+    a.y = {(R)ta, (R)sa, (R)ya, (R)0, (R)1, (R)0, cz, snt};
+    if (__any(a.cloudy)) {
+        double rl = par.re_liq, ri = par.re_ice, rain = 0.0;
+        if (a.cloudy) rc.props(rp.nrl - 1 - k, par.re_liq, par.re_ice, rl, ri, rain);
+        sw_cloud<R>(T, B, (double)row.f(SF_LIQ), rl, (double)row.f(SF_ICE), ri, a.y.ctau, a.y.cssa, a.y.casy, rain);
+    }
+}
+// gas and Rayleigh optical depths of g-points g0 .. g0 + CH - 1
+template <typename R, int B, bool SURR, int CH, typename BT>
+__device__ __forceinline__ void sw_tgtr(const Tabs<R> *__restrict__ T, const BT &Bt, const Surr &sg, int table, size_t s, int k,
+                                        int lt, const SwLay<R> &L, int g0, R *tg, R *tr)
+{
+    if (SURR && !table) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const R tau = (R)__expf(surr_out(sg, 280 + SW_NS[B] + g0 + j, s));
+            const R ssa = (R)fminf(1.0f, fmaxf(0.0f, surr_out(sg, 392 + SW_NS[B] + g0 + j, s)));
+            tr[j] = tau * ssa;
+            tg[j] = tau - tr[j];
+        }
+    } else {
+        sw_optics_t<R, B, CH>(T, Bt, L, k + 1, lt, tg, tr, g0);
+    }
+}
+
+// Pool slot of one SW wave: per layer and g-point the reflectances (direct, diffuse) of everything below the
+// layer; FP32 also the layer's R/T, which the top-down sweep would otherwise evaluate again (in FP64 the
+// bytes cost more than the evaluation).
+constexpr int SW_NV = 2;
+template <typename R> constexpr int sw_nv_mc() { return sizeof(R) == 4 ? SW_NV + 5 : SW_NV; }
+template <typename R, int NG> struct SwSlot {
+    WR_G char *p;
+    int lane, nk;
+    __device__ __forceinline__ void put(int k, int g, R pb, R pd, const R *rt) const  // rt: rb, rd, tb, td, ld
+    {
+        const size_t e = ((size_t)k * NG + g) * 64 + lane;
+        if constexpr (sizeof(R) == 4) {
+            ((WR_G f32x4v *)p)[e] = (f32x4v){pb, pd, rt[0], rt[1]};
+            WR_G float *q = (WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
+            q[0] = rt[2], q[1] = rt[3], q[2] = rt[4];
+        } else {
+            ((WR_G f64x2v *)p)[e] = (f64x2v){pb, pd};
+        }
+    }
+    __device__ __forceinline__ void get(int k, int g, R &pb, R &pd, R *rt) const
+    {
+        const size_t e = ((size_t)k * NG + g) * 64 + lane;
+        if constexpr (sizeof(R) == 4) {
+            const f32x4v v = ((const WR_G f32x4v *)p)[e];
+            const WR_G float *q = (const WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
+            pb = v.x, pd = v.y, rt[0] = v.z, rt[1] = v.w, rt[2] = q[0], rt[3] = q[1], rt[4] = q[2];
+        } else {
+            const f64x2v v = ((const WR_G f64x2v *)p)[e];
+            pb = v.x, pd = v.y;
+        }
+    }
+};
+
+// The adding method over one column: bottom-up reflectances to the slot, then the direct and diffuse beams
+// top-down with the level fluxes.  layer(k) gives a layer, rt_at(layer, k, g0, o) its R/T of a chunk, sun(g)
+// the solar source of a g-point; emit(level, up, down) takes a level's fluxes, top level first.
+template <typename R, int NG, int CH, typename LAYER, typename RT, typename SUN, typename EMIT>
+__device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG> &slot, LAYER &&layer, RT &&rt_at, SUN &&sun,
+                                          EMIT &&emit)
+{
+    R pb[NG], pd[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) pb[g] = asfc, pd[g] = asfc;
+    for (int k = 0; k < nrl; ++k) {
+        auto a = layer(k);
+#pragma unroll
+        for (int g0 = 0; g0 < NG; g0 += CH) {
+            RtV<R, CH> o;
+            rt_at(a, k, g0, o);
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const int g = g0 + j;
+                const R rt[5] = {o.rb[j], o.rd[j], o.tb[j], o.td[j], o.ld[j]};
+                slot.put(k, g, pb[g], pd[g], rt);
+                const R zden1 = rdiv<R>((R)1, (R)1 - pd[g] * o.rd[j]);
+                const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * pd[g] + o.ld[j] * pb[g])) * zden1;
+                const R nd = o.rd[j] + o.td[j] * o.td[j] * pd[g] * zden1;
+                pb[g] = nb, pd[g] = nd;
+            }
+            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    R tdbt[NG], tdn[NG], rdnd[NG], zsolar[NG];
+    R su = (R)0, sd = (R)0;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0, zsolar[g] = sun(g);
+        su = su + zsolar[g] * pb[g];
+        sd = sd + zsolar[g];
+    }
+    emit(nrl, su, sd);
+    for (int k = nrl - 1; k >= 0; --k) {
+        su = (R)0, sd = (R)0;
+        auto chunk = [&](int g0, auto &&get) {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const int g = g0 + j;
+                R zb, zd, rt[5];
+                get(g, j, zb, zd, rt);
+                const R tdbt_s = rt[4] * tdbt[g];
+                const R zden0 = rdiv<R>((R)1, (R)1 - rt[1] * rdnd[g]);
+                const R tdn_s = tdbt[g] * rt[2] + (rt[3] * ((tdn[g] - tdbt[g]) + tdbt[g] * rt[0] * rdnd[g])) * zden0;
+                const R rdnd_s = rt[1] + rt[3] * rt[3] * rdnd[g] * zden0;
+                tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
+                const R zden1 = rdiv<R>((R)1, (R)1 - rdnd_s * zd);
+                const R zfu = (tdbt_s * zb + (tdn_s - tdbt_s) * zd) * zden1;
+                const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * zb * rdnd_s) * zden1;
+                su = su + zsolar[g] * zfu;
+                sd = sd + zsolar[g] * zfd;
+            }
+        };
+        if constexpr (sizeof(R) == 4) {
+#pragma unroll
+            for (int g0 = 0; g0 < NG; g0 += CH) {
+                chunk(g0, [&](int g, int, R &zb, R &zd, R *rt) { slot.get(k, g, zb, zd, rt); });
+                if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            auto a = layer(k);
+#pragma unroll
+            for (int g0 = 0; g0 < NG; g0 += CH) {
+                RtV<R, CH> o;
+                rt_at(a, k, g0, o);
+                chunk(g0, [&](int g, int j, R &zb, R &zd, R *rt) {
+                    slot.get(k, g, zb, zd, nullptr);
+                    rt[0] = o.rb[j], rt[1] = o.rd[j], rt[2] = o.tb[j], rt[3] = o.td[j], rt[4] = o.ld[j];
+                });
+                if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        emit(k, su, sd);
+    }
+}
+
+// What the SW sweeps of one day column need besides its layers.
+template <typename R> struct SwCol {
+    int i, t, lt;
+    R cz, snt, asfc, ssolar;
+};
+template <typename R, int B>
+__device__ __forceinline__ void sw_col(const ColIn &in, const RunPar &par, int col0, const ColScal &cs, int t, SwCol<R> &c)
+{
+    c.i = col0 + t, c.t = t;
+    const double czd = in.cosz[c.i];
+    c.cz = (R)czd, c.snt = (R)(1.0 / czd);
+    c.ssolar = (R)((par.solcon / S0) * czd);
+    const double alb = in.alb[c.i];
+    c.asfc = (R)((SW_IDXSFC[B] != 0) ? alb : 0.5 * (alb + alb));
+    c.lt = cs.sw_laytrop[t];
+}
+
+// One day column of one SW band (spcvrtc, McICA).
+template <typename R, int B, bool SURR, typename BT>
+__device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par, int col0,
+                                          int n, const ColScal &cs, const RecPtrs &rp, const R *__restrict__ sflux,
+                                          const AccT<R> &acc, const Surr &sg, int blk, int lane, WR_G char *slot, Fix64 *fx)
+{
+    constexpr int NG = SW_NG[B], CH = sw_chunk<R, B>();
+    if (blk * 64 + lane >= *cs.nday) return;
+    const int t = cs.dlist[blk * 64 + lane], nrl = rp.nrl;
+    SwCol<R> c;
+    sw_col<R, B>(in, par, col0, cs, t, c);
+    const int table = SURR ? sg.table(t, 16 + B) : 1;
+    acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
+    struct Lay {
+        SwLayer<R> y;
+        uint32_t bits;
+    };
+    sw_adding<R, NG, CH>(
+        nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2},
+        [&](int k) {
+            Lay a;
+            sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, lane, k, a.y);
+            a.bits = a.y.cloudy ? mword(rp.msw, rp.row(blk, k), MROW_SW, B, lane) : 0u;
+            return a;
+        },
+        [&](const Lay &a, int k, int g0, RtV<R, CH> &o) {
+            R tg[CH], tr[CH];
+            sw_tgtr<R, B, SURR, CH>(T, Bt, sg, table, (size_t)k * n + t, k, c.lt, a.y.L, g0, tg, tr);
+            layer_rt_sky<R, CH>(T, tr, tg, a.y.y, a.bits >> g0, o, fx);
+        },
+        [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
+        [&](int lev, R su, R sd) {
+            acc.sw_up[(size_t)lev * n + t] = su;
+            acc.sw_dn[(size_t)lev * n + t] = sd;
+        });
+}
+
 // SW band kernel: blocks of 64 day-list entries, a grid no larger than the pool's slot count.
 template <typename R, int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__(64, (sw_waves<R, B>())) k_sw(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
-                                           int n, ColScal cs, const R *__restrict__ sflux, AccT<R> acc, Surr sg,
+                                           int n, ColScal cs, RecPtrs rp, const R *__restrict__ sflux, AccT<R> acc, Surr sg,
                                            char *__restrict__ pool)
 {
+    __shared__ Fix64 fx[1];
     const ColIn in = band_in<EXT>(in_);
-    const LaneCache<R> cc = lane_cache<R>(pool, sw_nv_mc<R>(), SW_NG[B], in.nlay + 2);
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
-    for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x) {
-        const int tt = blk * 64 + threadIdx.x;
-        if (tt < nday) sw_column<R, B, SURR>(T, T->sw[B], in, par, col0, n, cs, sflux, acc, sg, cs.dlist[tt], cc);
-    }
+    for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x)
+        sw_column<R, B, SURR>(T, T->sw[B], in, par, col0, n, cs, rp, sflux, acc, sg, blk, (int)threadIdx.x, slot, fx);
 }
 
 // The SW band tables of an LDS image (the SwImg order); FP64 keeps absb in global memory.  A table the
@@ -1125,23 +1341,20 @@ sw_lds_band(const WR_L R *lt, const SwImg<R> &im, const SwBand<R> &G)
 template <typename R, int B> constexpr int swl_wpg() { return 4 * sw_waves<R, B>(); }
 template <typename R, int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__((64 * swl_wpg<R, B>()), (sw_waves<R, B>()))
-    k_swl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, const R *__restrict__ sflux,
-          AccT<R> acc, Surr sg, char *__restrict__ pool)
+    k_swl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp,
+          const R *__restrict__ sflux, AccT<R> acc, Surr sg, char *__restrict__ pool)
 {
     extern __shared__ float4 swl_tab[];
     const ColIn in = band_in<EXT>(in_);
     lds_fill<R>(swl_tab, T->sw_img[B]);
     const auto Bl = sw_lds_band<R>((const WR_L R *)swl_tab, T->sw_img[B], T->sw[B]);
     constexpr int WPG = swl_wpg<R, B>();
-    const int lane = threadIdx.x % 64, slot = blockIdx.x * WPG + threadIdx.x / 64;
-    LaneCache<R> cc;
-    cc.p = (WR_G R *)(pool + (size_t)slot * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R))) + lane;
-    cc.nv = sw_nv_mc<R>();
+    __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
+    const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
-    for (int blk = slot; blk * 64 < nday; blk += gridDim.x * WPG) {
-        const int tt = blk * 64 + lane;
-        if (tt < nday) sw_column<R, B, SURR>(T, Bl, in, par, col0, n, cs, sflux, acc, sg, cs.dlist[tt], cc);
-    }
+    for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)
+        sw_column<R, B, SURR>(T, Bl, in, par, col0, n, cs, rp, sflux, acc, sg, blk, lane, slot, fx + (sizeof(R) == 4 ? wv : 0));
 }
 
 // ---- post: FP64 fluxes -> heating rates, top-first outputs -------------------------------------------

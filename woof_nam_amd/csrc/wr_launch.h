@@ -76,6 +76,7 @@ struct BandJob {
     RunPar par;
     int col0, n;
     ColScal cs;
+    RecPtrs rp;
     BandAcc ba;
     Surr sg;
     Rtr<R> rt;
@@ -127,7 +128,7 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                 return;
             }
         }
-        if constexpr (B < 16 && sizeof(R) == 4 && lw_gsplit<R>() == 1) {
+        if constexpr (B < 16 && sizeof(R) == 4) {
             // k_lwl: as many persistent workgroups as the CUs hold at once (the runtime's occupancy for
             // the kernel's registers and LDS), each wave with its own pool slot; at most as many as the
             // pool has slots for (none fit: k_lwc)
@@ -149,12 +150,12 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (((j.c->lw_lds >> B) & 1) && nwg > 0) {
                 hipLaunchKernelGGL((k_lwl<B, SURR, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, acc, j.sg, pool);
+                                   j.col0, j.n, j.cs, j.rp, acc, j.sg, pool);
             } else {
                 hipLaunchKernelGGL((k_lwc<B, SURR, EXT>), dim3(band_grid(j, LW_NV_F32, LW_NG[B])), dim3(64), 0, s, j.tabs,
-                                   j.in, j.par, j.col0, j.n, j.cs, acc, j.sg, pool);
+                                   j.in, j.par, j.col0, j.n, j.cs, j.rp, acc, j.sg, pool);
             }
-        } else if constexpr (B < 16 && sizeof(R) == 8 && lw_gsplit<R>() == 1) {
+        } else if constexpr (B < 16 && sizeof(R) == 8) {
             // k_lwl64: persistent workgroups, as many as the CUs hold at once
             constexpr unsigned WPG = lwl64_wpg<R, B>();
             const size_t lds = (size_t)j.c->host_d.lw_img[B].n * sizeof(double);
@@ -171,13 +172,13 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (((j.c->lw_lds64 >> B) & 1) && nwg > 0)
                 hipLaunchKernelGGL((k_lwl64<B, SURR, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, acc, j.sg);
+                                   j.col0, j.n, j.cs, j.rp, acc, j.sg);
             else
                 hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3((j.n + 63) / 64), dim3(64), 0, s, j.tabs, j.in, j.par, j.col0,
-                                   j.n, j.cs, acc, j.sg);
+                                   j.n, j.cs, j.rp, acc, j.sg);
         } else if constexpr (B < 16)
-            hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3((j.n * lw_gsplit<R>() + 63) / 64), dim3(64), 0, s, j.tabs, j.in,
-                               j.par, j.col0, j.n, j.cs, acc, j.sg);
+            hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3((j.n + 63) / 64), dim3(64), 0, s, j.tabs, j.in,
+                               j.par, j.col0, j.n, j.cs, j.rp, acc, j.sg);
         else {
             // k_swl: persistent workgroups, as many as the CUs hold at once and the pool has slots for
             constexpr int S = B < 16 ? 0 : B - 16;
@@ -205,10 +206,10 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (on && nwg > 0)
                 hipLaunchKernelGGL((k_swl<R, S, SURR, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, j.sflux, acc, j.sg, pool);
+                                   j.col0, j.n, j.cs, j.rp, j.sflux, acc, j.sg, pool);
             else
                 hipLaunchKernelGGL((k_sw<R, S, SURR, EXT>), dim3(band_grid(j, sw_nv_mc<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
-                                   j.in, j.par, j.col0, j.n, j.cs, j.sflux, acc, j.sg, pool);
+                                   j.in, j.par, j.col0, j.n, j.cs, j.rp, j.sflux, acc, j.sg, pool);
         }
         tend(j.c, s);
     }
@@ -245,10 +246,10 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (on && nwg > 0)
                 hipLaunchKernelGGL((k_lwrl<R, B, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, acc, j.rt);
+                                   j.col0, j.n, j.cs, j.rp, acc, j.rt);
             else
                 hipLaunchKernelGGL((k_lwr<R, B, EXT>), dim3((j.n + 63) / 64), dim3(64), 0, s, j.tabs, j.in, j.par, j.col0,
-                                   j.n, j.cs, acc, j.rt);
+                                   j.n, j.cs, j.rp, acc, j.rt);
         } else {
             // k_swrl: persistent workgroups with the band's tables in LDS, within the pool's slots
             constexpr int S = B < 16 ? 0 : B - 16;
@@ -276,10 +277,10 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (on && nwg > 0)
                 hipLaunchKernelGGL((k_swrl<R, S, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, j.sflux, acc, pool);
+                                   j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
             else
                 hipLaunchKernelGGL((k_swr<R, S, EXT>), dim3(band_grid(j, sw_nv_mc<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
-                                   j.in, j.par, j.col0, j.n, j.cs, j.sflux, acc, pool);
+                                   j.in, j.par, j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
         }
         tend(j.c, s);
     }
@@ -326,6 +327,30 @@ int run_bands(wr_ctx *c, int band, hipStream_t s, F &&one)
     return WR_OK;
 }
 
+// What the band kernels of a tile read: LW records, column scalars, day list, SW records, solar source and
+// (McICA) the cloud words.
+template <typename R> void launch_prep(const BandJob<R> &j, hipStream_t s)
+{
+    wr_ctx *c = j.c;
+    const unsigned nb = (unsigned)(j.n + 63) / 64, nl = (unsigned)(j.rp.nrl + 3) / 4;
+    tbeg(c, KID_COLPREP, s);
+    hipLaunchKernelGGL((k_layers<R>), dim3(nb, nl), dim3(64, 4), 0, s, j.tabs, j.in, j.par, j.col0, j.n, j.cs, j.rp);
+    hipLaunchKernelGGL(k_colprep, dim3((j.n + 255) / 256), dim3(256), 0, s, j.in, j.col0, j.n, j.cs);
+    tend(c, s);
+    tbeg(c, KID_DAYLIST, s);
+    launch_daylist(j.cs, j.n, s);
+    tend(c, s);
+    tbeg(c, KID_SWPREP, s);
+    hipLaunchKernelGGL((k_layers_sw<R>), dim3(nb, nl), dim3(64, 4), 0, s, j.tabs, j.in, j.par, j.col0, j.n, j.cs, j.rp);
+    hipLaunchKernelGGL((k_sflux<R>), dim3(nb, 14), dim3(64), 0, s, j.tabs, j.in, j.par, j.col0, j.n, j.cs, (R *)j.sflux);
+    tend(c, s);
+    if (j.par.mcica) {
+        tbeg(c, KID_MCICA, s);
+        hipLaunchKernelGGL(k_mcica, dim3(nb, 30), dim3(64), 0, s, j.in, j.par, j.col0, j.n, j.cs, j.rp);
+        tend(c, s);
+    }
+}
+
 // Whether a tile of n columns runs all its bands in one launch (wr_many.h)
 inline bool use_many(const wr_ctx *c, int n, int band) { return band < 0 && n <= c->many_cols && !c->lw_glane; }
 
@@ -337,14 +362,10 @@ int launch_tile(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, const
                 int col0, int n, int band, hipStream_t s, const Surr &sg = Surr{})
 {
     const int nrl = in.nlay + 1;
-    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), tile_planes(c, n, nrl, band), sg, Rtr<R>{},
+    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, n, nrl, (int)sizeof(R)),
+                 tile_planes(c, n, nrl, band), sg, Rtr<R>{},
                  tile_lwrec<R>(c, n, nrl)};
-    tbeg(c, KID_COLPREP, s);
-    hipLaunchKernelGGL((k_colprep<R>), dim3((n + 255) / 256), dim3(256), 0, s, tabs, in, par, col0, n, j.cs, sflux);
-    tend(c, s);
-    tbeg(c, KID_DAYLIST, s);
-    launch_daylist(j.cs, n, s);
-    tend(c, s);
+    launch_prep(j, s);
     if (c->lw_glane && (band < 0 || band < 16)) {
         tbeg(c, KID_LWREC, s);
         hipLaunchKernelGGL((k_lwrec<R>), dim3((n + 63) / 64), dim3(64), 0, s, tabs, in, par, col0, n, j.cs, j.rec);
@@ -372,13 +393,9 @@ int launch_tile_nam(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, c
     rt.lstu = gptr((uint64_t *)((char *)c->rtr + sizeof(double) * 12 * (NL + 3) * (size_t)c->max_cols));
     rt.lstd = rt.lstu + c->max_cols;
     rt.n = n;
-    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), tile_planes(c, n, nrl, band), Surr{}, rt, LwRec<R>{}};
-    tbeg(c, KID_COLPREP, s);
-    hipLaunchKernelGGL((k_colprep<R>), dim3((n + 255) / 256), dim3(256), 0, s, tabs, in, par, col0, n, j.cs, sflux);
-    tend(c, s);
-    tbeg(c, KID_DAYLIST, s);
-    launch_daylist(j.cs, n, s);
-    tend(c, s);
+    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, n, nrl, (int)sizeof(R)),
+                 tile_planes(c, n, nrl, band), Surr{}, rt, LwRec<R>{}};
+    launch_prep(j, s);
     tbeg(c, KID_RTRFAC, s);
     hipLaunchKernelGGL((k_rtr_fac<R>), dim3((n + 63) / 64), dim3(64), 0, s, in, col0, n, rt);
     tend(c, s);

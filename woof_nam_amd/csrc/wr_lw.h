@@ -117,10 +117,14 @@ __device__ __forceinline__ void lw_layer(const Tabs<R> *__restrict__ T, const Ra
     lw_layer<R>(T, rc.lay(kin), par, la, L);
 }
 
-// reference ratio chi_mls(a, lev) / chi_mls(b, lev) (setcoef rfrate, FP64)
-__device__ __forceinline__ double chirat(const WR_G double *__restrict__ chi, int a, int b, int lev)
+// row of T->chir with the reference ratio chi_mls(a, lev) / chi_mls(b, lev) (setcoef rfrate) of a gas pair
+constexpr int CHI_PAIRS = 6;
+constexpr int CHI_PAIR[CHI_PAIRS][2] = {{1, 2}, {3, 2}, {1, 3}, {1, 6}, {1, 4}, {4, 2}};
+constexpr int chi_row(int a, int b)
 {
-    return chi[(lev - 1) * 7 + (a - 1)] / chi[(lev - 1) * 7 + (b - 1)];
+    for (int p = 0; p < CHI_PAIRS; ++p)
+        if (CHI_PAIR[p][0] == a && CHI_PAIR[p][1] == b) return p;
+    return -1;
 }
 
 template <typename R> __device__ __forceinline__ R planck(const Tabs<R> *__restrict__ T, int b, double temp)
@@ -131,31 +135,31 @@ template <typename R> __device__ __forceinline__ R planck(const Tabs<R> *__restr
     return T->delwave[b] * (tp[ind - 1] + fr * (tp[ind] - tp[ind - 1]));
 }
 
-// LW cloud optical depth of band b (phys_rrtm_lw_cldprop.cu:79, ilwcliq = 1, ilwcice = 1)
+// LW cloud optical depth of band b (phys_rrtm_lw_cldprop.cu:79, ilwcliq = 1, ilwcice = 1) of a layer with
+// cloud: liquid and ice paths, their radii, rain path
 template <typename R>
-__device__ __forceinline__ R lw_taucld(const Tabs<R> *__restrict__ T, int b, int lcf1, double ct, double cldliq,
-                                       double cldice, double refliq, double refice, double cldran = 0.0)
+__device__ __forceinline__ R lw_taucld_r(const Tabs<R> *__restrict__ T, int b, R cldliq, R cldice, double refliq,
+                                         double refice, double cldran)
 {
-    if (!lcf1 || !(ct > 0.0)) return (R)0;
     R tauliq = 0, tauice = 0;
-    if (cldliq > 0.0) {
+    if (cldliq > (R)0) {
         const double factor = refliq - 1.5;
         const int index = imax(1, imin(57, (int)factor));
         const R fint = (R)(factor - (double)index);
         const R a1 = T->absliq1[b * 58 + (index - 1)];
         const R a2 = T->absliq1[b * 58 + index];
-        tauliq = fmax((R)0, (R)cldliq * (a1 + fint * (a2 - a1)));
+        tauliq = fmax((R)0, cldliq * (a1 + fint * (a2 - a1)));
     }
-    if (cldice > 0.0) {
+    if (cldice > (R)0) {
         const R ri = (R)fmin(130.0, fmax(13.0, refice));
         const int ia0 = T->ipat[b] - 1;
-        tauice = fmax((R)0, (R)cldice * (T->absice1[ia0 * 2 + 0] + T->absice1[ia0 * 2 + 1] / ri));
+        tauice = fmax((R)0, cldice * (T->absice1[ia0 * 2 + 0] + T->absice1[ia0 * 2 + 1] / ri));
     }
     const R tauran = (R)(0.33e-3 * cldran);  // absrain (NCAR) x rain path
     return tauice + tauliq + tauran + (R)0;  // + tausnw (snow path 0)
 }
 
-// lw_taucld of radiation layer kin of column rc, with the layer's radii and rain path (path form)
+// lw_taucld_r of radiation layer kin of column rc, with the layer's radii and rain path (path form)
 // loaded only for a cloudy layer
 template <typename R, typename L_T, typename RC_T, typename P_T>
 __device__ __forceinline__ R lw_taucld_l(const Tabs<R> *__restrict__ T, int b, int lcf1, const L_T &L, const RC_T &rc,
@@ -164,7 +168,7 @@ __device__ __forceinline__ R lw_taucld_l(const Tabs<R> *__restrict__ T, int b, i
     if (!lcf1 || !(L.ct > 0.0)) return (R)0;
     double rl, ri, rp;
     rc.props(kin, par.re_liq, par.re_ice, rl, ri, rp);
-    return lw_taucld<R>(T, b, 1, L.ct, L.clwp, L.ciwp, rl, ri, rp);
+    return lw_taucld_r<R>(T, b, (R)L.clwp, (R)L.ciwp, rl, ri, rp);
 }
 
 // ---- band optics ------------------------------------------------------------------------------
@@ -256,6 +260,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
     const R sf = L.selffac, sfr = L.selffrac, ff = L.forfac, ffr = L.forfrac, mf = L.minorfrac;
     const R *ca = L.colamt;
     const WR_G double *chi = T->chi_mls;
+#define CHR(a, b, lev) T->chir[chi_row(a, b) * 59 + (lev) - 1]
 #define SELF(g) (sf * (T2(Bt.selfref, inds, g, ng) + sfr * (T2(Bt.selfref, indsp, g, ng) - T2(Bt.selfref, inds, g, ng))))
 #define FOR(g) (ff * (T2(Bt.forref, indf, g, ng) + ffr * (T2(Bt.forref, indfp, g, ng) - T2(Bt.forref, indf, g, ng))))
 #define MIN1(tab, g) (T2(tab, indm, g, ng) + mf * (T2(tab, indmp, g, ng) - T2(tab, indm, g, ng)))
@@ -310,7 +315,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         const R ratn2o = ca[3] / p;
         const R adjcoln2o = (ratn2o > (R)1.5) ? ((R)0.5 + M<R>::pow(ratn2o - (R)0.5, (R)0.65)) * p : ca[3];
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jpp), ca[1], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)8);
             const Eta<R> em = eta<R>(ca[0], Bt.refrat_m_a, ca[1], (R)8), ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[1], (R)8);
             const Sel<R> s0 = sel_one<R>(e0.specparm, e0.fs, l0 * 9 + e0.js);
             const Sel<R> s1 = sel_one<R>(e1.specparm, e1.fs, l1 * 9 + e1.js);
@@ -324,7 +329,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
                 fr[jj] = FRACA(ep, g);
             }
         } else {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jpp), ca[1], (R)4);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)4);
             const Eta<R> em = eta<R>(ca[0], Bt.refrat_m_b, ca[1], (R)4), ep = eta<R>(ca[0], Bt.refrat_planck_b, ca[1], (R)4);
             const int i0 = u0 * 5 + e0.js, i1 = u1 * 5 + e1.js;
 #pragma unroll
@@ -339,7 +344,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 3) {
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jpp), ca[1], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)8);
             const Eta<R> ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[1], (R)8);
             const Sel<R> s0 = sel_one<R>(e0.specparm, e0.fs, l0 * 9 + e0.js);
             const Sel<R> s1 = sel_one<R>(e1.specparm, e1.fs, l1 * 9 + e1.js);
@@ -352,7 +357,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
                 fr[jj] = FRACA(ep, g);
             }
         } else {
-            const Eta<R> e0 = eta<R>(ca[2], (R)chirat(chi, 3, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[2], (R)chirat(chi, 3, 2, jpp), ca[1], (R)4);
+            const Eta<R> e0 = eta<R>(ca[2], CHR(3, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[2], CHR(3, 2, jpp), ca[1], (R)4);
             const Eta<R> ep = eta<R>(ca[2], Bt.refrat_planck_b, ca[1], (R)4);
             const int i0 = u0 * 5 + e0.js, i1 = u1 * 5 + e1.js;
 #pragma unroll
@@ -373,7 +378,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
     } else if constexpr (B == 4) {
         const R wxk = L.wx[0];
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jpp), ca[1], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)8);
             const Eta<R> em = eta<R>(ca[0], Bt.refrat_m_a, ca[1], (R)8), ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[1], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -386,7 +391,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
                 fr[jj] = FRACA(ep, g);
             }
         } else {
-            const Eta<R> e0 = eta<R>(ca[2], (R)chirat(chi, 3, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[2], (R)chirat(chi, 3, 2, jpp), ca[1], (R)4);
+            const Eta<R> e0 = eta<R>(ca[2], CHR(3, 2, jp), ca[1], (R)4), e1 = eta<R>(ca[2], CHR(3, 2, jpp), ca[1], (R)4);
             const Eta<R> ep = eta<R>(ca[2], Bt.refrat_planck_b, ca[1], (R)4);
             const int i0 = u0 * 5 + e0.js, i1 = u1 * 5 + e1.js;
 #pragma unroll
@@ -423,7 +428,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         const R ratco2 = ca[1] / temp;
         if (lower) {
             const R adjcolco2 = (ratco2 > (R)3) ? ((R)3 + M<R>::pow(ratco2 - (R)3, (R)0.79)) * temp : ca[1];
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 3, jp), ca[2], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 3, jpp), ca[2], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 3, jp), ca[2], (R)8), e1 = eta<R>(ca[0], CHR(1, 3, jpp), ca[2], (R)8);
             const Eta<R> em = eta<R>(ca[0], Bt.refrat_m_a, ca[2], (R)8), ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[2], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -481,7 +486,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         const R ratn2o = ca[3] / temp;
         const R adjcoln2o = (ratn2o > (R)1.5) ? ((R)0.5 + M<R>::pow(ratn2o - (R)0.5, (R)0.65)) * temp : ca[3];
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 6, jp), ca[4], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 6, jpp), ca[4], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 6, jp), ca[4], (R)8), e1 = eta<R>(ca[0], CHR(1, 6, jpp), ca[4], (R)8);
             const Eta<R> em = eta<R>(ca[0], Bt.refrat_m_a, ca[4], (R)8), ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[4], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -538,7 +543,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 11) {
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 2, jpp), ca[1], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)8);
             const Eta<R> ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[1], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -558,7 +563,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
             const R temp = L.coldry * (R)3.55e-4;
             const R ratco2 = ca[1] / temp;
             const R adjcolco2 = (ratco2 > (R)3) ? ((R)2 + M<R>::pow(ratco2 - (R)2, (R)0.68)) * temp : ca[1];
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 4, jp), ca[3], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 4, jpp), ca[3], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 4, jp), ca[3], (R)8), e1 = eta<R>(ca[0], CHR(1, 4, jpp), ca[3], (R)8);
             const Eta<R> emc2 = eta<R>(ca[0], Bt.refrat_m_a, ca[3], (R)8), emc = eta<R>(ca[0], Bt.refrat_m_a3, ca[3], (R)8);
             const Eta<R> ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[3], (R)8);
             Sel<R> s0, s1;
@@ -599,7 +604,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
     } else if constexpr (B == 14) {
         if (lower) {
             const R scalen2 = L.colbrd * L.scaleminor;
-            const Eta<R> e0 = eta<R>(ca[3], (R)chirat(chi, 4, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[3], (R)chirat(chi, 4, 2, jpp), ca[1], (R)8);
+            const Eta<R> e0 = eta<R>(ca[3], CHR(4, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[3], CHR(4, 2, jpp), ca[1], (R)8);
             const Eta<R> em = eta<R>(ca[3], Bt.refrat_m_a, ca[1], (R)8), ep = eta<R>(ca[3], Bt.refrat_planck_a, ca[1], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -617,7 +622,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 15) {
         if (lower) {
-            const Eta<R> e0 = eta<R>(ca[0], (R)chirat(chi, 1, 6, jp), ca[4], (R)8), e1 = eta<R>(ca[0], (R)chirat(chi, 1, 6, jpp), ca[4], (R)8);
+            const Eta<R> e0 = eta<R>(ca[0], CHR(1, 6, jp), ca[4], (R)8), e1 = eta<R>(ca[0], CHR(1, 6, jpp), ca[4], (R)8);
             const Eta<R> ep = eta<R>(ca[0], Bt.refrat_planck_a, ca[4], (R)8);
             Sel<R> s0, s1;
             sel_joint<R>(e0.specparm, e0.fs, l0 * 9 + e0.js, e1.specparm, e1.fs, l1 * 9 + e1.js, s0, s1);
@@ -638,6 +643,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
             }
         }
     }
+#undef CHR
 #undef SELF
 #undef FOR
 #undef MIN1

@@ -35,6 +35,7 @@ template <typename R> struct ManyArgs {
     RunPar par;
     int col0, n, blk0, nblk;  // blocks blk0 .. blk0 + nblk - 1 of 64 columns
     ColScal cs;
+    RecPtrs rp;
     BandAcc ba;
     Surr sg;
     Rtr<R> rt;
@@ -42,38 +43,31 @@ template <typename R> struct ManyArgs {
 };
 
 template <typename R, bool NAM, bool SURR, int P>
-__device__ __forceinline__ void many_run(const ManyArgs<R> &a, int pos, int b, size_t before)
+__device__ __forceinline__ void many_run(const ManyArgs<R> &a, int pos, int b, size_t before, Fix64 *fx)
 {
     if constexpr (P < 30) {
         constexpr int id = MANY_ORDER[P];
         if (pos != P) {
-            many_run<R, NAM, SURR, P + 1>(a, pos, b, before + many_slot<R, NAM>(id, 1));
+            many_run<R, NAM, SURR, P + 1>(a, pos, b, before + many_slot<R, NAM>(id, 1), fx);
             return;
         }
         const int nk = a.in.nlay + 2;
-        char *slot = a.pool + (before * a.nblk + many_slot<R, NAM>(id, 1) * b) * nk;
         const AccT<R> acc = band_acc<R>(a.ba, id);
-        LaneCache<R> cc;
-        cc.p = (WR_G R *)slot + threadIdx.x;
-        const int t = (a.blk0 + b) * 64 + threadIdx.x;
+        WR_G char *slot = (WR_G char *)(a.pool + (before * a.nblk + many_slot<R, NAM>(id, 1) * b) * nk);
+        const int blk = a.blk0 + b, lane = (int)threadIdx.x;
         if constexpr (id < 16) {
-            if constexpr (NAM) {
-                lwr_column<R, id>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, acc, a.rt, t);
-            } else if constexpr (sizeof(R) == 4) {
-                cc.nv = LW_NV_F32;
-                if (t < valid_cols(a.in, a.col0, a.n))
-                    lw_column_f32c<id, SURR>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, acc, a.sg, t, cc);
-            } else {
-                lw_column<R, id, SURR>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, acc, a.sg, t);
-            }
+            if constexpr (NAM)
+                lwr_column<R, id>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, a.rp, acc, a.rt, blk, lane);
+            else if constexpr (sizeof(R) == 4)
+                lw_column_f32c<id, SURR>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, a.rp, acc, a.sg, blk, lane, slot);
+            else
+                lw_column<R, id, SURR>(a.T, a.T->lw[id], a.in, a.par, a.col0, a.n, a.cs, a.rp, acc, a.sg, blk, lane);
         } else {
             constexpr int S = id - 16;
-            cc.nv = sw_nv_mc<R>();
-            if (t >= *a.cs.nday) return;
             if constexpr (NAM)
-                swr_column<R, S>(a.T, a.T->sw[S], a.in, a.par, a.col0, a.n, a.cs, a.sflux, acc, a.cs.dlist[t], cc);
+                swr_column<R, S>(a.T, a.T->sw[S], a.in, a.par, a.col0, a.n, a.cs, a.rp, a.sflux, acc, blk, lane, slot, fx);
             else
-                sw_column<R, S, SURR>(a.T, a.T->sw[S], a.in, a.par, a.col0, a.n, a.cs, a.sflux, acc, a.sg, a.cs.dlist[t], cc);
+                sw_column<R, S, SURR>(a.T, a.T->sw[S], a.in, a.par, a.col0, a.n, a.cs, a.rp, a.sflux, acc, a.sg, blk, lane, slot, fx);
         }
     }
 }
@@ -81,13 +75,14 @@ __device__ __forceinline__ void many_run(const ManyArgs<R> &a, int pos, int b, s
 template <typename R, bool NAM, bool SURR>
 __global__ void __launch_bounds__(64, sizeof(R) == 4 && !NAM ? 2 : 1) k_many(ManyArgs<R> a)
 {
-    many_run<R, NAM, SURR, 0>(a, (int)(blockIdx.x / a.nblk), (int)(blockIdx.x % a.nblk), 0);
+    __shared__ Fix64 fx[1];
+    many_run<R, NAM, SURR, 0>(a, (int)(blockIdx.x / a.nblk), (int)(blockIdx.x % a.nblk), 0, fx);
 }
 
 // The bands of a tile, as many 64-column blocks at once as the pool has room for.
 template <typename R, bool NAM, bool SURR> int launch_many(const BandJob<R> &j, hipStream_t s)
 {
-    ManyArgs<R> a{j.tabs, j.sflux, j.in, j.par, j.col0, j.n, 0, 0, j.cs, j.ba, j.sg, j.rt, j.c->pool[0]};
+    ManyArgs<R> a{j.tabs, j.sflux, j.in, j.par, j.col0, j.n, 0, 0, j.cs, j.rp, j.ba, j.sg, j.rt, j.c->pool[0]};
     const int nb = (j.n + 63) / 64;
     const size_t room = j.c->pool_all / many_block_bytes<R, NAM>(j.in.nlay + 2);
     const int per = (size_t)nb < room ? nb : (int)room;

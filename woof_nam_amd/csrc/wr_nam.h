@@ -144,28 +144,6 @@ __global__ void __launch_bounds__(64) k_rtr_fac(ColIn in, int col0, int n, Rtr<R
     }
 }
 
-// total-sky transmittance, source factor and absorptance of odtot (rtrnmr's cloudy branch)
-template <typename R>
-__device__ __forceinline__ void lw_tot3(const Tabs<R> *__restrict__ T, R odtot, R &totfac, R &atrtot, R &trnt)
-{
-    if (odtot < (R)0.06) {
-        totfac = (R)0.166667 * odtot;
-        atrtot = odtot - (R)0.5 * odtot * odtot;
-        trnt = (R)1 - atrtot;
-    } else {
-        const R tblind = odtot / ((R)(1.0 / 0.278) + odtot);
-        const int ittot = imin(NTBL, (int)((R)10000 * tblind + (R)0.5));
-        if constexpr (sizeof(R) == 4) {
-            const LutF l = lut_f32(ittot, true);
-            totfac = l.tfn, trnt = l.e;
-        } else {
-            totfac = T->tfn_tbl[ittot];
-            trnt = T->exp_tbl[ittot];
-        }
-        atrtot = (R)1 - trnt;
-    }
-}
-
 // ---- LW band kernel of the NAM route (rtrnmr) ---------------------------------------------------
 // Per-band optics chunks (g-points, 0 = whole band) and wave bounds, by precision, as for the McICA
 // route's LW kernels: a second resident wave covers the table-gather waits where the registers allow.
@@ -174,10 +152,10 @@ __device__ __forceinline__ void lw_tot3(const Tabs<R> *__restrict__ T, R odtot, 
 // FP32 bands 3 and 5 and most FP64 bands were fastest as they were (FP64 bands 6 and 11 gain 9 and
 // 17 %).
 // WR_LWR_WAVES > 0 or WR_LWR_CHUNK >= 0 override the tables for every band (tuning builds).
-constexpr int LWR64_WAVES[16] = {1, 1, 1, 1, 1, 2, 1, 1, 1, 1, 2, 1, 1, 1, 1, 1};
-constexpr int LWR64_CHUNK[16] = {0, 0, 0, 0, 0, 2, 0, 0, 0, 0, 4, 0, 0, 0, 0, 0};
-constexpr int LWR32_WAVES[16] = {2, 2, 1, 2, 1, 1, 2, 2, 2, 1, 1, 2, 1, 1, 1, 3};
-constexpr int LWR32_CHUNK[16] = {4, 4, 0, 2, 0, 0, 2, 4, 2, 0, 0, 4, 0, 0, 0, 0};
+constexpr int LWR64_WAVES[16] = {1, 1, 1, 1, 1, 2, 1, 2, 1, 2, 2, 2, 2, 2, 2, 2};
+constexpr int LWR64_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
+constexpr int LWR32_WAVES[16] = {3, 2, 2, 2, 2, 3, 2, 3, 2, 4, 3, 3, 4, 4, 4, 4};
+constexpr int LWR32_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
 #ifndef WR_LWR_WAVES
 #define WR_LWR_WAVES 0
 #endif
@@ -193,189 +171,119 @@ template <typename R, int B> constexpr int lwr_chunk()
     return chunk_of(LW_NG[B], WR_LWR_CHUNK >= 0 ? WR_LWR_CHUNK : (sizeof(R) == 8 ? LWR64_CHUNK[B] : LWR32_CHUNK[B]));
 }
 
-// One column of LW band B on the NAM route (rtrnmr), optics from the band tables Bt.
+// One column of LW band B on the NAM route (rtrnmr), optics from the band tables Bt: down sweep, surface, up
+// sweep with the optics evaluated again, in chunks of g-points without per-g-point branches (as lw_column).
 template <typename R, int B, typename BT>
 __device__ __forceinline__ void lwr_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par,
-                                           int col0, int n, const ColScal &cs, const AccT<R> &acc, const Rtr<R> &rt, int t)
+                                           int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
+                                           const Rtr<R> &rt, int blk, int lane)
 {
-    constexpr int NG = LW_NG[B];
+    constexpr int NG = LW_NG[B], CH = lwr_chunk<R, B>();
+    const int t = blk * 64 + lane;
     if (t >= valid_cols(in, col0, n)) return;
-    const int i = col0 + t;
-    const RadCol rc{in, i, in.nlay + 1};
-    const int nrl = rc.nrl;
-    const int lcf1 = cs.lcf1[t];
-    const double pwv = cs.pwv[t];
-    const R sdif = (R)((B == 0 || B == 3 || B == 9) ? 1.66 : fmin(1.80, fmax(1.50, LW_A0[B] + LW_A1[B] * exp_d(LW_A2[B] * pwv))));
-    const double sfe = in.emis[i];
-    const R semis = (R)((sfe > EPS && sfe <= 1.0) ? sfe : 1.0);
+    const Surr none{};
+    const LwCol<R> c = lw_col<R, B, false>(in, col0, cs, none, t);
+    const int nrl = c.nrl;
+    const RadCol rcol{in, c.i, nrl};
     const uint64_t lstu = rt.lstu[t], lstd = rt.lstd[t];
-    const R eps = (R)1.0e-6;
-
     acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
-    // ---- down sweep, top to surface ----
-    R radtotd[NG], totradd[NG], clrradd[NG], rad[NG];
+    // radiances per g-point: total, its cloudy and clear parts, the overlap correction between them
+    R tot[NG], cld[NG], clr[NG], rad[NG];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) radtotd[g] = totradd[g] = clrradd[g] = rad[g] = (R)0;
-    // layer inputs: cur = layer kin, nxt = kin + 1 (loaded an iteration ahead), nn = kin + 2
-    LayV cur = rc.lay(0), nxt = cur;
-    if (nrl > 1) nxt = rc.lay(1);
-    double tz_top = cs.tz[t], la_nx = cs.la[t], tz_nx = 0.0;
-    if constexpr (sizeof(R) != 8) tz_nx = cs.tz[(size_t)n + t];
-    for (int kin = 0; kin < nrl; ++kin) {
-        const int kk = nrl - kin;  // 1-based surface-first layer
-        LayV nn = nxt;
-        if (kin + 2 < nrl) nn = rc.lay(kin + 2);
-        // this layer's log pressure and bottom level temperature: FP32 kernels load k_colprep's values an
-        // iteration ahead; FP64 kernels evaluate them here by the same operations (measured faster there)
-        double la_c, tz_bot;
-        if constexpr (sizeof(R) == 8) {
-            la_c = la_nx;
-            if (kin + 1 < nrl) {
-                la_nx = log_d(nxt.pl);
-                tz_bot = tlvl_v(nxt.t, cur.t, log_d(cur.pb), la_nx, la_c);
-            } else {
-                tz_bot = rc.tskn();
-            }
-        } else {
-            la_c = la_nx, tz_bot = tz_nx;
-            if (kin + 1 < nrl) la_nx = cs.la[(size_t)(kin + 1) * n + t], tz_nx = cs.tz[(size_t)(kin + 2) * n + t];
+    for (int g = 0; g < NG; ++g) tot[g] = cld[g] = clr[g] = rad[g] = (R)0;
+    // one layer of a sweep; q0, idx: the overlap factors of its direction; start: a cloud block starts here
+    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, int q0, int idx, bool start, bool sfc, R pk0, R &s, R &s0) {
+        s = (R)0, s0 = (R)0;
+        const bool some = __any(y.cloudy);
+        R clfr = (R)0, cld1 = (R)0, cld2 = (R)0, clr1 = (R)0, clr2 = (R)0, cmb1 = (R)0, cmb2 = (R)0;
+        if (some) {
+            clfr = (R)rcol.cfrac(nrl - 1 - k);
+            cld1 = rt.at(q0, idx, t), cld2 = rt.at(q0 + 1, idx, t), clr1 = rt.at(q0 + 2, idx, t);
+            clr2 = rt.at(q0 + 3, idx, t), cmb1 = rt.at(q0 + 4, idx, t), cmb2 = rt.at(q0 + 5, idx, t);
         }
-        LwLay<R> L;
-        lw_layer<R>(T, cur, par, la_c, L);
-        R tau[NG], fr[NG];
-        lw_optics_ch<R, B, NG, lwr_chunk<R, B>()>(T, Bt, L, tau, fr, 0);
-        const R blay = planck<R>(T, B, L.tavel);
-        const R dplnkd = planck<R>(T, B, tz_bot) - blay;
-        const R taucld = lw_taucld_l<R>(T, B, lcf1, L, rc, kin, par);
-        const R taer = (R)rc.aer_lw_tau(B, kin);  // tautot = taug + tauaer
-        const R clfr = (R)lw_cldfrc(rc, kk);
-        const bool top = (lstd >> (kk - 1)) & 1;
-        const R c1 = rt.at(FCLR1D, kk - 1, t), d1 = rt.at(FCLD1D, kk - 1, t), m1 = rt.at(FCMB1D, kk - 1, t);
-        const R m2 = rt.at(FCMB2D, kk - 1, t), c2 = rt.at(FCLR2D, kk - 1, t), d2 = rt.at(FCLD2D, kk - 1, t);
-        R s = (R)0;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const GasT<R> q = lw_gas<R>(T, sdif, tau[g] + taer);
-            const R gassrcd = fr[g] * (blay + dplnkd * q.gasfac) * q.atrgas;
-            if (top) {
-                totradd[g] = clfr * radtotd[g];
-                clrradd[g] = radtotd[g] - totradd[g];
-                rad[g] = (R)0;
+        for (int g0 = 0; g0 < NG; g0 += CH) {
+            R tau[CH], fr[CH];
+            lw_taufr<R, B, false, CH>(T, Bt, none, c, n, k, y.L, g0, tau, fr);
+            GasV<R, CH> q;
+            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
+            if (sfc) {  // surface emission and reflection
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int g = g0 + j;
+                    const R r0 = c.semis * fr[j] * pk0;
+                    tot[g] = r0 + c.reflct * tot[g];
+                    cld[g] = clr[g] = rad[g] = (R)0;
+                    s0 = s0 + tot[g];
+                }
             }
-            if (clfr >= eps) {
-                const R odcld = sdif * taucld;
-                R totfac, atrtot, trnt;
-                lw_tot3<R>(T, q.odepth + odcld, totfac, atrtot, trnt);
-                const R totsrcd = fr[g] * (blay + dplnkd * totfac) * atrtot;
-                totradd[g] = totradd[g] * trnt + clfr * totsrcd;
-                clrradd[g] = clrradd[g] * q.trng + ((R)1 - clfr) * gassrcd;
-                radtotd[g] = totradd[g] + clrradd[g];
-                s = s + radtotd[g];
-                const R radmod = rad[g] * (c1 * q.trng + d1 * trnt) - m1 * gassrcd + m2 * totsrcd;
-                rad[g] = -radmod + c2 * (clrradd[g] + radmod) - d2 * (totradd[g] - radmod);
-                totradd[g] = totradd[g] + rad[g];
-                clrradd[g] = clrradd[g] - rad[g];
-            } else {
-                radtotd[g] = radtotd[g] * q.trng + gassrcd;
-                s = s + radtotd[g];
+            R gas[CH], nt[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                gas[j] = fr[j] * (y.blay + dplnk * q.gf[j]) * q.at[j];
+                nt[j] = tot[g0 + j] * q.tr[j] + gas[j];
             }
+            if (some) {
+                R tr[CH], at[CH], gf[CH];
+                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int g = g0 + j;
+                    const R src = fr[j] * (y.blay + dplnk * gf[j]) * at[j];
+                    R a = cld[g], b = clr[g], r = rad[g];
+                    if (start) {
+                        a = clfr * tot[g];
+                        b = tot[g] - a;
+                        r = (R)0;
+                    }
+                    R na = a * tr[j] + clfr * src;
+                    R nb = b * q.tr[j] + ((R)1 - clfr) * gas[j];
+                    const R ntot = na + nb;
+                    const R mod = r * (clr1 * q.tr[j] + cld1 * tr[j]) - cmb1 * gas[j] + cmb2 * src;
+                    const R nr = -mod + clr2 * (nb + mod) - cld2 * (na - mod);
+                    na = na + nr;
+                    nb = nb - nr;
+                    nt[j] = y.cloudy ? ntot : nt[j];
+                    cld[g] = y.cloudy ? na : a;
+                    clr[g] = y.cloudy ? nb : b;
+                    rad[g] = y.cloudy ? nr : r;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                tot[g0 + j] = nt[j];
+                s = s + nt[j];
+            }
+            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
         }
-        acc.lw_dn[(size_t)(kk - 1) * n + t] = s;
-        tz_top = tz_bot;
-        cur = nxt, nxt = nn;
+    };
+    R s, s0;
+    for (int k = nrl - 1; k >= 0; --k) {  // down sweep, top to surface
+        LwLayer<R> y;
+        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        sweep(k, y, y.bbot - y.blay, FCLD1D, k, (lstd >> k) & 1, false, (R)0, s, s0);
+        acc.lw_dn[(size_t)k * n + t] = s;
     }
-    // ---- up sweep, surface to top ----
-    const R reflct = (R)1 - semis;
-    R radtotu[NG], totradu[NG], clrradu[NG];
-    double tz_bot = cs.tz[(size_t)nrl * n + t];
-    // layer inputs: cur = layer kin, nxt = kin - 1 (loaded an iteration ahead), nn = kin - 2
-    cur = rc.lay(nrl - 1), nxt = cur;
-    if (nrl > 1) nxt = rc.lay(nrl - 2);
-    if constexpr (sizeof(R) == 8)
-        la_nx = log_d(cur.pl);
-    else
-        la_nx = cs.la[(size_t)(nrl - 1) * n + t], tz_nx = cs.tz[(size_t)(nrl - 1) * n + t];
-    for (int kin = nrl - 1; kin >= 0; --kin) {
-        const int kk = nrl - kin;
-        LayV nn = nxt;
-        if (kin >= 2) nn = rc.lay(kin - 2);
-        const double la_c = la_nx;
-        if constexpr (sizeof(R) == 8) {
-            if (kin > 0) {
-                la_nx = log_d(nxt.pl);
-                tz_top = tlvl_v(cur.t, nxt.t, log_d(cur.pt), la_c, la_nx);
-            } else {
-                tz_top = cur.t;
-            }
-        } else {
-            tz_top = tz_nx;
-            if (kin > 0) la_nx = cs.la[(size_t)(kin - 1) * n + t], tz_nx = cs.tz[(size_t)(kin - 1) * n + t];
+    for (int k = 0; k < nrl; ++k) {  // up sweep, surface to top
+        LwLayer<R> y;
+        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        R btop = y.blay;  // above the top layer, its own temperature
+        if (k + 1 < nrl) {
+            const LRow<R> up = lrow<R>(rp, blk, k + 1, lane);
+            btop = planck_of<R>(T, B, (int)(up.w(1) & 255u), up.f(LF_PB));
         }
-        LwLay<R> L;
-        lw_layer<R>(T, cur, par, la_c, L);
-        R tau[NG], fr[NG];
-        lw_optics_ch<R, B, NG, lwr_chunk<R, B>()>(T, Bt, L, tau, fr, 0);
-        const R blay = planck<R>(T, B, L.tavel);
-        const R dplnku = planck<R>(T, B, tz_top) - blay;
-        if (kk == 1) {  // surface emission and reflection
-            const R pk0 = planck<R>(T, B, rc.tskn());
-            R s0 = (R)0;
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                const R rad0 = semis * fr[g] * pk0;
-                radtotu[g] = rad0 + reflct * radtotd[g];
-                totradu[g] = clrradu[g] = (R)0;
-                rad[g] = (R)0;
-                s0 = s0 + radtotu[g];
-            }
-            acc.lw_up[t] = s0;
-        }
-        const R taucld = lw_taucld_l<R>(T, B, lcf1, L, rc, kin, par);
-        const R taer = (R)rc.aer_lw_tau(B, kin);  // tautot = taug + tauaer
-        const R clfr = (R)lw_cldfrc(rc, kk);
-        const bool bot = (lstu >> (kk - 1)) & 1;
-        const R c1 = rt.at(FCLR1U, kk + 1, t), d1 = rt.at(FCLD1U, kk + 1, t), m1 = rt.at(FCMB1U, kk + 1, t);
-        const R m2 = rt.at(FCMB2U, kk + 1, t), c2 = rt.at(FCLR2U, kk + 1, t), d2 = rt.at(FCLD2U, kk + 1, t);
-        R s = (R)0;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const GasT<R> q = lw_gas<R>(T, sdif, tau[g] + taer);
-            const R gasu = fr[g] * (blay + dplnku * q.gasfac) * q.atrgas;
-            if (bot) {
-                totradu[g] = clfr * radtotu[g];
-                clrradu[g] = radtotu[g] - totradu[g];
-                rad[g] = (R)0;
-            }
-            if (clfr >= eps) {
-                const R odcld = sdif * taucld;
-                R totfac, atrtot, trnt;
-                lw_tot3<R>(T, q.odepth + odcld, totfac, atrtot, trnt);
-                const R totu = fr[g] * (blay + dplnku * totfac) * atrtot;
-                totradu[g] = totradu[g] * trnt + clfr * totu;
-                clrradu[g] = clrradu[g] * q.trng + ((R)1 - clfr) * gasu;
-                radtotu[g] = totradu[g] + clrradu[g];
-                s = s + radtotu[g];
-                const R radmod = rad[g] * (c1 * q.trng + d1 * trnt) - m1 * gasu + m2 * totu;
-                rad[g] = -radmod + c2 * (clrradu[g] + radmod) - d2 * (totradu[g] - radmod);
-                totradu[g] = totradu[g] + rad[g];
-                clrradu[g] = clrradu[g] - rad[g];
-            } else {
-                radtotu[g] = radtotu[g] * q.trng + gasu;
-                s = s + radtotu[g];
-            }
-        }
-        acc.lw_up[(size_t)kk * n + t] = s;
-        tz_bot = tz_top;
-        cur = nxt, nxt = nn;
+        sweep(k, y, btop - y.blay, FCLD1U, k + 2, (lstu >> k) & 1, k == 0, y.bbot, s, s0);
+        if (k == 0) acc.lw_up[t] = s0;
+        acc.lw_up[(size_t)(k + 1) * n + t] = s;
     }
 }
 
 template <typename R, int B, bool EXT = true>
 __global__ void __launch_bounds__(64, (lwr_waves<R, B>())) k_lwr(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
-                                            int n, ColScal cs, AccT<R> acc, Rtr<R> rt)
+                                            int n, ColScal cs, RecPtrs rp, AccT<R> acc, Rtr<R> rt)
 {
     const ColIn in = band_in<EXT>(in_);
-    lwr_column<R, B>(T, T->lw[B], in, par, col0, n, cs, acc, rt, blockIdx.x * blockDim.x + threadIdx.x);
+    lwr_column<R, B>(T, T->lw[B], in, par, col0, n, cs, rp, acc, rt, (int)blockIdx.x, (int)threadIdx.x);
 }
 
 // k_lwr with the band's tables in LDS (the image of k_lwl / k_lwl64: FP64 keeps absb in global
@@ -384,7 +292,8 @@ __global__ void __launch_bounds__(64, (lwr_waves<R, B>())) k_lwr(const Tabs<R> *
 template <typename R, int B> constexpr int lwrl_wpg() { return 4 * lwr_waves<R, B>(); }
 template <typename R, int B, bool EXT = true>
 __global__ void __launch_bounds__((64 * lwrl_wpg<R, B>()), (lwr_waves<R, B>()))
-    k_lwrl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, AccT<R> acc, Rtr<R> rt)
+    k_lwrl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp, AccT<R> acc,
+           Rtr<R> rt)
 {
     extern __shared__ float4 lwrl_tab[];
     const ColIn in = band_in<EXT>(in_);
@@ -395,181 +304,96 @@ __global__ void __launch_bounds__((64 * lwrl_wpg<R, B>()), (lwr_waves<R, B>()))
     const int lane = threadIdx.x % 64;
     if constexpr (sizeof(R) == 4) {
         const auto Bl = lds_band<R>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
-        for (int blk = blockIdx.x * WPG + threadIdx.x / 64; blk * 64 < n; blk += gridDim.x * WPG)
-            lwr_column<R, B>(T, Bl, in, par, col0, n, cs, acc, rt, blk * 64 + lane);
+        for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
+            lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     } else {
         const auto Bl = lds_band<R>(lt, im, T->lw[B], T->lw[B].absb);
-        for (int blk = blockIdx.x * WPG + threadIdx.x / 64; blk * 64 < n; blk += gridDim.x * WPG)
-            lwr_column<R, B>(T, Bl, in, par, col0, n, cs, acc, rt, blk * 64 + lane);
+        for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
+            lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     }
 }
 
 // ---- SW band kernel of the NAM route (spcvrtc with cldfrc mixing and zcf1/zcf0 weighting) -------
-// R/T of layer k (surface-first): pass 0 clear sky; pass 1 total sky, the cloudy R/T mixed with the
-// clear ones by the layer cloud fraction zc1 = cfrac / zcf1 (phys_rrtm_sw_spcvrtc.cu, cloudy block)
-template <typename R, int B, typename BT>
-__device__ __forceinline__ void swr_layer(const Tabs<R> *__restrict__ T, const BT &Bt, const RadCol &rc, const RunPar &par, int k,
-                                          int lt, int pass, double cf1, R cz, R snt, SwLayerRT<R, B> &o, double la)
-{
-    constexpr int NG = SW_NG[B];
-    const int kin = rc.nrl - 1 - k;
-    SwLay<R> L;
-    sw_layer<R>(T, rc, par, kin, la, L);
-    R tg[NG], tr[NG];
-    sw_optics_t<R, B>(T, Bt, L, k + 1, lt, tg, tr);
-    double ta, sa, ya;
-    rc.aer_sw3(B, kin, ta, sa, ya);
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-        layer_rt_eval<R>(T, tr[g], tg[g], (R)ta, (R)sa, (R)ya, false, (R)0, (R)1, (R)0, cz, snt, o.rb[g], o.rd[g], o.tb[g],
-                         o.td[g], o.ld[g]);
-    if (pass == 0) return;
-    const double zc1d = rc.cfrac(kin) / cf1;
-    if (!(zc1d > FTINY)) return;
-    const R zc1 = (R)zc1d, zc0 = (R)(1.0 - zc1d);
-    R ctau = (R)0, cssa = (R)1, casy = (R)0;
-    sw_cloud_l<R>(T, B, L, rc, kin, par, ctau, cssa, casy);
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        R rb, rd, tb, td, ld;
-        layer_rt_eval<R>(T, tr[g], tg[g], (R)ta, (R)sa, (R)ya, true, ctau, cssa, casy, cz, snt, rb, rd, tb, td, ld);
-        o.rb[g] = zc0 * o.rb[g] + zc1 * rb;
-        o.rd[g] = zc0 * o.rd[g] + zc1 * rd;
-        o.tb[g] = zc0 * o.tb[g] + zc1 * tb;
-        o.td[g] = zc0 * o.td[g] + zc1 * td;
-        o.ld[g] = zc0 * o.ld[g] + zc1 * ld;
-    }
-}
-
-// One day column of one SW band on the NAM route: clear-sky pass, then (cloudy columns) the
-// total-sky pass; each pass is the bottom-up adding sweep (level reflectances to the lane cache) and
-// the top-down sweep with the layer R/T recomputed.
+// One day column of one SW band on the NAM route: clear-sky pass, then (cloudy columns) the total-sky pass,
+// whose layers mix the cloudy R/T with the clear ones by the layer's cloud fraction over the column's
+// cover, zc1 = cfrac / zcf1 (phys_rrtm_sw_spcvrtc.cu, cloudy block); each pass is the adding method.
 template <typename R, int B, typename BT>
 __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par, int col0,
-                                           int n, const ColScal &cs, const R *__restrict__ sflux, const AccT<R> &acc, int t,
-                                           const LaneCache<R> &cc)
+                                           int n, const ColScal &cs, const RecPtrs &rp, const R *__restrict__ sflux,
+                                           const AccT<R> &acc, int blk, int lane, WR_G char *slot, Fix64 *fx)
 {
-    constexpr bool CACHE_RT = sw_nv_mc<R>() > SW_NV;  // FP32: layer R/T kept for the top-down sweep
-    constexpr int NG = SW_NG[B];
-    constexpr int NS = SW_NS[B];
-    const int i = col0 + t;
-    const RadCol rc{in, i, in.nlay + 1};
-    const int nrl = rc.nrl, nlp1 = nrl + 1;
-    const double czd = in.cosz[i];
-    const R cz = (R)czd, snt = (R)(1.0 / czd);
-    const double ssolar = (par.solcon / S0) * czd;
-    const double alb = in.alb[i];
-    const R asfc = (R)((SW_IDXSFC[B] != 0) ? alb : 0.5 * (alb + alb));
+    constexpr int NG = SW_NG[B], CH = sw_chunk<R, B, true>();
+    if (blk * 64 + lane >= *cs.nday) return;
+    const int t = cs.dlist[blk * 64 + lane], nrl = rp.nrl;
+    SwCol<R> c;
+    sw_col<R, B>(in, par, col0, cs, t, c);
+    const RadCol rcol{in, c.i, nrl};
     const double cf1 = cs.zcf1[t], cf0 = cs.zcf0[t];
     const bool total = cf1 > EPS;
-    const int lt = cs.sw_laytrop[t];
-    R zsolar[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) zsolar[g] = (R)ssolar * sflux[(size_t)(NS + g) * n + t];
-
+    const Surr none{};
+    struct Lay {
+        SwLayer<R> y;
+        R zc1, zc0;
+        bool mix;
+    };
     for (int pass = 0; pass < (total ? 2 : 1); ++pass) {
-        // bottom-up (swflux sweep 1); zrupb/zrupd of level L (surface L = 1) at cache entry L - 1,
-        // the latest level also in pb/pd
-        R pb[NG], pd[NG];
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            pb[g] = asfc, pd[g] = asfc;
-            cc.at(0, NG, g, 0) = asfc;
-            cc.at(1, NG, g, 0) = asfc;
-        }
-        for (int k = 0; k < nrl; ++k) {
-            SwLayerRT<R, B> o;
-            swr_layer<R, B>(T, Bt, rc, par, k, lt, pass, cf1, cz, snt, o, cs.la[(size_t)(nrl - 1 - k) * n + t]);
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                const R zden1 = (R)1 / ((R)1 - pd[g] * o.rd[g]);
-                const R nb = o.rb[g] + (o.td[g] * ((o.tb[g] - o.ld[g]) * pd[g] + o.ld[g] * pb[g])) * zden1;
-                const R nd = o.rd[g] + o.td[g] * o.td[g] * pd[g] * zden1;
-                pb[g] = nb, pd[g] = nd;
-                cc.at(0, NG, g, k + 1) = nb;
-                cc.at(1, NG, g, k + 1) = nd;
-                if constexpr (CACHE_RT) {
-                    cc.at(2, NG, g, k) = o.rb[g];
-                    cc.at(3, NG, g, k) = o.rd[g];
-                    cc.at(4, NG, g, k) = o.tb[g];
-                    cc.at(5, NG, g, k) = o.td[g];
-                    cc.at(6, NG, g, k) = o.ld[g];
+        sw_adding<R, NG, CH>(
+            nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2},
+            [&](int k) {
+                Lay a;
+                sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, lane, k, a.y);
+                a.mix = false, a.zc1 = (R)0, a.zc0 = (R)1;
+                if (pass && __any(a.y.cloudy)) {
+                    const double zc1 = rcol.cfrac(nrl - 1 - k) / cf1;
+                    a.mix = zc1 > FTINY, a.zc1 = (R)zc1, a.zc0 = (R)(1.0 - zc1);
                 }
-            }
-        }
-        // top-down and level fluxes (layer R/T recomputed); pass 0 leaves the clear-sky fluxes in the
-        // band planes, which pass 1 reads back and mixes with the cloudy ones
-        R tdbt[NG], tdn[NG], rdnd[NG];
-        R su = (R)0, sd = (R)0;
+                return a;
+            },
+            [&](const Lay &a, int k, int g0, RtV<R, CH> &o) {
+                R tg[CH], tr[CH];
+                sw_tgtr<R, B, false, CH>(T, Bt, none, 1, 0, k, c.lt, a.y.L, g0, tg, tr);
+                layer_rt_sky<R, CH>(T, tr, tg, a.y.y, 0u, o, fx);
+                if (__any(a.mix)) {
+                    RtV<R, CH> d;
+                    layer_rt_sky<R, CH>(T, tr, tg, a.y.y, ~0u, d, fx);
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0;
-            const R zden1 = (R)1 / ((R)1 - rdnd[g] * pd[g]);
-            const R zfu = (tdbt[g] * pb[g] + (tdn[g] - tdbt[g]) * pd[g]) * zden1;
-            const R zfd = tdbt[g] + (tdn[g] - tdbt[g] + tdbt[g] * pb[g] * rdnd[g]) * zden1;
-            su = su + zsolar[g] * zfu;
-            sd = sd + zsolar[g] * zfd;
-        }
-        for (int s = nrl; s >= 0; --s) {
-            if (s < nrl) {
-                SwLayerRT<R, B> o;
-                if constexpr (CACHE_RT) {
-#pragma unroll
-                    for (int g = 0; g < NG; ++g) {
-                        o.rb[g] = cc.at(2, NG, g, s), o.rd[g] = cc.at(3, NG, g, s), o.tb[g] = cc.at(4, NG, g, s);
-                        o.td[g] = cc.at(5, NG, g, s), o.ld[g] = cc.at(6, NG, g, s);
+                    for (int j = 0; j < CH; ++j) {
+                        o.rb[j] = a.mix ? a.zc0 * o.rb[j] + a.zc1 * d.rb[j] : o.rb[j];
+                        o.rd[j] = a.mix ? a.zc0 * o.rd[j] + a.zc1 * d.rd[j] : o.rd[j];
+                        o.tb[j] = a.mix ? a.zc0 * o.tb[j] + a.zc1 * d.tb[j] : o.tb[j];
+                        o.td[j] = a.mix ? a.zc0 * o.td[j] + a.zc1 * d.td[j] : o.td[j];
+                        o.ld[j] = a.mix ? a.zc0 * o.ld[j] + a.zc1 * d.ld[j] : o.ld[j];
                     }
+                }
+            },
+            [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
+            [&](int lev, R su, R sd) {
+                // pass 0 leaves the clear-sky fluxes in the band planes, which pass 1 reads back and mixes
+                const size_t p = (size_t)lev * n + t;
+                if (pass == 0) {
+                    if (lev == 0) acc.sw_clr0[t] = sd;
+                    acc.sw_up[p] = su;
+                    acc.sw_dn[p] = sd;
                 } else {
-                    swr_layer<R, B>(T, Bt, rc, par, s, lt, pass, cf1, cz, snt, o, cs.la[(size_t)(nrl - 1 - s) * n + t]);
+                    acc.sw_up[p] = (R)(cf1 * (double)su + cf0 * (double)acc.sw_up[p]);
+                    acc.sw_dn[p] = (R)(cf1 * (double)sd + cf0 * (double)acc.sw_dn[p]);
                 }
-                su = (R)0, sd = (R)0;
-#pragma unroll
-                for (int g = 0; g < NG; ++g) {
-                    const R tdbt_s = o.ld[g] * tdbt[g];
-                    R tdn_s, rdnd_s;
-                    if (s == nrl - 1) {
-                        tdn_s = o.tb[g];
-                        rdnd_s = o.rd[g];
-                    } else {
-                        const R zden1 = (R)1 / ((R)1 - o.rd[g] * rdnd[g]);
-                        tdn_s = tdbt[g] * o.tb[g] + (o.td[g] * ((tdn[g] - tdbt[g]) + tdbt[g] * o.rb[g] * rdnd[g])) * zden1;
-                        rdnd_s = o.rd[g] + o.td[g] * o.td[g] * rdnd[g] * zden1;
-                    }
-                    tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
-                    const R zb = cc.at(0, NG, g, s), zd = cc.at(1, NG, g, s);  // level s + 1
-                    const R zden1 = (R)1 / ((R)1 - rdnd_s * zd);
-                    const R zfu = (tdbt_s * zb + (tdn_s - tdbt_s) * zd) * zden1;
-                    const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * zb * rdnd_s) * zden1;
-                    su = su + zsolar[g] * zfu;
-                    sd = sd + zsolar[g] * zfd;
-                }
-            }
-            const size_t o = (size_t)s * n + t;  // level s (surface-first)
-            if (pass == 0 && s == 0) acc.sw_clr0[t] = sd;
-            if (pass == 0) {
-                acc.sw_up[o] = su;
-                acc.sw_dn[o] = sd;
-            } else {
-                acc.sw_up[o] = (R)(cf1 * (double)su + cf0 * (double)acc.sw_up[o]);
-                acc.sw_dn[o] = (R)(cf1 * (double)sd + cf0 * (double)acc.sw_dn[o]);
-            }
-        }
+            });
     }
 }
 
 // SW band kernel of the NAM route: blocks of 64 day-list entries looped over a pool-sized grid.
 template <typename R, int B, bool EXT = true>
 __global__ void __launch_bounds__(64, (sw_waves<R, B, true>())) k_swr(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
-                                            int n, ColScal cs, const R *__restrict__ sflux, AccT<R> acc,
+                                            int n, ColScal cs, RecPtrs rp, const R *__restrict__ sflux, AccT<R> acc,
                                             char *__restrict__ pool)
 {
+    __shared__ Fix64 fx[1];
     const ColIn in = band_in<EXT>(in_);
-    const LaneCache<R> cc = lane_cache<R>(pool, sw_nv_mc<R>(), SW_NG[B], in.nlay + 2);
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
-    for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x) {
-        const int tt = blk * 64 + threadIdx.x;
-        if (tt < nday) swr_column<R, B>(T, T->sw[B], in, par, col0, n, cs, sflux, acc, cs.dlist[tt], cc);
-    }
+    for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x)
+        swr_column<R, B>(T, T->sw[B], in, par, col0, n, cs, rp, sflux, acc, blk, (int)threadIdx.x, slot, fx);
 }
 
 // k_swr with the band's tables in LDS (the images of k_swl): persistent workgroups of 4 x the band's
@@ -577,23 +401,20 @@ __global__ void __launch_bounds__(64, (sw_waves<R, B, true>())) k_swr(const Tabs
 template <typename R, int B> constexpr int swrl_wpg() { return 4 * sw_waves<R, B, true>(); }
 template <typename R, int B, bool EXT = true>
 __global__ void __launch_bounds__((64 * swrl_wpg<R, B>()), (sw_waves<R, B, true>()))
-    k_swrl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, const R *__restrict__ sflux,
-           AccT<R> acc, char *__restrict__ pool)
+    k_swrl(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp,
+           const R *__restrict__ sflux, AccT<R> acc, char *__restrict__ pool)
 {
     extern __shared__ float4 swrl_tab[];
     const ColIn in = band_in<EXT>(in_);
     lds_fill<R>(swrl_tab, T->sw_img[B]);
     const auto Bl = sw_lds_band<R>((const WR_L R *)swrl_tab, T->sw_img[B], T->sw[B]);
     constexpr int WPG = swrl_wpg<R, B>();
-    const int lane = threadIdx.x % 64, slot = blockIdx.x * WPG + threadIdx.x / 64;
-    LaneCache<R> cc;
-    cc.p = (WR_G R *)(pool + (size_t)slot * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R))) + lane;
-    cc.nv = sw_nv_mc<R>();
+    __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
+    const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
-    for (int blk = slot; blk * 64 < nday; blk += gridDim.x * WPG) {
-        const int tt = blk * 64 + lane;
-        if (tt < nday) swr_column<R, B>(T, Bl, in, par, col0, n, cs, sflux, acc, cs.dlist[tt], cc);
-    }
+    for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)
+        swr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, sflux, acc, blk, lane, slot, fx + (sizeof(R) == 4 ? wv : 0));
 }
 
 }  // namespace wr

@@ -4,7 +4,7 @@
 // sw_optics: taumol16..29 (phys_rrtm_sw_taumolNN.cu), the MINVAL(laytrop) group of bands
 //            19/23/25/28 taken per column (one-column groups), so columns are independent.
 // sw_cloud:  cldprop (phys_rrtm_sw_cldprop.cu:76), iswcliq = 1, iswcice = 3.
-// layer_rt:  delta scaling, PIFM (iswmode 2) and swc_layer_rt (phys_rrtm_sw_spcvrtc.cu:112-173).
+// (the layer's two-stream solution is in wr_kernels.h)
 #pragma once
 #include "wr_dev.h"
 
@@ -129,11 +129,11 @@ template <typename R> __device__ __forceinline__ int jsfs(R specmult, R &fs)
     return 1 + jsi;
 }
 
-// gas (tg) and Rayleigh (tr) optical depths of band B (index 0..13 = bands 16..29), layer kk (1-based),
-// from the band tables Bt (global or staged in LDS)
-template <typename R, int B, typename BT>
+// gas (tg) and Rayleigh (tr) optical depths of g-points g0 .. g0 + NGL - 1 of band B (index 0..13 = bands
+// 16..29), layer kk (1-based), from the band tables Bt (global or staged in LDS)
+template <typename R, int B, int NGL, typename BT>
 __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const BT &Bt, const SwLay<R> &L, int kk, int Lt,
-                                            R *tg, R *tr)
+                                            R *tg, R *tr, int g0)
 {
     constexpr int ng = SW_NG[B];
     const int jp = L.jp, jt = L.jt, jt1 = L.jt1;
@@ -156,87 +156,87 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
     int id[8];
     R fs;
     if constexpr (B == 0) { /* band 16 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[4];
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (sf * SELFI(g) + ff * FORI(g));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         }
         if (kk >= Lt)
-            for (int g = 0; g < ng; ++g) tg[g] = ca[4] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[4] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11);
     } else if constexpr (B == 1) { /* band 17 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * (R)6.86e-10;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)6.86e-10;
         const R speccomb = ca[0] + Bt.strrat * ca[1];
         if (kk <= Lt) {
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(((jp - 1) * 5 + (jt - 1)) * 9, (jp * 5 + (jt1 - 1)) * 9, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) {
-                const R forpart = FORI(g);
-                const R selfpart = (inds > 0) ? sf * SELFI(g) : (R)0;
-                tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (selfpart + ff * forpart);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                const R forpart = FORI(g0 + jj);
+                const R selfpart = (inds > 0) ? sf * SELFI(g0 + jj) : (R)0;
+                tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (selfpart + ff * forpart);
             }
         } else {
             const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(((jp - 13) * 5 + (jt - 1)) * 5, ((jp - 12) * 5 + (jt1 - 1)) * 5, js, 1175, 5, 6, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absb, ng, g, id, fc) + (ca[0] * ff) * FORI(g);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc) + (ca[0] * ff) * FORI(g0 + jj);
         }
     } else if constexpr (B == 2) { /* band 18 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[4];
             const R ratio = (speccomb > (R)0) ? (ca[0] / speccomb) : (R)0;
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ratio), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (sf * SELFI(g) + ff * FORI(g));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         } else {
-            for (int g = 0; g < ng; ++g) tg[g] = ca[4] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[4] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11);
         }
     } else if constexpr (B == 3) { /* band 19 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * (R)2.29e-09;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)2.29e-09;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[1];
             const int js = jsfs<R>((R)8 * fmin((R)0.999999, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (sf * SELFI(g) + ff * FORI(g));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         } else {
-            for (int g = 0; g < ng; ++g) tg[g] = ca[1] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[1] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11);
         }
     } else if constexpr (B == 4) { /* band 20 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         if (kk <= Lt) {
-            for (int g = 0; g < ng; ++g) {
-                const R absterm = abs4<R>(Bt.absa, ng, g, id0, id1, 65, f00, f01, f10, f11);
-                tg[g] = ca[0] * ((absterm) + sf * (SELFI(g)) + ff * (FORI(g))) + ca[4] * Bt.absch4[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                const R absterm = abs4<R>(Bt.absa, ng, g0 + jj, id0, id1, 65, f00, f01, f10, f11);
+                tg[jj] = ca[0] * ((absterm) + sf * (SELFI(g0 + jj)) + ff * (FORI(g0 + jj))) + ca[4] * Bt.absch4[g0 + jj];
             }
         } else {
-            for (int g = 0; g < ng; ++g) {
-                const R absterm = abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11);
-                tg[g] = ca[0] * ((absterm) + ff * (FORI(g))) + ca[4] * Bt.absch4[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                const R absterm = abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11);
+                tg[jj] = ca[0] * ((absterm) + ff * (FORI(g0 + jj))) + ca[4] * Bt.absch4[g0 + jj];
             }
         }
     } else if constexpr (B == 5) { /* band 21 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * (R)9.41e-09;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)9.41e-09;
         const R speccomb = ca[0] + Bt.strrat * ca[1];
         if (kk < Lt) {
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (sf * SELFI(g) + ff * FORI(g));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         }
         if (kk >= Lt) {
             const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 1175, 5, 6, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absb, ng, g, id, fc) + ca[0] * ff * FORI(g);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc) + ca[0] * ff * FORI(g0 + jj);
         }
     } else if constexpr (B == 6) { /* band 22 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * (R)1.54e-08;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)1.54e-08;
         const R o2cont = (R)(4.35e-4 / (350.0 * 2.0)) * ca[5];
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[5];
@@ -244,18 +244,18 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ratio), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g)
-                tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[0] * (sf * SELFI(g) + ff * FORI(g)) + o2cont;
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj)
+                tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj)) + o2cont;
         } else {
-            for (int g = 0; g < ng; ++g) tg[g] = ca[5] * (R)1.6 * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11) + o2cont;
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[5] * (R)1.6 * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11) + o2cont;
         }
     } else if constexpr (B == 7) { /* band 23 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl_v[g];
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl_v[g0 + jj];
         if (kk <= Lt) {
-            for (int g = 0; g < ng; ++g)
-                tg[g] = ca[0] * ((R)1.029 * abs4<R>(Bt.absa, ng, g, id0, id1, 65, f00, f01, f10, f11) + sf * SELFI(g) + ff * FORI(g));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj)
+                tg[jj] = ca[0] * ((R)1.029 * abs4<R>(Bt.absa, ng, g0 + jj, id0, id1, 65, f00, f01, f10, f11) + sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         } else {
-            for (int g = 0; g < ng; ++g) tg[g] = (R)0;
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = (R)0;
         }
     } else if constexpr (B == 8) { /* band 24 */
         if (kk <= Lt) {
@@ -263,59 +263,59 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) {
-                tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc) + ca[2] * Bt.abso3a[g] + ca[0] * (sf * SELFI(g) + ff * FORI(g));
-                const R ray0 = Bt.rayla[(js - 1) * 8 + g], ray1 = Bt.rayla[js * 8 + g];
-                tr[g] = cm * (ray0 + fs * (ray1 - ray0));
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[2] * Bt.abso3a[g0 + jj] + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
+                const R ray0 = Bt.rayla[(js - 1) * 8 + g0 + jj], ray1 = Bt.rayla[js * 8 + g0 + jj];
+                tr[jj] = cm * (ray0 + fs * (ray1 - ray0));
             }
         } else {
-            for (int g = 0; g < ng; ++g) {
-                tg[g] = ca[5] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11) + ca[2] * Bt.abso3b[g];
-                tr[g] = cm * Bt.raylb[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                tg[jj] = ca[5] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11) + ca[2] * Bt.abso3b[g0 + jj];
+                tr[jj] = cm * Bt.raylb[g0 + jj];
             }
         }
     } else if constexpr (B == 9) { /* band 25 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl_v[g];
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl_v[g0 + jj];
         if (kk <= Lt) {
-            for (int g = 0; g < ng; ++g)
-                tg[g] = ca[0] * abs4<R>(Bt.absa, ng, g, id0, id1, 65, f00, f01, f10, f11) + ca[2] * Bt.abso3a[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj)
+                tg[jj] = ca[0] * abs4<R>(Bt.absa, ng, g0 + jj, id0, id1, 65, f00, f01, f10, f11) + ca[2] * Bt.abso3a[g0 + jj];
         } else {
-            for (int g = 0; g < ng; ++g) tg[g] = ca[2] * Bt.abso3b[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[2] * Bt.abso3b[g0 + jj];
         }
     } else if constexpr (B == 10) { /* band 26 */
-        for (int g = 0; g < ng; ++g) tg[g] = (R)0, tr[g] = cm * Bt.rayl_v[g];
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = (R)0, tr[jj] = cm * Bt.rayl_v[g0 + jj];
     } else if constexpr (B == 11) { /* band 27 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl_v[g];
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl_v[g0 + jj];
         if (kk < Lt)
-            for (int g = 0; g < ng; ++g) tg[g] = ca[2] * abs4<R>(Bt.absa, ng, g, id0, id1, 65, f00, f01, f10, f11);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[2] * abs4<R>(Bt.absa, ng, g0 + jj, id0, id1, 65, f00, f01, f10, f11);
         if (kk >= Lt)
-            for (int g = 0; g < ng; ++g) tg[g] = ca[2] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = ca[2] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11);
     } else if constexpr (B == 12) { /* band 28 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * Bt.rayl;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         const R speccomb = ca[2] + Bt.strrat * ca[5];
         if (kk <= Lt) {
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[2] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absa, ng, g, id, fc);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc);
         } else {
             const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[2] / speccomb), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 1175, 5, 6, id);
-            for (int g = 0; g < ng; ++g) tg[g] = speccomb * sum8<R>(Bt.absb, ng, g, id, fc);
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc);
         }
     } else if constexpr (B == 13) { /* band 29 */
-        for (int g = 0; g < ng; ++g) tr[g] = cm * (R)9.30e-11;
+        _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)9.30e-11;
         if (kk <= Lt) {
             const int isp = imin(inds + 1, 10), ifp = imin(indf + 1, 4);
-            for (int g = 0; g < ng; ++g) {
-                const R selfv = S2(Bt.selfref, inds, g, ng) + sfr * (S2(Bt.selfref, isp, g, ng) - S2(Bt.selfref, inds, g, ng));
-                const R forv = S2(Bt.forref, indf, g, ng) + ffr * (S2(Bt.forref, ifp, g, ng) - S2(Bt.forref, indf, g, ng));
-                tg[g] = ca[0] * ((abs4<R>(Bt.absa, ng, g, id0, id1, 65, f00, f01, f10, f11)) + sf * selfv + ff * forv) + ca[1] * Bt.absco2[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
+                const R selfv = S2(Bt.selfref, inds, g0 + jj, ng) + sfr * (S2(Bt.selfref, isp, g0 + jj, ng) - S2(Bt.selfref, inds, g0 + jj, ng));
+                const R forv = S2(Bt.forref, indf, g0 + jj, ng) + ffr * (S2(Bt.forref, ifp, g0 + jj, ng) - S2(Bt.forref, indf, g0 + jj, ng));
+                tg[jj] = ca[0] * ((abs4<R>(Bt.absa, ng, g0 + jj, id0, id1, 65, f00, f01, f10, f11)) + sf * selfv + ff * forv) + ca[1] * Bt.absco2[g0 + jj];
             }
         } else {
-            for (int g = 0; g < ng; ++g)
-                tg[g] = ca[1] * abs4<R>(Bt.absb, ng, g, id0, id1, 235, f00, f01, f10, f11) + ca[0] * Bt.absh2o[g];
+            _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj)
+                tg[jj] = ca[1] * abs4<R>(Bt.absb, ng, g0 + jj, id0, id1, 235, f00, f01, f10, f11) + ca[0] * Bt.absh2o[g0 + jj];
         }
     }
 #undef SELFI
@@ -325,7 +325,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
 template <typename R, int B>
 __device__ __forceinline__ void sw_optics(const Tabs<R> *__restrict__ T, const SwLay<R> &L, int kk, int Lt, R *tg, R *tr)
 {
-    sw_optics_t<R, B>(T, T->sw[B], L, kk, Lt, tg, tr);
+    sw_optics_t<R, B, SW_NG[B]>(T, T->sw[B], L, kk, Lt, tg, tr, 0);
 }
 
 // cloud optical properties of band B for one layer (taucw, ssacw = tau*ssa, asycw = tau*ssa*g)
@@ -378,85 +378,6 @@ __device__ __forceinline__ void sw_cloud_l(const Tabs<R> *__restrict__ T, int B,
     double rl, ri, rp;
     rc.props(kin, par.re_liq, par.re_ice, rl, ri, rp);
     sw_cloud<R>(T, B, L.cwp, rl, L.cip, ri, tau, ssa, asy, rp);
-}
-
-template <typename R> __device__ __forceinline__ R expm(R zb, const WR_G R *__restrict__ tbl)
-{
-    if (zb <= (R)0.06) return (R)1 - zb + (R)0.5 * zb * zb;
-    const R ftind = zb / ((R)(1.0 / 0.278) + zb);
-    const int itind = imax(0, imin(10000, (int)((R)0.5 + (R)10000 * ftind)));
-    if constexpr (sizeof(R) == 4) return lut_f32(itind, false).e;
-    return tbl[itind];
-}
-
-// delta scaling + PIFM + layer R/T (zssaw < zcrit branch; the conservative branch is unreachable
-// behind the 1 - 1e-6 clamp of zssaw, phys_rrtm_sw_spcvrtc.cu:54,117)
-template <typename R>
-__device__ __forceinline__ void layer_rt(R ztau0, R zssa0, R zasy0, R cz, R snt, const WR_G R *__restrict__ tbl, R &rb, R &rd,
-                                         R &tb, R &td, R &zldbt, bool *ill = nullptr)
-{
-    const R zssaw = fmin((R)ONEMINUS, zssa0 / ztau0);
-    const R zasyw = zasy0 / fmax((R)FTINY, zssa0);
-    const R za1s = zasyw * zasyw;
-    const R za2s = zssaw * za1s;
-    const R ztau1 = ((R)1 - za2s) * ztau0;
-    const R zssa1 = (zssaw - za2s) / ((R)1 - za2s);
-    const R zasy1 = zasyw / ((R)1 + zasyw);
-    const R zasy3 = (R)0.75 * zasy1;
-    const R zgam1 = (R)2 - zssa1 * ((R)1.25 + zasy3);
-    const R zgam2 = (R)0.75 * zssa1 * ((R)1 - zasy1);
-    const R zgam3 = (R)0.5 - zasy3 * cz;
-    const R zgam4 = (R)1 - zgam3;
-    const R eps1 = (R)1.0e-8;
-    const R za1 = zgam1 * zgam4 + zgam2 * zgam3;
-    const R za2 = zgam1 * zgam3 + zgam2 * zgam4;
-    const R zrk = sqrt((zgam1 - zgam2) * (zgam1 + zgam2));
-    const R zrk2 = (R)2 * zrk;
-    const R zrp = zrk * cz;
-    const R zrp1 = (R)1 + zrp;
-    const R zrm1 = (R)1 - zrp;
-    R zrpp = (R)1 - zrp * zrp;
-    // FP32 near the two-stream singularity k mu = 1: numerator and denominator of the direct-beam
-    // terms both vanish there, so the caller re-evaluates the layer in FP64
-    if (ill && fabs(zrpp) < (R)1.0e-2) {
-        *ill = true;
-        return;
-    }
-    if (fabs(zrpp) < eps1) zrpp = (zrpp < (R)0) ? -eps1 : eps1;
-    const R zrkg1 = zrk + zgam1;
-    const R zrkg3 = zrk * zgam3;
-    const R zrkg4 = zrk * zgam4;
-    const R zr1 = zrm1 * (za2 + zrkg3);
-    const R zr2 = zrp1 * (za2 - zrkg3);
-    const R zr3 = zrk2 * (zgam3 - za2 * cz);
-    const R zr4 = zrpp * zrkg1;
-    const R zr5 = zrpp * (zrk - zgam1);
-    const R zt1 = zrp1 * (za1 + zrkg4);
-    const R zt2 = zrm1 * (za1 - zrkg4);
-    const R zt3 = zrk2 * (zgam4 + za1 * cz);
-    // FP32: cap the exponents at 80 so exp(-zb) stays a normal number and 1/exp(-zb) finite (the
-    // FP32 table underflows to 0 past about 103); the R/T expressions depend on the capped terms
-    // only through factors below exp(-160)
-    const R zcap = (sizeof(R) < sizeof(double)) ? (R)80 : (R)500;
-    const R zb1 = fmin(zrk * ztau1, zcap);
-    const R zexm1 = expm<R>(zb1, tbl);
-    const R zexp1 = (R)1 / zexm1;
-    const R zb2 = fmin(ztau1 * snt, zcap);
-    const R zexm2 = expm<R>(zb2, tbl);
-    const R zexp2 = (R)1 / zexm2;
-    const R ze1r45 = zr4 * zexp1 + zr5 * zexm1;
-    if (ze1r45 >= -eps1 && ze1r45 <= eps1) {
-        rb = eps1;
-        tb = zexm2;
-    } else {
-        const R zden1 = zssa1 / ze1r45;
-        rb = fmax((R)0, fmin((R)1, (zr1 * zexp1 - zr2 * zexm1 - zr3 * zexm2) * zden1));
-        tb = fmax((R)0, fmin((R)1, zexm2 * ((R)1 - (zt1 * zexp1 - zt2 * zexm1 - zt3 * zexp2) * zden1)));
-    }
-    const R zden1d = zr4 / (ze1r45 * zrkg1);
-    rd = fmax((R)0, fmin((R)1, zgam2 * (zexp1 - zexm1) * zden1d));
-    td = fmax((R)0, fmin((R)1, zrk2 * zden1d));
-    zldbt = expm<R>(ztau1 * snt, tbl);
 }
 
 }  // namespace wr
