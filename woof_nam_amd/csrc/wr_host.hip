@@ -544,15 +544,15 @@ int many_cols_env()
     const char *e = getenv("WR_MANY_COLS");
     return e ? std::max(0, atoi(e)) : MANY_COLS_DEFAULT;
 }
-constexpr size_t MANY_BLOCK = std::max(many_block_bytes<double, false>(64 + 1), many_block_bytes<float, false>(64 + 1));
+constexpr size_t MANY_BLOCK = std::max(many_block_bytes<double, false>(64), many_block_bytes<double, true>(64));
 
 // Device bytes of a context's tile work space for tiles of m columns, and the band-stream count.
 struct Sizes {
-    size_t acc, iws, dws, rtr, sflux_d, sflux_f, rec, lwrec, pool, pool_all;
+    size_t acc, iws, dws, rtr, sflux, rec, lwrec, pool, pool_all;
     int naux;
     size_t total() const
     {
-        return acc + iws + dws + rtr + sflux_d + sflux_f + rec + lwrec + pool_all;
+        return acc + iws + dws + rtr + sflux + rec + lwrec + pool_all;
     }
 };
 Sizes sizes(int32_t max_cols)
@@ -560,21 +560,23 @@ Sizes sizes(int32_t max_cols)
     const size_t m = (size_t)max_cols;
     Sizes z;
     z.acc = sizeof(double) * (60 * (NL + 1) + 14) * m;                        // band flux planes
-    z.iws = sizeof(int) * 7 * m;                                              // 6 column words + day-list segments
+    z.iws = sizeof(int) * 8 * m;                                              // column words, day-list segments
     z.dws = sizeof(double) * (4 + 2 * (size_t)NL) * m;                        // column words, layer logs, tz
-    z.rtr = (sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m;      // NAM-route overlap factors
-    z.sflux_d = sizeof(double) * 112 * m;
-    z.sflux_f = sizeof(float) * 112 * m;
-    z.rec = rec_block_bytes((int)sizeof(double)) * 64 * ((m + 63) / 64);     // layer records, up to 64 layers
+    const size_t rows = (m + 63) / 64 * 64;                                   // record rows: blocks x up to 64 layers
+    // NAM-route overlap factors, or the McICA route's words
+    z.rtr = std::max((sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m, rows * mrow_bytes());
+    z.sflux = sizeof(double) * 112 * m;
+    z.rec = std::max(rec_row_bytes(8), rec_row_bytes(4)) * rows;              // layer records
     z.lwrec = lw_glane_env() ? lwrec_bytes_per_col<double>(64 + 1) * m + 3 * 256 : 0;  // LW layer records
     // level pool: room for every 64-column block of a tile in the largest slot layout (FP64 SW:
-    // 2 values, FP32 SW: 7 values, x 16 g x levels), at most WR_POOL_GB (default 6) GB per stream
+    // 2 values, FP32 SW: 7 values, x 16 g x levels), at most WR_POOL_GB (default 3) GB per stream:
+    // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB
     const int nl_max = 64;
     const size_t lane_max = std::max(cache_slot_bytes(SW_NV, 16, nl_max + 1, (int)sizeof(double)),
                                      cache_slot_bytes(sw_nv_mc<float>(), 16, nl_max + 1, (int)sizeof(float)));
     const size_t need = (m + 63) / 64 * lane_max;
     const char *pe = getenv("WR_POOL_GB");
-    const double gb = pe ? atof(pe) : 6.0;
+    const double gb = pe ? atof(pe) : 3.0;
     size_t cap = (size_t)(gb * 1e9);
     if (cap < lane_max) cap = lane_max;
     z.pool = need < cap ? need : cap;
@@ -607,17 +609,17 @@ constexpr NaLayout na_layout()
     NaLayout z{};
     size_t off = 0;
     z.acc = off, off += na_al(sizeof(float) * (60 * (NL + 1) + 14) * m);
-    z.iws = off, off += na_al(sizeof(int) * 7 * m);
+    z.iws = off, off += na_al(sizeof(int) * 8 * m);
     z.dws = off, off += na_al(sizeof(double) * (4 + 2 * (size_t)NL) * m);
-    z.rtr = off, off += na_al((sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m);
+    z.rtr = off, off += na_al(std::max((sizeof(double) * 12 * (NL + 3) + 2 * sizeof(uint64_t)) * m, m * mrow_bytes()));
     z.sflux = off, off += na_al(sizeof(float) * 112 * m);
-    z.rec = off, off += na_al(rec_block_bytes((int)sizeof(float)) * 64 * ((m + 63) / 64));
-    z.pool = off, off += NA_BLOCKS * many_block_bytes<float, false>(64 + 1);
+    z.rec = off, off += na_al(rec_row_bytes((int)sizeof(float)) * m);
+    z.pool = off, off += NA_BLOCKS * many_block_bytes<float, false>(64);
     z.total = off;
     return z;
 }
 constexpr NaLayout NA = na_layout();
-static_assert(NA.total <= ((size_t)448 << 20), "the no-alloc work space stays under 448 MiB");
+static_assert(NA.total <= ((size_t)512 << 20), "the no-alloc work space stays under 512 MiB");
 
 static __device__ __align__(256) char scratch[NA.total];
 
@@ -681,10 +683,10 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
     if (rc == WR_OK) {
         if (hipMalloc((void **)&c->acc, z.acc) != hipSuccess || hipMalloc((void **)&c->iws, z.iws) != hipSuccess ||
             hipMalloc((void **)&c->dws, z.dws) != hipSuccess || hipMalloc(&c->rtr, z.rtr) != hipSuccess ||
-            hipMalloc((void **)&c->sflux_d, z.sflux_d) != hipSuccess ||
-            hipMalloc((void **)&c->sflux_f, z.sflux_f) != hipSuccess ||
+            hipMalloc((void **)&c->sflux_d, z.sflux) != hipSuccess ||
             hipMalloc((void **)&c->rec, z.rec) != hipSuccess || (z.lwrec && hipMalloc(&c->lwrec, z.lwrec) != hipSuccess))
             rc = WR_ERR_NOMEM;
+        c->sflux_f = (float *)c->sflux_d;
         c->lw_glane = z.lwrec > 0;
         if (hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
             hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
@@ -719,6 +721,7 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
     }
     if (rc == WR_OK && hipDeviceSynchronize() != hipSuccess) rc = WR_ERR_HIP;
     if (rc != WR_OK) {
+        (void)hipGetLastError();  // a failed allocation is reported here, not by the next launch's check
         wr_destroy(c);
         return rc;
     }
@@ -935,7 +938,6 @@ void wr_destroy(wr_ctx *c)
     (void)hipFree(c->dws);
     (void)hipFree(c->rtr);
     (void)hipFree(c->sflux_d);
-    (void)hipFree(c->sflux_f);
     (void)hipFree(c->rec);
     (void)hipFree(c->lwrec);
     (void)hipFree(c->sx);

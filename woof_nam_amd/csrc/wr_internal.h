@@ -21,12 +21,12 @@ struct wr_ctx {
     wr::Tabs<float> host_f;
     // tile work space
     double *acc;                     // band flux planes: 60 x [NL + 1][max_cols] + 14 x [max_cols]
-    int *iws;                        // 7 x [max_cols]: 6 column words, then day-list segment counts
+    int *iws;                        // 8 x [max_cols]: 6 column words, day-list segment counts, cloud blocks
     double *dws;                     // (4 + 2 NL) x [max_cols]: 3 column words, layer logs, level temperatures
-    void *rtr;                       // maximum-random overlap factors of the NAM LW route
-    double *sflux_d;                 // [112][max_cols]
-    float *sflux_f;
-    char *rec;                       // layer records and McICA words of a tile (wr_rec.h), sized for FP64
+    void *rtr;                       // NAM route: maximum-random overlap factors; McICA route: McICA words
+    double *sflux_d;                 // [112][max_cols] solar source
+    float *sflux_f;                  // the same space for the FP32 kernels
+    char *rec;                       // layer records of a tile (wr_rec.h), sized for FP64
     void *lwrec;                     // LW layer records of a tile (g-lane LW kernels), sized for FP64
     int lw_glane;                    // 1: McICA LW bands as g-lane kernels over the layer records
     uint32_t lw_lds;                 // bit B: the FP32 McICA kernel of LW band B + 1 stages its tables in LDS
@@ -105,6 +105,7 @@ inline ColScal colscal(wr_ctx *c)
     s.sw_laytrop = gptr(c->iws + 3 * m);
     s.dlist = gptr(c->iws + 4 * m);
     s.nday = gptr(c->iws + 5 * m);
+    s.cblk = gptr((uint32_t *)(c->iws + 7 * m));
     s.pwv = gptr(c->dws + 0 * m);
     s.zcf1 = gptr(c->dws + 1 * m);
     s.zcf0 = gptr(c->dws + 2 * m);

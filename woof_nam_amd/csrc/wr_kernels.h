@@ -84,7 +84,9 @@ static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int 
     const double tem2c = 1.0e-20 * 1.0e3 * CON_AVGD;
     double tem1 = 0.0, tem2 = 0.0, z0 = 1.0, z1 = 1.0;
     int lt = 0, lcf = 0, swlt = nrl;
+    uint32_t blocks = 0;
     double pb = rc.plvl(nrl);
+#pragma unroll 4
     for (int k = 0; k < nrl; ++k) {
         const int kin = nrl - 1 - k;
         const double pt = rc.plvl(kin);
@@ -103,6 +105,7 @@ static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int 
         }
         const double ct = rc.cfrac(kin);
         if (ct > EPS) lcf = 1;
+        if (ct > 0.0) blocks |= 1u << (k >> 2);
         if (ct > FTINY) {
             z1 = fmin(z1, 1.0 - ct);
         } else if (z1 < 1.0) {
@@ -112,6 +115,7 @@ static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int 
     }
     cs.lw_laytrop[t] = lt;
     cs.lcf1[t] = lcf;
+    cs.cblk[t] = blocks;
     const double tem0p = 10.0 * tem2 / (AMDW * tem1 * CON_G);
     cs.pwv[t] = tem0p * rc.plvl(nrl);
     const int day = in.cosz[i] >= 1.0e-4;
@@ -151,12 +155,12 @@ __global__ void __launch_bounds__(64) k_sflux(const Tabs<R> *__restrict__ T, Col
     const WR_G R *tab = upper ? T->sf02 : T->sf03;
     const int mfs = upper ? 5 : 9, k0 = upper ? swlt : 1, k1 = upper ? nrl - 1 : swlt - 1;
     int ks = upper ? nrl : swlt;
-    for (int k = k0, prev = jp(k0 - 1); k <= k1; ++k) {
+    bool found = false;  // no early exit, so that the loads of several layers are in flight
+    int prev = jp(k0 - 1);
+#pragma unroll 8
+    for (int k = k0; k <= k1; ++k) {
         const int cur = jp(k);
-        if (prev < lr && cur >= lr) {
-            ks = k + 1;
-            break;
-        }
+        if (!found && prev < lr && cur >= lr) ks = k + 1, found = true;
         prev = cur;
     }
     SwLay<R> L;
@@ -170,7 +174,7 @@ __global__ void __launch_bounds__(64) k_sflux(const Tabs<R> *__restrict__ T, Col
         colm2 = m == i2 ? L.colamt[m] : colm2;
     }
     const R speccomb = colm1 + T->sw_strrat[b] * colm2;
-    const R specmult = T->sw_specwt[b] * fmin((R)0.999999, colm1 / speccomb);
+    const R specmult = T->sw_specwt[b] * fmin((R)0.999999, rdiv<R>(colm1, speccomb));
     const int jsi = (int)specmult;
     const int js = 1 + jsi;
     const R fs = specmult - (R)jsi;
@@ -187,6 +191,33 @@ __global__ void __launch_bounds__(64) k_sflux(const Tabs<R> *__restrict__ T, Col
 // block), one workgroup's exclusive scan of the counts, then each segment writes its day columns in
 // column order.  The result is the same ordered list whatever the launch shape.
 constexpr int DAY_T = 256, DAY_IT = 8, DAY_SEG = DAY_T * DAY_IT;
+
+// the whole list of a tile of up to DAY_SMALL columns by one workgroup
+constexpr int DAY_SMALL = 16384;
+static __global__ void __launch_bounds__(1024) k_daylist_small(const int *__restrict__ day, int n, int *__restrict__ nday,
+                                                               int *__restrict__ dlist)
+{
+    __shared__ int cnt[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int base = 0;
+    for (int j0 = 0; j0 < n; j0 += 1024) {
+        const int j = j0 + (int)threadIdx.x;
+        const bool f = j < n && day[j] != 0;
+        const uint64_t m = __ballot(f);
+        if (lane == 0) cnt[w] = __popcll(m);
+        __syncthreads();
+        int before = 0, total = 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            before += q < w ? cnt[q] : 0;
+            total += cnt[q];
+        }
+        if (f) dlist[base + before + __popcll(m & (((uint64_t)1 << lane) - 1))] = j;
+        base += total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *nday = base;
+}
 
 // exclusive prefix of v over the 256 threads of the block (4 waves); total = the block sum
 __device__ __forceinline__ int block_excl_scan256(int v, int *lds, int &total)
@@ -413,6 +444,63 @@ template <typename R, int B> constexpr int lw_chunk_r()
 {
     return sizeof(R) == 8 ? chunk_of(LW_NG[B], WR_LW64_CHUNK >= 0 ? WR_LW64_CHUNK : LW64_CHUNK[B]) : lw_chunk<B>();
 }
+// ---- level sums over the g-points of a band ---------------------------------------------------------
+// A band's level flux is the sum of its g-points' contributions in g order.  A lane either holds all NG
+// g-points of its column (GW = NG) and adds them itself, or GW of them, the others being with the other
+// waves of its workgroup (k_many): then the contributions of SUM_LEVELS levels are left in LDS, and after a
+// barrier each wave adds those of its levels, again in g order, so that the sums are the same bits.
+// NQ: quantities per level.  The levels come in order row0, row0 + step, ...; emit(row, sums) stores one.
+constexpr int SUM_LEVELS = 4;
+template <typename R> constexpr size_t sum_lds_bytes() { return sizeof(R) * SUM_LEVELS * 64 * 24; }  // LW 16 g, SW 2 x 12 g
+template <typename R> struct Share {  // a wave's part of a column's g-points (split bands)
+    R *xs;         // LDS of the workgroup, sum_lds_bytes
+    int g0, wave;  // first g-point, wave index
+};
+template <typename R, int NG, int GW, int NQ> struct LevelSum {
+    Share<R> sh;
+    int lane, row, step, cnt;
+    __device__ __forceinline__ void begin(int row0, int step_) { row = row0, step = step_, cnt = 0; }
+    template <typename EMIT> __device__ __forceinline__ void put(const R (&v)[NQ][GW], EMIT &&emit)
+    {
+        if constexpr (GW == NG) {
+            R sum[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                sum[q] = (R)0;
+#pragma unroll
+                for (int j = 0; j < GW; ++j) sum[q] = sum[q] + v[q][j];
+            }
+            emit(row, sum);
+            row += step;
+        } else {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int j = 0; j < GW; ++j) sh.xs[((cnt * NQ + q) * NG + sh.g0 + j) * 64 + lane] = v[q][j];
+            if (++cnt == SUM_LEVELS) finish(emit);
+        }
+    }
+    template <typename EMIT> __device__ __forceinline__ void finish(EMIT &&emit)
+    {
+        if constexpr (GW < NG) {
+            __syncthreads();
+            for (int l = sh.wave; l < cnt; l += NG / GW) {
+                R sum[NQ];
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) {
+                    sum[q] = (R)0;
+#pragma unroll
+                    for (int g = 0; g < NG; ++g) sum[q] = sum[q] + sh.xs[((l * NQ + q) * NG + g) * 64 + lane];
+                }
+                emit(row + step * l, sum);
+            }
+            __syncthreads();
+            row += step * cnt;
+            cnt = 0;
+        }
+    }
+};
+
 // ---- LW band kernels (rtrnmc, McICA) ------------------------------------------------------------
 // One lane per column, one wave per 64-column block; the layer's set-up comes from its record row
 // (wr_rec.h), the McICA bits of the band's g-points from one word per layer.  The g-points of a layer run
@@ -534,7 +622,7 @@ __device__ __forceinline__ void lw_get(const Tabs<R> *__restrict__ T, const ColI
 {
     const LRow<R> row = lrow<R>(rp, blk, k, lane);
     const uint32_t w0 = row.w(0), w1 = row.w(1);
-    lrow_get<R>(row, w0, y.L);
+    lrow_get<R>(row, w0, par, y.L);
     y.blay = planck_of<R>(T, B, (int)(w0 >> 22), row.f(LF_PL));
     y.bbot = planck_of<R>(T, B, (int)(w1 & 255u), row.f(LF_PB));
     y.cloudy = (w1 & 256u) != 0;
@@ -566,22 +654,24 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
                                           int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
                                           const Surr &sg, int blk, int lane)
 {
-    constexpr int NG = LW_NG[B], CH = lw_chunk_r<R, B>();
-    const int t = blk * 64 + lane;
-    if (t >= valid_cols(in, col0, n)) return;
+    constexpr int NG = LW_NG[B], GW = NG, CH = lw_chunk_r<R, B>();
+    const Share<R> sh{nullptr, 0, 0};
+    const int nv = valid_cols(in, col0, n);
+    if (blk * 64 >= nv) return;
+    const bool ok = blk * 64 + lane < nv;  // lanes past the last column repeat it and store nothing
+    const int rl = ok ? lane : nv - 1 - blk * 64, t = blk * 64 + rl;
     const LwCol<R> c = lw_col<R, B, SURR>(in, col0, cs, sg, t);
     const int nrl = c.nrl;
-    acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
-    R rad[NG];
+    if (ok) acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
+    R rad[1][GW], sfc0[1][GW];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) rad[g] = (R)0;
-    // one layer of a sweep: dir 0 down (source between the layer and the level below), 1 up
-    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, uint32_t bits, bool sfc, R pk0, R &s, R &s0) {
-        s = (R)0, s0 = (R)0;
+    for (int g = 0; g < GW; ++g) rad[0][g] = (R)0;
+    // one layer of a sweep: the source lies between the layer and the level the radiation leaves through
+    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, uint32_t bits, bool sfc, R pk0) {
         R ecld = (R)1;
         if (__any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
 #pragma unroll
-        for (int g0 = 0; g0 < NG; g0 += CH) {
+        for (int g0 = 0; g0 < GW; g0 += CH) {
             R tau[CH], fr[CH];
             lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
             GasV<R, CH> q;
@@ -590,8 +680,8 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
                     const R rad0 = c.semis * fr[j] * pk0;
-                    rad[g0 + j] = rad0 + c.reflct * rad[g0 + j];
-                    s0 = s0 + rad[g0 + j];
+                    rad[0][g0 + j] = rad0 + c.reflct * rad[0][g0 + j];
+                    sfc0[0][g0 + j] = rad[0][g0 + j];
                 }
             }
             R nr[CH], gas[CH];
@@ -599,9 +689,10 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
             for (int j = 0; j < CH; ++j) {
                 const R bb = fr[j] * (y.blay + dplnk * q.gf[j]);
                 gas[j] = bb * q.at[j];
-                nr[j] = rad[g0 + j] * q.tr[j] + gas[j];
+                nr[j] = rad[0][g0 + j] * q.tr[j] + gas[j];
             }
-            if (__any((bits >> g0) & ((1u << CH) - 1u))) {
+            const uint32_t cb = bits >> g0;
+            if (__any(cb & ((1u << CH) - 1u))) {
                 R tr[CH], at[CH], gf[CH];
                 lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
                 const R efclrfr = (R)1 - ((R)1 - ecld);
@@ -609,40 +700,47 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
                 for (int j = 0; j < CH; ++j) {
                     const R bbt = fr[j] * (y.blay + dplnk * gf[j]);
                     const R tot = bbt * at[j];
-                    const R rc = rad[g0 + j] * q.tr[j] * efclrfr + gas[j] + (tot - gas[j]);
-                    nr[j] = (bits >> (g0 + j)) & 1u ? rc : nr[j];
+                    const R rc = rad[0][g0 + j] * q.tr[j] * efclrfr + gas[j] + (tot - gas[j]);
+                    nr[j] = (cb >> j) & 1u ? rc : nr[j];
                 }
             }
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                rad[g0 + j] = nr[j];
-                s = s + nr[j];
-            }
-            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < CH; ++j) rad[0][g0 + j] = nr[j];
+            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
     };
-    R s, s0;
+    LevelSum<R, NG, GW, 1> sum{sh, lane, 0, 0, 0};
+    auto dn = [&](int row, const R *s) {
+        if (ok) acc.lw_dn[(size_t)row * n + t] = s[0];
+    };
+    auto up = [&](int row, const R *s) {
+        if (ok) acc.lw_up[(size_t)row * n + t] = s[0];
+    };
+    sum.begin(nrl - 1, -1);
     for (int k = nrl - 1; k >= 0; --k) {  // down sweep, top to surface
         LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
-        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
-        sweep(k, y, y.bbot - y.blay, bits, false, (R)0, s, s0);
-        acc.lw_dn[(size_t)k * n + t] = s;
+        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl) : 0u;
+        sweep(k, y, y.bbot - y.blay, bits, false, (R)0);
+        sum.put(rad, dn);
     }
+    sum.finish(dn);
+    sum.begin(0, 1);
     for (int k = 0; k < nrl; ++k) {  // up sweep, surface to top
         LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
-        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
+        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl) : 0u;
         // the level above is the next layer's lower level; above the top layer, its own temperature
         R btop = y.blay;
         if (k + 1 < nrl) {
-            const LRow<R> up = lrow<R>(rp, blk, k + 1, lane);
-            btop = planck_of<R>(T, B, (int)(up.w(1) & 255u), up.f(LF_PB));
+            const LRow<R> nx = lrow<R>(rp, blk, k + 1, rl);
+            btop = planck_of<R>(T, B, (int)(nx.w(1) & 255u), nx.f(LF_PB));
         }
-        sweep(k, y, btop - y.blay, bits, k == 0, y.bbot, s, s0);  // the level below the lowest layer is the skin
-        if (k == 0) acc.lw_up[t] = s0;
-        acc.lw_up[(size_t)(k + 1) * n + t] = s;
+        sweep(k, y, btop - y.blay, bits, k == 0, y.bbot);  // the level below the lowest layer is the skin
+        if (k == 0) sum.put(sfc0, up);
+        sum.put(rad, up);
     }
+    sum.finish(up);
 }
 
 template <typename R, int B, bool SURR = false, bool EXT = true>
@@ -710,89 +808,113 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
 // with no optics.  The FP64 kernels recompute the upward optics instead: their sums follow the reference's
 // operation order, and twice the bytes would not pay.
 constexpr int LW_NV_F32 = 2;
+// transmittance a and the downward and upward sources (gas plus cloud) of CH g-points of a layer
+template <int CH>
+__device__ __forceinline__ void lw_chunk_f32(const Tabs<float> *__restrict__ T, const LwLayer<float> &y, float sdif, float dd, float du,
+                                             float ecld, uint32_t cb, const float *tau, const float *fr, float *a, float *bd,
+                                             float *bu)
+{
+    using R = float;
+    GasV<R, CH> q;
+    lw_gas_v<R, CH>(T, sdif, y.taer, tau, q);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const R fa = fr[j] * q.at[j];
+        bd[j] = fa * (y.blay + dd * q.gf[j]);
+        bu[j] = fa * (y.blay + du * q.gf[j]);
+        a[j] = q.tr[j];
+    }
+    if (__any(cb & ((1u << CH) - 1u))) {
+        R tr[CH], at[CH], gf[CH];
+        lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool cl = (cb >> j) & 1u;
+            const R fa = fr[j] * at[j];
+            const R td = fa * (y.blay + dd * gf[j]), tu = fa * (y.blay + du * gf[j]);
+            a[j] = cl ? q.tr[j] * ecld : a[j];
+            bd[j] = cl ? td : bd[j];
+            bu[j] = cl ? tu : bu[j];
+        }
+    }
+}
+
 template <int B, bool SURR, typename BT>
 __device__ __forceinline__ void lw_column_f32c(const Tabs<float> *__restrict__ T, const BT &Bt, const ColIn &in,
                                                const RunPar &par, int col0, int n, const ColScal &cs, const RecPtrs &rp,
                                                const AccT<float> &acc, const Surr &sg, int blk, int lane, WR_G char *slot)
 {
     using R = float;
-    constexpr int NG = LW_NG[B], CH = lw_chunk<B>();
-    const int t = blk * 64 + lane;
-    if (t >= valid_cols(in, col0, n)) return;
+    constexpr int NG = LW_NG[B], GW = NG, CH = lw_chunk<B>();
+    const Share<R> sh{nullptr, 0, 0};
+    const int nv = valid_cols(in, col0, n);
+    if (blk * 64 >= nv) return;
+    const bool ok = blk * 64 + lane < nv;  // lanes past the last column repeat it and store nothing
+    const int rl = ok ? lane : nv - 1 - blk * 64, t = blk * 64 + rl;
     const LwCol<R> c = lw_col<R, B, SURR>(in, col0, cs, sg, t);
     const int nrl = c.nrl;
     WR_G f32x2v *ab = (WR_G f32x2v *)slot + lane;  // [layer][g][lane]
-    acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
-    R rad[NG];
+    if (ok) acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
+    R rad[1][GW];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) rad[g] = (R)0;
+    for (int g = 0; g < GW; ++g) rad[0][g] = (R)0;
+    LevelSum<R, NG, GW, 1> sum{sh, lane, 0, 0, 0};
+    auto dn = [&](int row, const R *s) {
+        if (ok) acc.lw_dn[(size_t)row * n + t] = s[0];
+    };
+    auto up = [&](int row, const R *s) {
+        if (ok) acc.lw_up[(size_t)row * n + t] = s[0];
+    };
     R btop = (R)0;  // Planck function at the level above the layer
+    sum.begin(nrl - 1, -1);
     for (int k = nrl - 1; k >= 0; --k) {
         LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
-        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, lane) : 0u;
+        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
+        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl) : 0u;
         if (k == nrl - 1) btop = y.blay;
         const R dd = y.bbot - y.blay, du = btop - y.blay;
         R ecld = (R)1;
         if (__any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
-        R s = (R)0, s0 = (R)0;
+        R sfc0[GW];
 #pragma unroll
-        for (int g0 = 0; g0 < NG; g0 += CH) {
+        for (int g0 = 0; g0 < GW; g0 += CH) {
             R tau[CH], fr[CH];
             lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
-            GasV<R, CH> q;
-            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
             R a[CH], bd[CH], bu[CH];
+            lw_chunk_f32<CH>(T, y, c.sdif, dd, du, ecld, bits >> g0, tau, fr, a, bd, bu);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
-                const R fa = fr[j] * q.at[j];
-                bd[j] = fa * (y.blay + dd * q.gf[j]);
-                bu[j] = fa * (y.blay + du * q.gf[j]);
-                a[j] = q.tr[j];
-            }
-            if (__any((bits >> g0) & ((1u << CH) - 1u))) {
-                R tr[CH], at[CH], gf[CH];
-                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const bool cl = (bits >> (g0 + j)) & 1u;
-                    const R fa = fr[j] * at[j];
-                    const R td = fa * (y.blay + dd * gf[j]), tu = fa * (y.blay + du * gf[j]);
-                    a[j] = cl ? q.tr[j] * ecld : a[j];
-                    bd[j] = cl ? td : bd[j];
-                    bu[j] = cl ? tu : bu[j];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const R r = rad[g0 + j] * a[j] + bd[j];
-                rad[g0 + j] = r;
-                s = s + r;
+                rad[0][g0 + j] = rad[0][g0 + j] * a[j] + bd[j];
                 ab[((size_t)k * NG + g0 + j) * 64] = (f32x2v){a[j], bu[j]};
             }
             if (k == 0) {  // surface emission and reflection start the upward sweep
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
-                    rad[g0 + j] = c.semis * fr[j] * y.bbot + c.reflct * rad[g0 + j];
-                    s0 = s0 + rad[g0 + j];
+                    const R rad0 = c.semis * fr[j] * y.bbot;
+                    sfc0[g0 + j] = rad0 + c.reflct * rad[0][g0 + j];
                 }
             }
-            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
-        acc.lw_dn[(size_t)k * n + t] = s;
-        if (k == 0) acc.lw_up[t] = s0;
+        sum.put(rad, dn);
+        if (k == 0) {
+#pragma unroll
+            for (int g = 0; g < GW; ++g) rad[0][g] = sfc0[g];
+        }
         btop = y.bbot;
     }
+    sum.finish(dn);
+    sum.begin(0, 1);
+    sum.put(rad, up);
     for (int k = 0; k < nrl; ++k) {  // up sweep over the cached layers
-        R s = (R)0;
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
+        for (int g = 0; g < GW; ++g) {
             const f32x2v v = ab[((size_t)k * NG + g) * 64];
-            rad[g] = rad[g] * v.x + v.y;
-            s = s + rad[g];
+            rad[0][g] = rad[0][g] * v.x + v.y;
         }
-        acc.lw_up[(size_t)(k + 1) * n + t] = s;
+        sum.put(rad, up);
     }
+    sum.finish(up);
 }
 
 template <int B, bool SURR = false, bool EXT = true>
@@ -896,12 +1018,6 @@ __device__ __forceinline__ void expm_v(const R *z, const WR_G R *__restrict__ tb
             e[j] = !(z[j] <= (R)0.06) ? v : e[j];
         }
     }
-}
-
-template <typename R> __device__ __forceinline__ R rdiv(R a, R b)
-{
-    if constexpr (sizeof(R) == 4) return a * __builtin_amdgcn_rcpf(b);
-    return a / b;
 }
 
 // layer_rt (delta scaling, PIFM, layer R/T) for CH g-points; FP32 flags a g-point near the two-stream
@@ -1102,7 +1218,7 @@ __device__ __forceinline__ void sw_get(const Tabs<R> *__restrict__ T, const ColI
                                        int i, R cz, R snt, int blk, int lane, int k, SwLayer<R> &a)
 {
     const LRow<R> row = srow<R>(rp, blk, k, lane);
-    srow_get<R>(row, row.w(0), a.L);
+    srow_get<R>(row, row.w(0), par, a.L);
     a.cloudy = row.w(1) != 0;
     const RadCol rc{in, i, rp.nrl};
     double ta, sa, ya;
@@ -1137,16 +1253,19 @@ __device__ __forceinline__ void sw_tgtr(const Tabs<R> *__restrict__ T, const BT 
 // bytes cost more than the evaluation).
 constexpr int SW_NV = 2;
 template <typename R> constexpr int sw_nv_mc() { return sizeof(R) == 4 ? SW_NV + 5 : SW_NV; }
-template <typename R, int NG> struct SwSlot {
+// KEEP: with the layer's R/T.
+template <typename R, int NG, bool KEEP> struct SwSlot {
     WR_G char *p;
     int lane, nk;
     __device__ __forceinline__ void put(int k, int g, R pb, R pd, const R *rt) const  // rt: rb, rd, tb, td, ld
     {
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
-        if constexpr (sizeof(R) == 4) {
+        if constexpr (KEEP) {
             ((WR_G f32x4v *)p)[e] = (f32x4v){pb, pd, rt[0], rt[1]};
             WR_G float *q = (WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
             q[0] = rt[2], q[1] = rt[3], q[2] = rt[4];
+        } else if constexpr (sizeof(R) == 4) {
+            ((WR_G f32x2v *)p)[e] = (f32x2v){pb, pd};
         } else {
             ((WR_G f64x2v *)p)[e] = (f64x2v){pb, pd};
         }
@@ -1154,10 +1273,13 @@ template <typename R, int NG> struct SwSlot {
     __device__ __forceinline__ void get(int k, int g, R &pb, R &pd, R *rt) const
     {
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
-        if constexpr (sizeof(R) == 4) {
+        if constexpr (KEEP) {
             const f32x4v v = ((const WR_G f32x4v *)p)[e];
             const WR_G float *q = (const WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
             pb = v.x, pd = v.y, rt[0] = v.z, rt[1] = v.w, rt[2] = q[0], rt[3] = q[1], rt[4] = q[2];
+        } else if constexpr (sizeof(R) == 4) {
+            const f32x2v v = ((const WR_G f32x2v *)p)[e];
+            pb = v.x, pd = v.y;
         } else {
             const f64x2v v = ((const WR_G f64x2v *)p)[e];
             pb = v.x, pd = v.y;
@@ -1166,45 +1288,46 @@ template <typename R, int NG> struct SwSlot {
 };
 
 // The adding method over one column: bottom-up reflectances to the slot, then the direct and diffuse beams
-// top-down with the level fluxes.  layer(k) gives a layer, rt_at(layer, k, g0, o) its R/T of a chunk, sun(g)
-// the solar source of a g-point; emit(level, up, down) takes a level's fluxes, top level first.
-template <typename R, int NG, int CH, typename LAYER, typename RT, typename SUN, typename EMIT>
-__device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG> &slot, LAYER &&layer, RT &&rt_at, SUN &&sun,
-                                          EMIT &&emit)
+// top-down with the level fluxes.  layer(k) gives a layer, rt_at(layer, k, g0, o) its R/T of a chunk of the
+// lane's g-points, sun(g) the solar source of one; emit(level, {up, down}) takes a level's fluxes, top first.
+// KEEP: the top-down sweep takes the R/T from the slot instead of from rt_at again.
+template <typename R, int NG, int GW, int CH, bool KEEP, typename LAYER, typename RT, typename SUN, typename EMIT>
+__device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG, KEEP> &slot, const Share<R> &sh, LAYER &&layer, RT &&rt_at,
+                                          SUN &&sun, EMIT &&emit)
 {
-    R pb[NG], pd[NG];
+    R pb[GW], pd[GW];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) pb[g] = asfc, pd[g] = asfc;
+    for (int g = 0; g < GW; ++g) pb[g] = asfc, pd[g] = asfc;
     for (int k = 0; k < nrl; ++k) {
         auto a = layer(k);
 #pragma unroll
-        for (int g0 = 0; g0 < NG; g0 += CH) {
+        for (int g0 = 0; g0 < GW; g0 += CH) {
             RtV<R, CH> o;
             rt_at(a, k, g0, o);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 const int g = g0 + j;
                 const R rt[5] = {o.rb[j], o.rd[j], o.tb[j], o.td[j], o.ld[j]};
-                slot.put(k, g, pb[g], pd[g], rt);
+                slot.put(k, sh.g0 + g, pb[g], pd[g], rt);
                 const R zden1 = rdiv<R>((R)1, (R)1 - pd[g] * o.rd[j]);
                 const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * pd[g] + o.ld[j] * pb[g])) * zden1;
                 const R nd = o.rd[j] + o.td[j] * o.td[j] * pd[g] * zden1;
                 pb[g] = nb, pd[g] = nd;
             }
-            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    R tdbt[NG], tdn[NG], rdnd[NG], zsolar[NG];
-    R su = (R)0, sd = (R)0;
+    R tdbt[GW], tdn[GW], rdnd[GW], zsolar[GW], f[2][GW];
+    LevelSum<R, NG, GW, 2> sum{sh, slot.lane, 0, 0, 0};
+    sum.begin(nrl, -1);
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
+    for (int g = 0; g < GW; ++g) {
         tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0, zsolar[g] = sun(g);
-        su = su + zsolar[g] * pb[g];
-        sd = sd + zsolar[g];
+        f[0][g] = zsolar[g] * pb[g];
+        f[1][g] = zsolar[g];
     }
-    emit(nrl, su, sd);
+    sum.put(f, emit);
     for (int k = nrl - 1; k >= 0; --k) {
-        su = (R)0, sd = (R)0;
         auto chunk = [&](int g0, auto &&get) {
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
@@ -1219,31 +1342,32 @@ __device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG> &
                 const R zden1 = rdiv<R>((R)1, (R)1 - rdnd_s * zd);
                 const R zfu = (tdbt_s * zb + (tdn_s - tdbt_s) * zd) * zden1;
                 const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * zb * rdnd_s) * zden1;
-                su = su + zsolar[g] * zfu;
-                sd = sd + zsolar[g] * zfd;
+                f[0][g] = zsolar[g] * zfu;
+                f[1][g] = zsolar[g] * zfd;
             }
         };
-        if constexpr (sizeof(R) == 4) {
+        if constexpr (KEEP) {
 #pragma unroll
-            for (int g0 = 0; g0 < NG; g0 += CH) {
-                chunk(g0, [&](int g, int, R &zb, R &zd, R *rt) { slot.get(k, g, zb, zd, rt); });
-                if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            for (int g0 = 0; g0 < GW; g0 += CH) {
+                chunk(g0, [&](int g, int, R &zb, R &zd, R *rt) { slot.get(k, sh.g0 + g, zb, zd, rt); });
+                if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
             }
         } else {
             auto a = layer(k);
 #pragma unroll
-            for (int g0 = 0; g0 < NG; g0 += CH) {
+            for (int g0 = 0; g0 < GW; g0 += CH) {
                 RtV<R, CH> o;
                 rt_at(a, k, g0, o);
                 chunk(g0, [&](int g, int j, R &zb, R &zd, R *rt) {
-                    slot.get(k, g, zb, zd, nullptr);
+                    slot.get(k, sh.g0 + g, zb, zd, nullptr);
                     rt[0] = o.rb[j], rt[1] = o.rd[j], rt[2] = o.tb[j], rt[3] = o.td[j], rt[4] = o.ld[j];
                 });
-                if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
             }
         }
-        emit(k, su, sd);
+        sum.put(f, emit);
     }
+    sum.finish(emit);
 }
 
 // What the SW sweeps of one day column need besides its layers.
@@ -1270,22 +1394,26 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
                                           const AccT<R> &acc, const Surr &sg, int blk, int lane, WR_G char *slot, Fix64 *fx)
 {
     constexpr int NG = SW_NG[B], CH = sw_chunk<R, B>();
-    if (blk * 64 + lane >= *cs.nday) return;
-    const int t = cs.dlist[blk * 64 + lane], nrl = rp.nrl;
+    constexpr bool KEEP = sw_nv_mc<R>() > SW_NV;
+    const int nday = *cs.nday;
+    if (blk * 64 >= nday) return;
+    const bool ok = blk * 64 + lane < nday;  // lanes past the last day column repeat it and store nothing
+    const int rl = ok ? lane : nday - 1 - blk * 64;
+    const int t = cs.dlist[blk * 64 + rl], nrl = rp.nrl;
     SwCol<R> c;
     sw_col<R, B>(in, par, col0, cs, t, c);
     const int table = SURR ? sg.table(t, 16 + B) : 1;
-    acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
+    if (ok) acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
     struct Lay {
         SwLayer<R> y;
         uint32_t bits;
     };
-    sw_adding<R, NG, CH>(
-        nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2},
+    sw_adding<R, NG, NG, CH, KEEP>(
+        nrl, c.asfc, SwSlot<R, NG, KEEP>{slot, lane, in.nlay + 2}, Share<R>{nullptr, 0, 0},
         [&](int k) {
             Lay a;
-            sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, lane, k, a.y);
-            a.bits = a.y.cloudy ? mword(rp.msw, rp.row(blk, k), MROW_SW, B, lane) : 0u;
+            sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
+            a.bits = a.y.cloudy ? mword(rp.msw, rp.row(blk, k), MROW_SW, B, rl) : 0u;
             return a;
         },
         [&](const Lay &a, int k, int g0, RtV<R, CH> &o) {
@@ -1294,9 +1422,11 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
             layer_rt_sky<R, CH>(T, tr, tg, a.y.y, a.bits >> g0, o, fx);
         },
         [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
-        [&](int lev, R su, R sd) {
-            acc.sw_up[(size_t)lev * n + t] = su;
-            acc.sw_dn[(size_t)lev * n + t] = sd;
+        [&](int lev, const R *f) {
+            if (ok) {
+                acc.sw_up[(size_t)lev * n + t] = f[0];
+                acc.sw_dn[(size_t)lev * n + t] = f[1];
+            }
         });
 }
 
@@ -1361,6 +1491,9 @@ __global__ void __launch_bounds__((64 * swl_wpg<R, B>()), (sw_waves<R, B>()))
 struct OutPtrs {
     WR_G double *hr_lw, *hr_sw, *flw_up, *flw_dn, *fsw_up, *fsw_dn, *fsw_dn_sfc_clr;
 };
+// One thread per column and segment of levels (gridDim.y segments; one for large tiles, whose planes bound the
+// kernel: 13 GB in FP32, 26 GB in FP64 for 796,590 columns).  A segment after the first evaluates the level
+// below it once more.  Small tiles take 16: a column's 62 levels one after the other were 139 us.
 template <typename P>
 __global__ void __launch_bounds__(256) k_post(ColIn in, int col0, int n, ColScal cs, BandAcc ba, OutPtrs out)
 {
@@ -1394,11 +1527,16 @@ __global__ void __launch_bounds__(256) k_post(ColIn in, int col0, int n, ColScal
         }
         return v;
     };
-    const double up0 = lwsum(0, 0), dn0 = lwsum(1, 0);
+    const int len = (nrl + (int)gridDim.y - 1) / (int)gridDim.y, k0 = (int)blockIdx.y * len, k1 = imin(nrl, k0 + len);
+    const bool first = blockIdx.y == 0;
+    if (k0 >= k1) return;
+    const double up0 = lwsum(0, k0), dn0 = lwsum(1, k0);
     double fprev = up0 * flxfac - dn0 * flxfac;
-    out.flw_up[(size_t)nrl * nc + i] = up0 * flxfac;
-    out.flw_dn[(size_t)nrl * nc + i] = dn0 * flxfac;
-    for (int k = 1; k <= nrl; ++k) {
+    if (first) {
+        out.flw_up[(size_t)nrl * nc + i] = up0 * flxfac;
+        out.flw_dn[(size_t)nrl * nc + i] = dn0 * flxfac;
+    }
+    for (int k = k0 + 1; k <= k1; ++k) {
         const double fu = lwsum(0, k) * flxfac, fd = lwsum(1, k) * flxfac;
         out.flw_up[(size_t)(nrl - k) * nc + i] = fu;
         out.flw_dn[(size_t)(nrl - k) * nc + i] = fd;
@@ -1410,10 +1548,12 @@ __global__ void __launch_bounds__(256) k_post(ColIn in, int col0, int n, ColScal
         fprev = fnet;
     }
     if (cs.day[t]) {
-        double fu0 = swsum(0, 0), fd0 = swsum(1, 0);
-        out.fsw_up[(size_t)nrl * nc + i] = fu0;
-        out.fsw_dn[(size_t)nrl * nc + i] = fd0;
-        for (int k = 0; k < nrl; ++k) {
+        double fu0 = swsum(0, k0), fd0 = swsum(1, k0);
+        if (first) {
+            out.fsw_up[(size_t)nrl * nc + i] = fu0;
+            out.fsw_dn[(size_t)nrl * nc + i] = fd0;
+        }
+        for (int k = k0; k < k1; ++k) {
             const double fu1 = swsum(0, k + 1), fd1 = swsum(1, k + 1);
             out.fsw_up[(size_t)(nrl - 1 - k) * nc + i] = fu1;
             out.fsw_dn[(size_t)(nrl - 1 - k) * nc + i] = fd1;
@@ -1423,7 +1563,7 @@ __global__ void __launch_bounds__(256) k_post(ColIn in, int col0, int n, ColScal
             if (k < nm) out.hr_sw[(size_t)(nm - 1 - k) * nc + i] = h;
             fu0 = fu1, fd0 = fd1;
         }
-        if (out.fsw_dn_sfc_clr) {
+        if (first && out.fsw_dn_sfc_clr) {
             double v = 0.0;
 #pragma unroll
             for (int b = 0; b < 14; ++b) {
@@ -1433,9 +1573,10 @@ __global__ void __launch_bounds__(256) k_post(ColIn in, int col0, int n, ColScal
             out.fsw_dn_sfc_clr[i] = v;
         }
     } else {
-        for (int L = 0; L <= nrl; ++L) out.fsw_up[(size_t)L * nc + i] = 0.0, out.fsw_dn[(size_t)L * nc + i] = 0.0;
-        for (int k0 = 0; k0 < nm; ++k0) out.hr_sw[(size_t)k0 * nc + i] = 0.0;
-        if (out.fsw_dn_sfc_clr) out.fsw_dn_sfc_clr[i] = 0.0;
+        for (int L = first ? k0 : k0 + 1; L <= k1; ++L)
+            out.fsw_up[(size_t)L * nc + i] = 0.0, out.fsw_dn[(size_t)L * nc + i] = 0.0;
+        for (int q = k0; q < imin(k1, nm); ++q) out.hr_sw[(size_t)q * nc + i] = 0.0;
+        if (first && out.fsw_dn_sfc_clr) out.fsw_dn_sfc_clr[i] = 0.0;
     }
 }
 

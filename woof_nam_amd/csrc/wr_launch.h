@@ -47,6 +47,10 @@ static_assert(band_plan_complete(), "every band kernel appears exactly once in B
 // scatter.
 inline void launch_daylist(const ColScal &cs, int n, hipStream_t s)
 {
+    if (n <= DAY_SMALL) {
+        hipLaunchKernelGGL(k_daylist_small, dim3(1), dim3(1024), 0, s, (const int *)cs.day, n, (int *)cs.nday, (int *)cs.dlist);
+        return;
+    }
     const int nseg = (n + DAY_SEG - 1) / DAY_SEG;
     int *seg = (int *)cs.nday + 1;
     hipLaunchKernelGGL(k_daycount, dim3(nseg), dim3(DAY_T), 0, s, (const int *)cs.day, n, seg);
@@ -327,6 +331,13 @@ int run_bands(wr_ctx *c, int band, hipStream_t s, F &&one)
     return WR_OK;
 }
 
+// k_post's grid: columns x level segments, as many segments (at most 16, of 4 levels or more) as give the chip
+// about 65,536 threads; a segment costs one level more than it owns, so large tiles take one.
+inline dim3 post_grid(int n, int nrl)
+{
+    return dim3((unsigned)(n + 255) / 256, (unsigned)std::max(1, std::min({16, nrl / 4, 65536 / std::max(n, 1)})));
+}
+
 // What the band kernels of a tile read: LW records, column scalars, day list, SW records, solar source and
 // (McICA) the cloud words.
 template <typename R> void launch_prep(const BandJob<R> &j, hipStream_t s)
@@ -362,7 +373,7 @@ int launch_tile(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, const
                 int col0, int n, int band, hipStream_t s, const Surr &sg = Surr{})
 {
     const int nrl = in.nlay + 1;
-    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, n, nrl, (int)sizeof(R)),
+    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, (char *)c->rtr, n, nrl, (int)sizeof(R)),
                  tile_planes(c, n, nrl, band), sg, Rtr<R>{},
                  tile_lwrec<R>(c, n, nrl)};
     launch_prep(j, s);
@@ -376,7 +387,7 @@ int launch_tile(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, const
                  : run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band<R, SURR, EXT>(j, id, q, pool); });
     if (rc != WR_OK) return rc;
     tbeg(c, KID_POST, s);
-    hipLaunchKernelGGL(k_post<R>, dim3((n + 255) / 256), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);
+    hipLaunchKernelGGL(k_post<R>, post_grid(n, nrl), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);
     tend(c, s);
     return hipGetLastError() == hipSuccess ? WR_OK : WR_ERR_HIP;
 }
@@ -393,7 +404,7 @@ int launch_tile_nam(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, c
     rt.lstu = gptr((uint64_t *)((char *)c->rtr + sizeof(double) * 12 * (NL + 3) * (size_t)c->max_cols));
     rt.lstd = rt.lstu + c->max_cols;
     rt.n = n;
-    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, n, nrl, (int)sizeof(R)),
+    BandJob<R> j{c, tabs, sflux, in, par, col0, n, colscal(c), rec_ptrs(c->rec, (char *)c->rtr, n, nrl, (int)sizeof(R)),
                  tile_planes(c, n, nrl, band), Surr{}, rt, LwRec<R>{}};
     launch_prep(j, s);
     tbeg(c, KID_RTRFAC, s);
@@ -404,7 +415,7 @@ int launch_tile_nam(wr_ctx *c, const Tabs<R> *tabs, R *sflux, const ColIn &in, c
                  : run_bands(c, band, s, [&](int id, hipStream_t q, char *pool) { launch_band_nam<R, EXT>(j, id, q, pool); });
     if (rc != WR_OK) return rc;
     tbeg(c, KID_POST, s);
-    hipLaunchKernelGGL(k_post<R>, dim3((n + 255) / 256), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);
+    hipLaunchKernelGGL(k_post<R>, post_grid(n, nrl), dim3(256), 0, s, in, col0, n, j.cs, j.ba, out);
     tend(c, s);
     return hipGetLastError() == hipSuccess ? WR_OK : WR_ERR_HIP;
 }

@@ -153,7 +153,7 @@ __device__ __forceinline__ R lw_taucld_r(const Tabs<R> *__restrict__ T, int b, R
     if (cldice > (R)0) {
         const R ri = (R)fmin(130.0, fmax(13.0, refice));
         const int ia0 = T->ipat[b] - 1;
-        tauice = fmax((R)0, cldice * (T->absice1[ia0 * 2 + 0] + T->absice1[ia0 * 2 + 1] / ri));
+        tauice = fmax((R)0, cldice * (T->absice1[ia0 * 2 + 0] + rdiv<R>(T->absice1[ia0 * 2 + 1], ri)));
     }
     const R tauran = (R)(0.33e-3 * cldran);  // absrain (NCAR) x rain path
     return tauice + tauliq + tauran + (R)0;  // + tausnw (snow path 0)
@@ -214,7 +214,7 @@ template <typename R> __device__ __forceinline__ Eta<R> eta(R a, R ratio, R b, R
 {
     Eta<R> e;
     e.speccomb = a + ratio * b;
-    e.specparm = a / e.speccomb;
+    e.specparm = rdiv<R>(a, e.speccomb);
     const R specmult = mult * fmin(e.specparm, (R)ONEMINUS);
     e.js = 1 + (int)specmult;
     e.fs = specmult - (R)((int)specmult);
@@ -275,7 +275,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         const R pp = L.pavel;
         const R scalen2 = L.colbrd * L.scaleminorn2;
         if (lower) {
-            const R corradj = (pp < (R)250) ? ((R)1 - (R)0.15 * ((R)250 - pp) / (R)154.4) : (R)1;
+            const R corradj = (pp < (R)250) ? ((R)1 - rdiv<R>((R)0.15 * ((R)250 - pp), (R)154.4)) : (R)1;
 #pragma unroll
             for (int jj = 0; jj < NGL; ++jj) {
                 const int g = g0 + jj;
@@ -284,7 +284,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
                 fr[jj] = Bt.fracrefa[g];
             }
         } else {
-            const R corradj = (R)1 - (R)0.15 * (pp / (R)95.6);
+            const R corradj = (R)1 - (R)0.15 * rdiv<R>(pp, (R)95.6);
 #pragma unroll
             for (int jj = 0; jj < NGL; ++jj) {
                 const int g = g0 + jj;
@@ -295,7 +295,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 1) {
         if (lower) {
-            const R corradj = (R)1 - (R)0.05 * (L.pavel - (R)100) / (R)900;
+            const R corradj = (R)1 - rdiv<R>((R)0.05 * (L.pavel - (R)100), (R)900);
 #pragma unroll
             for (int jj = 0; jj < NGL; ++jj) {
                 const int g = g0 + jj;
@@ -312,7 +312,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 2) {
         const R p = L.coldry * (R)chi[jp * 7 + 3];
-        const R ratn2o = ca[3] / p;
+        const R ratn2o = rdiv<R>(ca[3], p);
         const R adjcoln2o = (ratn2o > (R)1.5) ? ((R)0.5 + M<R>::pow(ratn2o - (R)0.5, (R)0.65)) * p : ca[3];
         if (lower) {
             const Eta<R> e0 = eta<R>(ca[0], CHR(1, 2, jp), ca[1], (R)8), e1 = eta<R>(ca[0], CHR(1, 2, jpp), ca[1], (R)8);
@@ -406,7 +406,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         const R wx2 = L.wx[1], wx3 = L.wx[2];
         if (lower) {
             const R temp = L.coldry * (R)chi[jp * 7 + 1];
-            const R ratco2 = ca[1] / temp;
+            const R ratco2 = rdiv<R>(ca[1], temp);
             const R adjcolco2 = (ratco2 > (R)3) ? ((R)2 + M<R>::pow(ratco2 - (R)2, (R)0.77)) * temp : ca[1];
 #pragma unroll
             for (int jj = 0; jj < NGL; ++jj) {
@@ -425,7 +425,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 6) {
         const R temp = L.coldry * (R)chi[jp * 7 + 1];
-        const R ratco2 = ca[1] / temp;
+        const R ratco2 = rdiv<R>(ca[1], temp);
         if (lower) {
             const R adjcolco2 = (ratco2 > (R)3) ? ((R)3 + M<R>::pow(ratco2 - (R)3, (R)0.79)) * temp : ca[1];
             const Eta<R> e0 = eta<R>(ca[0], CHR(1, 3, jp), ca[2], (R)8), e1 = eta<R>(ca[0], CHR(1, 3, jpp), ca[2], (R)8);
@@ -458,7 +458,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 7) {
         const R temp = L.coldry * (R)chi[jp * 7 + 1];
-        const R ratco2 = ca[1] / temp;
+        const R ratco2 = rdiv<R>(ca[1], temp);
         const R adjcolco2 = (ratco2 > (R)3) ? ((R)2 + M<R>::pow(ratco2 - (R)2, (R)0.65)) * temp : ca[1];
         const R w3 = L.wx[2], w4 = L.wx[3];
         if (lower) {
@@ -483,7 +483,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
         }
     } else if constexpr (B == 8) {
         const R temp = L.coldry * (R)chi[jp * 7 + 3];
-        const R ratn2o = ca[3] / temp;
+        const R ratn2o = rdiv<R>(ca[3], temp);
         const R adjcoln2o = (ratn2o > (R)1.5) ? ((R)0.5 + M<R>::pow(ratn2o - (R)0.5, (R)0.65)) * temp : ca[3];
         if (lower) {
             const Eta<R> e0 = eta<R>(ca[0], CHR(1, 6, jp), ca[4], (R)8), e1 = eta<R>(ca[0], CHR(1, 6, jpp), ca[4], (R)8);
@@ -561,7 +561,7 @@ __device__ __forceinline__ void lw_optics_t(const Tabs<R> *__restrict__ T, const
     } else if constexpr (B == 12) {
         if (lower) {
             const R temp = L.coldry * (R)3.55e-4;
-            const R ratco2 = ca[1] / temp;
+            const R ratco2 = rdiv<R>(ca[1], temp);
             const R adjcolco2 = (ratco2 > (R)3) ? ((R)2 + M<R>::pow(ratco2 - (R)2, (R)0.68)) * temp : ca[1];
             const Eta<R> e0 = eta<R>(ca[0], CHR(1, 4, jp), ca[3], (R)8), e1 = eta<R>(ca[0], CHR(1, 4, jpp), ca[3], (R)8);
             const Eta<R> emc2 = eta<R>(ca[0], Bt.refrat_m_a, ca[3], (R)8), emc = eta<R>(ca[0], Bt.refrat_m_a3, ca[3], (R)8);

@@ -97,6 +97,15 @@ template <> struct M<float> {
     __device__ static __forceinline__ float pow(float x, float y) { return __expf(y * __logf(x)); }
 };
 
+// a / b in precision R.  FP32: the hardware reciprocal (1 ulp) and a product; the compiler's own FP32 division
+// expands differently from one place to the next (a constant divisor, a known range), so that two kernels
+// evaluating one expression could differ in the last bit.
+template <typename R> __device__ __forceinline__ R rdiv(R a, R b)
+{
+    if constexpr (sizeof(R) == 4) return a * __builtin_amdgcn_rcpf(b);
+    return a / b;
+}
+
 __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                                               uint32_t k1, uint32_t out[4])
 {

@@ -171,6 +171,42 @@ template <typename R, int B> constexpr int lwr_chunk()
     return chunk_of(LW_NG[B], WR_LWR_CHUNK >= 0 ? WR_LWR_CHUNK : (sizeof(R) == 8 ? LWR64_CHUNK[B] : LWR32_CHUNK[B]));
 }
 
+// the overlap factors of one step of a sweep and the layer's cloud fraction
+template <typename R> struct RtrStep {
+    R clfr, cld1, cld2, clr1, clr2, cmb1, cmb2;
+    bool start;  // a cloud block starts here
+};
+template <typename R>
+__device__ __forceinline__ RtrStep<R> rtr_step(const Rtr<R> &rt, int q0, int idx, int t, R clfr, bool start)
+{
+    return {clfr, rt.at(q0, idx, t), rt.at(q0 + 1, idx, t), rt.at(q0 + 2, idx, t), rt.at(q0 + 3, idx, t), rt.at(q0 + 4, idx, t),
+            rt.at(q0 + 5, idx, t), start};
+}
+// radiances of one g-point through a layer with cloud in some lane: total (tot), its cloudy and clear parts,
+// the overlap correction; gas and src the clear and cloudy sources, tr and trc the transmittances
+template <typename R>
+__device__ __forceinline__ void rtr_update(const RtrStep<R> &f, bool cloudy, R gas, R src, R tr, R trc, R &tot, R &cld, R &clr, R &rad)
+{
+    const R clear = tot * tr + gas;
+    R a = cld, b = clr, r = rad;
+    if (f.start) {
+        a = f.clfr * tot;
+        b = tot - a;
+        r = (R)0;
+    }
+    R na = a * trc + f.clfr * src;
+    R nb = b * tr + ((R)1 - f.clfr) * gas;
+    const R ntot = na + nb;
+    const R mod = r * (f.clr1 * tr + f.cld1 * trc) - f.cmb1 * gas + f.cmb2 * src;
+    const R nr = -mod + f.clr2 * (nb + mod) - f.cld2 * (na - mod);
+    na = na + nr;
+    nb = nb - nr;
+    tot = cloudy ? ntot : clear;
+    cld = cloudy ? na : a;
+    clr = cloudy ? nb : b;
+    rad = cloudy ? nr : r;
+}
+
 // One column of LW band B on the NAM route (rtrnmr), optics from the band tables Bt: down sweep, surface, up
 // sweep with the optics evaluated again, in chunks of g-points without per-g-point branches (as lw_column).
 template <typename R, int B, typename BT>
@@ -178,31 +214,29 @@ __device__ __forceinline__ void lwr_column(const Tabs<R> *__restrict__ T, const 
                                            int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
                                            const Rtr<R> &rt, int blk, int lane)
 {
-    constexpr int NG = LW_NG[B], CH = lwr_chunk<R, B>();
-    const int t = blk * 64 + lane;
-    if (t >= valid_cols(in, col0, n)) return;
+    constexpr int NG = LW_NG[B], GW = NG, CH = lwr_chunk<R, B>();
+    const Share<R> sh{nullptr, 0, 0};
+    const int nv = valid_cols(in, col0, n);
+    if (blk * 64 >= nv) return;
+    const bool ok = blk * 64 + lane < nv;  // lanes past the last column repeat it and store nothing
+    const int rl = ok ? lane : nv - 1 - blk * 64, t = blk * 64 + rl;
     const Surr none{};
     const LwCol<R> c = lw_col<R, B, false>(in, col0, cs, none, t);
     const int nrl = c.nrl;
     const RadCol rcol{in, c.i, nrl};
     const uint64_t lstu = rt.lstu[t], lstd = rt.lstd[t];
-    acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
+    if (ok) acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
     // radiances per g-point: total, its cloudy and clear parts, the overlap correction between them
-    R tot[NG], cld[NG], clr[NG], rad[NG];
+    R tot[1][GW], cld[GW], clr[GW], rad[GW], sfc0[1][GW];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) tot[g] = cld[g] = clr[g] = rad[g] = (R)0;
+    for (int g = 0; g < GW; ++g) tot[0][g] = cld[g] = clr[g] = rad[g] = (R)0;
     // one layer of a sweep; q0, idx: the overlap factors of its direction; start: a cloud block starts here
-    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, int q0, int idx, bool start, bool sfc, R pk0, R &s, R &s0) {
-        s = (R)0, s0 = (R)0;
+    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, int q0, int idx, bool start, bool sfc, R pk0) {
         const bool some = __any(y.cloudy);
-        R clfr = (R)0, cld1 = (R)0, cld2 = (R)0, clr1 = (R)0, clr2 = (R)0, cmb1 = (R)0, cmb2 = (R)0;
-        if (some) {
-            clfr = (R)rcol.cfrac(nrl - 1 - k);
-            cld1 = rt.at(q0, idx, t), cld2 = rt.at(q0 + 1, idx, t), clr1 = rt.at(q0 + 2, idx, t);
-            clr2 = rt.at(q0 + 3, idx, t), cmb1 = rt.at(q0 + 4, idx, t), cmb2 = rt.at(q0 + 5, idx, t);
-        }
+        RtrStep<R> f{};
+        if (some) f = rtr_step<R>(rt, q0, idx, t, (R)rcol.cfrac(nrl - 1 - k), start);
 #pragma unroll
-        for (int g0 = 0; g0 < NG; g0 += CH) {
+        for (int g0 = 0; g0 < GW; g0 += CH) {
             R tau[CH], fr[CH];
             lw_taufr<R, B, false, CH>(T, Bt, none, c, n, k, y.L, g0, tau, fr);
             GasV<R, CH> q;
@@ -212,70 +246,59 @@ __device__ __forceinline__ void lwr_column(const Tabs<R> *__restrict__ T, const 
                 for (int j = 0; j < CH; ++j) {
                     const int g = g0 + j;
                     const R r0 = c.semis * fr[j] * pk0;
-                    tot[g] = r0 + c.reflct * tot[g];
+                    tot[0][g] = r0 + c.reflct * tot[0][g];
                     cld[g] = clr[g] = rad[g] = (R)0;
-                    s0 = s0 + tot[g];
+                    sfc0[0][g] = tot[0][g];
                 }
             }
-            R gas[CH], nt[CH];
+            R gas[CH];
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                gas[j] = fr[j] * (y.blay + dplnk * q.gf[j]) * q.at[j];
-                nt[j] = tot[g0 + j] * q.tr[j] + gas[j];
-            }
+            for (int j = 0; j < CH; ++j) gas[j] = fr[j] * (y.blay + dplnk * q.gf[j]) * q.at[j];
             if (some) {
-                R tr[CH], at[CH], gf[CH];
-                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+                R trc[CH], at[CH], gf[CH];
+                lw_tot_v<R, CH>(T, q.od, y.odcld, trc, at, gf);
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
                     const int g = g0 + j;
                     const R src = fr[j] * (y.blay + dplnk * gf[j]) * at[j];
-                    R a = cld[g], b = clr[g], r = rad[g];
-                    if (start) {
-                        a = clfr * tot[g];
-                        b = tot[g] - a;
-                        r = (R)0;
-                    }
-                    R na = a * tr[j] + clfr * src;
-                    R nb = b * q.tr[j] + ((R)1 - clfr) * gas[j];
-                    const R ntot = na + nb;
-                    const R mod = r * (clr1 * q.tr[j] + cld1 * tr[j]) - cmb1 * gas[j] + cmb2 * src;
-                    const R nr = -mod + clr2 * (nb + mod) - cld2 * (na - mod);
-                    na = na + nr;
-                    nb = nb - nr;
-                    nt[j] = y.cloudy ? ntot : nt[j];
-                    cld[g] = y.cloudy ? na : a;
-                    clr[g] = y.cloudy ? nb : b;
-                    rad[g] = y.cloudy ? nr : r;
+                    rtr_update<R>(f, y.cloudy, gas[j], src, q.tr[j], trc[j], tot[0][g], cld[g], clr[g], rad[g]);
                 }
-            }
+            } else {
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                tot[g0 + j] = nt[j];
-                s = s + nt[j];
+                for (int j = 0; j < CH; ++j) tot[0][g0 + j] = tot[0][g0 + j] * q.tr[j] + gas[j];
             }
-            if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
     };
-    R s, s0;
+    LevelSum<R, NG, GW, 1> sum{sh, lane, 0, 0, 0};
+    auto dn = [&](int row, const R *s) {
+        if (ok) acc.lw_dn[(size_t)row * n + t] = s[0];
+    };
+    auto up = [&](int row, const R *s) {
+        if (ok) acc.lw_up[(size_t)row * n + t] = s[0];
+    };
+    sum.begin(nrl - 1, -1);
     for (int k = nrl - 1; k >= 0; --k) {  // down sweep, top to surface
         LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
-        sweep(k, y, y.bbot - y.blay, FCLD1D, k, (lstd >> k) & 1, false, (R)0, s, s0);
-        acc.lw_dn[(size_t)k * n + t] = s;
+        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
+        sweep(k, y, y.bbot - y.blay, FCLD1D, k, (lstd >> k) & 1, false, (R)0);
+        sum.put(tot, dn);
     }
+    sum.finish(dn);
+    sum.begin(0, 1);
     for (int k = 0; k < nrl; ++k) {  // up sweep, surface to top
         LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, lane, k, y);
+        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
         R btop = y.blay;  // above the top layer, its own temperature
         if (k + 1 < nrl) {
-            const LRow<R> up = lrow<R>(rp, blk, k + 1, lane);
-            btop = planck_of<R>(T, B, (int)(up.w(1) & 255u), up.f(LF_PB));
+            const LRow<R> nx = lrow<R>(rp, blk, k + 1, rl);
+            btop = planck_of<R>(T, B, (int)(nx.w(1) & 255u), nx.f(LF_PB));
         }
-        sweep(k, y, btop - y.blay, FCLD1U, k + 2, (lstu >> k) & 1, k == 0, y.bbot, s, s0);
-        if (k == 0) acc.lw_up[t] = s0;
-        acc.lw_up[(size_t)(k + 1) * n + t] = s;
+        sweep(k, y, btop - y.blay, FCLD1U, k + 2, (lstu >> k) & 1, k == 0, y.bbot);
+        if (k == 0) sum.put(sfc0, up);
+        sum.put(tot, up);
     }
+    sum.finish(up);
 }
 
 template <typename R, int B, bool EXT = true>
@@ -314,6 +337,19 @@ __global__ void __launch_bounds__((64 * lwrl_wpg<R, B>()), (lwr_waves<R, B>()))
 }
 
 // ---- SW band kernel of the NAM route (spcvrtc with cldfrc mixing and zcf1/zcf0 weighting) -------
+// o = zc0 o + zc1 d: the cloudy R/T of a layer mixed into the clear ones
+template <typename R, int CH> __device__ __forceinline__ void rt_mix(bool mix, R zc0, R zc1, const RtV<R, CH> &d, RtV<R, CH> &o)
+{
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        o.rb[j] = mix ? zc0 * o.rb[j] + zc1 * d.rb[j] : o.rb[j];
+        o.rd[j] = mix ? zc0 * o.rd[j] + zc1 * d.rd[j] : o.rd[j];
+        o.tb[j] = mix ? zc0 * o.tb[j] + zc1 * d.tb[j] : o.tb[j];
+        o.td[j] = mix ? zc0 * o.td[j] + zc1 * d.td[j] : o.td[j];
+        o.ld[j] = mix ? zc0 * o.ld[j] + zc1 * d.ld[j] : o.ld[j];
+    }
+}
+
 // One day column of one SW band on the NAM route: clear-sky pass, then (cloudy columns) the total-sky pass,
 // whose layers mix the cloudy R/T with the clear ones by the layer's cloud fraction over the column's
 // cover, zc1 = cfrac / zcf1 (phys_rrtm_sw_spcvrtc.cu, cloudy block); each pass is the adding method.
@@ -323,8 +359,12 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
                                            const AccT<R> &acc, int blk, int lane, WR_G char *slot, Fix64 *fx)
 {
     constexpr int NG = SW_NG[B], CH = sw_chunk<R, B, true>();
-    if (blk * 64 + lane >= *cs.nday) return;
-    const int t = cs.dlist[blk * 64 + lane], nrl = rp.nrl;
+    constexpr bool KEEP = sw_nv_mc<R>() > SW_NV;
+    const int nday = *cs.nday;
+    if (blk * 64 >= nday) return;
+    const bool ok = blk * 64 + lane < nday;  // lanes past the last day column repeat it and store nothing
+    const int rl = ok ? lane : nday - 1 - blk * 64;
+    const int t = cs.dlist[blk * 64 + rl], nrl = rp.nrl;
     SwCol<R> c;
     sw_col<R, B>(in, par, col0, cs, t, c);
     const RadCol rcol{in, c.i, nrl};
@@ -336,16 +376,17 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
         R zc1, zc0;
         bool mix;
     };
-    for (int pass = 0; pass < (total ? 2 : 1); ++pass) {
-        sw_adding<R, NG, CH>(
-            nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2},
+    const int passes = __any(total) ? 2 : 1;  // a column without cloud stores nothing in the second pass
+    for (int pass = 0; pass < passes; ++pass) {
+        sw_adding<R, NG, NG, CH, KEEP>(
+            nrl, c.asfc, SwSlot<R, NG, KEEP>{slot, lane, in.nlay + 2}, Share<R>{nullptr, 0, 0},
             [&](int k) {
                 Lay a;
-                sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, lane, k, a.y);
+                sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
                 a.mix = false, a.zc1 = (R)0, a.zc0 = (R)1;
                 if (pass && __any(a.y.cloudy)) {
                     const double zc1 = rcol.cfrac(nrl - 1 - k) / cf1;
-                    a.mix = zc1 > FTINY, a.zc1 = (R)zc1, a.zc0 = (R)(1.0 - zc1);
+                    a.mix = total && zc1 > FTINY, a.zc1 = (R)zc1, a.zc0 = (R)(1.0 - zc1);
                 }
                 return a;
             },
@@ -356,27 +397,20 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
                 if (__any(a.mix)) {
                     RtV<R, CH> d;
                     layer_rt_sky<R, CH>(T, tr, tg, a.y.y, ~0u, d, fx);
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) {
-                        o.rb[j] = a.mix ? a.zc0 * o.rb[j] + a.zc1 * d.rb[j] : o.rb[j];
-                        o.rd[j] = a.mix ? a.zc0 * o.rd[j] + a.zc1 * d.rd[j] : o.rd[j];
-                        o.tb[j] = a.mix ? a.zc0 * o.tb[j] + a.zc1 * d.tb[j] : o.tb[j];
-                        o.td[j] = a.mix ? a.zc0 * o.td[j] + a.zc1 * d.td[j] : o.td[j];
-                        o.ld[j] = a.mix ? a.zc0 * o.ld[j] + a.zc1 * d.ld[j] : o.ld[j];
-                    }
+                    rt_mix<R, CH>(a.mix, a.zc0, a.zc1, d, o);
                 }
             },
             [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
-            [&](int lev, R su, R sd) {
+            [&](int lev, const R *f) {
                 // pass 0 leaves the clear-sky fluxes in the band planes, which pass 1 reads back and mixes
                 const size_t p = (size_t)lev * n + t;
-                if (pass == 0) {
-                    if (lev == 0) acc.sw_clr0[t] = sd;
-                    acc.sw_up[p] = su;
-                    acc.sw_dn[p] = sd;
-                } else {
-                    acc.sw_up[p] = (R)(cf1 * (double)su + cf0 * (double)acc.sw_up[p]);
-                    acc.sw_dn[p] = (R)(cf1 * (double)sd + cf0 * (double)acc.sw_dn[p]);
+                if (ok && pass == 0) {
+                    if (lev == 0) acc.sw_clr0[t] = f[1];
+                    acc.sw_up[p] = f[0];
+                    acc.sw_dn[p] = f[1];
+                } else if (ok && total) {
+                    acc.sw_up[p] = (R)(cf1 * (double)f[0] + cf0 * (double)acc.sw_up[p]);
+                    acc.sw_dn[p] = (R)(cf1 * (double)f[1] + cf0 * (double)acc.sw_dn[p]);
                 }
             });
     }

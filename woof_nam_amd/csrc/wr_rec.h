@@ -21,6 +21,7 @@ namespace wr {
 
 struct ColScal {
     WR_G int *lw_laytrop, *lcf1, *day, *sw_laytrop, *dlist, *nday;
+    WR_G uint32_t *cblk;  // 4-layer blocks (from the surface) that hold cloud
     WR_G double *pwv, *zcf1, *zcf0;
     // per tile column, written by k_layers: la[kin * n + t] = log of the layer pressure (layer kin,
     // top-first); tz[L * n + t] = LW level temperature, L = 0 the top layer's temperature, L = kin + 1
@@ -28,32 +29,37 @@ struct ColScal {
     WR_G double *la, *tz;
 };
 
-enum { LF_F00 = 0, LF_F01, LF_F10, LF_F11, LF_SF, LF_SFR, LF_FF, LF_FFR, LF_MF, LF_SCM, LF_SCN2, LF_CA, LF_WX = LF_CA + 7,
-       LF_DRY = LF_WX + 4, LF_BRD, LF_P, LF_PL, LF_PB, LF_LIQ, LF_ICE, LF_N };
-enum { SF_F00 = 0, SF_F01, SF_F10, SF_F11, SF_SF, SF_SFR, SF_FF, SF_FFR, SF_CA, SF_MOL = SF_CA + 6, SF_LIQ, SF_ICE, SF_N };
+// Fields of a row.  The last ones are for FP32 only: column amounts that follow from the dry column and the
+// call's mixing ratios, which the FP64 kernels form themselves (the same two operations) instead of loading
+// 8 bytes each; in FP32 they are roundings of FP64 products, so they are kept.
+enum { LF_F00 = 0, LF_F01, LF_F10, LF_F11, LF_SF, LF_SFR, LF_FF, LF_FFR, LF_MF, LF_SCM, LF_SCN2, LF_CA0, LF_CA2, LF_DRY, LF_BRD,
+       LF_P, LF_PL, LF_PB, LF_LIQ, LF_ICE, LF_N64, LF_CA1 = LF_N64, LF_CA3, LF_WX = LF_CA3 + 4, LF_N32 = LF_WX + 4 };
+// SF_MOL: FP32 dry plus water vapour column, FP64 the dry column
+enum { SF_F00 = 0, SF_F01, SF_F10, SF_F11, SF_SF, SF_SFR, SF_FF, SF_FFR, SF_CA0, SF_CA2, SF_MOL, SF_LIQ, SF_ICE, SF_N64,
+       SF_CA1 = SF_N64, SF_CA3, SF_N32 = SF_CA3 + 3 };
 
 // bytes of a row (one layer of one 64-column block): index words, then the fields
-template <typename R> constexpr int lrow_bytes() { return 64 * (2 * 4 + LF_N * (int)sizeof(R)); }
-template <typename R> constexpr int srow_bytes() { return 64 * (2 * 4 + SF_N * (int)sizeof(R)); }
+constexpr int lrow_size(int rbytes) { return 64 * (2 * 4 + (rbytes == 4 ? LF_N32 : LF_N64) * rbytes); }
+constexpr int srow_size(int rbytes) { return 64 * (2 * 4 + (rbytes == 4 ? SF_N32 : SF_N64) * rbytes); }
+template <typename R> constexpr int lrow_bytes() { return lrow_size((int)sizeof(R)); }
+template <typename R> constexpr int srow_bytes() { return srow_size((int)sizeof(R)); }
 constexpr int MROW_LW = 16 * 64 * 2, MROW_SW = 14 * 64 * 2;  // McICA words of a row
-// bytes of a tile's records and words per 64-column block and layer
-constexpr size_t rec_block_bytes(int rbytes)
-{
-    return (size_t)64 * (4 * 4 + (LF_N + SF_N) * rbytes) + MROW_LW + MROW_SW;
-}
+// bytes of a tile's records per 64-column block and layer, in the larger precision, and of its words
+constexpr size_t rec_row_bytes(int rbytes) { return (size_t)lrow_size(rbytes) + srow_size(rbytes); }
+constexpr size_t mrow_bytes() { return MROW_LW + MROW_SW; }
 
 struct RecPtrs {
     WR_G char *lw, *sw, *mlw, *msw;  // [block][layer, surface first] rows
     int nrl;
     __device__ __forceinline__ size_t row(int blk, int k) const { return (size_t)blk * nrl + k; }
 };
-inline RecPtrs rec_ptrs(char *base, int n, int nrl, int rbytes)
+inline RecPtrs rec_ptrs(char *rec, char *words, int n, int nrl, int rbytes)
 {
     RecPtrs r;
     const size_t rows = (size_t)((n + 63) / 64) * nrl;
-    r.lw = gptr(base);
-    r.sw = r.lw + rows * 64 * (2 * 4 + LF_N * rbytes);
-    r.mlw = r.sw + rows * 64 * (2 * 4 + SF_N * rbytes);
+    r.lw = gptr(rec);
+    r.sw = r.lw + rows * lrow_size(rbytes);
+    r.mlw = gptr(words);
     r.msw = r.mlw + rows * MROW_LW;
     r.nrl = nrl;
     return r;
@@ -102,32 +108,55 @@ __device__ __forceinline__ R planck_of(const Tabs<R> *__restrict__ T, int b, int
 }
 
 // the layer quantities the band optics use, from a record row (unused fields are never loaded)
-template <typename R> __device__ __forceinline__ void lrow_get(const LRow<R> &r, uint32_t w, LwLay<R> &L)
+template <typename R>
+__device__ __forceinline__ void lrow_get(const LRow<R> &r, uint32_t w, const RunPar &par, LwLay<R> &L)
 {
     L.jp = w & 63, L.jt = ((w >> 6) & 3) + 1, L.jt1 = ((w >> 8) & 3) + 1, L.indself = (w >> 10) & 15;
     L.indfor = (w >> 14) & 3, L.indminor = (w >> 16) & 31, L.lower = (w >> 21) & 1;
     L.fac00 = r.f(LF_F00), L.fac01 = r.f(LF_F01), L.fac10 = r.f(LF_F10), L.fac11 = r.f(LF_F11);
     L.selffac = r.f(LF_SF), L.selffrac = r.f(LF_SFR), L.forfac = r.f(LF_FF), L.forfrac = r.f(LF_FFR);
     L.minorfrac = r.f(LF_MF), L.scaleminor = r.f(LF_SCM), L.scaleminorn2 = r.f(LF_SCN2);
-#pragma unroll
-    for (int m = 0; m < 7; ++m) L.colamt[m] = r.f(LF_CA + m);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) L.wx[m] = r.f(LF_WX + m);
     L.coldry = r.f(LF_DRY), L.colbrd = r.f(LF_BRD), L.pavel = r.f(LF_P);
+    L.colamt[0] = r.f(LF_CA0), L.colamt[2] = r.f(LF_CA2);
+    if constexpr (sizeof(R) == 4) {
+        L.colamt[1] = r.f(LF_CA1);
+#pragma unroll
+        for (int m = 3; m < 7; ++m) L.colamt[m] = r.f(LF_CA3 + m - 3);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) L.wx[m] = r.f(LF_WX + m);
+    } else {  // lw_layer's operations on the same dry column
+        const double floor = 1.0e-12 * L.coldry;
+        L.colamt[1] = fmax(floor, L.coldry * par.vmr[0]);
+        L.colamt[3] = fmax(floor, L.coldry * par.vmr[1]), L.colamt[4] = fmax(floor, L.coldry * par.vmr[2]);
+        L.colamt[5] = fmax(0.0, L.coldry * par.vmr[3]), L.colamt[6] = fmax(0.0, L.coldry * par.vmr[4]);
+        L.wx[0] = fmax(0.0, L.coldry * par.vmr[8]), L.wx[1] = fmax(0.0, L.coldry * par.vmr[5]);
+        L.wx[2] = fmax(0.0, L.coldry * par.vmr[6]), L.wx[3] = fmax(0.0, L.coldry * par.vmr[7]);
+    }
 }
-template <typename R> __device__ __forceinline__ void srow_get(const LRow<R> &r, uint32_t w, SwLay<R> &L)
+template <typename R>
+__device__ __forceinline__ void srow_get(const LRow<R> &r, uint32_t w, const RunPar &par, SwLay<R> &L)
 {
     L.jp = w & 63, L.jt = ((w >> 6) & 3) + 1, L.jt1 = ((w >> 8) & 3) + 1, L.indself = (w >> 10) & 15;
     L.indfor = (w >> 14) & 3;
     L.fac00 = r.f(SF_F00), L.fac01 = r.f(SF_F01), L.fac10 = r.f(SF_F10), L.fac11 = r.f(SF_F11);
     L.selffac = r.f(SF_SF), L.selffrac = r.f(SF_SFR), L.forfac = r.f(SF_FF), L.forfrac = r.f(SF_FFR);
+    L.colamt[0] = r.f(SF_CA0), L.colamt[2] = r.f(SF_CA2);
+    if constexpr (sizeof(R) == 4) {
+        L.colmol = r.f(SF_MOL);
+        L.colamt[1] = r.f(SF_CA1);
 #pragma unroll
-    for (int m = 0; m < 6; ++m) L.colamt[m] = r.f(SF_CA + m);
-    L.colmol = r.f(SF_MOL);
+        for (int m = 3; m < 6; ++m) L.colamt[m] = r.f(SF_CA3 + m - 3);
+    } else {  // sw_layer's operations on the same dry column
+        const double cd = r.f(SF_MOL), floor = 1.0e-12 * cd;
+        L.colmol = cd + L.colamt[0];
+        L.colamt[1] = fmax(floor, cd * par.vmr[0]);
+        L.colamt[3] = fmax(floor, cd * par.vmr[1]), L.colamt[4] = fmax(floor, cd * par.vmr[2]);
+        L.colamt[5] = fmax(floor, cd * par.vmr[3]);
+    }
 }
 
 // ---- LW records, layer logs and level temperatures: one thread per (column, layer) ----------------
-// Bound by the stores (124 bytes per layer and column in FP32, 240 in FP64).
+// Bound by the stores (124 bytes per layer and column in FP32, 168 in FP64).
 template <typename R>
 __global__ void __launch_bounds__(256) k_layers(const Tabs<R> *__restrict__ T, ColIn in, RunPar par, int col0, int n,
                                                 ColScal cs, RecPtrs rp)
@@ -160,10 +189,14 @@ __global__ void __launch_bounds__(256) k_layers(const Tabs<R> *__restrict__ T, C
     put(LF_F00, L.fac00), put(LF_F01, L.fac01), put(LF_F10, L.fac10), put(LF_F11, L.fac11);
     put(LF_SF, L.selffac), put(LF_SFR, L.selffrac), put(LF_FF, L.forfac), put(LF_FFR, L.forfrac);
     put(LF_MF, L.minorfrac), put(LF_SCM, L.scaleminor), put(LF_SCN2, L.scaleminorn2);
+    put(LF_CA0, L.colamt[0]), put(LF_CA2, L.colamt[2]);
+    if constexpr (sizeof(R) == 4) {
+        put(LF_CA1, L.colamt[1]);
 #pragma unroll
-    for (int m = 0; m < 7; ++m) put(LF_CA + m, L.colamt[m]);
+        for (int m = 3; m < 7; ++m) put(LF_CA3 + m - 3, L.colamt[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) put(LF_WX + m, L.wx[m]);
+        for (int m = 0; m < 4; ++m) put(LF_WX + m, L.wx[m]);
+    }
     put(LF_DRY, L.coldry), put(LF_BRD, L.colbrd), put(LF_P, L.pavel), put(LF_PL, fl), put(LF_PB, fb);
     put(LF_LIQ, (R)L.clwp), put(LF_ICE, (R)L.ciwp);
 }
@@ -189,21 +222,22 @@ __global__ void __launch_bounds__(256) k_layers_sw(const Tabs<R> *__restrict__ T
     auto put = [&](int i, R x) { f[i * 64] = x; };
     put(SF_F00, L.fac00), put(SF_F01, L.fac01), put(SF_F10, L.fac10), put(SF_F11, L.fac11);
     put(SF_SF, L.selffac), put(SF_SFR, L.selffrac), put(SF_FF, L.forfac), put(SF_FFR, L.forfrac);
+    put(SF_CA0, L.colamt[0]), put(SF_CA2, L.colamt[2]);
+    if constexpr (sizeof(R) == 4) {
+        put(SF_CA1, L.colamt[1]);
 #pragma unroll
-    for (int m = 0; m < 6; ++m) put(SF_CA + m, L.colamt[m]);
-    put(SF_MOL, L.colmol), put(SF_LIQ, (R)L.cwp), put(SF_ICE, (R)L.cip);
+        for (int m = 3; m < 6; ++m) put(SF_CA3 + m - 3, L.colamt[m]);
+    }
+    put(SF_MOL, sizeof(R) == 4 ? L.colmol : L.coldry), put(SF_LIQ, (R)L.cwp), put(SF_ICE, (R)L.cip);
 }
 
 // ---- McICA words: one thread per (column or day-list entry, band) ----------------------------------
 // The same draws and rule as mcica_g.  Bound by the Philox multiplies of the cloudy blocks.
 template <int NG>
-__device__ __forceinline__ void mcica_words(const RadCol &rc, uint64_t col, uint64_t seed, int kind, int g0, int iovr,
+__device__ __forceinline__ void mcica_words(const RadCol &rc, uint32_t blocks, uint64_t col, uint64_t seed, int kind, int g0, int iovr,
                                             WR_G char *m, size_t row0, int rowbytes, int b, int lane)
 {
     const int nrl = rc.nrl;
-    uint32_t blocks = 0;  // 4-layer blocks (from the surface) that hold cloud
-    for (int k = 0; k < nrl; ++k)
-        if (rc.cfrac(nrl - 1 - k) > 0.0) blocks |= 1u << (k >> 2);
     double prev[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) prev[g] = 0.0;
@@ -243,15 +277,15 @@ __device__ __forceinline__ void mcica_words(const RadCol &rc, uint64_t col, uint
     }
 }
 template <int B>
-__device__ __forceinline__ void mcica_band(int b, const RadCol &rc, uint64_t col, uint64_t seed, int iovr, const RecPtrs &rp,
+__device__ __forceinline__ void mcica_band(int b, const RadCol &rc, uint32_t blocks, uint64_t col, uint64_t seed, int iovr, const RecPtrs &rp,
                                            size_t row0, int lane)
 {
     if constexpr (B < 30) {
-        if (b != B) return mcica_band<B + 1>(b, rc, col, seed, iovr, rp, row0, lane);
+        if (b != B) return mcica_band<B + 1>(b, rc, blocks, col, seed, iovr, rp, row0, lane);
         if constexpr (B < 16)
-            mcica_words<LW_NG[B]>(rc, col, seed, 0, LW_NS[B], iovr, rp.mlw, row0, MROW_LW, B, lane);
+            mcica_words<LW_NG[B]>(rc, blocks, col, seed, 0, LW_NS[B], iovr, rp.mlw, row0, MROW_LW, B, lane);
         else
-            mcica_words<SW_NG[B - 16]>(rc, col, seed, 1, SW_NS[B - 16], iovr, rp.msw, row0, MROW_SW, B - 16, lane);
+            mcica_words<SW_NG[B - 16]>(rc, blocks, col, seed, 1, SW_NS[B - 16], iovr, rp.msw, row0, MROW_SW, B - 16, lane);
     }
 }
 static __global__ void __launch_bounds__(64) k_mcica(ColIn in, RunPar par, int col0, int n, ColScal cs,
@@ -264,7 +298,7 @@ static __global__ void __launch_bounds__(64) k_mcica(ColIn in, RunPar par, int c
     const RadCol rc{in, col0 + t, rp.nrl};
     const uint64_t col = in.col_id ? in.col_id[col0 + t] : (uint64_t)(col0 + t);
     const uint64_t seed = in.seed_dev ? *in.seed_dev : par.seed;
-    mcica_band<0>(b, rc, col, seed, par.iovr, rp, rp.row(blk, 0), lane);
+    mcica_band<0>(b, rc, cs.cblk[t], col, seed, par.iovr, rp, rp.row(blk, 0), lane);
 }
 
 }  // namespace wr

@@ -19,7 +19,7 @@ constexpr int SW_IDXSFC[14] = {1, 1, 1, 1, 1, 1, 1, 1, 0, 2, 2, 2, 2, 1};
 template <typename R> struct SwLay {
     int jp, jt, jt1, indself, indfor;
     R fac00, fac01, fac10, fac11, selffac, selffrac, forfac, forfrac;
-    R colamt[6], colmol;
+    R colamt[6], colmol, coldry;
     double ct, cwp, cip, delp;
 };
 
@@ -47,6 +47,7 @@ __device__ __forceinline__ void sw_layer(const Tabs<R> *__restrict__ T, const Ra
     ca[4] = fmax(tc, cd * par.vmr[2]);
     ca[5] = fmax(tc, cd * par.vmr[3]);
     L.colmol = (R)(cd + ca[0]);
+    L.coldry = (R)cd;
 #pragma unroll
     for (int m = 0; m < 6; ++m) L.colamt[m] = (R)ca[m];
     L.delp = dl;
@@ -159,7 +160,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[4];
-            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
@@ -170,7 +171,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)6.86e-10;
         const R speccomb = ca[0] + Bt.strrat * ca[1];
         if (kk <= Lt) {
-            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(((jp - 1) * 5 + (jt - 1)) * 9, (jp * 5 + (jt1 - 1)) * 9, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
@@ -179,7 +180,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
                 tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (selfpart + ff * forpart);
             }
         } else {
-            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(((jp - 13) * 5 + (jt - 1)) * 5, ((jp - 12) * 5 + (jt1 - 1)) * 5, js, 1175, 5, 6, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc) + (ca[0] * ff) * FORI(g0 + jj);
@@ -188,7 +189,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[4];
-            const R ratio = (speccomb > (R)0) ? (ca[0] / speccomb) : (R)0;
+            const R ratio = (speccomb > (R)0) ? (rdiv<R>(ca[0], speccomb)) : (R)0;
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ratio), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
@@ -200,7 +201,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)2.29e-09;
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[1];
-            const int js = jsfs<R>((R)8 * fmin((R)0.999999, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)0.999999, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
@@ -224,13 +225,13 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * (R)9.41e-09;
         const R speccomb = ca[0] + Bt.strrat * ca[1];
         if (kk < Lt) {
-            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc) + ca[0] * (sf * SELFI(g0 + jj) + ff * FORI(g0 + jj));
         }
         if (kk >= Lt) {
-            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 1175, 5, 6, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc) + ca[0] * ff * FORI(g0 + jj);
@@ -240,7 +241,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         const R o2cont = (R)(4.35e-4 / (350.0 * 2.0)) * ca[5];
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[5];
-            const R ratio = (speccomb > (R)0) ? (ca[0] / speccomb) : (R)0;
+            const R ratio = (speccomb > (R)0) ? (rdiv<R>(ca[0], speccomb)) : (R)0;
             const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ratio), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
@@ -260,7 +261,7 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
     } else if constexpr (B == 8) { /* band 24 */
         if (kk <= Lt) {
             const R speccomb = ca[0] + Bt.strrat * ca[5];
-            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[0] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, rdiv<R>(ca[0], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) {
@@ -294,12 +295,12 @@ __device__ __forceinline__ void sw_optics_t(const Tabs<R> *__restrict__ T, const
         _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tr[jj] = cm * Bt.rayl;
         const R speccomb = ca[2] + Bt.strrat * ca[5];
         if (kk <= Lt) {
-            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, ca[2] / speccomb), fs);
+            const int js = jsfs<R>((R)8 * fmin((R)ONEMINUS, rdiv<R>(ca[2], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 585, 9, 10, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absa, ng, g0 + jj, id, fc);
         } else {
-            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, ca[2] / speccomb), fs);
+            const int js = jsfs<R>((R)4 * fmin((R)ONEMINUS, rdiv<R>(ca[2], speccomb)), fs);
             fac8<R>(fs, f00, f01, f10, f11, fc);
             ind8(id0, id1, js, 1175, 5, 6, id);
             _Pragma("unroll") for (int jj = 0; jj < NGL; ++jj) tg[jj] = speccomb * sum8<R>(Bt.absb, ng, g0 + jj, id, fc);
