@@ -79,21 +79,28 @@ __device__ __forceinline__ LutF lut_f32(int i, bool lw_cap)
 #define WR_L
 #endif
 // The tables of one LW band; P is the pointer type (global by default, LDS in the staged kernels),
-// PB that of absb.
-template <typename R, typename P = const WR_G R *, typename PB = P> struct LwBandT {
+// PB that of absb, PM that of ka_m.
+template <typename R, typename P = const WR_G R *, typename PB = P, typename PM = P> struct LwBandT {
     P absa;
     PB absb;
     P selfref, forref, fracrefa, fracrefb;
-    P ka_m[3], kb_m[3];
+    PM ka_m[3];
+    P kb_m[3];
     P x1, x2;
+    P etab;  // exp_tbl
     R refrat_planck_a, refrat_planck_b, refrat_m_a, refrat_m_b, refrat_m_a3;
 };
 template <typename R> using LwBand = LwBandT<R>;
 // The same tables packed into one image: 14 tables (absa absb selfref forref fracrefa fracrefb
 // ka_m[0..2] kb_m[0..2] x1 x2) at element offsets off[] (multiples of 4, -1 where the image does not
 // hold one), n elements in all (a multiple of 4), from a 256-byte aligned base.  The FP64 image leaves
-// absb out.
+// absb out, and ka_m of the bands that would not leave room for the transmittance table (lw64_kam).
 constexpr int LW_IMG_T = 14;
+// bytes of exp_tbl in LDS, behind a band's FP64 image (16-byte words)
+constexpr size_t ETAB_LDS = ((NTBL + 1) * sizeof(double) + 15) & ~(size_t)15;
+// FP64: whether the band's image holds ka_m.  Bands 3 and 5 (16 g-points, 9 mixtures of two gases) have 22 KB of
+// it beside 78 KB of other tables; with the 80 KB of exp_tbl that is more than the 160 KB of a CU.
+__host__ __device__ constexpr bool lw64_kam(int band0) { return band0 != 2 && band0 != 4; }
 template <typename R> struct LwImg {
     const WR_G R *base;
     int n;
@@ -123,7 +130,6 @@ template <typename R> struct Tabs {
     const WR_G int32_t *ipat, *layreffr, *ix1, *ix2, *ibx;
     const WR_G R *exp_tbl, *tfn_tbl, *tau_tbl, *sw_exp_tbl;
     const WR_G R *chir;    // [6][59] reference ratios of the binary gas pairs (chi_row in wr_lw.h)
-    const WR_G R *lut4;    // FP64: [NTBL + 1]{exp, tfn, tau, 0}, the LW tables of one index side by side
     const WR_G double *sw_exp_tbl64;  // FP64 SW exp table (layers that take the FP64 R/T branch)
     const WR_G R *sf01, *sf02, *sf03, *sw_strrat, *sw_specwt;
     const WR_G R *extliq1, *ssaliq1, *asyliq1, *extice3, *ssaice3, *asyice3;

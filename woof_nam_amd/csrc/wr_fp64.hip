@@ -7,7 +7,7 @@ namespace {
 using namespace wr;
 
 // rlwinit / rswinit look-up tables (phys_rrtm_lw_rtrnmr.py:97-132, phys_rrtm_sw_rswinit.cu:310-345)
-__global__ void k_luts(double *exp_tbl, double *tfn_tbl, double *tau_tbl, double *sw_exp_tbl, double *lut4)
+__global__ void k_luts(double *exp_tbl, double *tfn_tbl, double *tau_tbl, double *sw_exp_tbl)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i > NTBL) return;
@@ -25,15 +25,13 @@ __global__ void k_luts(double *exp_tbl, double *tfn_tbl, double *tau_tbl, double
         tfn_tbl[i] = (tau < 0.06) ? tau / 6.0 : 1.0 - 2.0 * ((1.0 / tau) - (e / (1.0 - e)));
         sw_exp_tbl[i] = exp_d(-(bpade * tfn));
     }
-    lut4[4 * i] = exp_tbl[i], lut4[4 * i + 1] = tfn_tbl[i], lut4[4 * i + 2] = tau_tbl[i], lut4[4 * i + 3] = 0.0;
 }
 }  // namespace
 
 int wr_init_luts(wr_ctx *c, hipStream_t s)
 {
     hipLaunchKernelGGL(k_luts, dim3((wr::NTBL + 256) / 256), dim3(256), 0, s, (double *)c->host_d.exp_tbl,
-                       (double *)c->host_d.tfn_tbl, (double *)c->host_d.tau_tbl, (double *)c->host_d.sw_exp_tbl,
-                       (double *)c->host_d.lut4);
+                       (double *)c->host_d.tfn_tbl, (double *)c->host_d.tau_tbl, (double *)c->host_d.sw_exp_tbl);
     return hipGetLastError() == hipSuccess ? WR_OK : WR_ERR_HIP;
 }
 

@@ -210,11 +210,11 @@ template <typename R> int bind_tables(const TFile &f, Blob &b, Tabs<R> &T)
     T.tfn_tbl = b.reserve<R>(NTBL + 1);
     T.tau_tbl = b.reserve<R>(NTBL + 1);
     T.sw_exp_tbl = b.reserve<R>(NTBL + 1);
-    if (sizeof(R) == 8) T.lut4 = b.reserve<R>(4 * (NTBL + 1));
 
     for (int k = 0; k < 16; ++k) {
         LwBand<R> &B = T.lw[k];
         const int bn = k + 1;
+        B.etab = T.exp_tbl;
         B.absa = d.need<R>(bname("lw", bn, "absa", true));
         B.absb = (k != 5 && k != 11 && k != 12 && k != 14) ? d.need<R>(bname("lw", bn, "absb", true))
                                                              : d.opt<R>(bname("lw", bn, "absb", true));
@@ -257,7 +257,7 @@ template <typename R> int bind_tables(const TFile &f, Blob &b, Tabs<R> &T)
         for (const Slot &s : slots)
             if (s.band == k + 1)
                 ent[s.kind == 0 ? 6 + s.idx : s.kind == 1 ? 9 + s.idx : s.kind == 2 ? 12 : 13] =
-                    d.find(bname("lw", s.band, s.key, true));
+                    sizeof(R) == 8 && s.kind == 0 && !lw64_kam(k) ? nullptr : d.find(bname("lw", s.band, s.key, true));
         LwImg<R> &im = T.lw_img[k];
         int n = 0;
         for (int j = 0; j < LW_IMG_T; ++j) {
@@ -516,7 +516,7 @@ bool lw_glane_env()
 // WR_LW_LDS64 does the same for the FP64 McICA LW kernels (k_lwl64 in place of k_lw).  The defaults
 // are the measured choice per band on the 954x835x60 grid: every FP32 band (LW sum 101 -> 97 ms per
 // call), every FP64 band but 14 (LW sum 233 -> 216 ms; band 14 ran 7 % slower).
-constexpr uint32_t LW_LDS_DEFAULT = 0xffffu, LW_LDS64_DEFAULT = 0xffffu & ~(1u << 13);
+constexpr uint32_t LW_LDS_DEFAULT = 0xffffu, LW_LDS64_DEFAULT = 0xffffu;
 // WR_SW_LDS / WR_SW_LDS64 (bit B = band B + 16) choose k_swl over k_sw the same way.  Measured per
 // band (serialised, 954x835x60): FP64 SW bands 17-24 and 29 run 3-9 % faster from LDS, 25, 26, 28
 // slower (the FP64 call 320 -> 312 ms with this mask); in FP32 the SW sum went 62.0 -> 65.4 ms, so
@@ -527,12 +527,12 @@ constexpr uint32_t LWR_LDS_DEFAULT = 0xffffu, LWR_LDS64_DEFAULT = 0xffffu;
 // WR_SWR_LDS / WR_SWR_LDS64: the NAM route's SW kernels (k_swrl over k_swr), on the SW images.
 constexpr uint32_t SWR_LDS_DEFAULT = 0x0u, SWR_LDS64_DEFAULT = 0x3fffu;
 template <typename R, typename I>
-uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_max)
+uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_max, size_t more = 0)
 {
     const char *e = getenv(env);
     uint32_t m = e ? (uint32_t)strtoul(e, nullptr, 16) : dflt;
     for (int b = 0; b < nb; ++b)
-        if (img[b].n <= 0 || (size_t)img[b].n * sizeof(R) > (size_t)lds_max) m &= ~(1u << b);
+        if (img[b].n <= 0 || (size_t)img[b].n * sizeof(R) + more > (size_t)lds_max) m &= ~(1u << b);
     return m & ((1u << nb) - 1u);
 }
 
@@ -569,11 +569,12 @@ Sizes sizes(int32_t max_cols)
     z.rec = std::max(rec_row_bytes(8), rec_row_bytes(4)) * rows;              // layer records
     z.lwrec = lw_glane_env() ? lwrec_bytes_per_col<double>(64 + 1) * m + 3 * 256 : 0;  // LW layer records
     // level pool: room for every 64-column block of a tile in the largest slot layout (FP64 SW:
-    // 2 values, FP32 SW: 7 values, x 16 g x levels), at most WR_POOL_GB (default 3) GB per stream:
+    // 2 values, FP32 SW: 5 values, x 16 g x levels; FP64 LW), at most WR_POOL_GB (default 3) GB per stream:
     // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB
     const int nl_max = 64;
-    const size_t lane_max = std::max(cache_slot_bytes(SW_NV, 16, nl_max + 1, (int)sizeof(double)),
-                                     cache_slot_bytes(sw_nv_mc<float>(), 16, nl_max + 1, (int)sizeof(float)));
+    const size_t lane_max = std::max({cache_slot_bytes(sw_nv<double>(), 16, nl_max + 1, (int)sizeof(double)),
+                                      cache_slot_bytes(sw_nv<float>(), 16, nl_max + 1, (int)sizeof(float)),
+                                      lw64_slot_bytes(16, nl_max + 1)});
     const size_t need = (m + 63) / 64 * lane_max;
     const char *pe = getenv("WR_POOL_GB");
     const double gb = pe ? atof(pe) : 3.0;
@@ -692,10 +693,10 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
             hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
             rc = WR_ERR_HIP;
         c->lw_lds = lds_mask<float>("WR_LW_LDS", LW_LDS_DEFAULT, c->host_f.lw_img, 16, c->lds_max);
-        c->lw_lds64 = lds_mask<double>("WR_LW_LDS64", LW_LDS64_DEFAULT, c->host_d.lw_img, 16, c->lds_max);
+        c->lw_lds64 = lds_mask<double>("WR_LW_LDS64", LW_LDS64_DEFAULT, c->host_d.lw_img, 16, c->lds_max, ETAB_LDS);
         c->sw_lds = lds_mask<float>("WR_SW_LDS", SW_LDS_DEFAULT, c->host_f.sw_img, 14, c->lds_max);
         c->lwr_lds = lds_mask<float>("WR_LWR_LDS", LWR_LDS_DEFAULT, c->host_f.lw_img, 16, c->lds_max);
-        c->lwr_lds64 = lds_mask<double>("WR_LWR_LDS64", LWR_LDS64_DEFAULT, c->host_d.lw_img, 16, c->lds_max);
+        c->lwr_lds64 = lds_mask<double>("WR_LWR_LDS64", LWR_LDS64_DEFAULT, c->host_d.lw_img, 16, c->lds_max, ETAB_LDS);
         c->swr_lds = lds_mask<float>("WR_SWR_LDS", SWR_LDS_DEFAULT, c->host_f.sw_img, 14, c->lds_max);
         c->swr_lds64 = lds_mask<double>("WR_SWR_LDS64", SWR_LDS64_DEFAULT, c->host_d.sw_img, 14, c->lds_max);
         c->sw_lds64 = lds_mask<double>("WR_SW_LDS64", SW_LDS64_DEFAULT, c->host_d.sw_img, 14, c->lds_max);

@@ -511,10 +511,12 @@ template <typename R, int NG, int GW, int NQ> struct LevelSum {
 // is skipped as a whole.
 
 // Transmittance, source factor and optical depth of the LW tables at od (rtrnmc's tblind quantisation).
-// FP64 reads the table the oracle reproduces; FP32 evaluates the entry.  FP32: tblind of the largest
+// FP64 takes the transmittance from the table etab that the oracle reproduces (LDS in the staged kernels) and evaluates
+// the rest of the entry (lut_rest): the gather of whole entries from L2, 64 lanes on 64 lines, bound the FP64 kernels
+// (15 TB/s of L2 reads at 0.34 of the issue slots).  FP32 evaluates the entry.  FP32: tblind of the largest
 // depths rounds to 1, where the table ends in (1e-20, 1, 1e10); the index stops just below it, which gives
 // those values to FP32 accuracy.  tau and 1 / tau share one reciprocal.
-template <typename R> __device__ __forceinline__ void lw_lut(const Tabs<R> *__restrict__ T, R od, R &e, R &tfn, R &tau)
+template <typename R, typename PE> __device__ __forceinline__ void lw_lut(PE etab, R od, R &e, R &tfn, R &tau)
 {
     if constexpr (sizeof(R) == 4) {
         const R tb = od * __builtin_amdgcn_rcpf((R)(1.0 / 0.278) + od);
@@ -528,16 +530,17 @@ template <typename R> __device__ __forceinline__ void lw_lut(const Tabs<R> *__re
         tfn = tau < (R)0.06 ? tau * (R)(1.0 / 6.0) : big;
     } else {
         const R tb = od / ((R)(1.0 / 0.278) + od);
-        const f64x4v q = ((const WR_G f64x4v *)T->lut4)[imin(NTBL, (int)((R)NTBL * tb + (R)0.5))];
-        e = q.x, tfn = q.y, tau = q.z;
+        const int i = imin(NTBL, (int)((R)NTBL * tb + (R)0.5));
+        e = etab[i];
+        lut_rest(i, NTBL, e, tfn, tau);
     }
 }
 
 template <typename R, int CH> struct GasV {  // CH g-points: transmittance, absorptance, source factor, optical depth
     R tr[CH], at[CH], gf[CH], od[CH];
 };
-template <typename R, int CH>
-__device__ __forceinline__ void lw_gas_v(const Tabs<R> *__restrict__ T, R sdif, R taer, const R *tau, GasV<R, CH> &q)
+template <typename R, int CH, typename PE>
+__device__ __forceinline__ void lw_gas_v(PE etab, R sdif, R taer, const R *tau, GasV<R, CH> &q)
 {
     bool any = false;
 #pragma unroll
@@ -553,7 +556,7 @@ __device__ __forceinline__ void lw_gas_v(const Tabs<R> *__restrict__ T, R sdif, 
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             R e, tfn, ta;
-            lw_lut<R>(T, q.od[j], e, tfn, ta);
+            lw_lut<R>(etab, q.od[j], e, tfn, ta);
             const bool big = !(q.od[j] <= (R)0.06);
             q.tr[j] = big ? e : q.tr[j];
             q.at[j] = big ? (R)1 - e : q.at[j];
@@ -563,8 +566,8 @@ __device__ __forceinline__ void lw_gas_v(const Tabs<R> *__restrict__ T, R sdif, 
     }
 }
 // the same for the total (gas plus cloud) optical depth: transmittance, absorptance, source factor
-template <typename R, int CH>
-__device__ __forceinline__ void lw_tot_v(const Tabs<R> *__restrict__ T, const R *od, R odcld, R *tr, R *at, R *gf)
+template <typename R, int CH, typename PE>
+__device__ __forceinline__ void lw_tot_v(PE etab, const R *od, R odcld, R *tr, R *at, R *gf)
 {
     bool any = false;
 #pragma unroll
@@ -580,7 +583,7 @@ __device__ __forceinline__ void lw_tot_v(const Tabs<R> *__restrict__ T, const R 
         for (int j = 0; j < CH; ++j) {
             const R x = od[j] + odcld;
             R e, tfn, ta;
-            lw_lut<R>(T, x, e, tfn, ta);
+            lw_lut<R>(etab, x, e, tfn, ta);
             const bool big = !(x < (R)0.06);
             tr[j] = big ? e : tr[j];
             at[j] = big ? (R)1 - e : at[j];
@@ -647,12 +650,16 @@ __device__ __forceinline__ void lw_taufr(const Tabs<R> *__restrict__ T, const BT
         lw_optics_t<R, B, CH>(T, Bt, L, tau, fr, g0);
 }
 
-// One column of LW band B in FP64, optics from the band tables Bt: down sweep, surface, up sweep with the
-// optics evaluated again.  Every sum and product in the reference's order.
+// One column of LW band B in FP64, optics from the band tables Bt: the down sweep also forms each layer's
+// upward gas source and, where a g-point has cloud, the cloud correction, and leaves them with the transmittance
+// in the wave's pool slot, so that the up sweep needs no optics.  Every sum and product in the reference's order.
+// Slot, per lane: [layer][g] {transmittance, upward gas source}; [layer][g] cloud minus gas source, written and
+// read only where a chunk has cloud; [layer] cloud transmittance.
+__host__ __device__ constexpr size_t lw64_slot_bytes(int ng, int nk) { return (size_t)64 * sizeof(double) * nk * (3 * ng + 1); }
 template <typename R, int B, bool SURR, typename BT>
 __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par,
                                           int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
-                                          const Surr &sg, int blk, int lane)
+                                          const Surr &sg, int blk, int lane, WR_G char *slot)
 {
     constexpr int NG = LW_NG[B], GW = NG, CH = lw_chunk_r<R, B>();
     const Share<R> sh{nullptr, 0, 0};
@@ -662,53 +669,12 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
     const int rl = ok ? lane : nv - 1 - blk * 64, t = blk * 64 + rl;
     const LwCol<R> c = lw_col<R, B, SURR>(in, col0, cs, sg, t);
     const int nrl = c.nrl;
+    WR_G f64x2v *const tg = (WR_G f64x2v *)slot + lane;
+    WR_G R *const cg = (WR_G R *)((WR_G f64x2v *)slot + (size_t)nrl * NG * 64) + lane, *const ef = cg + (size_t)nrl * NG * 64;
     if (ok) acc.lw_dn[(size_t)nrl * n + t] = (R)0;  // no downward LW at the top
-    R rad[1][GW], sfc0[1][GW];
+    R rad[1][GW];
 #pragma unroll
     for (int g = 0; g < GW; ++g) rad[0][g] = (R)0;
-    // one layer of a sweep: the source lies between the layer and the level the radiation leaves through
-    auto sweep = [&](int k, const LwLayer<R> &y, R dplnk, uint32_t bits, bool sfc, R pk0) {
-        R ecld = (R)1;
-        if (__any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
-#pragma unroll
-        for (int g0 = 0; g0 < GW; g0 += CH) {
-            R tau[CH], fr[CH];
-            lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
-            GasV<R, CH> q;
-            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
-            if (sfc) {  // surface emission and reflection
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const R rad0 = c.semis * fr[j] * pk0;
-                    rad[0][g0 + j] = rad0 + c.reflct * rad[0][g0 + j];
-                    sfc0[0][g0 + j] = rad[0][g0 + j];
-                }
-            }
-            R nr[CH], gas[CH];
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const R bb = fr[j] * (y.blay + dplnk * q.gf[j]);
-                gas[j] = bb * q.at[j];
-                nr[j] = rad[0][g0 + j] * q.tr[j] + gas[j];
-            }
-            const uint32_t cb = bits >> g0;
-            if (__any(cb & ((1u << CH) - 1u))) {
-                R tr[CH], at[CH], gf[CH];
-                lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
-                const R efclrfr = (R)1 - ((R)1 - ecld);
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const R bbt = fr[j] * (y.blay + dplnk * gf[j]);
-                    const R tot = bbt * at[j];
-                    const R rc = rad[0][g0 + j] * q.tr[j] * efclrfr + gas[j] + (tot - gas[j]);
-                    nr[j] = (cb >> j) & 1u ? rc : nr[j];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < CH; ++j) rad[0][g0 + j] = nr[j];
-            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
-        }
-    };
     LevelSum<R, NG, GW, 1> sum{sh, lane, 0, 0, 0};
     auto dn = [&](int row, const R *s) {
         if (ok) acc.lw_dn[(size_t)row * n + t] = s[0];
@@ -716,28 +682,93 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
     auto up = [&](int row, const R *s) {
         if (ok) acc.lw_up[(size_t)row * n + t] = s[0];
     };
+    R btop = (R)0;  // Planck function at the level above the layer; above the top layer its own temperature's
     sum.begin(nrl - 1, -1);
     for (int k = nrl - 1; k >= 0; --k) {  // down sweep, top to surface
         LwLayer<R> y;
         lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
         const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl) : 0u;
-        sweep(k, y, y.bbot - y.blay, bits, false, (R)0);
+        if (k == nrl - 1) btop = y.blay;
+        const R dd = y.bbot - y.blay, du = btop - y.blay;
+        R efclrfr = (R)1;
+        if (__any(y.cloudy)) {
+            efclrfr = (R)1 - ((R)1 - M<R>::exp(-y.odcld));
+            ef[(size_t)k * 64] = efclrfr;
+        }
+        R sfc0[GW];
+#pragma unroll
+        for (int g0 = 0; g0 < GW; g0 += CH) {
+            R tau[CH], fr[CH];
+            lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
+            GasV<R, CH> q;
+            lw_gas_v<R, CH>(Bt.etab, c.sdif, y.taer, tau, q);
+            R nr[CH], gas[CH], gup[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                gas[j] = fr[j] * (y.blay + dd * q.gf[j]) * q.at[j];
+                gup[j] = fr[j] * (y.blay + du * q.gf[j]) * q.at[j];
+                tg[((size_t)k * NG + g0 + j) * 64] = (f64x2v){q.tr[j], gup[j]};
+                nr[j] = rad[0][g0 + j] * q.tr[j] + gas[j];
+            }
+            const uint32_t cb = bits >> g0;
+            if (__any(cb & ((1u << CH) - 1u))) {
+                R tr[CH], at[CH], gf[CH];
+                lw_tot_v<R, CH>(Bt.etab, q.od, y.odcld, tr, at, gf);
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const R td = fr[j] * (y.blay + dd * gf[j]) * at[j], tu = fr[j] * (y.blay + du * gf[j]) * at[j];
+                    cg[((size_t)k * NG + g0 + j) * 64] = tu - gup[j];
+                    const R rc = rad[0][g0 + j] * q.tr[j] * efclrfr + gas[j] + (td - gas[j]);
+                    nr[j] = (cb >> j) & 1u ? rc : nr[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                rad[0][g0 + j] = nr[j];
+                if (k == 0) {  // surface emission and reflection start the upward sweep
+                    const R rad0 = c.semis * fr[j] * y.bbot;
+                    sfc0[g0 + j] = rad0 + c.reflct * nr[j];
+                }
+            }
+            if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
+        }
         sum.put(rad, dn);
+        if (k == 0) {
+#pragma unroll
+            for (int g = 0; g < GW; ++g) rad[0][g] = sfc0[g];
+        }
+        btop = y.bbot;
     }
     sum.finish(dn);
     sum.begin(0, 1);
+    sum.put(rad, up);
     for (int k = 0; k < nrl; ++k) {  // up sweep, surface to top
-        LwLayer<R> y;
-        lw_get<R, B>(T, in, par, rp, c, blk, rl, k, y);
-        const uint32_t bits = y.cloudy ? mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl) : 0u;
-        // the level above is the next layer's lower level; above the top layer, its own temperature
-        R btop = y.blay;
-        if (k + 1 < nrl) {
-            const LRow<R> nx = lrow<R>(rp, blk, k + 1, rl);
-            btop = planck_of<R>(T, B, (int)(nx.w(1) & 255u), nx.f(LF_PB));
+        const bool cloudy = (lrow<R>(rp, blk, k, rl).w(1) & 256u) != 0;
+        uint32_t bits = 0;
+        R efclrfr = (R)1;
+        if (__any(cloudy)) {
+            efclrfr = ef[(size_t)k * 64];
+            if (cloudy) bits = mword(rp.mlw, rp.row(blk, k), MROW_LW, B, rl);
         }
-        sweep(k, y, btop - y.blay, bits, k == 0, y.bbot);  // the level below the lowest layer is the skin
-        if (k == 0) sum.put(sfc0, up);
+#pragma unroll
+        for (int g0 = 0; g0 < GW; g0 += CH) {
+            const uint32_t cb = bits >> g0;
+            f64x2v v[CH];
+            R nr[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) v[j] = tg[((size_t)k * NG + g0 + j) * 64];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) nr[j] = rad[0][g0 + j] * v[j].x + v[j].y;
+            if (__any(cb & ((1u << CH) - 1u))) {
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const R rc = rad[0][g0 + j] * v[j].x * efclrfr + v[j].y + cg[((size_t)k * NG + g0 + j) * 64];
+                    nr[j] = (cb >> j) & 1u ? rc : nr[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; ++j) rad[0][g0 + j] = nr[j];
+        }
         sum.put(rad, up);
     }
     sum.finish(up);
@@ -745,24 +776,30 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
 
 template <typename R, int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__(64, (lw_waves<R, B>())) k_lw(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
-                                           int n, ColScal cs, RecPtrs rp, AccT<R> acc, Surr sg)
+                                           int n, ColScal cs, RecPtrs rp, AccT<R> acc, Surr sg, char *__restrict__ pool)
 {
     const ColIn in = band_in<EXT>(in_);
-    lw_column<R, B, SURR>(T, T->lw[B], in, par, col0, n, cs, rp, acc, sg, (int)blockIdx.x, (int)threadIdx.x);
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * lw64_slot_bytes(LW_NG[B], in.nlay + 2));
+    for (int blk = blockIdx.x; blk * 64 < n; blk += gridDim.x)
+        lw_column<R, B, SURR>(T, T->lw[B], in, par, col0, n, cs, rp, acc, sg, blk, (int)threadIdx.x, slot);
 }
 
 // The band tables of an LDS image (the LwImg order), absb from PB: the image's when the image holds it,
 // the global table otherwise.  A table the band does not have points at the image start and is never
 // read.  The offsets are multiples of 4 elements (the & ~3 states it, so that 4 g-points of a row
 // load as one 16-byte read).
-template <typename R, typename PB>
-__device__ __forceinline__ LwBandT<R, const WR_L R *, PB> lds_band(const WR_L R *lt, const LwImg<R> &im, const LwBand<R> &G,
-                                                                   PB absb)
+template <typename R, int B, typename PB>
+__device__ __forceinline__ auto lds_band(const WR_L R *lt, const LwImg<R> &im, const LwBand<R> &G, PB absb)
 {
-    LwBandT<R, const WR_L R *, PB> Bl;
+    constexpr bool KAM = sizeof(R) == 4 || lw64_kam(B);
+    LwBandT<R, const WR_L R *, PB, typename std::conditional<KAM, const WR_L R *, const WR_G R *>::type> Bl;
     auto at = [&](int j) { return lt + (imax(0, im.off[j]) & ~3); };
     Bl.absa = at(0), Bl.absb = absb, Bl.selfref = at(2), Bl.forref = at(3), Bl.fracrefa = at(4), Bl.fracrefb = at(5);
-    Bl.ka_m[0] = at(6), Bl.ka_m[1] = at(7), Bl.ka_m[2] = at(8);
+    if constexpr (KAM)
+        Bl.ka_m[0] = at(6), Bl.ka_m[1] = at(7), Bl.ka_m[2] = at(8);
+    else
+        Bl.ka_m[0] = G.ka_m[0], Bl.ka_m[1] = G.ka_m[1], Bl.ka_m[2] = G.ka_m[2];
+    Bl.etab = lt + im.n;  // FP64: behind the image (lds_fill_lw); FP32 reads none
     Bl.kb_m[0] = at(9), Bl.kb_m[1] = at(10), Bl.kb_m[2] = at(11);
     Bl.x1 = at(12), Bl.x2 = at(13);
     Bl.refrat_planck_a = G.refrat_planck_a, Bl.refrat_planck_b = G.refrat_planck_b;
@@ -780,6 +817,15 @@ template <typename R, typename I> __device__ __forceinline__ void lds_fill(float
     for (int q = threadIdx.x; q < n4; q += blockDim.x) dst[q] = src[q];
     __syncthreads();
 }
+// LW: FP64 with exp_tbl behind the image (ETAB_LDS bytes; the last word holds one entry)
+template <typename R> __device__ __forceinline__ void lds_fill_lw(float4 *dst, const LwImg<R> &im, const WR_G R *etab)
+{
+    if constexpr (sizeof(R) == 8) {
+        WR_L R *e = (WR_L R *)dst + im.n;
+        for (int q = threadIdx.x; q <= NTBL; q += blockDim.x) e[q] = etab[q];
+    }
+    lds_fill<R>(dst, im);
+}
 
 // k_lw (FP64, one lane per column) with the band's tables other than absb in LDS (absb, the tables of
 // the layers above laytrop, stays in global memory: the FP64 image of every band then fits in LDS).
@@ -789,17 +835,18 @@ template <typename R, int B> constexpr int lwl64_wpg() { return 4 * lw_waves<R, 
 template <int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<double, B>()))
     k_lwl64(const Tabs<double> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp,
-            AccT<double> acc, Surr sg)
+            AccT<double> acc, Surr sg, char *__restrict__ pool)
 {
     extern __shared__ float4 lwl64_tab[];
     const ColIn in = band_in<EXT>(in_);
     const LwImg<double> &im = T->lw_img[B];
-    lds_fill<double>(lwl64_tab, im);
-    const auto Bl = lds_band<double>((const WR_L double *)lwl64_tab, im, T->lw[B], T->lw[B].absb);
+    lds_fill_lw<double>(lwl64_tab, im, T->exp_tbl);
+    const auto Bl = lds_band<double, B>((const WR_L double *)lwl64_tab, im, T->lw[B], T->lw[B].absb);
     constexpr int WPG = lwl64_wpg<double, B>();
-    const int lane = threadIdx.x % 64;
-    for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
-        lw_column<double, B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane);
+    const int lane = threadIdx.x % 64, w = blockIdx.x * WPG + wave_id();
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * lw64_slot_bytes(LW_NG[B], in.nlay + 2));
+    for (int blk = w; blk * 64 < n; blk += gridDim.x * WPG)
+        lw_column<double, B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane, slot);
 }
 
 // FP32 LW band kernel with a cached upward sweep.  The down sweep also forms, per layer and g-point,
@@ -810,13 +857,13 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
 constexpr int LW_NV_F32 = 2;
 // transmittance a and the downward and upward sources (gas plus cloud) of CH g-points of a layer
 template <int CH>
-__device__ __forceinline__ void lw_chunk_f32(const Tabs<float> *__restrict__ T, const LwLayer<float> &y, float sdif, float dd, float du,
+__device__ __forceinline__ void lw_chunk_f32(const LwLayer<float> &y, float sdif, float dd, float du,
                                              float ecld, uint32_t cb, const float *tau, const float *fr, float *a, float *bd,
                                              float *bu)
 {
     using R = float;
     GasV<R, CH> q;
-    lw_gas_v<R, CH>(T, sdif, y.taer, tau, q);
+    lw_gas_v<R, CH>(nullptr, sdif, y.taer, tau, q);
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
         const R fa = fr[j] * q.at[j];
@@ -826,7 +873,7 @@ __device__ __forceinline__ void lw_chunk_f32(const Tabs<float> *__restrict__ T, 
     }
     if (__any(cb & ((1u << CH) - 1u))) {
         R tr[CH], at[CH], gf[CH];
-        lw_tot_v<R, CH>(T, q.od, y.odcld, tr, at, gf);
+        lw_tot_v<R, CH>(nullptr, q.od, y.odcld, tr, at, gf);
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             const bool cl = (cb >> j) & 1u;
@@ -881,7 +928,7 @@ __device__ __forceinline__ void lw_column_f32c(const Tabs<float> *__restrict__ T
             R tau[CH], fr[CH];
             lw_taufr<R, B, SURR, CH>(T, Bt, sg, c, n, k, y.L, g0, tau, fr);
             R a[CH], bd[CH], bu[CH];
-            lw_chunk_f32<CH>(T, y, c.sdif, dd, du, ecld, bits >> g0, tau, fr, a, bd, bu);
+            lw_chunk_f32<CH>(y, c.sdif, dd, du, ecld, bits >> g0, tau, fr, a, bd, bu);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 rad[0][g0 + j] = rad[0][g0 + j] * a[j] + bd[j];
@@ -944,7 +991,7 @@ __global__ void __launch_bounds__(64 * lwl_wpg<B>(), lwc_waves<B>())
     const LwImg<float> &im = T->lw_img[B];
     lds_fill<float>(lwl_tab, im);
     const WR_L float *lt = (const WR_L float *)lwl_tab;
-    const auto Bl = lds_band<float>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
+    const auto Bl = lds_band<float, B>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
     constexpr int WPG = lwl_wpg<B>();
     const int lane = threadIdx.x % 64, w = blockIdx.x * WPG + wave_id();
     WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(LW_NV_F32, LW_NG[B], in.nlay + 2, 4));
@@ -1248,58 +1295,58 @@ __device__ __forceinline__ void sw_tgtr(const Tabs<R> *__restrict__ T, const BT 
     }
 }
 
-// Pool slot of one SW wave: per layer and g-point the reflectances (direct, diffuse) of everything below the
-// layer; FP32 also the layer's R/T, which the top-down sweep would otherwise evaluate again (in FP64 the
-// bytes cost more than the evaluation).
-constexpr int SW_NV = 2;
-template <typename R> constexpr int sw_nv_mc() { return sizeof(R) == 4 ? SW_NV + 5 : SW_NV; }
-// KEEP: with the layer's R/T.
-template <typename R, int NG, bool KEEP> struct SwSlot {
+// What the bottom-up sweep leaves per layer and g-point for the top-down one: the reflectances (direct pb,
+// diffuse pd) of everything below the layer and, in FP32, what carries the beams through it.  With S the direct
+// and F the diffuse radiation that enter at the layer's top, those that leave at its bottom are
+//   S' = ld S,   F' = al F + be S,   al = td / (1 - rd pd),   be = ((tb - ld) + rd ld pb) / (1 - rd pd)
+// (the diffuse beam is transmitted, gains what the layer scatters out of the direct one, and what the layer
+// reflects back of S' pb + F' pd), and the fluxes at that level are S' pb + F' pd up and S' + F' down.  The
+// denominator is the one that the bottom-up step divides by anyway, so FP32 spends one reciprocal per layer where
+// the reference's order (the reflectance of everything above, vrtqdr) takes three, and 5 values per g-point
+// and layer where that needs 7.  FP64 keeps the reference's order, which its outputs reproduce bit for
+// bit, and evaluates the layer's R/T again (the bytes cost more than the evaluation).
+template <typename R> constexpr int sw_nv() { return sizeof(R) == 4 ? 5 : 2; }
+// Pool slot of one SW wave.
+template <typename R, int NG> struct SwSlot {
     WR_G char *p;
     int lane, nk;
-    __device__ __forceinline__ void put(int k, int g, R pb, R pd, const R *rt) const  // rt: rb, rd, tb, td, ld
+    __device__ __forceinline__ void put(int k, int g, const R (&v)[sw_nv<R>()]) const  // pb, pd; FP32 al, be, ld
     {
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
-        if constexpr (KEEP) {
-            ((WR_G f32x4v *)p)[e] = (f32x4v){pb, pd, rt[0], rt[1]};
-            WR_G float *q = (WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
-            q[0] = rt[2], q[1] = rt[3], q[2] = rt[4];
-        } else if constexpr (sizeof(R) == 4) {
-            ((WR_G f32x2v *)p)[e] = (f32x2v){pb, pd};
+        if constexpr (sizeof(R) == 4) {
+            ((WR_G f32x4v *)p)[e] = (f32x4v){v[0], v[1], v[2], v[3]};
+            ((WR_G float *)(p + (size_t)nk * NG * 64 * 16))[e] = v[4];
         } else {
-            ((WR_G f64x2v *)p)[e] = (f64x2v){pb, pd};
+            ((WR_G f64x2v *)p)[e] = (f64x2v){v[0], v[1]};
         }
     }
-    __device__ __forceinline__ void get(int k, int g, R &pb, R &pd, R *rt) const
+    __device__ __forceinline__ void get(int k, int g, R (&v)[sw_nv<R>()]) const
     {
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
-        if constexpr (KEEP) {
-            const f32x4v v = ((const WR_G f32x4v *)p)[e];
-            const WR_G float *q = (const WR_G float *)(p + (size_t)nk * NG * 64 * 16) + e * 3;
-            pb = v.x, pd = v.y, rt[0] = v.z, rt[1] = v.w, rt[2] = q[0], rt[3] = q[1], rt[4] = q[2];
-        } else if constexpr (sizeof(R) == 4) {
-            const f32x2v v = ((const WR_G f32x2v *)p)[e];
-            pb = v.x, pd = v.y;
+        if constexpr (sizeof(R) == 4) {
+            const f32x4v q = ((const WR_G f32x4v *)p)[e];
+            v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+            v[4] = ((const WR_G float *)(p + (size_t)nk * NG * 64 * 16))[e];
         } else {
-            const f64x2v v = ((const WR_G f64x2v *)p)[e];
-            pb = v.x, pd = v.y;
+            const f64x2v q = ((const WR_G f64x2v *)p)[e];
+            v[0] = q.x, v[1] = q.y;
         }
     }
 };
 
 // The adding method over one column: bottom-up reflectances to the slot, then the direct and diffuse beams
-// top-down with the level fluxes.  layer(k) gives a layer, rt_at(layer, k, g0, o) its R/T of a chunk of the
-// lane's g-points, sun(g) the solar source of one; emit(level, {up, down}) takes a level's fluxes, top first.
-// KEEP: the top-down sweep takes the R/T from the slot instead of from rt_at again.
-template <typename R, int NG, int GW, int CH, bool KEEP, typename LAYER, typename RT, typename SUN, typename EMIT>
-__device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG, KEEP> &slot, const Share<R> &sh, LAYER &&layer, RT &&rt_at,
+// top-down with the level fluxes.  layer(k, step) gives a layer (step: the sweep's direction), rt_at(layer, k, g0, o)
+// its R/T of a chunk of the lane's g-points, sun(g) the solar source of one; emit(level, {up, down}) takes a
+// level's fluxes, top first.
+template <typename R, int NG, int GW, int CH, typename SLOT, typename LAYER, typename RT, typename SUN, typename EMIT>
+__device__ __forceinline__ void sw_adding(int nrl, R asfc, SLOT &&slot, int lane, const Share<R> &sh, LAYER &&layer, RT &&rt_at,
                                           SUN &&sun, EMIT &&emit)
 {
     R pb[GW], pd[GW];
 #pragma unroll
     for (int g = 0; g < GW; ++g) pb[g] = asfc, pd[g] = asfc;
     for (int k = 0; k < nrl; ++k) {
-        auto a = layer(k);
+        auto a = layer(k, 1);
 #pragma unroll
         for (int g0 = 0; g0 < GW; g0 += CH) {
             RtV<R, CH> o;
@@ -1307,65 +1354,78 @@ __device__ __forceinline__ void sw_adding(int nrl, R asfc, const SwSlot<R, NG, K
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 const int g = g0 + j;
-                const R rt[5] = {o.rb[j], o.rd[j], o.tb[j], o.td[j], o.ld[j]};
-                slot.put(k, sh.g0 + g, pb[g], pd[g], rt);
                 const R zden1 = rdiv<R>((R)1, (R)1 - pd[g] * o.rd[j]);
-                const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * pd[g] + o.ld[j] * pb[g])) * zden1;
-                const R nd = o.rd[j] + o.td[j] * o.td[j] * pd[g] * zden1;
-                pb[g] = nb, pd[g] = nd;
+                if constexpr (sizeof(R) == 4) {
+                    const R sc = o.tb[j] - o.ld[j], lb = o.ld[j] * pb[g], al = o.td[j] * zden1;
+                    slot.put(k, g, {pb[g], pd[g], al, (sc + o.rd[j] * lb) * zden1, o.ld[j]});
+                    pb[g] = o.rb[j] + al * (sc * pd[g] + lb);
+                    pd[g] = o.rd[j] + al * o.td[j] * pd[g];
+                } else {
+                    slot.put(k, g, {pb[g], pd[g]});
+                    const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * pd[g] + o.ld[j] * pb[g])) * zden1;
+                    const R nd = o.rd[j] + o.td[j] * o.td[j] * pd[g] * zden1;
+                    pb[g] = nb, pd[g] = nd;
+                }
             }
             if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    R tdbt[GW], tdn[GW], rdnd[GW], zsolar[GW], f[2][GW];
-    LevelSum<R, NG, GW, 2> sum{sh, slot.lane, 0, 0, 0};
+    R zsolar[GW], f[2][GW];
+    LevelSum<R, NG, GW, 2> sum{sh, lane, 0, 0, 0};
     sum.begin(nrl, -1);
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
-        tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0, zsolar[g] = sun(g);
+        zsolar[g] = sun(g);
         f[0][g] = zsolar[g] * pb[g];
         f[1][g] = zsolar[g];
     }
     sum.put(f, emit);
-    for (int k = nrl - 1; k >= 0; --k) {
-        auto chunk = [&](int g0, auto &&get) {
+    if constexpr (sizeof(R) == 4) {
+        R s[GW], d[GW];  // direct and diffuse beams
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const int g = g0 + j;
-                R zb, zd, rt[5];
-                get(g, j, zb, zd, rt);
-                const R tdbt_s = rt[4] * tdbt[g];
-                const R zden0 = rdiv<R>((R)1, (R)1 - rt[1] * rdnd[g]);
-                const R tdn_s = tdbt[g] * rt[2] + (rt[3] * ((tdn[g] - tdbt[g]) + tdbt[g] * rt[0] * rdnd[g])) * zden0;
-                const R rdnd_s = rt[1] + rt[3] * rt[3] * rdnd[g] * zden0;
-                tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
-                const R zden1 = rdiv<R>((R)1, (R)1 - rdnd_s * zd);
-                const R zfu = (tdbt_s * zb + (tdn_s - tdbt_s) * zd) * zden1;
-                const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * zb * rdnd_s) * zden1;
-                f[0][g] = zsolar[g] * zfu;
-                f[1][g] = zsolar[g] * zfd;
-            }
-        };
-        if constexpr (KEEP) {
+        for (int g = 0; g < GW; ++g) s[g] = zsolar[g], d[g] = (R)0;
+        for (int k = nrl - 1; k >= 0; --k) {
 #pragma unroll
-            for (int g0 = 0; g0 < GW; g0 += CH) {
-                chunk(g0, [&](int g, int, R &zb, R &zd, R *rt) { slot.get(k, sh.g0 + g, zb, zd, rt); });
-                if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
+            for (int g = 0; g < GW; ++g) {
+                R v[5];
+                slot.get(k, g, v);
+                d[g] = v[2] * d[g] + v[3] * s[g];
+                s[g] = v[4] * s[g];
+                f[0][g] = s[g] * v[0] + d[g] * v[1];
+                f[1][g] = s[g] + d[g];
             }
-        } else {
-            auto a = layer(k);
+            sum.put(f, emit);
+        }
+    } else {
+        R tdbt[GW], tdn[GW], rdnd[GW];
+#pragma unroll
+        for (int g = 0; g < GW; ++g) tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0;
+        for (int k = nrl - 1; k >= 0; --k) {
+            auto a = layer(k, -1);
 #pragma unroll
             for (int g0 = 0; g0 < GW; g0 += CH) {
                 RtV<R, CH> o;
                 rt_at(a, k, g0, o);
-                chunk(g0, [&](int g, int j, R &zb, R &zd, R *rt) {
-                    slot.get(k, sh.g0 + g, zb, zd, nullptr);
-                    rt[0] = o.rb[j], rt[1] = o.rd[j], rt[2] = o.tb[j], rt[3] = o.td[j], rt[4] = o.ld[j];
-                });
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int g = g0 + j;
+                    R z[2];
+                    slot.get(k, g, z);
+                    const R tdbt_s = o.ld[j] * tdbt[g];
+                    const R zden0 = (R)1 / ((R)1 - o.rd[j] * rdnd[g]);
+                    const R tdn_s = tdbt[g] * o.tb[j] + (o.td[j] * ((tdn[g] - tdbt[g]) + tdbt[g] * o.rb[j] * rdnd[g])) * zden0;
+                    const R rdnd_s = o.rd[j] + o.td[j] * o.td[j] * rdnd[g] * zden0;
+                    tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
+                    const R zden1 = (R)1 / ((R)1 - rdnd_s * z[1]);
+                    const R zfu = (tdbt_s * z[0] + (tdn_s - tdbt_s) * z[1]) * zden1;
+                    const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * z[0] * rdnd_s) * zden1;
+                    f[0][g] = zsolar[g] * zfu;
+                    f[1][g] = zsolar[g] * zfd;
+                }
                 if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
             }
+            sum.put(f, emit);
         }
-        sum.put(f, emit);
     }
     sum.finish(emit);
 }
@@ -1394,7 +1454,6 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
                                           const AccT<R> &acc, const Surr &sg, int blk, int lane, WR_G char *slot, Fix64 *fx)
 {
     constexpr int NG = SW_NG[B], CH = sw_chunk<R, B>();
-    constexpr bool KEEP = sw_nv_mc<R>() > SW_NV;
     const int nday = *cs.nday;
     if (blk * 64 >= nday) return;
     const bool ok = blk * 64 + lane < nday;  // lanes past the last day column repeat it and store nothing
@@ -1408,9 +1467,9 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
         SwLayer<R> y;
         uint32_t bits;
     };
-    sw_adding<R, NG, NG, CH, KEEP>(
-        nrl, c.asfc, SwSlot<R, NG, KEEP>{slot, lane, in.nlay + 2}, Share<R>{nullptr, 0, 0},
-        [&](int k) {
+    sw_adding<R, NG, NG, CH>(
+        nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
+        [&](int k, int) {
             Lay a;
             sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
             a.bits = a.y.cloudy ? mword(rp.msw, rp.row(blk, k), MROW_SW, B, rl) : 0u;
@@ -1438,7 +1497,7 @@ __global__ void __launch_bounds__(64, (sw_waves<R, B>())) k_sw(const Tabs<R> *__
 {
     __shared__ Fix64 fx[1];
     const ColIn in = band_in<EXT>(in_);
-    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x)
         sw_column<R, B, SURR>(T, T->sw[B], in, par, col0, n, cs, rp, sflux, acc, sg, blk, (int)threadIdx.x, slot, fx);
@@ -1481,7 +1540,7 @@ __global__ void __launch_bounds__((64 * swl_wpg<R, B>()), (sw_waves<R, B>()))
     constexpr int WPG = swl_wpg<R, B>();
     __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
     const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
-    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)
         sw_column<R, B, SURR>(T, Bl, in, par, col0, n, cs, rp, sflux, acc, sg, blk, lane, slot, fx + (sizeof(R) == 4 ? wv : 0));

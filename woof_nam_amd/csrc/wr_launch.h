@@ -107,13 +107,16 @@ inline LwRec<R> tile_lwrec(wr_ctx *c, int n, int nk)
 // McICA route band kernels (k_lw / k_sw), dispatched from a runtime id to the template instance.
 // Grid of a band kernel: one 64-lane block per 64 columns, at most one block per pool slot (the
 // kernels loop over the remaining blocks).
-template <typename R>
-inline unsigned band_grid(const BandJob<R> &j, int nv, int ng)
+template <typename R> inline unsigned pool_grid(const BandJob<R> &j, size_t slot)
 {
-    const size_t slot = cache_slot_bytes(nv, ng, j.in.nlay + 2, (int)sizeof(R));
     const size_t nslot = j.c->pool_bytes / slot;
     const size_t nblk = (size_t)(j.n + 63) / 64;
     return (unsigned)(nblk < nslot ? nblk : nslot);
+}
+template <typename R>
+inline unsigned band_grid(const BandJob<R> &j, int nv, int ng)
+{
+    return pool_grid(j, cache_slot_bytes(nv, ng, j.in.nlay + 2, (int)sizeof(R)));
 }
 
 template <typename R, bool SURR, bool EXT, int B = 0>
@@ -162,7 +165,7 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
         } else if constexpr (B < 16 && sizeof(R) == 8) {
             // k_lwl64: persistent workgroups, as many as the CUs hold at once
             constexpr unsigned WPG = lwl64_wpg<R, B>();
-            const size_t lds = (size_t)j.c->host_d.lw_img[B].n * sizeof(double);
+            const size_t lds = (size_t)j.c->host_d.lw_img[B].n * sizeof(double) + ETAB_LDS;
             static std::atomic<int> per_cu{-1};  // workgroups per CU, once per instance (one table set per process)
             if (per_cu < 0 && ((j.c->lw_lds64 >> B) & 1)) {
                 int nb = 0;
@@ -171,19 +174,19 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                     nb = 0;
                 per_cu = nb;
             }
+            const size_t slot = lw64_slot_bytes(LW_NG[B], j.in.nlay + 2);
+            const size_t nwg_pool = j.c->pool_bytes / slot / WPG;
             const size_t nwg_cols = ((size_t)j.n + 64 * WPG - 1) / (64 * WPG);
             size_t nwg = (size_t)(j.c->n_cu > 0 ? j.c->n_cu : 1) * (size_t)std::max(per_cu.load(), 0);
+            nwg = nwg < nwg_pool ? nwg : nwg_pool;
             nwg = nwg < nwg_cols ? nwg : nwg_cols;
             if (((j.c->lw_lds64 >> B) & 1) && nwg > 0)
                 hipLaunchKernelGGL((k_lwl64<B, SURR, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
-                                   j.col0, j.n, j.cs, j.rp, acc, j.sg);
+                                   j.col0, j.n, j.cs, j.rp, acc, j.sg, pool);
             else
-                hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3((j.n + 63) / 64), dim3(64), 0, s, j.tabs, j.in, j.par, j.col0,
-                                   j.n, j.cs, j.rp, acc, j.sg);
-        } else if constexpr (B < 16)
-            hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3((j.n + 63) / 64), dim3(64), 0, s, j.tabs, j.in,
-                               j.par, j.col0, j.n, j.cs, j.rp, acc, j.sg);
-        else {
+                hipLaunchKernelGGL((k_lw<R, B, SURR, EXT>), dim3(pool_grid(j, slot)), dim3(64), 0, s, j.tabs, j.in, j.par,
+                                   j.col0, j.n, j.cs, j.rp, acc, j.sg, pool);
+        } else {
             // k_swl: persistent workgroups, as many as the CUs hold at once and the pool has slots for
             constexpr int S = B < 16 ? 0 : B - 16;
             constexpr unsigned WPG = swl_wpg<R, S>();
@@ -202,7 +205,7 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                     nb = 0;
                 per_cu = nb;
             }
-            const size_t slot = cache_slot_bytes(sw_nv_mc<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
+            const size_t slot = cache_slot_bytes(sw_nv<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
             const size_t nwg_pool = j.c->pool_bytes / slot / WPG;
             const size_t nwg_cols = ((size_t)j.n + 64 * WPG - 1) / (64 * WPG);
             size_t nwg = (size_t)(j.c->n_cu > 0 ? j.c->n_cu : 1) * (size_t)std::max(per_cu.load(), 0);
@@ -212,7 +215,7 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                 hipLaunchKernelGGL((k_swl<R, S, SURR, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
                                    j.col0, j.n, j.cs, j.rp, j.sflux, acc, j.sg, pool);
             else
-                hipLaunchKernelGGL((k_sw<R, S, SURR, EXT>), dim3(band_grid(j, sw_nv_mc<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
+                hipLaunchKernelGGL((k_sw<R, S, SURR, EXT>), dim3(band_grid(j, sw_nv<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
                                    j.in, j.par, j.col0, j.n, j.cs, j.rp, j.sflux, acc, j.sg, pool);
         }
         tend(j.c, s);
@@ -236,7 +239,7 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                 img_n = j.c->host_f.lw_img[B].n;
             else
                 img_n = j.c->host_d.lw_img[B].n;
-            const size_t lds = (size_t)img_n * sizeof(R);
+            const size_t lds = (size_t)img_n * sizeof(R) + (sizeof(R) == 8 ? ETAB_LDS : 0);
             static std::atomic<int> per_cu{-1};  // workgroups per CU, once per instance (one table set per process)
             if (per_cu < 0 && on) {
                 int nb = 0;
@@ -273,7 +276,7 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                     nb = 0;
                 per_cu = nb;
             }
-            const size_t slot = cache_slot_bytes(sw_nv_mc<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
+            const size_t slot = cache_slot_bytes(sw_nv<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
             const size_t nwg_pool = j.c->pool_bytes / slot / WPG;
             const size_t nwg_cols = ((size_t)j.n + 64 * WPG - 1) / (64 * WPG);
             size_t nwg = (size_t)(j.c->n_cu > 0 ? j.c->n_cu : 1) * (size_t)std::max(per_cu.load(), 0);
@@ -283,7 +286,7 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                 hipLaunchKernelGGL((k_swrl<R, S, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
                                    j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
             else
-                hipLaunchKernelGGL((k_swr<R, S, EXT>), dim3(band_grid(j, sw_nv_mc<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
+                hipLaunchKernelGGL((k_swr<R, S, EXT>), dim3(band_grid(j, sw_nv<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
                                    j.in, j.par, j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
         }
         tend(j.c, s);

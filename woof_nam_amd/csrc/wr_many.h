@@ -33,11 +33,12 @@ constexpr int MANY_ORDER[30] = {17, 29, 21, 20, 23, 2,  4,  3,  24, 8,  6,  19, 
 template <typename R, bool NAM> constexpr int many_vl() { return NAM ? 6 : sizeof(R) == 4 ? 3 : 5; }
 template <bool NAM> constexpr int many_vs() { return NAM ? 10 : 5; }
 // pool values of one 64-column block, per lane: [140][nrl][VL], surface source [140], cloud transmittance
-// [16][nrl], SW [112][nrl][VS], reflectances [112][nlay + 2][2]
+// [16][nrl], SW [112][nrl][VS], FP64 reflectances [112][nrl][2] (the FP32 sweep leaves its 5 values in the
+// place of the layer's R/T)
 template <typename R, bool NAM> constexpr size_t many_lane_values(int nrl)
 {
     return (size_t)140 * nrl * many_vl<R, NAM>() + 140 + (size_t)16 * nrl + (size_t)112 * nrl * many_vs<NAM>() +
-           (size_t)112 * (nrl + 1) * SW_NV;
+           (sizeof(R) == 8 ? (size_t)112 * nrl * sw_nv<R>() : 0);
 }
 template <typename R, bool NAM> constexpr size_t many_block_bytes(int nrl)
 {
@@ -73,9 +74,9 @@ template <typename R, bool NAM> struct ManyBlk {
     {
         return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + ((size_t)g * nrl + k) * VS) * 64 + lane;
     }
-    __device__ __forceinline__ WR_G R *refl(int g) const  // reflectance pairs of the band that starts at g
+    __device__ __forceinline__ WR_G R *refl(int g, int k, int lane) const
     {
-        return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + (size_t)112 * nrl * VS + (size_t)g * (nrl + 1) * SW_NV) * 64;
+        return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + (size_t)112 * nrl * VS + ((size_t)g * nrl + k) * 2) * 64 + lane;
     }
 };
 template <typename R, bool NAM>
@@ -120,7 +121,7 @@ __device__ __forceinline__ void lay_lw(const ManyArgs<R> &a, int b, int k, int l
         }
         if constexpr (!NAM && sizeof(R) == 4) {
             R ta[CH], bd[CH], bu[CH];
-            lw_chunk_f32<CH>(a.T, y, c.sdif, dd, du, ecld, bits >> g0, tau, fr, ta, bd, bu);
+            lw_chunk_f32<CH>(y, c.sdif, dd, du, ecld, bits >> g0, tau, fr, ta, bd, bu);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 WR_G R *q = m.lw(NS + g0 + j, k, lane);
@@ -128,7 +129,7 @@ __device__ __forceinline__ void lay_lw(const ManyArgs<R> &a, int b, int k, int l
             }
         } else {
             GasV<R, CH> q;
-            lw_gas_v<R, CH>(a.T, c.sdif, y.taer, tau, q);
+            lw_gas_v<R, CH>(a.T->exp_tbl, c.sdif, y.taer, tau, q);
             R gd[CH], gu[CH], trc[CH], sd[CH], su[CH];
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
@@ -139,7 +140,7 @@ __device__ __forceinline__ void lay_lw(const ManyArgs<R> &a, int b, int k, int l
             const uint32_t cb = NAM ? (y.cloudy ? ~0u : 0u) : bits >> g0;
             if (__any(cb & ((1u << CH) - 1u))) {
                 R at[CH], gf[CH];
-                lw_tot_v<R, CH>(a.T, q.od, y.odcld, trc, at, gf);
+                lw_tot_v<R, CH>(a.T->exp_tbl, q.od, y.odcld, trc, at, gf);
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
                     const R td = fr[j] * (y.blay + dd * gf[j]) * at[j], tu = fr[j] * (y.blay + du * gf[j]) * at[j];
@@ -319,6 +320,69 @@ __device__ __forceinline__ void sweep_lw(const ManyArgs<R> &a, int b, int lane, 
     sum.finish(up);
 }
 
+// The slot of a sweep's g-points: FP32 in the place of the layer's R/T (the direct transmission, its fifth value, stays).
+// The top-down sweep's reads run SWEEP_AHEAD layers ahead of their use, as do those of the R/T (RtAhead).
+constexpr int SWEEP_AHEAD = 3;
+template <typename R, bool NAM, int GW> struct ManySlot {
+    static constexpr int NV = sw_nv<R>();
+    ManyBlk<R, NAM> m;
+    int g0, lane, pass;
+    R v[GW][SWEEP_AHEAD][NV];
+    __device__ __forceinline__ WR_G R *at(int k, int g) const
+    {
+        return sizeof(R) == 4 ? m.sw(g0 + g, k, lane) + pass * 320 : m.refl(g0 + g, k, lane);
+    }
+    __device__ __forceinline__ void put(int k, int g, const R (&x)[NV]) const
+    {
+        WR_G R *q = at(k, g);
+        q[0] = x[0], q[64] = x[1];
+        if constexpr (NV == 5) q[128] = x[2], q[192] = x[3];
+    }
+    __device__ __forceinline__ void load(int k, int g, R (&x)[NV]) const
+    {
+        const WR_G R *q = at(imax(k, 0), g);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) x[i] = q[64 * i];
+    }
+    __device__ __forceinline__ void get(int k, int g, R (&x)[NV])
+    {
+        if (k == m.nrl - 1)
+#pragma unroll
+            for (int d = 0; d < SWEEP_AHEAD; ++d) load(k - d, g, v[g][d]);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            x[i] = v[g][0][i];
+#pragma unroll
+            for (int d = 0; d + 1 < SWEEP_AHEAD; ++d) v[g][d][i] = v[g][d + 1][i];
+        }
+        load(k - SWEEP_AHEAD, g, v[g][SWEEP_AHEAD - 1]);
+    }
+};
+template <typename R, bool NAM, int GW> struct RtAhead {
+    ManyBlk<R, NAM> m;
+    int g0, lane, pass;
+    RtV<R, GW> v[SWEEP_AHEAD];
+    __device__ __forceinline__ void load(int k, RtV<R, GW> &o) const
+    {
+#pragma unroll
+        for (int j = 0; j < GW; ++j) {
+            const WR_G R *q = m.sw(g0 + j, imin(imax(k, 0), m.nrl - 1), lane) + pass * 320;
+            o.rb[j] = q[0], o.rd[j] = q[64], o.tb[j] = q[128], o.td[j] = q[192], o.ld[j] = q[256];
+        }
+    }
+    __device__ __forceinline__ RtV<R, GW> next(int k, int step)
+    {
+        if (k == (step > 0 ? 0 : m.nrl - 1))
+#pragma unroll
+            for (int d = 0; d < SWEEP_AHEAD; ++d) load(k + d * step, v[d]);
+        const RtV<R, GW> o = v[0];
+#pragma unroll
+        for (int d = 0; d + 1 < SWEEP_AHEAD; ++d) v[d] = v[d + 1];
+        load(k + SWEEP_AHEAD * step, v[SWEEP_AHEAD - 1]);
+        return o;
+    }
+};
+
 template <typename R, int B, bool NAM>
 __device__ __forceinline__ void sweep_sw(const ManyArgs<R> &a, int b, int lane, const Share<R> &sh)
 {
@@ -334,18 +398,13 @@ __device__ __forceinline__ void sweep_sw(const ManyArgs<R> &a, int b, int lane, 
     const double cf1 = a.cs.zcf1[t], cf0 = a.cs.zcf0[t];
     const bool total = NAM && cf1 > EPS;
     if (!NAM && ok) acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
-    const SwSlot<R, NG, false> slot{(WR_G char *)m.refl(NS), lane, nrl + 1};
     const int passes = __any(total) ? 2 : 1;
-    for (int pass = 0; pass < passes; ++pass)
-        sw_adding<R, NG, GW, GW, false>(
-            nrl, c.asfc, slot, sh, [](int k) { return k; },
-            [&](int, int k, int g0, RtV<R, GW> &o) {
-#pragma unroll
-                for (int j = 0; j < GW; ++j) {
-                    const WR_G R *q = m.sw(NS + sh.g0 + j, k, lane) + pass * 320;
-                    o.rb[j] = q[0], o.rd[j] = q[64], o.tb[j] = q[128], o.td[j] = q[192], o.ld[j] = q[256];
-                }
-            },
+    for (int pass = 0; pass < passes; ++pass) {
+        ManySlot<R, NAM, GW> slot{m, NS + sh.g0, lane, pass, {}};
+        RtAhead<R, NAM, GW> rt{m, NS + sh.g0, lane, pass, {}};
+        sw_adding<R, NG, GW, GW>(
+            nrl, c.asfc, slot, lane, sh, [&](int k, int step) { return rt.next(k, step); },
+            [](const RtV<R, GW> &v, int, int, RtV<R, GW> &o) { o = v; },
             [&](int g) { return c.ssolar * a.sflux[(size_t)(NS + sh.g0 + g) * a.n + t]; },
             [&](int lev, const R *f) {
                 const size_t p = (size_t)lev * a.n + t;
@@ -358,6 +417,7 @@ __device__ __forceinline__ void sweep_sw(const ManyArgs<R> &a, int b, int lane, 
                     acc.sw_dn[p] = (R)(cf1 * (double)f[1] + cf0 * (double)acc.sw_dn[p]);
                 }
             });
+    }
 }
 
 template <typename R, bool NAM, int P>

@@ -106,6 +106,36 @@ template <typename R> __device__ __forceinline__ R rdiv(R a, R b)
     return a / b;
 }
 
+// The other two values of the LW table at index i (0 < i), whose transmittance e = exp_tbl[i] is given: tau =
+// bpade (i / (NTBL - i)) and tfn = 1 - 2 (1 / tau - e / (1 - e)), tau / 6 below 0.06, bit for bit those of
+// k_luts.  All quotients share one reciprocal, of (NTBL - i) i (1 - e): two Newton steps, then for each quotient q
+// of a and b the correction q + (a - b q) / b with a fused multiply-add (Markstein), which rounds correctly; the
+// 9,999 indices have been compared exhaustively.  About 45 issue slots, against two 16-byte gathers from L2
+// whose 64 lanes touch up to 64 lines.
+__device__ __forceinline__ void lut_rest(int i, int ntbl, double e, double &tfn, double &tau)
+{
+#pragma clang fp contract(off)
+    const double bpade = 1.0 / 0.278;
+    const double fi = (double)i, ci = (double)(ntbl - i), d = 1.0 - e;
+    const double p = ci * fi, pd = p * d;
+    double y = __builtin_amdgcn_rcp(pd);
+    y = __builtin_fma(__builtin_fma(-pd, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-pd, y, 1.0), y, y);
+    const double yd = p * y, yp = d * y, yc = fi * yp;
+    double t = fi * yc;
+    t = __builtin_fma(__builtin_fma(-ci, t, fi), yc, t);
+    tau = bpade * t;
+    double it = (ci * 0.278) * (ci * yp);
+    it = __builtin_fma(__builtin_fma(-tau, it, 1.0), it, it);
+    it = __builtin_fma(__builtin_fma(-tau, it, 1.0), it, it);
+    double ed = e * yd;
+    ed = __builtin_fma(__builtin_fma(-d, ed, e), yd, ed);
+    double q = tau * (1.0 / 6.0);
+    q = __builtin_fma(__builtin_fma(-6.0, q, tau), 1.0 / 6.0, q);
+    tfn = tau < 0.06 ? q : 1.0 - 2.0 * (it - ed);
+    if (i >= ntbl) tau = 1.0e10, tfn = 1.0;
+}
+
 __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                                               uint32_t k1, uint32_t out[4])
 {

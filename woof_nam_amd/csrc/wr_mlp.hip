@@ -21,8 +21,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_SILU = 2, EPI_DSILU = 3 };
-constexpr int GK = 32;      // K per step (one MFMA's depth)
-constexpr int GLD = GK + 8; // LDS row stride in BF16 elements: 80 bytes, rows 16-byte aligned
+constexpr int GK = 64;      // K per step (two MFMAs deep)
+constexpr int GLD = GK + 8; // LDS row stride in BF16 elements: 144 bytes, rows 16-byte aligned
 
 struct GemmArgs {
     int M, N, K;
@@ -71,27 +71,47 @@ __device__ __forceinline__ bf16x8 run8(const __bf16 *p, long long stride, int cn
     return v;
 }
 
-// Stage a 64 x GK block of an operand into S[row][k] (rows: M of A, N of B).  rows_contig: the row
-// index is the unit-stride one (a run of 8 rows at one k); otherwise a run of 8 k at one row.
+// A thread's part of a 64 x GK block of an operand on its way to S[row][k] (rows: M of A, N of B): two runs of 8.
+// rows_contig: the row index is the unit-stride one (runs of 8 rows at one k); otherwise runs of 8 k at one row.
+struct Staged {
+    bf16x8 v[2];
+};
 template <typename T>
-__device__ __forceinline__ void stage(const T *X, long long ld_row, long long ld_k, int nrow, int r0, int kk,
-                                      int k_end, bool rows_contig, __bf16 (*S)[GLD], int tid)
+__device__ __forceinline__ Staged stage_load(const T *X, long long ld_row, long long ld_k, int nrow, int r0, int kk, int k_end,
+                                             bool rows_contig, int tid)
 {
-    if (rows_contig) {
-        const int c = tid >> 3, r = (tid & 7) * 8;
-        const int row = r0 + r, k = kk + c;
-        const int cnt = k < k_end ? max(0, min(8, nrow - row)) : 0;
-        const bf16x8 v = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_row, cnt);
+    Staged s;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) S[r + j][c] = v[j];
-    } else {
-        const int r = tid >> 2, c = (tid & 3) * 8;
-        const int row = r0 + r, k = kk + c;
-        const int cnt = row < nrow ? max(0, min(8, k_end - k)) : 0;
-        *(bf16x8 *)&S[r][c] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_k, cnt);
+    for (int u = 0; u < 2; ++u) {
+        if (rows_contig) {
+            const int row = r0 + (tid & 7) * 8, k = kk + (tid >> 3) + u * 32;
+            const int cnt = k < k_end ? max(0, min(8, nrow - row)) : 0;
+            s.v[u] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_row, cnt);
+        } else {
+            const int row = r0 + (tid >> 2), k = kk + (tid & 3) * 8 + u * 32;
+            const int cnt = row < nrow ? max(0, min(8, k_end - k)) : 0;
+            s.v[u] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_k, cnt);
+        }
+    }
+    return s;
+}
+__device__ __forceinline__ void stage_store(const Staged &s, bool rows_contig, __bf16 (*S)[GLD], int tid)
+{
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if (rows_contig) {
+            const int r = (tid & 7) * 8, c = (tid >> 3) + u * 32;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) S[r + j][c] = s.v[u][j];
+        } else {
+            *(bf16x8 *)&S[tid >> 2][(tid & 3) * 8 + u * 32] = s.v[u];
+        }
     }
 }
 
+// 64 x 64 tile per workgroup.  The loads of the next K step are in flight while the MFMAs of this one run; a step
+// is GK = 64 deep, so that a split of a weight gradient (1,024 samples) is 16 of them.  Bound by the latency of a
+// step where the grid is small (the weight gradients), by the operands' bytes otherwise.
 template <typename TA, typename TB, int EPI>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
 {
@@ -112,21 +132,28 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
+    const int row = lane & 15, kq = (lane >> 4) * 8;  // the lane's row and first k of each operand fragment
+    Staged sa = stage_load(A, g.lda_m, g.lda_k, g.M, m0, k_begin, k_end, a_rows, tid);
+    Staged sb = stage_load(B, g.ldb_n, g.ldb_k, g.N, n0, k_begin, k_end, b_rows, tid);
     for (int kk = k_begin; kk < k_end; kk += GK) {
-        stage(A, g.lda_m, g.lda_k, g.M, m0, kk, k_end, a_rows, As, tid);
-        stage(B, g.ldb_n, g.ldb_k, g.N, n0, kk, k_end, b_rows, Bs, tid);
+        stage_store(sa, a_rows, As, tid);
+        stage_store(sb, b_rows, Bs, tid);
         __syncthreads();
-        // lane holds row (lane % 16) and k (lane / 16) * 8 + 0..7 of each operand tile
-        const int row = lane & 15, kq = (lane >> 4) * 8;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const bf16x8 a = *(const bf16x8 *)&As[wm + i * 16 + row][kq];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const bf16x8 b = *(const bf16x8 *)&Bs[wn + j * 16 + row][kq];
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i][j], 0, 0, 0);
-            }
+        if (kk + GK < k_end) {
+            sa = stage_load(A, g.lda_m, g.lda_k, g.M, m0, kk + GK, k_end, a_rows, tid);
+            sb = stage_load(B, g.ldb_n, g.ldb_k, g.N, n0, kk + GK, k_end, b_rows, tid);
         }
+#pragma unroll
+        for (int k2 = 0; k2 < GK; k2 += 32)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16x8 a = *(const bf16x8 *)&As[wm + i * 16 + row][k2 + kq];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const bf16x8 b = *(const bf16x8 *)&Bs[wn + j * 16 + row][k2 + kq];
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i][j], 0, 0, 0);
+                }
+            }
         __syncthreads();
     }
     // epilogue: lane holds D[4*(lane/16) + q][lane % 16] of each 16 x 16 tile
@@ -298,16 +325,19 @@ __global__ void k_splitk_reduce(const float *__restrict__ part, int splits, long
     const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (i >= n) return;
     float s = 0.f;
+#pragma unroll 8
     for (int k = 0; k < splits; ++k) s += part[k * stride + i];
     out[i] = s;
 }
 
-// Column sums db[n] = sum_m X[m * ld + n], in a fixed order.  A workgroup owns CS_N columns (64-byte row
+// Column sums db[n] = sum_m X[m * ld + n], in a fixed order.  A workgroup owns CS_N columns (32-byte row
 // segments) and its CS_R row groups walk every CS_R-th row with CS_U loads in flight, each into its own
 // sum; the sums of a column then meet in a tree through LDS.  One thread per column, as this ran
 // before, is one chain of M dependent loads on N / 64 waves: 3 ms for the 16,384 x 504 error of a
 // training step, against 20 us here (bound by the few workgroups that N / CS_N gives).
-constexpr int CS_N = 16, CS_R = 64, CS_U = 8;
+// 8 columns and 128 row groups: with 16 and 64 the 128-column sums of 16,384 rows took 28 us, a memory latency for each
+// of 32 rounds on 8 workgroups; 32 loads a thread in place of 8 took 76 us.
+constexpr int CS_N = 8, CS_R = 128, CS_U = 8;
 __global__ void __launch_bounds__(CS_N * CS_R) k_colsum(const float *__restrict__ X, int M, int N, long long ld,
                                                         float *__restrict__ out)
 {
@@ -340,13 +370,33 @@ __global__ void __launch_bounds__(CS_N * CS_R) k_colsum(const float *__restrict_
     if (r == 0 && n < N) out[n] = red[0][c];
 }
 
-// dY = 2 (Y - T) * scale; per-block partial sum of squared error
+// dY = 2 (Y - T) * scale; per-block partial sum of squared error.  Bound by its three streams (99 MB for 16,384 x
+// 504): 4 values a load where the pointers allow, two loads of each stream in flight.
 __global__ void k_mse(const float *__restrict__ Y, const float *__restrict__ T, long long n, float scale,
                       float *__restrict__ dY, float *__restrict__ part)
 {
     __shared__ float red[256];
     float s = 0.f;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const long long step = gridDim.x * (long long)blockDim.x, first = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    long long done = 0;
+    if ((((uintptr_t)Y | (uintptr_t)T | (uintptr_t)dY) & 15) == 0) {
+        const long long n4 = n / 4;
+        auto one = [&](float4 y, float4 t, long long i) {
+            const float4 d = {y.x - t.x, y.y - t.y, y.z - t.z, y.w - t.w};
+            ((float4 *)dY)[i] = (float4){2.f * d.x * scale, 2.f * d.y * scale, 2.f * d.z * scale, 2.f * d.w * scale};
+            s += d.x * d.x + d.y * d.y + (d.z * d.z + d.w * d.w);
+        };
+        const float4 *Y4 = (const float4 *)Y, *T4 = (const float4 *)T;
+        long long i = first;
+        for (; i + step < n4; i += 2 * step) {
+            const float4 y0 = Y4[i], t0 = T4[i], y1 = Y4[i + step], t1 = T4[i + step];
+            one(y0, t0, i);
+            one(y1, t1, i + step);
+        }
+        if (i < n4) one(Y4[i], T4[i], i);
+        done = n4 * 4;
+    }
+    for (long long i = done + first; i < n; i += step) {
         const float d = Y[i] - T[i];
         dY[i] = 2.f * d * scale;
         s += d * d;

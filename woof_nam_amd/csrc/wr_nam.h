@@ -240,7 +240,7 @@ __device__ __forceinline__ void lwr_column(const Tabs<R> *__restrict__ T, const 
             R tau[CH], fr[CH];
             lw_taufr<R, B, false, CH>(T, Bt, none, c, n, k, y.L, g0, tau, fr);
             GasV<R, CH> q;
-            lw_gas_v<R, CH>(T, c.sdif, y.taer, tau, q);
+            lw_gas_v<R, CH>(Bt.etab, c.sdif, y.taer, tau, q);
             if (sfc) {  // surface emission and reflection
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
@@ -256,7 +256,7 @@ __device__ __forceinline__ void lwr_column(const Tabs<R> *__restrict__ T, const 
             for (int j = 0; j < CH; ++j) gas[j] = fr[j] * (y.blay + dplnk * q.gf[j]) * q.at[j];
             if (some) {
                 R trc[CH], at[CH], gf[CH];
-                lw_tot_v<R, CH>(T, q.od, y.odcld, trc, at, gf);
+                lw_tot_v<R, CH>(Bt.etab, q.od, y.odcld, trc, at, gf);
 #pragma unroll
                 for (int j = 0; j < CH; ++j) {
                     const int g = g0 + j;
@@ -321,16 +321,16 @@ __global__ void __launch_bounds__((64 * lwrl_wpg<R, B>()), (lwr_waves<R, B>()))
     extern __shared__ float4 lwrl_tab[];
     const ColIn in = band_in<EXT>(in_);
     const LwImg<R> &im = T->lw_img[B];
-    lds_fill<R>(lwrl_tab, im);
+    lds_fill_lw<R>(lwrl_tab, im, T->exp_tbl);
     const WR_L R *lt = (const WR_L R *)lwrl_tab;
     constexpr int WPG = lwrl_wpg<R, B>();
     const int lane = threadIdx.x % 64;
     if constexpr (sizeof(R) == 4) {
-        const auto Bl = lds_band<R>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
+        const auto Bl = lds_band<R, B>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
         for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
             lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     } else {
-        const auto Bl = lds_band<R>(lt, im, T->lw[B], T->lw[B].absb);
+        const auto Bl = lds_band<R, B>(lt, im, T->lw[B], T->lw[B].absb);
         for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
             lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     }
@@ -359,7 +359,6 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
                                            const AccT<R> &acc, int blk, int lane, WR_G char *slot, Fix64 *fx)
 {
     constexpr int NG = SW_NG[B], CH = sw_chunk<R, B, true>();
-    constexpr bool KEEP = sw_nv_mc<R>() > SW_NV;
     const int nday = *cs.nday;
     if (blk * 64 >= nday) return;
     const bool ok = blk * 64 + lane < nday;  // lanes past the last day column repeat it and store nothing
@@ -378,9 +377,9 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
     };
     const int passes = __any(total) ? 2 : 1;  // a column without cloud stores nothing in the second pass
     for (int pass = 0; pass < passes; ++pass) {
-        sw_adding<R, NG, NG, CH, KEEP>(
-            nrl, c.asfc, SwSlot<R, NG, KEEP>{slot, lane, in.nlay + 2}, Share<R>{nullptr, 0, 0},
-            [&](int k) {
+        sw_adding<R, NG, NG, CH>(
+            nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
+            [&](int k, int) {
                 Lay a;
                 sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
                 a.mix = false, a.zc1 = (R)0, a.zc0 = (R)1;
@@ -424,7 +423,7 @@ __global__ void __launch_bounds__(64, (sw_waves<R, B, true>())) k_swr(const Tabs
 {
     __shared__ Fix64 fx[1];
     const ColIn in = band_in<EXT>(in_);
-    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x)
         swr_column<R, B>(T, T->sw[B], in, par, col0, n, cs, rp, sflux, acc, blk, (int)threadIdx.x, slot, fx);
@@ -445,7 +444,7 @@ __global__ void __launch_bounds__((64 * swrl_wpg<R, B>()), (sw_waves<R, B, true>
     constexpr int WPG = swrl_wpg<R, B>();
     __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
     const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
-    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv_mc<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)
         swr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, sflux, acc, blk, lane, slot, fx + (sizeof(R) == 4 ? wv : 0));

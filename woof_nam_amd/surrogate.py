@@ -139,7 +139,10 @@ class MLP:
     def _wgrad(self, dZ, H, n_out, n_in, out):
         """out[n_out][n_in] = dZ^T H over the batch (split-K partials, fixed-order sum)."""
         B = int(dZ.shape[0])
-        splits = max(1, min(64, B // 1024))
+        # about 1,024 workgroups of one 64 x 64 tile and one split, 256 samples or more each: a split is a serial
+        # chain of steps, and 16 splits of 1,024 samples (32 to 256 workgroups) took 41 to 50 us per product
+        tiles = -(-n_out // 64) * -(-n_in // 64)
+        splits = max(1, min(64, 1024 // tiles, B // 256))
         part = self._buf(f"part{n_out}x{n_in}", (splits, n_out, n_in), torch.float32)
         gemm(n_out, n_in, B, dZ, 1, n_out, H, n_in, 1, part, None, n_in, 1, splits=splits,
              split_stride=n_out * n_in)
