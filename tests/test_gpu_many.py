@@ -1,4 +1,4 @@
-"""Small tiles: every band of a tile in one launch against the per-band launches.
+"""Small tiles: all bands of a tile in two launches against the per-band launches.
 
 WR_MANY_COLS=0 (read when a context is created) keeps the per-band kernels; both run the same column
 functions, so every output is the same bits, at the edges of a 64-column block, for both precisions and
@@ -31,7 +31,7 @@ def columns(n, seed, ext, device):
 
 @pytest.mark.parametrize("mcica,ext", [(1, False), (0, False), (1, True), (0, True)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_one_launch_equals_per_band_launches(gpu_device, monkeypatch, precision, mcica, ext):
+def test_two_launches_equal_per_band_launches(gpu_device, monkeypatch, precision, mcica, ext):
     p = Radiation.default_params(mcica=mcica, seed=11)
     rads = []
     for env in ("0", None):
@@ -39,7 +39,7 @@ def test_one_launch_equals_per_band_launches(gpu_device, monkeypatch, precision,
         rads.append(Radiation(0, max_cols=700))
     try:
         for n in (1, 63, 64, 65, 701):              # 701: a full tile and a one-column tile
-            print(f"case one launch {precision} mcica={mcica} ext={ext} ncol={n}", flush=True)
+            print(f"case two launches {precision} mcica={mcica} ext={ext} ncol={n}", flush=True)
             cols = columns(n, 50 + n, ext, gpu_device)
             a, b = (r.run(cols, params=p, precision=precision)[0] for r in rads)
             torch.cuda.synchronize()
@@ -48,3 +48,25 @@ def test_one_launch_equals_per_band_launches(gpu_device, monkeypatch, precision,
     finally:
         for r in rads:
             r.close()
+
+
+@pytest.mark.parametrize("mcica", [1, 0])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_tiles_of_any_size_agree(gpu_device, monkeypatch, precision, mcica):
+    """One set of columns in large and in smaller tiles: the band kernels over more blocks than their grid has
+    waves (several rounds and a ragged last one), and the two launches over more blocks than the pool holds."""
+    n, p = 140_001, Radiation.default_params(mcica=mcica, seed=5)
+    cols = columns(n, 77, False, gpu_device)
+    out = []
+    for max_cols, env in ((n, "0"), (30_000, None), (9_000, "0")):
+        monkeypatch.setenv("WR_MANY_COLS", env) if env else monkeypatch.delenv("WR_MANY_COLS")
+        print(f"case tiles {precision} mcica={mcica} max_cols={max_cols} many={env}", flush=True)
+        rad = Radiation(0, max_cols=max_cols)
+        try:
+            out.append(rad.run(cols, params=p, precision=precision)[0])
+            torch.cuda.synchronize()
+        finally:
+            rad.close()
+    for other in out[1:]:
+        for k in abi.OUTPUT_FIELDS:
+            assert torch.equal(out[0][k].view(torch.int64), other[k].view(torch.int64)), k

@@ -54,8 +54,8 @@ def hipcc() -> str:
 # The mixed-precision and surrogate units contract FP32 multiply-adds and use the hardware FP32
 # reciprocal/sqrt; the FP64 index arithmetic inside them keeps contraction off by pragma.  The waves
 # per SIMD of every band kernel come from per-band tables in the sources (wr_kernels.h, wr_nam.h).
-# WR_LW_GSPLIT=2 (two lanes per column in LW, half of the g-points each) halves the LW registers but
-# measured 9 % slower: the per-layer column work then runs twice.
+# Contraction is per source expression ("on", not "fast"), so that two kernels that evaluate one expression
+# round it alike.
 _FP32_UNIT = ["-ffp-contract=on", "-fno-hip-fp32-correctly-rounded-divide-sqrt"]
 UNIT_FLAGS = {
     "wr_mixed.hip": _FP32_UNIT,

@@ -79,13 +79,12 @@ __device__ __forceinline__ LutF lut_f32(int i, bool lw_cap)
 #define WR_L
 #endif
 // The tables of one LW band; P is the pointer type (global by default, LDS in the staged kernels),
-// PB that of absb, PM that of ka_m.
+// PB that of absb, PM that of ka_m and kb_m.
 template <typename R, typename P = const WR_G R *, typename PB = P, typename PM = P> struct LwBandT {
     P absa;
     PB absb;
     P selfref, forref, fracrefa, fracrefb;
-    PM ka_m[3];
-    P kb_m[3];
+    PM ka_m[3], kb_m[3];
     P x1, x2;
     P etab;  // exp_tbl
     R refrat_planck_a, refrat_planck_b, refrat_m_a, refrat_m_b, refrat_m_a3;
@@ -94,13 +93,13 @@ template <typename R> using LwBand = LwBandT<R>;
 // The same tables packed into one image: 14 tables (absa absb selfref forref fracrefa fracrefb
 // ka_m[0..2] kb_m[0..2] x1 x2) at element offsets off[] (multiples of 4, -1 where the image does not
 // hold one), n elements in all (a multiple of 4), from a 256-byte aligned base.  The FP64 image leaves
-// absb out, and ka_m of the bands that would not leave room for the transmittance table (lw64_kam).
+// absb out, and ka_m and kb_m of the bands that would not leave room for the transmittance table (lw64_minor).
 constexpr int LW_IMG_T = 14;
 // bytes of exp_tbl in LDS, behind a band's FP64 image (16-byte words)
 constexpr size_t ETAB_LDS = ((NTBL + 1) * sizeof(double) + 15) & ~(size_t)15;
-// FP64: whether the band's image holds ka_m.  Bands 3 and 5 (16 g-points, 9 mixtures of two gases) have 22 KB of
-// it beside 78 KB of other tables; with the 80 KB of exp_tbl that is more than the 160 KB of a CU.
-__host__ __device__ constexpr bool lw64_kam(int band0) { return band0 != 2 && band0 != 4; }
+// FP64: whether the band's image holds ka_m and kb_m.  Bands 3 and 5 (16 g-points, 9 mixtures of two gases) have up
+// to 34 KB of them beside 78 KB of other tables; with the 80 KB of exp_tbl that is more than the 160 KB of a CU.
+__host__ __device__ constexpr bool lw64_minor(int band0) { return band0 != 2 && band0 != 4; }
 template <typename R> struct LwImg {
     const WR_G R *base;
     int n;

@@ -257,7 +257,7 @@ template <typename R> int bind_tables(const TFile &f, Blob &b, Tabs<R> &T)
         for (const Slot &s : slots)
             if (s.band == k + 1)
                 ent[s.kind == 0 ? 6 + s.idx : s.kind == 1 ? 9 + s.idx : s.kind == 2 ? 12 : 13] =
-                    sizeof(R) == 8 && s.kind == 0 && !lw64_kam(k) ? nullptr : d.find(bname("lw", s.band, s.key, true));
+                    sizeof(R) == 8 && s.kind < 2 && !lw64_minor(k) ? nullptr : d.find(bname("lw", s.band, s.key, true));
         LwImg<R> &im = T.lw_img[k];
         int n = 0;
         for (int j = 0; j < LW_IMG_T; ++j) {
@@ -536,11 +536,21 @@ uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_
     return m & ((1u << nb) - 1u);
 }
 
-// Tiles of up to this many columns run every band in one launch (wr_many.h); WR_MANY_COLS overrides it
-// at context creation (0: never).
-constexpr int MANY_COLS_DEFAULT = 8192;
+// Tiles of up to this many columns run all their bands in two launches (wr_many.h); WR_MANY_COLS overrides it at
+// context creation (0: never).  A context created under a WR_*_LDS* mask, which chooses between band kernels, runs the
+// band kernels at every size.  ms per call, band kernels / two launches:
+//   columns              8,192       20,000       48,000       64,000      110,889
+//   FP64 McICA      12.4 / 3.6   15.4 / 8.2   24.1 / 19.5   27.6 / 25.8   34.1 / 42.3
+//   mixed McICA      8.0 / 1.6    9.7 / 3.6   11.4 / 8.4    12.9 / 11.1   13.4 / 18.2
+//   FP64 NAM        23.0 / 5.8   24.5 / 11.1  34.0 / 26.2   40.0 / 35.1   51.5 / 73.1
+//   mixed NAM       14.9 / 2.9   16.8 / 5.8   20.8 / 13.9   22.0 / 18.5   25.2 / 34.2
+constexpr int MANY_COLS_DEFAULT = 65536;
+constexpr int MANY_POOL_COLS = 8192;  // columns whose pool values a context has room for at once (launch_many)
 int many_cols_env()
 {
+    for (const char *m : {"WR_LW_LDS", "WR_LW_LDS64", "WR_SW_LDS", "WR_SW_LDS64", "WR_LWR_LDS", "WR_LWR_LDS64", "WR_SWR_LDS",
+                          "WR_SWR_LDS64"})
+        if (getenv(m)) return 0;
     const char *e = getenv("WR_MANY_COLS");
     return e ? std::max(0, atoi(e)) : MANY_COLS_DEFAULT;
 }
@@ -572,8 +582,8 @@ Sizes sizes(int32_t max_cols)
     // 2 values, FP32 SW: 5 values, x 16 g x levels; FP64 LW), at most WR_POOL_GB (default 3) GB per stream:
     // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB
     const int nl_max = 64;
-    const size_t lane_max = std::max({cache_slot_bytes(sw_nv<double>(), 16, nl_max + 1, (int)sizeof(double)),
-                                      cache_slot_bytes(sw_nv<float>(), 16, nl_max + 1, (int)sizeof(float)),
+    const size_t lane_max = std::max({cache_slot_bytes(2 * sw_nv<double>(), 16, nl_max + 1, (int)sizeof(double)),
+                                      cache_slot_bytes(2 * sw_nv<float>(), 16, nl_max + 1, (int)sizeof(float)),
                                       lw64_slot_bytes(16, nl_max + 1)});
     const size_t need = (m + 63) / 64 * lane_max;
     const char *pe = getenv("WR_POOL_GB");
@@ -586,8 +596,8 @@ Sizes sizes(int32_t max_cols)
     const int na = e ? atoi(e) : WR_NAUX;
     z.naux = na < 0 ? 0 : (na > WR_NAUX ? WR_NAUX : na);
     // the streams' pools lie one after another; together they also hold every band's slots of the tiles
-    // that run their bands in one launch
-    const size_t many = (size_t)((std::min(max_cols, many_cols_env()) + 63) / 64) * MANY_BLOCK;
+    // that run their bands in two launches
+    const size_t many = (size_t)((std::min({max_cols, many_cols_env(), MANY_POOL_COLS}) + 63) / 64) * MANY_BLOCK;
     z.pool_all = std::max(z.pool * (size_t)(z.naux > 1 ? z.naux : 1), many);
     return z;
 }

@@ -46,7 +46,7 @@ struct wr_ctx {
     char *pool[WR_NAUX];
     size_t pool_bytes;
     size_t pool_all;                 // bytes from pool[0] on, pool[1..] among them: one launch may use them all
-    int many_cols;                   // tiles of up to this many columns run every band in one launch
+    int many_cols;                   // tiles of up to this many columns run all bands in two launches (wr_many.h)
     // band-kernel streams (default priority, non-blocking) and their fork/join events
     int naux;
     hipStream_t aux[WR_NAUX];
@@ -126,7 +126,7 @@ int wr_launch_fp64_ext(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, co
                        int band, hipStream_t s);
 int wr_launch_mixed_ext(wr_ctx *c, const wr::ColIn &in, const wr::RunPar &par, const wr::OutPtrs &out, int col0, int n,
                         int band, hipStream_t s);
-// every band of a small tile in one launch (wr_many.h), on the tile that launch_tile / launch_tile_nam set up
+// every band of a small tile in two launches (wr_many.h), on the tile that launch_tile / launch_tile_nam set up
 namespace wr {
 template <typename R> struct BandJob;
 template <typename R, bool NAM, bool SURR> int launch_many(const BandJob<R> &j, hipStream_t s);

@@ -1,19 +1,19 @@
 // wr_kernels.h -- kernels of the MI355X RRTMG radiation path (templated on the optics precision R).
 //
-// Per column tile (n columns starting at col0):
+// Per column tile (n columns starting at col0), after the layer records of wr_rec.h:
 //   k_colprep   column scalars: LW laytrop, precipitable water, cloud flag; SW day flag, column cloud
-//               cover (max-random), SW laytrop and the solar source of the 112 g-points
+//               cover (max-random), SW laytrop
+//   k_sflux     solar source of the 112 g-points of the day columns
 //   k_day*      ordered compaction of the day columns (count, scan, scatter; deterministic order)
-//   k_lw<B>     one thread per column, all g-points of band B in registers: McICA masks, then the
-//               rtrnmc down sweep and up sweep (optics recomputed per sweep); the band's level fluxes
-//               go to its own FP64 planes (FP64, and FP32 with two lanes per column)
-//   k_lwc<B>    FP32: as k_lw, with each layer's upward transmittance and source kept in the pool slot
+//   k_lw<B>, k_lwl64<B>  FP64: one lane per column, all g-points of band B in registers: the rtrnmc down
+//               sweep and up sweep; the band's level fluxes go to its own planes
+//   k_lwc<B>, k_lwl<B>  FP32: the same, with each layer's upward transmittance and source kept in the pool slot
 //               by the down sweep, so that the up sweep needs no optics
-//   k_sw<B>     one thread per day column: for each g-point of band B the two-stream adding method
+//   k_sw<B>, k_swl<B>  one lane per day column: for each g-point of band B the two-stream adding method
 //               as one bottom-up sweep (reflectance of the atmosphere below each level, to the pool
-//               slot; FP32 also the layer R/T) and one top-down sweep (direct/diffuse transmission
-//               and level fluxes)
-//   k_post      FP64 level fluxes -> heating rates, top-first outputs
+//               slot) and one top-down sweep (direct and diffuse beams, level fluxes)
+//   k_post      level fluxes -> heating rates, top-first outputs
+// (the kernels with an l read the band's tables from LDS).
 #pragma once
 #include <type_traits>
 
@@ -86,7 +86,7 @@ static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int 
     int lt = 0, lcf = 0, swlt = nrl;
     uint32_t blocks = 0;
     double pb = rc.plvl(nrl);
-#pragma unroll 4
+#pragma unroll 16
     for (int k = 0; k < nrl; ++k) {
         const int kin = nrl - 1 - k;
         const double pt = rc.plvl(kin);
@@ -390,24 +390,16 @@ __host__ __device__ constexpr size_t cache_slot_bytes(int nv, int ng, int nk, in
     return (size_t)64 * nv * ng * nk * rbytes;
 }
 
-// Optics chunks and wave bounds of the LW band kernels, per band.  These kernels wait on table gathers
-// most of the time, so a second resident wave per SIMD pays wherever the registers allow it:
-// * chunk: g-points per optics chunk (0 = the whole band at once).  A scheduling barrier between
-//   chunks keeps the gathers of one chunk from being hoisted above the arithmetic of the previous
-//   one, which bounds the registers the gathered values hold.  The arithmetic of every g-point is
-//   unchanged, so the FP64 results stay bit-identical;
-// * waves: waves per SIMD the compiler must fit.
-// FP32 cached kernel (k_lwc): the two-key-species bands 3, 4, 5, 7, 9 spill 18-80 registers at two
-// waves and still run 25-30 % faster.  The other bands reach two waves by their register count
-// (bands 6, 8, 12 through the chunks); for them the bound itself made the schedule 15-20 % slower,
-// and chunking bands 1, 2, 10, 11 only lowered the loads in flight.  The two-g-point bands 15 and 16
-// run 11-19 % faster at a three-wave bound (6-10 spilled registers).
-// FP64 recompute kernel (k_lw<double>): two-g-point chunks bring bands 1, 2, 6, 11 to two waves
-// without spills (26-33 % faster; band 1 needs the bound as well since the column body became a
-// function shared with the LDS-staged kernel); bands 8 and 12 gain 6-10 % from a two-wave bound
-// with spills.
-// The other bands stay at one wave unchunked: chunked at one wave they lost half their speed (fewer
-// gathers in flight, no second wave to cover the waits).
+// Optics chunks and wave bounds of the LW band kernels, per band.  These kernels wait on memory most of the time
+// (0.65 to 0.8 of the wave cycles on the 954x835x60 grid), so more resident waves per SIMD pay as far as the
+// registers allow:
+// * chunk: g-points whose optics are evaluated together, about four.  A scheduling barrier between chunks keeps
+//   the gathers of one from being hoisted above the arithmetic of the one before, which bounds the registers; within
+//   a chunk nothing branches per g-point, so that its chains overlap.  The arithmetic of every g-point is
+//   that of the whole band at once;
+// * waves: waves per SIMD the compiler must fit.  FP32: four, or three where four spilled (the 16 and 14 g-point
+//   bands of two gases).  FP64: two everywhere; at three the LW kernels of a 796,590-column call took 205 ms in
+//   place of 147, from up to 530 bytes of scratch a lane.
 // WR_LWC_WAVES / WR_LW64_WAVES > 0 or WR_LW_CHUNK / WR_LW64_CHUNK >= 0 override the tables for every
 // band (tuning builds).
 constexpr int LWC_WAVES[16] = {4, 4, 3, 3, 3, 4, 3, 4, 3, 4, 4, 4, 4, 4, 4, 4};
@@ -449,7 +441,7 @@ template <typename R, int B> constexpr int lw_chunk_r()
 // g-points of its column (GW = NG) and adds them itself, or GW of them, the others being with the other
 // waves of its workgroup (k_many): then the contributions of SUM_LEVELS levels are left in LDS, and after a
 // barrier each wave adds those of its levels, again in g order, so that the sums are the same bits.
-// NQ: quantities per level.  The levels come in order row0, row0 + step, ...; emit(row, sums) stores one.
+// NQ: quantities per level (4: two skies, with half as many levels between barriers).  The levels come in order row0, row0 + step, ...; emit(row, sums) stores one.
 constexpr int SUM_LEVELS = 4;
 template <typename R> constexpr size_t sum_lds_bytes() { return sizeof(R) * SUM_LEVELS * 64 * 24; }  // LW 16 g, SW 2 x 12 g
 template <typename R> struct Share {  // a wave's part of a column's g-points (split bands)
@@ -457,6 +449,7 @@ template <typename R> struct Share {  // a wave's part of a column's g-points (s
     int g0, wave;  // first g-point, wave index
 };
 template <typename R, int NG, int GW, int NQ> struct LevelSum {
+    static constexpr int SL = NQ > 2 ? SUM_LEVELS / 2 : SUM_LEVELS;
     Share<R> sh;
     int lane, row, step, cnt;
     __device__ __forceinline__ void begin(int row0, int step_) { row = row0, step = step_, cnt = 0; }
@@ -477,7 +470,7 @@ template <typename R, int NG, int GW, int NQ> struct LevelSum {
             for (int q = 0; q < NQ; ++q)
 #pragma unroll
                 for (int j = 0; j < GW; ++j) sh.xs[((cnt * NQ + q) * NG + sh.g0 + j) * 64 + lane] = v[q][j];
-            if (++cnt == SUM_LEVELS) finish(emit);
+            if (++cnt == SL) finish(emit);
         }
     }
     template <typename EMIT> __device__ __forceinline__ void finish(EMIT &&emit)
@@ -791,16 +784,18 @@ __global__ void __launch_bounds__(64, (lw_waves<R, B>())) k_lw(const Tabs<R> *__
 template <typename R, int B, typename PB>
 __device__ __forceinline__ auto lds_band(const WR_L R *lt, const LwImg<R> &im, const LwBand<R> &G, PB absb)
 {
-    constexpr bool KAM = sizeof(R) == 4 || lw64_kam(B);
-    LwBandT<R, const WR_L R *, PB, typename std::conditional<KAM, const WR_L R *, const WR_G R *>::type> Bl;
+    constexpr bool MINOR = sizeof(R) == 4 || lw64_minor(B);
+    LwBandT<R, const WR_L R *, PB, typename std::conditional<MINOR, const WR_L R *, const WR_G R *>::type> Bl;
     auto at = [&](int j) { return lt + (imax(0, im.off[j]) & ~3); };
     Bl.absa = at(0), Bl.absb = absb, Bl.selfref = at(2), Bl.forref = at(3), Bl.fracrefa = at(4), Bl.fracrefb = at(5);
-    if constexpr (KAM)
-        Bl.ka_m[0] = at(6), Bl.ka_m[1] = at(7), Bl.ka_m[2] = at(8);
-    else
-        Bl.ka_m[0] = G.ka_m[0], Bl.ka_m[1] = G.ka_m[1], Bl.ka_m[2] = G.ka_m[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        if constexpr (MINOR)
+            Bl.ka_m[i] = at(6 + i), Bl.kb_m[i] = at(9 + i);
+        else
+            Bl.ka_m[i] = G.ka_m[i], Bl.kb_m[i] = G.kb_m[i];
+    }
     Bl.etab = lt + im.n;  // FP64: behind the image (lds_fill_lw); FP32 reads none
-    Bl.kb_m[0] = at(9), Bl.kb_m[1] = at(10), Bl.kb_m[2] = at(11);
     Bl.x1 = at(12), Bl.x2 = at(13);
     Bl.refrat_planck_a = G.refrat_planck_a, Bl.refrat_planck_b = G.refrat_planck_b;
     Bl.refrat_m_a = G.refrat_m_a, Bl.refrat_m_b = G.refrat_m_b, Bl.refrat_m_a3 = G.refrat_m_a3;
@@ -808,6 +803,13 @@ __device__ __forceinline__ auto lds_band(const WR_L R *lt, const LwImg<R> &im, c
 }
 // the wave's index in its workgroup, as the wave-uniform value it is
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64)); }
+
+// The wave's number in a grid of persistent workgroups, workgroups first: consecutive numbers are on different
+// CUs, so that the last round of a large tile spreads over the whole chip instead of filling a few workgroups
+// (796,590 columns are 12,447 blocks, 159 more than six rounds of 2,048 waves).  A tile of fewer blocks than the grid
+// could hold keeps few and full workgroups, so that the band streams share the chip (one wave on each CU
+// instead: 40,000 columns of the FP64 NAM route in 44 ms, not 26).
+__device__ __forceinline__ int wave_slot() { return wave_id() * (int)gridDim.x + (int)blockIdx.x; }
 
 // copies the image into the workgroup's LDS (16-byte words) and waits for the whole workgroup
 template <typename R, typename I> __device__ __forceinline__ void lds_fill(float4 *dst, const I &im)
@@ -843,7 +845,7 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
     lds_fill_lw<double>(lwl64_tab, im, T->exp_tbl);
     const auto Bl = lds_band<double, B>((const WR_L double *)lwl64_tab, im, T->lw[B], T->lw[B].absb);
     constexpr int WPG = lwl64_wpg<double, B>();
-    const int lane = threadIdx.x % 64, w = blockIdx.x * WPG + wave_id();
+    const int lane = threadIdx.x % 64, w = wave_slot();
     WR_G char *slot = (WR_G char *)(pool + (size_t)w * lw64_slot_bytes(LW_NG[B], in.nlay + 2));
     for (int blk = w; blk * 64 < n; blk += gridDim.x * WPG)
         lw_column<double, B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane, slot);
@@ -993,20 +995,19 @@ __global__ void __launch_bounds__(64 * lwl_wpg<B>(), lwc_waves<B>())
     const WR_L float *lt = (const WR_L float *)lwl_tab;
     const auto Bl = lds_band<float, B>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
     constexpr int WPG = lwl_wpg<B>();
-    const int lane = threadIdx.x % 64, w = blockIdx.x * WPG + wave_id();
+    const int lane = threadIdx.x % 64, w = wave_slot();
     WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(LW_NV_F32, LW_NG[B], in.nlay + 2, 4));
     for (int blk = w; blk * 64 < n; blk += gridDim.x * WPG)
         lw_column_f32c<B, SURR>(T, Bl, in, par, col0, n, cs, rp, acc, sg, blk, lane, slot);
 }
 
-// Waves per SIMD the SW kernels are compiled for, per band, measured serialised on the 954x835x60
-// grid:
-// * FP64 (both routes): bands 16, 25, 26, 28 fit two waves with few spills (16-27 % faster each);
-// * FP32 McICA route: two waves for the bands that spill at one; bands 16, 18, 19, 22, 24, 25, 26 fit
-//   two waves by their register count, and the bound only slowed their schedule (8-14 %);
-// * FP32 NAM route: two waves for every band but 22 (one wave 25-45 % slower).
+// Waves per SIMD the SW kernels are compiled for, per band: what the registers allow without much scratch; two
+// g-points a chunk in both precisions.  FP64 McICA, one wave -> two, alone on 796,590 columns: bands 18, 19, 24, 27
+// 5.45 -> 5.10, 5.45 -> 5.22, 5.55 -> 5.38, 5.98 -> 5.00 ms; bands 17, 20, 21, 23, 29 lose (17: 8.9 -> 13.0 ms with
+// 628 bytes of scratch a lane).  The NAM route holds two skies, hence its own row.
 // WR_SW64_WAVES / WR_SW32_WAVES > 0 override the tables for every band (tuning builds).
-constexpr int SW64_WAVES[14] = {2, 1, 1, 1, 1, 1, 2, 1, 1, 2, 2, 1, 2, 1};
+constexpr int SW64_WAVES[14] = {2, 1, 2, 2, 1, 1, 2, 1, 2, 2, 2, 2, 2, 1};
+constexpr int SWR64_WAVES[14] = {2, 1, 1, 1, 1, 1, 2, 1, 1, 2, 2, 1, 2, 1};
 constexpr int SW32_WAVES[14] = {3, 2, 2, 2, 2, 2, 4, 2, 2, 3, 3, 2, 3, 2};
 constexpr int SWR32_WAVES[14] = {3, 2, 2, 2, 2, 2, 4, 2, 2, 3, 3, 2, 3, 2};
 // g-points per chunk of the layer R/T (0: the whole band), by precision and route
@@ -1023,7 +1024,7 @@ template <typename R, int B, bool NAM = false> constexpr int sw_chunk()
 #endif
 template <typename R, int B, bool NAM = false> constexpr int sw_waves()
 {
-    if (sizeof(R) == 8) return WR_SW64_WAVES > 0 ? WR_SW64_WAVES : SW64_WAVES[B];
+    if (sizeof(R) == 8) return WR_SW64_WAVES > 0 ? WR_SW64_WAVES : (NAM ? SWR64_WAVES[B] : SW64_WAVES[B]);
     return WR_SW32_WAVES > 0 ? WR_SW32_WAVES : (NAM ? SWR32_WAVES[B] : SW32_WAVES[B]);
 }
 
@@ -1310,8 +1311,10 @@ template <typename R> constexpr int sw_nv() { return sizeof(R) == 4 ? 5 : 2; }
 template <typename R, int NG> struct SwSlot {
     WR_G char *p;
     int lane, nk;
-    __device__ __forceinline__ void put(int k, int g, const R (&v)[sw_nv<R>()]) const  // pb, pd; FP32 al, be, ld
+    // sky 1 (NAM route: the total sky beside the clear one) lies behind sky 0
+    __device__ __forceinline__ void put(int k, int sky, int g, const R (&v)[sw_nv<R>()]) const  // pb, pd; FP32 al, be, ld
     {
+        WR_G char *const p = this->p + (size_t)sky * nk * NG * 64 * sw_nv<R>() * sizeof(R);
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
         if constexpr (sizeof(R) == 4) {
             ((WR_G f32x4v *)p)[e] = (f32x4v){v[0], v[1], v[2], v[3]};
@@ -1320,8 +1323,9 @@ template <typename R, int NG> struct SwSlot {
             ((WR_G f64x2v *)p)[e] = (f64x2v){v[0], v[1]};
         }
     }
-    __device__ __forceinline__ void get(int k, int g, R (&v)[sw_nv<R>()]) const
+    __device__ __forceinline__ void get(int k, int sky, int g, R (&v)[sw_nv<R>()]) const
     {
+        const WR_G char *const p = this->p + (size_t)sky * nk * NG * 64 * sw_nv<R>() * sizeof(R);
         const size_t e = ((size_t)k * NG + g) * 64 + lane;
         if constexpr (sizeof(R) == 4) {
             const f32x4v q = ((const WR_G f32x4v *)p)[e];
@@ -1335,92 +1339,119 @@ template <typename R, int NG> struct SwSlot {
 };
 
 // The adding method over one column: bottom-up reflectances to the slot, then the direct and diffuse beams
-// top-down with the level fluxes.  layer(k, step) gives a layer (step: the sweep's direction), rt_at(layer, k, g0, o)
-// its R/T of a chunk of the lane's g-points, sun(g) the solar source of one; emit(level, {up, down}) takes a
-// level's fluxes, top first.
-template <typename R, int NG, int GW, int CH, typename SLOT, typename LAYER, typename RT, typename SUN, typename EMIT>
-__device__ __forceinline__ void sw_adding(int nrl, R asfc, SLOT &&slot, int lane, const Share<R> &sh, LAYER &&layer, RT &&rt_at,
-                                          SUN &&sun, EMIT &&emit)
+// top-down with the level fluxes.  NP skies at once (the NAM route's clear and total sky, whose layers differ only
+// where there is cloud: one evaluation of the optics serves both; the second is skipped as a whole where two is
+// false).  layer(k, step) gives a layer (step: the sweep's direction), rt_at(layer, k, g0, o) its R/T of a chunk of
+// the lane's g-points in each sky, sun(g) the solar source of one; emit(level, {up, down of each sky}) takes
+// a level's fluxes, top first.
+template <typename R, int NG, int GW, int CH, int NP, typename SLOT, typename LAYER, typename RT, typename SUN, typename EMIT>
+__device__ __forceinline__ void sw_adding(int nrl, R asfc, bool two, SLOT &&slot, int lane, const Share<R> &sh, LAYER &&layer,
+                                          RT &&rt_at, SUN &&sun, EMIT &&emit)
 {
-    R pb[GW], pd[GW];
+    R pb[NP][GW], pd[NP][GW];
 #pragma unroll
-    for (int g = 0; g < GW; ++g) pb[g] = asfc, pd[g] = asfc;
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int g = 0; g < GW; ++g) pb[p][g] = asfc, pd[p][g] = asfc;
     for (int k = 0; k < nrl; ++k) {
         auto a = layer(k, 1);
 #pragma unroll
         for (int g0 = 0; g0 < GW; g0 += CH) {
-            RtV<R, CH> o;
-            rt_at(a, k, g0, o);
+            RtV<R, CH> os[NP];
+            rt_at(a, k, g0, os);
 #pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const int g = g0 + j;
-                const R zden1 = rdiv<R>((R)1, (R)1 - pd[g] * o.rd[j]);
-                if constexpr (sizeof(R) == 4) {
-                    const R sc = o.tb[j] - o.ld[j], lb = o.ld[j] * pb[g], al = o.td[j] * zden1;
-                    slot.put(k, g, {pb[g], pd[g], al, (sc + o.rd[j] * lb) * zden1, o.ld[j]});
-                    pb[g] = o.rb[j] + al * (sc * pd[g] + lb);
-                    pd[g] = o.rd[j] + al * o.td[j] * pd[g];
-                } else {
-                    slot.put(k, g, {pb[g], pd[g]});
-                    const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * pd[g] + o.ld[j] * pb[g])) * zden1;
-                    const R nd = o.rd[j] + o.td[j] * o.td[j] * pd[g] * zden1;
-                    pb[g] = nb, pd[g] = nd;
+            for (int p = 0; p < NP; ++p) {
+                if (p > 0 && !two) break;
+                const RtV<R, CH> &o = os[p];
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const int g = g0 + j;
+                    R &b = pb[p][g], &d = pd[p][g];
+                    const R zden1 = rdiv<R>((R)1, (R)1 - d * o.rd[j]);
+                    if constexpr (sizeof(R) == 4) {
+                        const R sc = o.tb[j] - o.ld[j], lb = o.ld[j] * b, al = o.td[j] * zden1;
+                        slot.put(k, p, g, {b, d, al, (sc + o.rd[j] * lb) * zden1, o.ld[j]});
+                        b = o.rb[j] + al * (sc * d + lb);
+                        d = o.rd[j] + al * o.td[j] * d;
+                    } else {
+                        slot.put(k, p, g, {b, d});
+                        const R nb = o.rb[j] + (o.td[j] * ((o.tb[j] - o.ld[j]) * d + o.ld[j] * b)) * zden1;
+                        const R nd = o.rd[j] + o.td[j] * o.td[j] * d * zden1;
+                        b = nb, d = nd;
+                    }
                 }
             }
             if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    R zsolar[GW], f[2][GW];
-    LevelSum<R, NG, GW, 2> sum{sh, lane, 0, 0, 0};
+    R zsolar[GW], f[2 * NP][GW];
+    LevelSum<R, NG, GW, 2 * NP> sum{sh, lane, 0, 0, 0};
     sum.begin(nrl, -1);
 #pragma unroll
     for (int g = 0; g < GW; ++g) {
         zsolar[g] = sun(g);
-        f[0][g] = zsolar[g] * pb[g];
-        f[1][g] = zsolar[g];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            f[2 * p][g] = zsolar[g] * pb[p][g];
+            f[2 * p + 1][g] = zsolar[g];
+        }
     }
     sum.put(f, emit);
     if constexpr (sizeof(R) == 4) {
-        R s[GW], d[GW];  // direct and diffuse beams
+        R s[NP][GW], d[NP][GW];  // direct and diffuse beams
 #pragma unroll
-        for (int g = 0; g < GW; ++g) s[g] = zsolar[g], d[g] = (R)0;
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int g = 0; g < GW; ++g) s[p][g] = zsolar[g], d[p][g] = (R)0;
         for (int k = nrl - 1; k >= 0; --k) {
 #pragma unroll
-            for (int g = 0; g < GW; ++g) {
-                R v[5];
-                slot.get(k, g, v);
-                d[g] = v[2] * d[g] + v[3] * s[g];
-                s[g] = v[4] * s[g];
-                f[0][g] = s[g] * v[0] + d[g] * v[1];
-                f[1][g] = s[g] + d[g];
+            for (int p = 0; p < NP; ++p) {
+                if (p > 0 && !two) break;
+#pragma unroll
+                for (int g = 0; g < GW; ++g) {
+                    R v[5];
+                    slot.get(k, p, g, v);
+                    d[p][g] = v[2] * d[p][g] + v[3] * s[p][g];
+                    s[p][g] = v[4] * s[p][g];
+                    f[2 * p][g] = s[p][g] * v[0] + d[p][g] * v[1];
+                    f[2 * p + 1][g] = s[p][g] + d[p][g];
+                }
             }
             sum.put(f, emit);
         }
     } else {
-        R tdbt[GW], tdn[GW], rdnd[GW];
+        R tdbt[NP][GW], tdn[NP][GW], rdnd[NP][GW];
 #pragma unroll
-        for (int g = 0; g < GW; ++g) tdbt[g] = (R)1, tdn[g] = (R)1, rdnd[g] = (R)0;
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int g = 0; g < GW; ++g) tdbt[p][g] = (R)1, tdn[p][g] = (R)1, rdnd[p][g] = (R)0;
         for (int k = nrl - 1; k >= 0; --k) {
             auto a = layer(k, -1);
 #pragma unroll
             for (int g0 = 0; g0 < GW; g0 += CH) {
-                RtV<R, CH> o;
-                rt_at(a, k, g0, o);
+                RtV<R, CH> os[NP];
+                rt_at(a, k, g0, os);
 #pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const int g = g0 + j;
-                    R z[2];
-                    slot.get(k, g, z);
-                    const R tdbt_s = o.ld[j] * tdbt[g];
-                    const R zden0 = (R)1 / ((R)1 - o.rd[j] * rdnd[g]);
-                    const R tdn_s = tdbt[g] * o.tb[j] + (o.td[j] * ((tdn[g] - tdbt[g]) + tdbt[g] * o.rb[j] * rdnd[g])) * zden0;
-                    const R rdnd_s = o.rd[j] + o.td[j] * o.td[j] * rdnd[g] * zden0;
-                    tdbt[g] = tdbt_s, tdn[g] = tdn_s, rdnd[g] = rdnd_s;
-                    const R zden1 = (R)1 / ((R)1 - rdnd_s * z[1]);
-                    const R zfu = (tdbt_s * z[0] + (tdn_s - tdbt_s) * z[1]) * zden1;
-                    const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * z[0] * rdnd_s) * zden1;
-                    f[0][g] = zsolar[g] * zfu;
-                    f[1][g] = zsolar[g] * zfd;
+                for (int p = 0; p < NP; ++p) {
+                    if (p > 0 && !two) break;
+                    const RtV<R, CH> &o = os[p];
+#pragma unroll
+                    for (int j = 0; j < CH; ++j) {
+                        const int g = g0 + j;
+                        R z[2];
+                        slot.get(k, p, g, z);
+                        const R db = tdbt[p][g], dn = tdn[p][g], rn = rdnd[p][g];
+                        const R tdbt_s = o.ld[j] * db;
+                        const R zden0 = (R)1 / ((R)1 - o.rd[j] * rn);
+                        const R tdn_s = db * o.tb[j] + (o.td[j] * ((dn - db) + db * o.rb[j] * rn)) * zden0;
+                        const R rdnd_s = o.rd[j] + o.td[j] * o.td[j] * rn * zden0;
+                        tdbt[p][g] = tdbt_s, tdn[p][g] = tdn_s, rdnd[p][g] = rdnd_s;
+                        const R zden1 = (R)1 / ((R)1 - rdnd_s * z[1]);
+                        const R zfu = (tdbt_s * z[0] + (tdn_s - tdbt_s) * z[1]) * zden1;
+                        const R zfd = tdbt_s + (tdn_s - tdbt_s + tdbt_s * z[0] * rdnd_s) * zden1;
+                        f[2 * p][g] = zsolar[g] * zfu;
+                        f[2 * p + 1][g] = zsolar[g] * zfd;
+                    }
                 }
                 if constexpr (CH < GW) __builtin_amdgcn_sched_barrier(0);
             }
@@ -1467,18 +1498,18 @@ __device__ __forceinline__ void sw_column(const Tabs<R> *__restrict__ T, const B
         SwLayer<R> y;
         uint32_t bits;
     };
-    sw_adding<R, NG, NG, CH>(
-        nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
+    sw_adding<R, NG, NG, CH, 1>(
+        nrl, c.asfc, false, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
         [&](int k, int) {
             Lay a;
             sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
             a.bits = a.y.cloudy ? mword(rp.msw, rp.row(blk, k), MROW_SW, B, rl) : 0u;
             return a;
         },
-        [&](const Lay &a, int k, int g0, RtV<R, CH> &o) {
+        [&](const Lay &a, int k, int g0, RtV<R, CH> (&o)[1]) {
             R tg[CH], tr[CH];
             sw_tgtr<R, B, SURR, CH>(T, Bt, sg, table, (size_t)k * n + t, k, c.lt, a.y.L, g0, tg, tr);
-            layer_rt_sky<R, CH>(T, tr, tg, a.y.y, a.bits >> g0, o, fx);
+            layer_rt_sky<R, CH>(T, tr, tg, a.y.y, a.bits >> g0, o[0], fx);
         },
         [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
         [&](int lev, const R *f) {
@@ -1539,7 +1570,7 @@ __global__ void __launch_bounds__((64 * swl_wpg<R, B>()), (sw_waves<R, B>()))
     const auto Bl = sw_lds_band<R>((const WR_L R *)swl_tab, T->sw_img[B], T->sw[B]);
     constexpr int WPG = swl_wpg<R, B>();
     __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
-    const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
+    const int lane = threadIdx.x % 64, wv = wave_id(), w = wave_slot();
     WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)

@@ -276,7 +276,7 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                     nb = 0;
                 per_cu = nb;
             }
-            const size_t slot = cache_slot_bytes(sw_nv<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
+            const size_t slot = cache_slot_bytes(2 * sw_nv<R>(), SW_NG[S], j.in.nlay + 2, (int)sizeof(R));
             const size_t nwg_pool = j.c->pool_bytes / slot / WPG;
             const size_t nwg_cols = ((size_t)j.n + 64 * WPG - 1) / (64 * WPG);
             size_t nwg = (size_t)(j.c->n_cu > 0 ? j.c->n_cu : 1) * (size_t)std::max(per_cu.load(), 0);
@@ -286,7 +286,7 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
                 hipLaunchKernelGGL((k_swrl<R, S, EXT>), dim3((unsigned)nwg), dim3(64 * WPG), lds, s, j.tabs, j.in, j.par,
                                    j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
             else
-                hipLaunchKernelGGL((k_swr<R, S, EXT>), dim3(band_grid(j, sw_nv<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
+                hipLaunchKernelGGL((k_swr<R, S, EXT>), dim3(band_grid(j, 2 * sw_nv<R>(), SW_NG[S])), dim3(64), 0, s, j.tabs,
                                    j.in, j.par, j.col0, j.n, j.cs, j.rp, j.sflux, acc, pool);
         }
         tend(j.c, s);
@@ -365,7 +365,7 @@ template <typename R> void launch_prep(const BandJob<R> &j, hipStream_t s)
     }
 }
 
-// Whether a tile of n columns runs all its bands in one launch (wr_many.h)
+// Whether a tile of n columns runs all its bands in the two launches of wr_many.h (the line: MANY_COLS_DEFAULT)
 inline bool use_many(const wr_ctx *c, int n, int band) { return band < 0 && n <= c->many_cols && !c->lw_glane; }
 
 // One tile of n columns from col0 (McICA route): column scalars, day list, band kernels, FP64 post.

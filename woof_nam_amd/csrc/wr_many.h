@@ -33,12 +33,12 @@ constexpr int MANY_ORDER[30] = {17, 29, 21, 20, 23, 2,  4,  3,  24, 8,  6,  19, 
 template <typename R, bool NAM> constexpr int many_vl() { return NAM ? 6 : sizeof(R) == 4 ? 3 : 5; }
 template <bool NAM> constexpr int many_vs() { return NAM ? 10 : 5; }
 // pool values of one 64-column block, per lane: [140][nrl][VL], surface source [140], cloud transmittance
-// [16][nrl], SW [112][nrl][VS], FP64 reflectances [112][nrl][2] (the FP32 sweep leaves its 5 values in the
-// place of the layer's R/T)
+// [16][nrl], SW [112][nrl][VS], FP64 reflectances [112][nrl][2] of each sky (the FP32
+// sweep leaves its 5 values in the place of the layer's R/T)
 template <typename R, bool NAM> constexpr size_t many_lane_values(int nrl)
 {
     return (size_t)140 * nrl * many_vl<R, NAM>() + 140 + (size_t)16 * nrl + (size_t)112 * nrl * many_vs<NAM>() +
-           (sizeof(R) == 8 ? (size_t)112 * nrl * sw_nv<R>() : 0);
+           (sizeof(R) == 8 ? (size_t)112 * nrl * sw_nv<R>() * (NAM ? 2 : 1) : 0);
 }
 template <typename R, bool NAM> constexpr size_t many_block_bytes(int nrl)
 {
@@ -74,9 +74,10 @@ template <typename R, bool NAM> struct ManyBlk {
     {
         return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + ((size_t)g * nrl + k) * VS) * 64 + lane;
     }
-    __device__ __forceinline__ WR_G R *refl(int g, int k, int lane) const
+    __device__ __forceinline__ WR_G R *refl(int g, int k, int sky, int lane) const
     {
-        return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + (size_t)112 * nrl * VS + ((size_t)g * nrl + k) * 2) * 64 + lane;
+        return p + ((size_t)140 * nrl * VL + 140 + (size_t)16 * nrl + (size_t)112 * nrl * VS +
+                    ((size_t)g * nrl + k) * (NAM ? 4 : 2) + 2 * sky) * 64 + lane;
     }
 };
 template <typename R, bool NAM>
@@ -107,7 +108,10 @@ __device__ __forceinline__ void lay_lw(const ManyArgs<R> &a, int b, int k, int l
     const R dd = y.bbot - y.blay, du = btop - y.blay;
     R ecld = (R)1;
     if (!NAM && __any(y.cloudy)) ecld = M<R>::exp(-y.odcld);
-    if constexpr (!NAM && sizeof(R) == 8) *m.ef(B, k, lane) = (R)1 - ((R)1 - ecld);
+    // what only clouds need is stored where the block's layer has any (many_cloud tells the sweeps)
+    const bool some = __any(y.cloudy);
+    if constexpr (!NAM && sizeof(R) == 8)
+        if (some) *m.ef(B, k, lane) = (R)1 - ((R)1 - ecld);
 #pragma unroll
     for (int g0 = 0; g0 < NG; g0 += CH) {
         R tau[CH], fr[CH];
@@ -155,8 +159,11 @@ __device__ __forceinline__ void lay_lw(const ManyArgs<R> &a, int b, int k, int l
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 WR_G R *w = m.lw(NS + g0 + j, k, lane);
-                w[0] = q.tr[j], w[64] = gd[j], w[128] = sd[j], w[192] = gu[j], w[256] = su[j];
-                if constexpr (NAM) w[320] = trc[j];
+                w[0] = q.tr[j], w[64] = gd[j], w[192] = gu[j];
+                if (some) {
+                    w[128] = sd[j], w[256] = su[j];
+                    if constexpr (NAM) w[320] = trc[j];
+                }
             }
         }
         if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
@@ -179,8 +186,9 @@ __device__ __forceinline__ void lay_sw(const ManyArgs<R> &a, int b, int k, int l
     uint32_t bits = 0;
     bool mix = false;
     R zc1 = (R)0, zc0 = (R)1;
+    const bool some = __any(y.cloudy);
     if constexpr (NAM) {
-        if (__any(y.cloudy)) {
+        if (some) {
             const RadCol rcol{a.in, c.i, a.rp.nrl};
             const double cf1 = a.cs.zcf1[t], z = rcol.cfrac(a.rp.nrl - 1 - k) / cf1;
             mix = cf1 > EPS && z > FTINY, zc1 = (R)z, zc0 = (R)(1.0 - z);
@@ -200,13 +208,13 @@ __device__ __forceinline__ void lay_sw(const ManyArgs<R> &a, int b, int k, int l
 #pragma unroll
         for (int j = 0; j < CH; ++j) put(m.sw(NS + g0 + j, k, lane), o, j);
         if constexpr (NAM) {
-            if (__any(mix)) {
+            if (some) {
                 RtV<R, CH> d;
                 layer_rt_sky<R, CH>(a.T, tr, tg, y.y, ~0u, d, fx);
                 rt_mix<R, CH>(mix, zc0, zc1, d, o);
-            }
 #pragma unroll
-            for (int j = 0; j < CH; ++j) put(m.sw(NS + g0 + j, k, lane) + 320, o, j);
+                for (int j = 0; j < CH; ++j) put(m.sw(NS + g0 + j, k, lane) + 320, o, j);
+            }
         }
         if constexpr (CH < NG) __builtin_amdgcn_sched_barrier(0);
     }
@@ -235,6 +243,18 @@ __global__ void __launch_bounds__(64 * MANY_LAYERS, sizeof(R) == 4 ? 3 : 2) k_la
 }
 
 // ---- sweeps of one block and band ----------------------------------------------------------------
+// The layers of a block that hold cloud in any of its columns (bit k).
+template <bool SW, typename R> __device__ __forceinline__ uint64_t many_cloud(const RecPtrs &rp, int blk, int lane)
+{
+    uint64_t m = 0;
+#pragma unroll 8
+    for (int k = 0; k < rp.nrl; ++k) {
+        const uint32_t w = SW ? srow<R>(rp, blk, k, lane).w(1) : lrow<R>(rp, blk, k, lane).w(1) & 256u;
+        m |= (uint64_t)(__any(w != 0) ? 1 : 0) << k;
+    }
+    return m;
+}
+
 template <typename R, int B, bool NAM>
 __device__ __forceinline__ void sweep_lw(const ManyArgs<R> &a, int b, int lane, const Share<R> &sh)
 {
@@ -261,13 +281,14 @@ __device__ __forceinline__ void sweep_lw(const ManyArgs<R> &a, int b, int lane, 
     uint64_t lstu = 0, lstd = 0;
     if constexpr (NAM) lstu = a.rt.lstu[t], lstd = a.rt.lstd[t];
     const RadCol rcol{a.in, c.i, nrl};
+    const uint64_t clouds = NAM || sizeof(R) == 8 ? many_cloud<false, R>(a.rp, blk, rl) : 0;
     // one layer; v: 0 the downward values, 1 the upward ones
     auto step = [&](int k, int v) {
         if constexpr (NAM) {
-            const R clfr = (R)rcol.cfrac(nrl - 1 - k);
-            const bool cloudy = clfr > (R)0;
             RtrStep<R> f{};
-            const bool some = __any(cloudy);
+            const bool some = (clouds >> k) & 1;
+            const R clfr = some ? (R)rcol.cfrac(nrl - 1 - k) : (R)0;
+            const bool cloudy = clfr > (R)0;
             if (some) f = rtr_step<R>(a.rt, v ? FCLD1U : FCLD1D, v ? k + 2 : k, t, clfr, ((v ? lstu : lstd) >> k) & 1);
 #pragma unroll
             for (int j = 0; j < GW; ++j) {
@@ -285,16 +306,24 @@ __device__ __forceinline__ void sweep_lw(const ManyArgs<R> &a, int b, int lane, 
                 rad[0][j] = rad[0][j] * q[0] + q[v ? 128 : 64];
             }
         } else {
-            // a clear g-point: cloud transmittance 1 and cloud source 0, which leave the value as it is
-            const R ef = *m.ef(B, k, lane);
-            const uint32_t w1 = lrow<R>(a.rp, blk, k, rl).w(1);
-            const uint32_t word = mword(a.rp.mlw, a.rp.row(blk, k), MROW_LW, B, rl);
-            const uint32_t bits = (w1 & 256u) ? word >> sh.g0 : 0u;
+            if ((clouds >> k) & 1) {
+                // a clear g-point: cloud transmittance 1 and cloud source 0, which leave the value as it is
+                const R ef = *m.ef(B, k, lane);
+                const uint32_t w1 = lrow<R>(a.rp, blk, k, rl).w(1);
+                const uint32_t word = mword(a.rp.mlw, a.rp.row(blk, k), MROW_LW, B, rl);
+                const uint32_t bits = (w1 & 256u) ? word >> sh.g0 : 0u;
 #pragma unroll
-            for (int j = 0; j < GW; ++j) {
-                const WR_G R *q = m.lw(gs + j, k, lane);
-                const R e = (bits >> j) & 1u ? ef : (R)1;
-                rad[0][j] = rad[0][j] * q[0] * e + q[v ? 192 : 64] + q[v ? 256 : 128];
+                for (int j = 0; j < GW; ++j) {
+                    const WR_G R *q = m.lw(gs + j, k, lane);
+                    const R e = (bits >> j) & 1u ? ef : (R)1;
+                    rad[0][j] = rad[0][j] * q[0] * e + q[v ? 192 : 64] + q[v ? 256 : 128];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < GW; ++j) {
+                    const WR_G R *q = m.lw(gs + j, k, lane);
+                    rad[0][j] = rad[0][j] * q[0] + q[v ? 192 : 64];
+                }
             }
         }
     };
@@ -320,66 +349,28 @@ __device__ __forceinline__ void sweep_lw(const ManyArgs<R> &a, int b, int lane, 
     sum.finish(up);
 }
 
-// The slot of a sweep's g-points: FP32 in the place of the layer's R/T (the direct transmission, its fifth value, stays).
-// The top-down sweep's reads run SWEEP_AHEAD layers ahead of their use, as do those of the R/T (RtAhead).
-constexpr int SWEEP_AHEAD = 3;
+// The slot of a sweep's g-points: FP32 in the place of the layer's R/T.  Reading the layers ahead of their use into
+// registers gained nothing (FP32 within 2 %; in FP64 the registers cost more than it gave).
 template <typename R, bool NAM, int GW> struct ManySlot {
     static constexpr int NV = sw_nv<R>();
     ManyBlk<R, NAM> m;
-    int g0, lane, pass;
-    R v[GW][SWEEP_AHEAD][NV];
-    __device__ __forceinline__ WR_G R *at(int k, int g) const
+    int g0, lane;
+    __device__ __forceinline__ WR_G R *at(int k, int sky, int g) const
     {
-        return sizeof(R) == 4 ? m.sw(g0 + g, k, lane) + pass * 320 : m.refl(g0 + g, k, lane);
+        return sizeof(R) == 4 ? m.sw(g0 + g, k, lane) + sky * 320 : m.refl(g0 + g, k, sky, lane);
     }
-    __device__ __forceinline__ void put(int k, int g, const R (&x)[NV]) const
+    __device__ __forceinline__ void put(int k, int sky, int g, const R (&x)[NV]) const
     {
-        WR_G R *q = at(k, g);
-        q[0] = x[0], q[64] = x[1];
-        if constexpr (NV == 5) q[128] = x[2], q[192] = x[3];
+        WR_G R *q = at(k, sky, g);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (i < 4 || sky) q[64 * i] = x[i];  // the fifth, the direct transmission, is in place already in sky 0
     }
-    __device__ __forceinline__ void load(int k, int g, R (&x)[NV]) const
+    __device__ __forceinline__ void get(int k, int sky, int g, R (&x)[NV]) const
     {
-        const WR_G R *q = at(imax(k, 0), g);
+        const WR_G R *q = at(k, sky, g);
 #pragma unroll
         for (int i = 0; i < NV; ++i) x[i] = q[64 * i];
-    }
-    __device__ __forceinline__ void get(int k, int g, R (&x)[NV])
-    {
-        if (k == m.nrl - 1)
-#pragma unroll
-            for (int d = 0; d < SWEEP_AHEAD; ++d) load(k - d, g, v[g][d]);
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            x[i] = v[g][0][i];
-#pragma unroll
-            for (int d = 0; d + 1 < SWEEP_AHEAD; ++d) v[g][d][i] = v[g][d + 1][i];
-        }
-        load(k - SWEEP_AHEAD, g, v[g][SWEEP_AHEAD - 1]);
-    }
-};
-template <typename R, bool NAM, int GW> struct RtAhead {
-    ManyBlk<R, NAM> m;
-    int g0, lane, pass;
-    RtV<R, GW> v[SWEEP_AHEAD];
-    __device__ __forceinline__ void load(int k, RtV<R, GW> &o) const
-    {
-#pragma unroll
-        for (int j = 0; j < GW; ++j) {
-            const WR_G R *q = m.sw(g0 + j, imin(imax(k, 0), m.nrl - 1), lane) + pass * 320;
-            o.rb[j] = q[0], o.rd[j] = q[64], o.tb[j] = q[128], o.td[j] = q[192], o.ld[j] = q[256];
-        }
-    }
-    __device__ __forceinline__ RtV<R, GW> next(int k, int step)
-    {
-        if (k == (step > 0 ? 0 : m.nrl - 1))
-#pragma unroll
-            for (int d = 0; d < SWEEP_AHEAD; ++d) load(k + d * step, v[d]);
-        const RtV<R, GW> o = v[0];
-#pragma unroll
-        for (int d = 0; d + 1 < SWEEP_AHEAD; ++d) v[d] = v[d + 1];
-        load(k + SWEEP_AHEAD * step, v[SWEEP_AHEAD - 1]);
-        return o;
     }
 };
 
@@ -398,26 +389,37 @@ __device__ __forceinline__ void sweep_sw(const ManyArgs<R> &a, int b, int lane, 
     const double cf1 = a.cs.zcf1[t], cf0 = a.cs.zcf0[t];
     const bool total = NAM && cf1 > EPS;
     if (!NAM && ok) acc.sw_clr0[t] = (R)0;  // clear-sky surface flux: NAM route only
-    const int passes = __any(total) ? 2 : 1;
-    for (int pass = 0; pass < passes; ++pass) {
-        ManySlot<R, NAM, GW> slot{m, NS + sh.g0, lane, pass, {}};
-        RtAhead<R, NAM, GW> rt{m, NS + sh.g0, lane, pass, {}};
-        sw_adding<R, NG, GW, GW>(
-            nrl, c.asfc, slot, lane, sh, [&](int k, int step) { return rt.next(k, step); },
-            [](const RtV<R, GW> &v, int, int, RtV<R, GW> &o) { o = v; },
-            [&](int g) { return c.ssolar * a.sflux[(size_t)(NS + sh.g0 + g) * a.n + t]; },
-            [&](int lev, const R *f) {
-                const size_t p = (size_t)lev * a.n + t;
-                if (ok && pass == 0) {
-                    if (NAM && lev == 0) acc.sw_clr0[t] = f[1];
-                    acc.sw_up[p] = f[0];
-                    acc.sw_dn[p] = f[1];
-                } else if (ok && total) {  // the clear-sky fluxes of pass 0 mixed with the cloudy ones
-                    acc.sw_up[p] = (R)(cf1 * (double)f[0] + cf0 * (double)acc.sw_up[p]);
-                    acc.sw_dn[p] = (R)(cf1 * (double)f[1] + cf0 * (double)acc.sw_dn[p]);
+    const bool two = NAM && __any(total);
+    constexpr int NP = NAM ? 2 : 1;
+    const uint64_t clouds = two ? many_cloud<true, R>(a.rp, blk, rl) : 0;  // layers whose total-sky R/T differ
+    sw_adding<R, NG, GW, GW, NP>(
+        nrl, c.asfc, two, ManySlot<R, NAM, GW>{m, NS + sh.g0, lane}, lane, sh, [](int k, int) { return k; },
+        [&](int, int k, int, RtV<R, GW> (&o)[NP]) {
+            auto one = [&](int sky) {
+#pragma unroll
+                for (int j = 0; j < GW; ++j) {
+                    const WR_G R *q = m.sw(NS + sh.g0 + j, k, lane) + sky * 320;
+                    RtV<R, GW> &r = o[sky];
+                    r.rb[j] = q[0], r.rd[j] = q[64], r.tb[j] = q[128], r.td[j] = q[192], r.ld[j] = q[256];
                 }
-            });
-    }
+            };
+            one(0);
+            if constexpr (NAM) {
+                if ((clouds >> k) & 1)
+                    one(1);
+                else
+                    o[1] = o[0];
+            }
+        },
+        [&](int g) { return c.ssolar * a.sflux[(size_t)(NS + sh.g0 + g) * a.n + t]; },
+        [&](int lev, const R *f) {
+            if constexpr (NAM) {
+                swr_emit<R>(acc, ok, total, cf1, cf0, lev, a.n, t, f);
+            } else if (ok) {
+                acc.sw_up[(size_t)lev * a.n + t] = f[0];
+                acc.sw_dn[(size_t)lev * a.n + t] = f[1];
+            }
+        });
 }
 
 template <typename R, bool NAM, int P>

@@ -1,4 +1,4 @@
-// wr_many_fp64.hip -- the one-launch band kernel of small tiles (FP64, McICA route).
+// wr_many_fp64.hip -- the optics and sweep kernels of small tiles (FP64, McICA route; wr_many.h).
 #include "wr_many.h"
 
 namespace wr {

@@ -145,12 +145,8 @@ __global__ void __launch_bounds__(64) k_rtr_fac(ColIn in, int col0, int n, Rtr<R
 }
 
 // ---- LW band kernel of the NAM route (rtrnmr) ---------------------------------------------------
-// Per-band optics chunks (g-points, 0 = whole band) and wave bounds, by precision, as for the McICA
-// route's LW kernels: a second resident wave covers the table-gather waits where the registers allow.
-// Chosen per band from serialised timings on the 954x835x60 grid (chunks of 2 or 4, bound 1 or 2):
-// FP32 bands 1, 2, 4, 7, 8, 9, 12 run 14-29 % faster at two waves, band 16 7 % faster at three; the
-// FP32 bands 3 and 5 and most FP64 bands were fastest as they were (FP64 bands 6 and 11 gain 9 and
-// 17 %).
+// Per-band optics chunks and wave bounds, by precision, as for the McICA route's LW kernels (same reasons); the
+// three radiances a g-point of a cloudy layer has (clear, cloudy, their overlap) leave room for fewer waves.
 // WR_LWR_WAVES > 0 or WR_LWR_CHUNK >= 0 override the tables for every band (tuning builds).
 constexpr int LWR64_WAVES[16] = {1, 1, 1, 1, 1, 2, 1, 2, 1, 2, 2, 2, 2, 2, 2, 2};
 constexpr int LWR64_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
@@ -327,11 +323,11 @@ __global__ void __launch_bounds__((64 * lwrl_wpg<R, B>()), (lwr_waves<R, B>()))
     const int lane = threadIdx.x % 64;
     if constexpr (sizeof(R) == 4) {
         const auto Bl = lds_band<R, B>(lt, im, T->lw[B], lt + (imax(0, im.off[1]) & ~3));
-        for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
+        for (int blk = wave_slot(); blk * 64 < n; blk += gridDim.x * WPG)
             lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     } else {
         const auto Bl = lds_band<R, B>(lt, im, T->lw[B], T->lw[B].absb);
-        for (int blk = blockIdx.x * WPG + wave_id(); blk * 64 < n; blk += gridDim.x * WPG)
+        for (int blk = wave_slot(); blk * 64 < n; blk += gridDim.x * WPG)
             lwr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, acc, rt, blk, lane);
     }
 }
@@ -350,9 +346,22 @@ template <typename R, int CH> __device__ __forceinline__ void rt_mix(bool mix, R
     }
 }
 
-// One day column of one SW band on the NAM route: clear-sky pass, then (cloudy columns) the total-sky pass,
+// The fluxes of a level, {clear up, clear down, total up, total down}, to the band planes.
+template <typename R>
+__device__ __forceinline__ void swr_emit(const AccT<R> &acc, bool ok, bool total, double cf1, double cf0, int lev, int n, int t,
+                                         const R *f)
+{
+    if (!ok) return;
+    const size_t p = (size_t)lev * n + t;
+    if (lev == 0) acc.sw_clr0[t] = f[1];
+    acc.sw_up[p] = total ? (R)(cf1 * (double)f[2] + cf0 * (double)f[0]) : f[0];
+    acc.sw_dn[p] = total ? (R)(cf1 * (double)f[3] + cf0 * (double)f[1]) : f[1];
+}
+
+// One day column of one SW band on the NAM route: the clear sky and, for cloudy columns, the total sky,
 // whose layers mix the cloudy R/T with the clear ones by the layer's cloud fraction over the column's
-// cover, zc1 = cfrac / zcf1 (phys_rrtm_sw_spcvrtc.cu, cloudy block); each pass is the adding method.
+// cover, zc1 = cfrac / zcf1 (phys_rrtm_sw_spcvrtc.cu, cloudy block).  Both skies go through the adding method
+// together, on one evaluation of the optics; the column's fluxes are cf1 x total + cf0 x clear.
 template <typename R, int B, typename BT>
 __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const BT &Bt, const ColIn &in, const RunPar &par, int col0,
                                            int n, const ColScal &cs, const RecPtrs &rp, const R *__restrict__ sflux,
@@ -375,44 +384,32 @@ __device__ __forceinline__ void swr_column(const Tabs<R> *__restrict__ T, const 
         R zc1, zc0;
         bool mix;
     };
-    const int passes = __any(total) ? 2 : 1;  // a column without cloud stores nothing in the second pass
-    for (int pass = 0; pass < passes; ++pass) {
-        sw_adding<R, NG, NG, CH>(
-            nrl, c.asfc, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
-            [&](int k, int) {
-                Lay a;
-                sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
-                a.mix = false, a.zc1 = (R)0, a.zc0 = (R)1;
-                if (pass && __any(a.y.cloudy)) {
-                    const double zc1 = rcol.cfrac(nrl - 1 - k) / cf1;
-                    a.mix = total && zc1 > FTINY, a.zc1 = (R)zc1, a.zc0 = (R)(1.0 - zc1);
-                }
-                return a;
-            },
-            [&](const Lay &a, int k, int g0, RtV<R, CH> &o) {
-                R tg[CH], tr[CH];
-                sw_tgtr<R, B, false, CH>(T, Bt, none, 1, 0, k, c.lt, a.y.L, g0, tg, tr);
-                layer_rt_sky<R, CH>(T, tr, tg, a.y.y, 0u, o, fx);
-                if (__any(a.mix)) {
-                    RtV<R, CH> d;
-                    layer_rt_sky<R, CH>(T, tr, tg, a.y.y, ~0u, d, fx);
-                    rt_mix<R, CH>(a.mix, a.zc0, a.zc1, d, o);
-                }
-            },
-            [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
-            [&](int lev, const R *f) {
-                // pass 0 leaves the clear-sky fluxes in the band planes, which pass 1 reads back and mixes
-                const size_t p = (size_t)lev * n + t;
-                if (ok && pass == 0) {
-                    if (lev == 0) acc.sw_clr0[t] = f[1];
-                    acc.sw_up[p] = f[0];
-                    acc.sw_dn[p] = f[1];
-                } else if (ok && total) {
-                    acc.sw_up[p] = (R)(cf1 * (double)f[0] + cf0 * (double)acc.sw_up[p]);
-                    acc.sw_dn[p] = (R)(cf1 * (double)f[1] + cf0 * (double)acc.sw_dn[p]);
-                }
-            });
-    }
+    const bool two = __any(total);
+    sw_adding<R, NG, NG, CH, 2>(
+        nrl, c.asfc, two, SwSlot<R, NG>{slot, lane, in.nlay + 2}, lane, Share<R>{nullptr, 0, 0},
+        [&](int k, int) {
+            Lay a;
+            sw_get<R, B>(T, in, par, rp, c.i, c.cz, c.snt, blk, rl, k, a.y);
+            a.mix = false, a.zc1 = (R)0, a.zc0 = (R)1;
+            if (two && __any(a.y.cloudy)) {
+                const double zc1 = rcol.cfrac(nrl - 1 - k) / cf1;
+                a.mix = total && zc1 > FTINY, a.zc1 = (R)zc1, a.zc0 = (R)(1.0 - zc1);
+            }
+            return a;
+        },
+        [&](const Lay &a, int k, int g0, RtV<R, CH> (&o)[2]) {
+            R tg[CH], tr[CH];
+            sw_tgtr<R, B, false, CH>(T, Bt, none, 1, 0, k, c.lt, a.y.L, g0, tg, tr);
+            layer_rt_sky<R, CH>(T, tr, tg, a.y.y, 0u, o[0], fx);
+            o[1] = o[0];
+            if (__any(a.mix)) {
+                RtV<R, CH> d;
+                layer_rt_sky<R, CH>(T, tr, tg, a.y.y, ~0u, d, fx);
+                rt_mix<R, CH>(a.mix, a.zc0, a.zc1, d, o[1]);
+            }
+        },
+        [&](int g) { return c.ssolar * sflux[(size_t)(SW_NS[B] + g) * n + t]; },
+        [&](int lev, const R *f) { swr_emit<R>(acc, ok, total, cf1, cf0, lev, n, t, f); });
 }
 
 // SW band kernel of the NAM route: blocks of 64 day-list entries looped over a pool-sized grid.
@@ -423,7 +420,7 @@ __global__ void __launch_bounds__(64, (sw_waves<R, B, true>())) k_swr(const Tabs
 {
     __shared__ Fix64 fx[1];
     const ColIn in = band_in<EXT>(in_);
-    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    WR_G char *slot = (WR_G char *)(pool + (size_t)blockIdx.x * cache_slot_bytes(2 * sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = blockIdx.x; blk * 64 < nday; blk += gridDim.x)
         swr_column<R, B>(T, T->sw[B], in, par, col0, n, cs, rp, sflux, acc, blk, (int)threadIdx.x, slot, fx);
@@ -443,8 +440,8 @@ __global__ void __launch_bounds__((64 * swrl_wpg<R, B>()), (sw_waves<R, B, true>
     const auto Bl = sw_lds_band<R>((const WR_L R *)swrl_tab, T->sw_img[B], T->sw[B]);
     constexpr int WPG = swrl_wpg<R, B>();
     __shared__ Fix64 fx[sizeof(R) == 4 ? WPG : 1];
-    const int lane = threadIdx.x % 64, wv = wave_id(), w = blockIdx.x * WPG + wv;
-    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
+    const int lane = threadIdx.x % 64, wv = wave_id(), w = wave_slot();
+    WR_G char *slot = (WR_G char *)(pool + (size_t)w * cache_slot_bytes(2 * sw_nv<R>(), SW_NG[B], in.nlay + 2, (int)sizeof(R)));
     const int nday = *cs.nday;
     for (int blk = w; blk * 64 < nday; blk += gridDim.x * WPG)
         swr_column<R, B>(T, Bl, in, par, col0, n, cs, rp, sflux, acc, blk, lane, slot, fx + (sizeof(R) == 4 ? wv : 0));
