@@ -41,22 +41,22 @@ OUT_ALL = (2 * NL + 4 * (NL + 2)) * 8
 # and WRITE_SIZE on a 160,000-column call, HBM bytes = 2 x FETCH + WRITE (calibrated on a 1 GiB
 # device copy); the tables and their commands are profiles/hbm_traffic_{fp64,mixed}_grid400x400.md.
 TRAFFIC_FP64 = {
-    "k_lw_b01": 11692, "k_lw_b02": 11410, "k_lw_b03": 7700, "k_lw_b04": 8552, "k_lw_b05": 8665,
-    "k_lw_b06": 9819, "k_lw_b07": 8433, "k_lw_b08": 11028, "k_lw_b09": 7461, "k_lw_b10": 9091,
-    "k_lw_b11": 9852, "k_lw_b12": 9941, "k_lw_b13": 8001, "k_lw_b14": 7667, "k_lw_b15": 8471, "k_lw_b16": 7477,
-    "k_sw_b16": 21335, "k_sw_b17": 33790, "k_sw_b18": 25222, "k_sw_b19": 25176, "k_sw_b20": 29498,
-    "k_sw_b21": 29547, "k_sw_b22": 12241, "k_sw_b23": 29526, "k_sw_b24": 26168, "k_sw_b25": 21989,
-    "k_sw_b26": 19979, "k_sw_b27": 26218, "k_sw_b28": 22202, "k_sw_b29": 33784,
+    "k_lw_b01": 36345, "k_lw_b02": 40010, "k_lw_b03": 67073, "k_lw_b04": 45583, "k_lw_b05": 68035,
+    "k_lw_b06": 30248, "k_lw_b07": 49089, "k_lw_b08": 30737, "k_lw_b09": 50282, "k_lw_b10": 24141,
+    "k_lw_b11": 30735, "k_lw_b12": 29762, "k_lw_b13": 20494, "k_lw_b14": 13899, "k_lw_b15": 15366,
+    "k_lw_b16": 14388, "k_sw_b16": 25226, "k_sw_b17": 36965, "k_sw_b18": 32370, "k_sw_b19": 33796,
+    "k_sw_b20": 33034, "k_sw_b21": 33051, "k_sw_b22": 17228, "k_sw_b23": 33035, "k_sw_b24": 37801,
+    "k_sw_b25": 22253, "k_sw_b26": 16920, "k_sw_b27": 26483, "k_sw_b28": 22215, "k_sw_b29": 36957,
 }
 
 
 TRAFFIC_MIXED = {
-    "k_lw_b01": 18810, "k_lw_b02": 21082, "k_lw_b03": 27694, "k_lw_b04": 24335, "k_lw_b05": 27629,
-    "k_lw_b06": 15479, "k_lw_b07": 21765, "k_lw_b08": 15993, "k_lw_b09": 21276, "k_lw_b10": 13113,
-    "k_lw_b11": 15546, "k_lw_b12": 15549, "k_lw_b13": 10506, "k_lw_b14": 7274, "k_lw_b15": 7757,
-    "k_lw_b16": 7272, "k_sw_b16": 25803, "k_sw_b17": 48094, "k_sw_b18": 33012, "k_sw_b19": 33008,
-    "k_sw_b20": 40600, "k_sw_b21": 40484, "k_sw_b22": 11371, "k_sw_b23": 40595, "k_sw_b24": 33465,
-    "k_sw_b25": 26281, "k_sw_b26": 25289, "k_sw_b27": 33459, "k_sw_b28": 26265, "k_sw_b29": 48029,
+    "k_lw_b01": 14852, "k_lw_b02": 16108, "k_lw_b03": 22358, "k_lw_b04": 18282, "k_lw_b05": 22598,
+    "k_lw_b06": 13216, "k_lw_b07": 17705, "k_lw_b08": 14014, "k_lw_b09": 18396, "k_lw_b10": 10003,
+    "k_lw_b11": 12702, "k_lw_b12": 12403, "k_lw_b13": 11776, "k_lw_b14": 6099, "k_lw_b15": 7075,
+    "k_lw_b16": 6343, "k_sw_b16": 18901, "k_sw_b17": 33597, "k_sw_b18": 23713, "k_sw_b19": 23713,
+    "k_sw_b20": 28640, "k_sw_b21": 28654, "k_sw_b22": 9002, "k_sw_b23": 28377, "k_sw_b24": 23937,
+    "k_sw_b25": 17855, "k_sw_b26": 16134, "k_sw_b27": 22473, "k_sw_b28": 17838, "k_sw_b29": 33542,
 }
 
 
@@ -90,20 +90,20 @@ VALU_PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3}
 # FP64 path: FP64 FLOPs.  Mixed path: FP32-equivalent FLOPs, FP32 + 2 x FP64 (FP64 issues at half the
 # FP32 rate), against the FP32 peak.
 FLOPS_FP64 = {
-    "k_lw_b01": 145539, "k_lw_b02": 152887, "k_lw_b03": 255119, "k_lw_b04": 208076, "k_lw_b05": 246546,
-    "k_lw_b06": 114218, "k_lw_b07": 188830, "k_lw_b08": 125292, "k_lw_b09": 195105, "k_lw_b10": 91067,
-    "k_lw_b11": 116786, "k_lw_b12": 159111, "k_lw_b13": 105033, "k_lw_b14": 58000, "k_lw_b15": 76799,
-    "k_lw_b16": 69924, "k_sw_b16": 267695, "k_sw_b17": 516824, "k_sw_b18": 346071, "k_sw_b19": 347459,
-    "k_sw_b20": 417488, "k_sw_b21": 428415, "k_sw_b22": 106142, "k_sw_b23": 411511, "k_sw_b24": 350855,
-    "k_sw_b25": 239041, "k_sw_b26": 226762, "k_sw_b27": 327658, "k_sw_b28": 261471, "k_sw_b29": 503154
+    "k_lw_b01": 103605, "k_lw_b02": 111543, "k_lw_b03": 207017, "k_lw_b04": 183854, "k_lw_b05": 194846,
+    "k_lw_b06": 66482, "k_lw_b07": 137974, "k_lw_b08": 75089, "k_lw_b09": 148142, "k_lw_b10": 57602,
+    "k_lw_b11": 78677, "k_lw_b12": 86424, "k_lw_b13": 53423, "k_lw_b14": 22997, "k_lw_b15": 28145,
+    "k_lw_b16": 25920, "k_sw_b16": 240578, "k_sw_b17": 486226, "k_sw_b18": 316040, "k_sw_b19": 317657,
+    "k_sw_b20": 376592, "k_sw_b21": 392305, "k_sw_b22": 81257, "k_sw_b23": 369338, "k_sw_b24": 319797,
+    "k_sw_b25": 210813, "k_sw_b26": 202525, "k_sw_b27": 295195, "k_sw_b28": 236466, "k_sw_b29": 468001,
 }
 FLOPS_MIXED = {
-    "k_lw_b01": 89332, "k_lw_b02": 88151, "k_lw_b03": 167792, "k_lw_b04": 129832, "k_lw_b05": 163931,
-    "k_lw_b06": 67145, "k_lw_b07": 121752, "k_lw_b08": 74139, "k_lw_b09": 124769, "k_lw_b10": 55205,
-    "k_lw_b11": 72732, "k_lw_b12": 81436, "k_lw_b13": 58433, "k_lw_b14": 33661, "k_lw_b15": 43539,
-    "k_lw_b16": 39158, "k_sw_b16": 136168, "k_sw_b17": 256402, "k_sw_b18": 166713, "k_sw_b19": 168384,
-    "k_sw_b20": 198289, "k_sw_b21": 196579, "k_sw_b22": 59655, "k_sw_b23": 213413, "k_sw_b24": 158891,
-    "k_sw_b25": 109955, "k_sw_b26": 249383, "k_sw_b27": 138230, "k_sw_b28": 121776, "k_sw_b29": 250155
+    "k_lw_b01": 57968, "k_lw_b02": 62523, "k_lw_b03": 124075, "k_lw_b04": 106701, "k_lw_b05": 120257,
+    "k_lw_b06": 39687, "k_lw_b07": 84748, "k_lw_b08": 46411, "k_lw_b09": 88385, "k_lw_b10": 31804,
+    "k_lw_b11": 44762, "k_lw_b12": 51327, "k_lw_b13": 32909, "k_lw_b14": 12278, "k_lw_b15": 16546,
+    "k_lw_b16": 15000, "k_sw_b16": 83940, "k_sw_b17": 173341, "k_sw_b18": 107556, "k_sw_b19": 108843,
+    "k_sw_b20": 128502, "k_sw_b21": 132268, "k_sw_b22": 28670, "k_sw_b23": 158044, "k_sw_b24": 105905,
+    "k_sw_b25": 74102, "k_sw_b26": 219026, "k_sw_b27": 92055, "k_sw_b28": 78923, "k_sw_b29": 164537,
 }
 
 

@@ -156,7 +156,7 @@ int wr_run_mixed(wr_ctx *ctx, const wr_columns *in, const wr_params *par, const 
  * reference.  For callers that cannot allocate device memory at call time (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation).  Same inputs, outputs and results
  * as wr_run_mixed (the same kernels), but the tile work space is a static device array of the library
- * (219 MB per device, held until the process ends) instead of the context's, and the band
+ * (414 MB per device, held until the process ends) instead of the context's, and the band
  * kernels run on the caller's stream.  At most WR_NOALLOC_MAX_COLS columns per call (more:
  * WR_ERR_TOO_LARGE) and 63 model layers.  The context supplies the tables; its own work space is not
  * touched.  Every call on one device shares that device's array: calls that overlap on one device

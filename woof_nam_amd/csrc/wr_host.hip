@@ -513,14 +513,12 @@ bool lw_glane_env()
 // FP32 McICA LW bands (bit B = band B + 1) that run k_lwl, the kernel with the band's tables in LDS:
 // WR_LW_LDS (a hexadecimal mask) overrides the default.  A band whose table image exceeds the
 // device's LDS per workgroup runs k_lwc.
-// WR_LW_LDS64 does the same for the FP64 McICA LW kernels (k_lwl64 in place of k_lw).  The defaults
-// are the measured choice per band on the 954x835x60 grid: every FP32 band (LW sum 101 -> 97 ms per
-// call), every FP64 band but 14 (LW sum 233 -> 216 ms; band 14 ran 7 % slower).
+// WR_LW_LDS64 does the same for the FP64 McICA LW kernels (k_lwl64 in place of k_lw), which also keep the
+// transmittance table there: band 3 takes 24.9 ms of a 954x835x60 call from global memory and 16.4 from LDS.
 constexpr uint32_t LW_LDS_DEFAULT = 0xffffu, LW_LDS64_DEFAULT = 0xffffu;
 // WR_SW_LDS / WR_SW_LDS64 (bit B = band B + 16) choose k_swl over k_sw the same way.  Measured per
 // band (serialised, 954x835x60): FP64 SW bands 17-24 and 29 run 3-9 % faster from LDS, 25, 26, 28
-// slower (the FP64 call 320 -> 312 ms with this mask); in FP32 the SW sum went 62.0 -> 65.4 ms, so
-// FP32 SW keeps its global-table kernels.
+// slower; in FP32 every band was slower, so FP32 SW keeps its global-table kernels.
 constexpr uint32_t SW_LDS_DEFAULT = 0x0u, SW_LDS64_DEFAULT = 0x21feu;
 // WR_LWR_LDS / WR_LWR_LDS64: the NAM route's LW kernels (k_lwrl over k_lwr), on the LW images.
 constexpr uint32_t LWR_LDS_DEFAULT = 0xffffu, LWR_LDS64_DEFAULT = 0xffffu;

