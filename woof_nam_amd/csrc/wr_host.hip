@@ -578,7 +578,8 @@ Sizes sizes(int32_t max_cols)
     z.lwrec = lw_glane_env() ? lwrec_bytes_per_col<double>(64 + 1) * m + 3 * 256 : 0;  // LW layer records
     // level pool: room for every 64-column block of a tile in the largest slot layout (FP64 SW:
     // 2 values, FP32 SW: 5 values, x 16 g x levels; FP64 LW), at most WR_POOL_GB (default 3) GB per stream:
-    // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB
+    // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB.  A multiple of 256 bytes: the streams' pools
+    // lie one after another, and their slots are read and written as 16-byte vectors
     const int nl_max = 64;
     const size_t lane_max = std::max({cache_slot_bytes(2 * sw_nv<double>(), 16, nl_max + 1, (int)sizeof(double)),
                                       cache_slot_bytes(2 * sw_nv<float>(), 16, nl_max + 1, (int)sizeof(float)),
@@ -586,8 +587,7 @@ Sizes sizes(int32_t max_cols)
     const size_t need = (m + 63) / 64 * lane_max;
     const char *pe = getenv("WR_POOL_GB");
     const double gb = pe ? atof(pe) : 3.0;
-    size_t cap = (size_t)(gb * 1e9);
-    if (cap < lane_max) cap = lane_max;
+    const size_t cap = std::max((size_t)(gb * 1e9) / 256 * 256, lane_max);  // lane_max: a multiple of 256
     z.pool = need < cap ? need : cap;
     // WR_BAND_STREAMS=0 keeps the band kernels on the caller's stream
     const char *e = getenv("WR_BAND_STREAMS");
