@@ -70,3 +70,25 @@ def test_tiles_of_any_size_agree(gpu_device, monkeypatch, precision, mcica):
     for other in out[1:]:
         for k in abi.OUTPUT_FIELDS:
             assert torch.equal(out[0][k].view(torch.int64), other[k].view(torch.int64)), k
+
+
+@pytest.mark.parametrize("mcica", [1, 0])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_small_pools_give_the_same_bits(gpu_device, monkeypatch, precision, mcica):
+    """WR_POOL_GB: 4 x 0.03 GB hold one or a few blocks of the two launches at once; 4 x 0.01 GB hold none, and the
+    band kernels then loop over the few slots that there are."""
+    n, p = 705, Radiation.default_params(mcica=mcica, seed=3)
+    cols = columns(n, 91, False, gpu_device)
+    out = []
+    for gb in (None, "0.03", "0.01"):
+        monkeypatch.setenv("WR_POOL_GB", gb) if gb else monkeypatch.delenv("WR_POOL_GB", raising=False)
+        print(f"case small pools {precision} mcica={mcica} gb={gb}", flush=True)
+        rad = Radiation(0, max_cols=n)
+        try:
+            out.append(rad.run(cols, params=p, precision=precision)[0])
+            torch.cuda.synchronize()
+        finally:
+            rad.close()
+    for other in out[1:]:
+        for k in abi.OUTPUT_FIELDS:
+            assert torch.equal(out[0][k].view(torch.int64), other[k].view(torch.int64)), k

@@ -122,6 +122,17 @@ def test_tile_sized_from_free_memory():
     assert L.wr_context_bytes(0) == 0
 
 
+@pytest.mark.parametrize("ncol,free_gb", [(4096, 0.8), (20_000, 1.0), (40_000, 1.2), (300_000, 5.0), (1000, 0.25)])
+def test_tile_shrinks_where_memory_is_short(ncol, free_gb):
+    """With little device memory free the hook takes smaller tiles instead of refusing the call."""
+    from woof_nam_amd import _lib
+    L, lm, free = _lib.load(), 60, free_gb * 1e9
+    per_call = rrtm_call.call_bytes_per_column(lm) * ncol
+    m = rrtm_call.tile_columns(ncol, lm, int(free))
+    assert 64 <= m <= ncol
+    assert L.wr_context_bytes(m) + per_call <= 0.9 * free
+
+
 def test_mcica_route_refused_by_the_hook():
     ctx = make_ctx()
     ctx.cfg.rrtm_mcica = 1

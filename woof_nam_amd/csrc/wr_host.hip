@@ -543,7 +543,14 @@ uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_
 //   FP64 NAM        23.0 / 5.8   24.5 / 11.1  34.0 / 26.2   40.0 / 35.1   51.5 / 73.1
 //   mixed NAM       14.9 / 2.9   16.8 / 5.8   20.8 / 13.9   22.0 / 18.5   25.2 / 34.2
 constexpr int MANY_COLS_DEFAULT = 65536;
-constexpr int MANY_POOL_COLS = 8192;  // columns whose pool values a context has room for at once (launch_many)
+// Pool bytes that a context of small tiles has for the two launches: the optics of as many 64-column blocks as fit are in
+// flight at once, and fewer blocks fill the chip less.  us per call with 0.25 / 0.5 / 1 / 2 / 4 / 10 GB:
+//   FP64 McICA  1,000 columns     968 /    778 /    739 /    735 /    737 /    734
+//               4,096           3,088 /  2,546 /  2,290 /  1,947 /  1,869 /  1,879
+//   FP64 NAM    4,096           6,583 /  4,458 /  3,269 /  2,832 /  2,564 /  2,424
+//               40,000         60,348 / 40,766 / 30,000 / 24,545 / 22,018 / 21,759
+//   mixed McICA 4,096             947 /    920 /    888 /    885 /    895 /    886
+constexpr size_t MANY_POOL = (size_t)2e9;
 int many_cols_env()
 {
     for (const char *m : {"WR_LW_LDS", "WR_LW_LDS64", "WR_SW_LDS", "WR_SW_LDS64", "WR_LWR_LDS", "WR_LWR_LDS64", "WR_SWR_LDS",
@@ -553,11 +560,13 @@ int many_cols_env()
     return e ? std::max(0, atoi(e)) : MANY_COLS_DEFAULT;
 }
 constexpr size_t MANY_BLOCK = std::max(many_block_bytes<double, false>(64), many_block_bytes<double, true>(64));
+constexpr int max_of(const int *v, int n) { return n == 1 ? v[0] : std::max(v[0], max_of(v + 1, n - 1)); }
+constexpr int LW_G = max_of(LW_NG, 16), SW_G = max_of(SW_NG, 14);  // g-points of the widest bands
 
 // Device bytes of a context's tile work space for tiles of m columns, and the band-stream count.
 struct Sizes {
     size_t acc, iws, dws, rtr, sflux, rec, lwrec, pool, pool_all;
-    int naux;
+    int naux, pools, many_cols;  // band streams, their pools, columns of a tile in two launches
     size_t total() const
     {
         return acc + iws + dws + rtr + sflux + rec + lwrec + pool_all;
@@ -577,13 +586,14 @@ Sizes sizes(int32_t max_cols)
     z.rec = std::max(rec_row_bytes(8), rec_row_bytes(4)) * rows;              // layer records
     z.lwrec = lw_glane_env() ? lwrec_bytes_per_col<double>(64 + 1) * m + 3 * 256 : 0;  // LW layer records
     // level pool: room for every 64-column block of a tile in the largest slot layout (FP64 SW:
-    // 2 values, FP32 SW: 5 values, x 16 g x levels; FP64 LW), at most WR_POOL_GB (default 3) GB per stream:
+    // 2 values, FP32 SW: 5 values, x g x levels, of two skies; FP64 LW), at most WR_POOL_GB (default 3) GB per stream:
     // the 2,048 waves the SIMDs hold of the widest FP32 SW band take 2.8 GB.  A multiple of 256 bytes: the streams' pools
     // lie one after another, and their slots are read and written as 16-byte vectors
     const int nl_max = 64;
-    const size_t lane_max = std::max({cache_slot_bytes(2 * sw_nv<double>(), 16, nl_max + 1, (int)sizeof(double)),
-                                      cache_slot_bytes(2 * sw_nv<float>(), 16, nl_max + 1, (int)sizeof(float)),
-                                      lw64_slot_bytes(16, nl_max + 1)});
+    const size_t lane_max = std::max({cache_slot_bytes(2 * sw_nv<double>(), SW_G, nl_max + 1, (int)sizeof(double)),
+                                      cache_slot_bytes(2 * sw_nv<float>(), SW_G, nl_max + 1, (int)sizeof(float)),
+                                      cache_slot_bytes(LW_NV_F32, LW_G, nl_max + 1, (int)sizeof(float)),
+                                      lw64_slot_bytes(LW_G, nl_max + 1)});
     const size_t need = (m + 63) / 64 * lane_max;
     const char *pe = getenv("WR_POOL_GB");
     const double gb = pe ? atof(pe) : 3.0;
@@ -593,10 +603,16 @@ Sizes sizes(int32_t max_cols)
     const char *e = getenv("WR_BAND_STREAMS");
     const int na = e ? atoi(e) : WR_NAUX;
     z.naux = na < 0 ? 0 : (na > WR_NAUX ? WR_NAUX : na);
-    // the streams' pools lie one after another; together they also hold every band's slots of the tiles
-    // that run their bands in two launches
-    const size_t many = (size_t)((std::min({max_cols, many_cols_env(), MANY_POOL_COLS}) + 63) / 64) * MANY_BLOCK;
-    z.pool_all = std::max(z.pool * (size_t)(z.naux > 1 ? z.naux : 1), many);
+    // Tiles that run their bands in two launches use the whole of the pool space: what their blocks take, at most MANY_POOL
+    // or what one pool per stream takes, whichever is larger, and at most the streams' limit.  A context whose tiles
+    // all run so has a band kernel only for a single band, on the caller's stream, and one pool of that kind.
+    const size_t ns = (size_t)std::max(z.naux, 1);
+    z.many_cols = z.lwrec ? 0 : many_cols_env();
+    const size_t blocks = (size_t)(std::min(max_cols, z.many_cols) + 63) / 64;
+    const size_t many = std::min({blocks * MANY_BLOCK, std::max(MANY_POOL, z.pool * ns), cap * ns});
+    z.pools = max_cols <= z.many_cols && many >= MANY_BLOCK ? 1 : (int)ns;
+    z.pool_all = std::max(z.pool * (size_t)z.pools, many);
+    if (z.pool_all < MANY_BLOCK) z.many_cols = 0;
     return z;
 }
 
@@ -712,8 +728,19 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
     if (rc == WR_OK) {
         c->pool_bytes = z.pool;
         c->pool_all = z.pool_all;
-        c->many_cols = many_cols_env();
-        if (hipMalloc((void **)&c->pool[0], c->pool_all) != hipSuccess) rc = WR_ERR_NOMEM;
+        c->many_cols = z.many_cols;
+        // short of memory: less room for the two launches, down to one block's, then none (band kernels)
+        const size_t least = z.pool * (size_t)z.pools;
+        while (hipMalloc((void **)&c->pool[0], c->pool_all) != hipSuccess) {
+            (void)hipGetLastError();
+            c->pool[0] = nullptr;
+            if (c->pool_all <= least) {
+                rc = WR_ERR_NOMEM;
+                break;
+            }
+            c->pool_all = std::max(c->pool_all / 2, least);
+        }
+        if (c->pool_all < MANY_BLOCK) c->many_cols = 0;
     }
     if (rc == WR_OK) {
         // WR_BAND_STREAMS=0 keeps the band kernels on the caller's stream
@@ -722,9 +749,9 @@ int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols
             if (hipStreamCreateWithFlags(&c->aux[q], hipStreamNonBlocking) != hipSuccess ||
                 hipEventCreateWithFlags(&c->join[q], hipEventDisableTiming) != hipSuccess)
                 rc = WR_ERR_HIP;
-        // one level pool per band stream (stream 0 shares the caller's), all allocated here: no later
-        // call allocates
-        for (int q = 1; q < c->naux && rc == WR_OK; ++q) c->pool[q] = c->pool[0] + (size_t)q * c->pool_bytes;
+        // one level pool per band stream that needs one (stream 0 shares the caller's), all allocated here: no
+        // later call allocates
+        for (int q = 1; q < z.pools && rc == WR_OK; ++q) c->pool[q] = c->pool[0] + (size_t)q * c->pool_bytes;
         if (rc == WR_OK && c->naux > 0 && hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess)
             rc = WR_ERR_HIP;
     }

@@ -77,18 +77,18 @@ def call_bytes_per_column(lm: int) -> int:
 def tile_columns(ncol: int, lm: int, free_bytes: int, cap: int = 1048576, margin: float = 0.9) -> int:
     """Largest tile (columns per library context) that fits the free device memory beside the call's
     own arrays, as namgpu/physics/rrtm/rrtm_call.py:183-203 (batch_count) sizes its batches from free
-    bytes.  Raises MemoryError when not even a 4,096-column tile fits."""
+    bytes.  Raises MemoryError when not even a 64-column tile fits (one block of the kernels' lanes)."""
     L = _lib.load()
     avail = int(margin * free_bytes) - call_bytes_per_column(lm) * ncol
     hi = max(1, min(ncol, cap))
     if L.wr_context_bytes(hi) <= avail:
         return hi
-    lo = min(4096, hi)
+    lo = min(64, hi)
     if L.wr_context_bytes(lo) > avail:
         raise MemoryError(f"rrtm-call: {ncol} columns need {call_bytes_per_column(lm) * ncol / 1e9:.1f} GB of "
                           f"column arrays and a {lo}-column context of {L.wr_context_bytes(lo) / 1e9:.1f} GB; "
                           f"{free_bytes / 1e9:.1f} GB free")
-    while hi - lo > 1024:                       # context bytes grow with the tile: bisect
+    while hi - lo > max(64, min(1024, lo // 8)):    # context bytes grow with the tile: bisect
         mid = (lo + hi) // 2
         if L.wr_context_bytes(mid) <= avail:
             lo = mid
