@@ -80,6 +80,19 @@ def test_colsum_matches_float64(gpu_device, M, N):
     assert (np.abs(out.cpu().numpy() - x.astype(np.float64).sum(0)) <= tol).all()
 
 
+@pytest.mark.parametrize("M", [2_147_483_521, 2_147_483_647])
+def test_colsum_of_the_longest_columns(gpu_device, M):
+    """Row counts at the end of the 32-bit range: a row stride of 0 reads one element M times, so that no 8.6 GB array
+    is needed.  Sums of 2^-20 are exact up to 2^24 terms, a thread's share; the 7 additions of the tree round."""
+    from woof_nam_amd import _lib
+    print(f"case colsum M={M} ld=0", flush=True)
+    x = torch.full((1,), 2.0 ** -20, dtype=torch.float32, device=gpu_device)
+    out = torch.zeros((1,), dtype=torch.float32, device=gpu_device)
+    _lib.check(_lib.load().wr_mlp_colsum(S._p(x), M, 1, 0, S._p(out), S._stream()), "wr_mlp_colsum")
+    torch.cuda.synchronize()
+    assert abs(float(out) - M * 2.0 ** -20) <= 7 * 2.0 ** -24 * 2048.0
+
+
 def test_gradients_match_cpu_oracle(gpu_device):
     print("case mlp gradients vs oracle", flush=True)
     m = S.MLP(gpu_device, seed=4)

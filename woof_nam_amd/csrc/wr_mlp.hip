@@ -343,12 +343,12 @@ __global__ void __launch_bounds__(CS_N * CS_R) k_colsum(const float *__restrict_
 {
     __shared__ float red[CS_R][CS_N + 1];
     const int c = threadIdx.x % CS_N, r = threadIdx.x / CS_N;
-    const int n = blockIdx.x * CS_N + c;
+    const long long n = (long long)blockIdx.x * CS_N + c;
     float s[CS_U];
 #pragma unroll
     for (int u = 0; u < CS_U; ++u) s[u] = 0.f;
     if (n < N) {
-        int m = r;
+        long long m = r;  // 64 bits: the index a step ahead passes 2^31 where M is near it
         for (; m + (CS_U - 1) * CS_R < M; m += CS_U * CS_R)
 #pragma unroll
             for (int u = 0; u < CS_U; ++u) s[u] += X[(size_t)(m + u * CS_R) * ld + n];
