@@ -66,6 +66,18 @@ def test_gemm_split_k_and_silu(gpu_device):
                                atol=1e-2)
 
 
+@pytest.mark.parametrize("K,splits", [(2_147_483_647, 65535), (2_147_483_600, 60_000)])
+def test_gemm_of_the_longest_sums(gpu_device, K, splits):
+    """K at the end of its 32-bit range, where the last splits begin past it (strides of 0: one element each).  A
+    split's sum is a whole number of at most 35,840, exact in FP32; the partials add up to K."""
+    print(f"case gemm K={K} splits={splits}", flush=True)
+    one = torch.ones((1,), dtype=torch.bfloat16, device=gpu_device)
+    part = torch.full((splits,), -7.0, dtype=torch.float32, device=gpu_device)
+    S.gemm(1, 1, K, one, 0, 0, one, 0, 0, part, None, 1, 1, splits=splits, split_stride=1)
+    torch.cuda.synchronize()
+    assert int(part.double().sum()) == K
+
+
 @pytest.mark.parametrize("M,N", [(1, 1), (63, 16), (64, 17), (513, 15), (4101, 504), (16384, 128)])
 def test_colsum_matches_float64(gpu_device, M, N):
     """wr_mlp_colsum at the edges of its 16-column workgroups and 512-row steps against a float64 sum.  A

@@ -36,7 +36,7 @@ struct GemmArgs {
     const float *bias;       // [N]
     float *Zout;             // EPI_BIAS_SILU: pre-activation, same strides as C
     const float *Zin;        // EPI_DSILU: pre-activation the derivative is taken at, same strides as C
-    int k_per_split;         // K range of one split (grid.z), a multiple of GK
+    unsigned k_per_split;    // K range of one split (grid.z), a multiple of GK
     long long split_stride;  // element offset between split partial outputs
 };
 
@@ -77,19 +77,21 @@ struct Staged {
     bf16x8 v[2];
 };
 template <typename T>
-__device__ __forceinline__ Staged stage_load(const T *X, long long ld_row, long long ld_k, int nrow, int r0, int kk, int k_end,
-                                             bool rows_contig, int tid)
+__device__ __forceinline__ Staged stage_load(const T *X, long long ld_row, long long ld_k, int nrow, int r0, unsigned kk,
+                                             unsigned k_end, bool rows_contig, int tid)
 {
     Staged s;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         if (rows_contig) {
-            const int row = r0 + (tid & 7) * 8, k = kk + (tid >> 3) + u * 32;
+            const int row = r0 + (tid & 7) * 8;
+            const unsigned k = kk + (tid >> 3) + u * 32;
             const int cnt = k < k_end ? max(0, min(8, nrow - row)) : 0;
             s.v[u] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_row, cnt);
         } else {
-            const int row = r0 + (tid >> 2), k = kk + (tid & 3) * 8 + u * 32;
-            const int cnt = row < nrow ? max(0, min(8, k_end - k)) : 0;
+            const int row = r0 + (tid >> 2);
+            const unsigned k = kk + (tid & 3) * 8 + u * 32;
+            const int cnt = row < nrow && k < k_end ? (int)min(8u, k_end - k) : 0;
             s.v[u] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_k, cnt);
         }
     }
@@ -120,8 +122,8 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;  // M on x: up to 2^31 rows
-    const int k_begin = blockIdx.z * g.k_per_split;
-    const int k_end = min(g.K, k_begin + g.k_per_split);
+    // unsigned: a step or a split past the end of a K near 2^31 stays above it (splits * k_per_split < 2^32)
+    const unsigned k_begin = blockIdx.z * g.k_per_split, k_end = min((unsigned)g.K, k_begin + g.k_per_split);
     const TA *A = (const TA *)g.A;
     const TB *B = (const TB *)g.B;
     const bool a_rows = g.lda_k != 1 && g.lda_m == 1, b_rows = g.ldb_k != 1 && g.ldb_n == 1;
@@ -135,7 +137,7 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
     const int row = lane & 15, kq = (lane >> 4) * 8;  // the lane's row and first k of each operand fragment
     Staged sa = stage_load(A, g.lda_m, g.lda_k, g.M, m0, k_begin, k_end, a_rows, tid);
     Staged sb = stage_load(B, g.ldb_n, g.ldb_k, g.N, n0, k_begin, k_end, b_rows, tid);
-    for (int kk = k_begin; kk < k_end; kk += GK) {
+    for (unsigned kk = k_begin; kk < k_end; kk += GK) {
         stage_store(sa, a_rows, As, tid);
         stage_store(sb, b_rows, Bs, tid);
         __syncthreads();
@@ -533,7 +535,7 @@ int wr_mlp_gemm(int32_t M, int32_t N, int32_t K, const void *A, int32_t a_bf16, 
     g.B = B, g.ldb_k = ldb_k, g.ldb_n = ldb_n;
     g.C = C, g.Cb = (__bf16 *)Cb, g.ldc_m = ldc_m, g.ldc_n = ldc_n;
     g.bias = bias, g.Zout = Zout, g.Zin = Zin;
-    const int kps = ((K + splits - 1) / splits + GK - 1) / GK * GK;
+    const unsigned kps = (((unsigned)K + (unsigned)splits - 1) / (unsigned)splits + GK - 1) / GK * GK;
     g.k_per_split = kps > 0 ? kps : GK;
     g.split_stride = split_stride;
     hipStream_t s = (hipStream_t)stream;
