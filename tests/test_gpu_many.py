@@ -3,11 +3,14 @@
 WR_MANY_COLS=0 (read when a context is created) keeps the per-band kernels; both run the same column
 functions, so every output is the same bits, at the edges of a 64-column block, for both precisions and
 routes, with and without the optional column inputs."""
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
 
 from woof_nam_amd import abi, gen
+from woof_nam_amd import surrogate as S
 from woof_nam_amd.radiation import Radiation
 
 pytestmark = pytest.mark.gpu
@@ -43,6 +46,31 @@ def test_two_launches_equal_per_band_launches(gpu_device, monkeypatch, precision
             cols = columns(n, 50 + n, ext, gpu_device)
             a, b = (r.run(cols, params=p, precision=precision)[0] for r in rads)
             torch.cuda.synchronize()
+            for k in abi.OUTPUT_FIELDS:
+                assert torch.equal(a[k].view(torch.int64), b[k].view(torch.int64)), (k, n)
+    finally:
+        for r in rads:
+            r.close()
+
+
+def test_surrogate_two_launches_equal_per_band_launches(gpu_device, monkeypatch):
+    """The learned optics in both forms: columns inside the training envelope, every third one outside it (table
+    optics), alone in a tile, at the edges of a block and in two tiles."""
+    net = S.MLP.load(Path(S.__file__).resolve().parent / "data" / "surrogate_rrtmg.npz", gpu_device)
+    rads = []
+    for env in ("0", None):
+        monkeypatch.setenv("WR_MANY_COLS", env) if env else monkeypatch.delenv("WR_MANY_COLS")
+        rads.append(Radiation(0, max_cols=700))
+        rads[-1].attach_surrogate(net)
+    try:
+        for n in (1, 63, 65, 701):
+            print(f"case two launches surrogate ncol={n}", flush=True)
+            cols = columns(n, 150 + n, False, gpu_device)
+            cols["t_lay"][:, 2::3] = 345.0              # far outside the training temperatures
+            (a, fa), (b, fb) = (r.run(cols, params=Radiation.default_params(seed=9), precision="surrogate") for r in rads)
+            torch.cuda.synchronize()
+            fa, fb = fa["fallback"], fb["fallback"]
+            assert torch.equal(fa, fb) and bool((fa[2::3] == 1).all()) and (n == 1 or int(fa.sum()) < n)
             for k in abi.OUTPUT_FIELDS:
                 assert torch.equal(a[k].view(torch.int64), b[k].view(torch.int64)), (k, n)
     finally:

@@ -59,24 +59,33 @@ def test_alone_equals_mix_equals_direct(gpu_device, precision):
     srv.close()
 
 
-def test_graph_replays_match_eager(gpu_device):
-    """Several replays with eager work and synchronisations in between all equal the eager call."""
-    print("case serve graph replays", flush=True)
+@pytest.mark.parametrize("many", [None, "0"], ids=["two_launches", "band_streams"])
+def test_graph_replays_match_eager(gpu_device, monkeypatch, many):
+    """Several replays with eager work and synchronisations in between all equal the eager call.  A tile of this size
+    captures two launches; under WR_MANY_COLS=0 the fork and join of the 30 band kernels over the context's streams, as
+    larger tiles do, which must also equal the eager call in two launches."""
+    print(f"case serve graph replays many={many}", flush=True)
     cols = dev_cols(2048, 4, gpu_device)
+    monkeypatch.delenv("WR_MANY_COLS", raising=False)
+    servers = [Server(0, tile=2048, slots=1, precision="mixed", graphs=False)]
+    if many:
+        monkeypatch.setenv("WR_MANY_COLS", many)
+        servers.append(Server(0, tile=2048, slots=1, precision="mixed", graphs=False))
+    refs = []
+    for srv in servers:
+        refs.append(Request(rid=0, kind="x", cols=cols, seed=3))
+        srv.submit(refs[-1])
+        srv.drain()
     srv_g = Server(0, tile=2048, slots=1, precision="mixed", graphs=True)
-    srv_e = Server(0, tile=2048, slots=1, precision="mixed", graphs=False)
-    ref = Request(rid=0, kind="x", cols=cols, seed=3)
-    srv_e.submit(ref)
-    srv_e.drain()
     for rep in range(4):
         r = Request(rid=rep, kind="x", cols=cols, seed=3)
         srv_g.submit(r)
         srv_g.drain()
         torch.cuda.synchronize()
-        assert same(r.out, ref.out), f"replay {rep} differs"
+        assert all(same(r.out, ref.out) for ref in refs), f"replay {rep} differs"
         _ = (cols["t_lay"] * 2.0).sum().item()      # eager work between replays
-    srv_g.close()
-    srv_e.close()
+    for srv in (srv_g, *servers):
+        srv.close()
 
 
 def test_budget_admission(gpu_device):
