@@ -55,8 +55,8 @@ __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
 
 // Entry i of the LW/SW look-up tables (transmittance e, Pade source factor tfn, optical depth tau at
 // tblind = i / 10000; the FP64 tables are built by k_luts), evaluated in FP32 where it is needed: the
-// FP32 kernels spend the few operations instead of three dependent table gathers per g-point.  The
-// FP64 kernels read the tables, which the CPU oracle reproduces bit for bit.
+// g-lane kernels (wr_glw.h) spend the few operations instead of three dependent table gathers per g-point; the other
+// kernels' form is lw_lut in wr_kernels.h.
 struct LutF {
     float e, tfn, tau;
 };

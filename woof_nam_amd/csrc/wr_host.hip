@@ -537,11 +537,12 @@ uint32_t lds_mask(const char *env, uint32_t dflt, const I *img, int nb, int lds_
 // Tiles of up to this many columns run all their bands in two launches (wr_many.h); WR_MANY_COLS overrides it at
 // context creation (0: never).  A context created under a WR_*_LDS* mask, which chooses between band kernels, runs the
 // band kernels at every size.  ms per call, band kernels / two launches:
-//   columns              8,192       20,000       48,000       64,000      110,889
-//   FP64 McICA      12.4 / 3.6   15.4 / 8.2   24.1 / 19.5   27.6 / 25.8   34.1 / 42.3
-//   mixed McICA      8.0 / 1.6    9.7 / 3.6   11.4 / 8.4    12.9 / 11.1   13.4 / 18.2
-//   FP64 NAM        23.0 / 5.8   24.5 / 11.1  34.0 / 26.2   40.0 / 35.1   51.5 / 73.1
-//   mixed NAM       14.9 / 2.9   16.8 / 5.8   20.8 / 13.9   22.0 / 18.5   25.2 / 34.2
+//   columns        8,192        20,000       48,000       64,000      110,889
+//   FP64 McICA  16.3 / 3.8    17.6 / 8.0   23.5 / 19.0  26.8 / 25.2  35.0 / 42.0
+//   mixed McICA  9.0 / 1.5     9.6 / 3.6   11.6 / 8.4   12.9 / 11.1  14.7 / 18.6
+//   surrogate   11.1 / 2.2    14.6 / 4.9   18.0 / 11.2  20.5 / 14.7  25.3 / 24.7
+//   FP64 NAM    23.2 / 5.2    24.4 / 11.9  34.0 / 26.8  40.8 / 34.5  55.3 / 57.3
+//   mixed NAM   15.6 / 2.8    16.7 / 6.0   20.7 / 13.2  21.9 / 16.8  25.0 / 30.3
 constexpr int MANY_COLS_DEFAULT = 65536;
 // Pool bytes that a context of small tiles has for the two launches: the optics of as many 64-column blocks as fit are in
 // flight at once, and fewer blocks fill the chip less.  us per call with 0.25 / 0.5 / 1 / 2 / 4 / 10 GB:
@@ -926,8 +927,8 @@ const char *wr_kernel_name(int32_t kid)
     if (kid == KID_MLP) return "mlp_gemm";
     if (kid == KID_RTRFAC) return "k_rtr_fac";
     if (kid == KID_LWREC) return "k_lwrec";
-    if (kid == KID_MANY) return "k_many";
-    if (kid == KID_SWPREP) return "k_swprep";
+    if (kid == KID_MANY) return "k_lay+k_sweep";
+    if (kid == KID_SWPREP) return "k_layers_sw+k_sflux";
     if (kid == KID_MCICA) return "k_mcica";
     return "?";
 }

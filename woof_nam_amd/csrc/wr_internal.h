@@ -42,7 +42,7 @@ struct wr_ctx {
     void *sy;                        // network outputs, bfloat16 [504][S]
     int *sflag;                      // [max_cols] per-column table-optics flag
     // per-stream cache pools of the band kernels (pool[0]: the caller's stream and aux stream 0;
-    // pool[q]: aux stream q), pool_bytes each, all allocated by wr_create
+    // pool[q]: aux stream q, null in a context of small tiles), pool_bytes each, all allocated by wr_create
     char *pool[WR_NAUX];
     size_t pool_bytes;
     size_t pool_all;                 // bytes from pool[0] on, pool[1..] among them: one launch may use them all

@@ -19,20 +19,11 @@
 
 #include "wr_rec.h"
 
-// Default minimum waves per SIMD of the LW band kernels (register budget 512 / waves).  One
-// keeps everything in registers (AGPRs included), with no scratch (private segment) that the runtime
-// must back on every HIP queue running the kernel.  The per-band tables below raise it to two where
-// that measured faster; the spills this costs stay at or below about 1.1 KB of scratch per lane.
-#ifndef WR_LW_WAVES
-#define WR_LW_WAVES 1
-#endif
-
 namespace wr {
 
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef double f64x2v __attribute__((ext_vector_type(2)));
-typedef double f64x4v __attribute__((ext_vector_type(4)));
 
 // Level fluxes of ONE band for one tile ([nrl+1][n] planes, written once per level; sw_clr0 [n]), in
 // the band kernel's precision P: FP64 planes for the FP64 kernels; FP32 planes for the FP32 kernels,
@@ -397,9 +388,12 @@ __host__ __device__ constexpr size_t cache_slot_bytes(int nv, int ng, int nk, in
 //   the gathers of one from being hoisted above the arithmetic of the one before, which bounds the registers; within
 //   a chunk nothing branches per g-point, so that its chains overlap.  The arithmetic of every g-point is
 //   that of the whole band at once;
-// * waves: waves per SIMD the compiler must fit.  FP32: four, or three where four spilled (the 16 and 14 g-point
-//   bands of two gases).  FP64: two everywhere; at three the LW kernels of a 796,590-column call took 205 ms in
-//   place of 147, from up to 530 bytes of scratch a lane.
+// * waves: waves per SIMD the compiler must fit.  FP32: three in the bands of two gases with 12 or more g-points (3, 5,
+//   7 and 9 still have 96 to 132 bytes of scratch a lane there), four in the others, of which 6, 8, 12 and 13 have 20 to
+//   140 bytes that three waves do not need.  Alone on 796,590 columns, four waves / three: band 1 2.54 / 2.62 ms, 2 2.75
+//   / 2.84, 6 2.30 / 2.32, 8 2.46 / 2.41, 10 1.74 / 1.79, 11 2.18 / 2.22, 12 2.25 / 2.35, 15 1.22 / 1.28, 16 1.11 / 1.19;
+//   only band 13, with 4 g-points, is much the slower at four: 2.64 / 1.70.  FP64: two everywhere; at three the LW
+//   kernels of a 796,590-column call took 205 ms in place of 147, from up to 530 bytes of scratch a lane.
 // WR_LWC_WAVES / WR_LW64_WAVES > 0 or WR_LW_CHUNK / WR_LW64_CHUNK >= 0 override the tables for every
 // band (tuning builds).
 constexpr int LWC_WAVES[16] = {4, 4, 3, 3, 3, 4, 3, 4, 3, 4, 4, 4, 4, 4, 4, 4};
@@ -419,10 +413,7 @@ constexpr int LW64_CHUNK[16] = {5, 4, 4, 2, 4, 4, 4, 4, 4, 3, 4, 4, 4, 2, 2, 2};
 #define WR_LW64_CHUNK -1
 #endif
 template <int B> constexpr int lwc_waves() { return WR_LWC_WAVES > 0 ? WR_LWC_WAVES : LWC_WAVES[B]; }
-template <typename R, int B> constexpr int lw_waves()
-{
-    return sizeof(R) == 8 ? (WR_LW64_WAVES > 0 ? WR_LW64_WAVES : LW64_WAVES[B]) : WR_LW_WAVES;
-}
+template <int B> constexpr int lw64_waves() { return WR_LW64_WAVES > 0 ? WR_LW64_WAVES : LW64_WAVES[B]; }
 // the smallest divisor of ngl that is >= want (ngl when want <= 0)
 constexpr int chunk_of(int ngl, int want)
 {
@@ -432,16 +423,14 @@ constexpr int chunk_of(int ngl, int want)
     return ngl;
 }
 template <int B> constexpr int lw_chunk() { return chunk_of(LW_NG[B], WR_LW_CHUNK >= 0 ? WR_LW_CHUNK : LWC_CHUNK[B]); }
-template <typename R, int B> constexpr int lw_chunk_r()
-{
-    return sizeof(R) == 8 ? chunk_of(LW_NG[B], WR_LW64_CHUNK >= 0 ? WR_LW64_CHUNK : LW64_CHUNK[B]) : lw_chunk<B>();
-}
+template <int B> constexpr int lw64_chunk() { return chunk_of(LW_NG[B], WR_LW64_CHUNK >= 0 ? WR_LW64_CHUNK : LW64_CHUNK[B]); }
 // ---- level sums over the g-points of a band ---------------------------------------------------------
 // A band's level flux is the sum of its g-points' contributions in g order.  A lane either holds all NG
 // g-points of its column (GW = NG) and adds them itself, or GW of them, the others being with the other
-// waves of its workgroup (k_many): then the contributions of SUM_LEVELS levels are left in LDS, and after a
+// waves of its workgroup (k_sweep): then the contributions of SUM_LEVELS levels are left in LDS, and after a
 // barrier each wave adds those of its levels, again in g order, so that the sums are the same bits.
-// NQ: quantities per level (4: two skies, with half as many levels between barriers).  The levels come in order row0, row0 + step, ...; emit(row, sums) stores one.
+// NQ: quantities per level (4: two skies, with half as many levels between barriers).  The levels come in order
+// row0, row0 + step, ...; emit(row, sums) stores one.
 constexpr int SUM_LEVELS = 4;
 template <typename R> constexpr size_t sum_lds_bytes() { return sizeof(R) * SUM_LEVELS * 64 * 24; }  // LW 16 g, SW 2 x 12 g
 template <typename R> struct Share {  // a wave's part of a column's g-points (split bands)
@@ -587,7 +576,7 @@ __device__ __forceinline__ void lw_tot_v(PE etab, const R *od, R odcld, R *tr, R
 
 // What the LW transfer of one column needs besides its layers.
 template <typename R> struct LwCol {
-    int i, t, nrl, lcf1, table;
+    int i, t, nrl, table;
     R sdif, semis, reflct;
 };
 template <typename R, int B, bool SURR>
@@ -595,7 +584,6 @@ __device__ __forceinline__ LwCol<R> lw_col(const ColIn &in, int col0, const ColS
 {
     LwCol<R> c;
     c.i = col0 + t, c.t = t, c.nrl = in.nlay + 1;
-    c.lcf1 = cs.lcf1[t];
     c.table = SURR ? sg.table(t, B) : 1;
     const double pwv = cs.pwv[t];
     c.sdif = (R)((B == 0 || B == 3 || B == 9) ? 1.66 : fmin(1.80, fmax(1.50, LW_A0[B] + LW_A1[B] * exp_d(LW_A2[B] * pwv))));
@@ -654,7 +642,7 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
                                           int col0, int n, const ColScal &cs, const RecPtrs &rp, const AccT<R> &acc,
                                           const Surr &sg, int blk, int lane, WR_G char *slot)
 {
-    constexpr int NG = LW_NG[B], GW = NG, CH = lw_chunk_r<R, B>();
+    constexpr int NG = LW_NG[B], GW = NG, CH = lw64_chunk<B>();
     const Share<R> sh{nullptr, 0, 0};
     const int nv = valid_cols(in, col0, n);
     if (blk * 64 >= nv) return;
@@ -768,7 +756,7 @@ __device__ __forceinline__ void lw_column(const Tabs<R> *__restrict__ T, const B
 }
 
 template <typename R, int B, bool SURR = false, bool EXT = true>
-__global__ void __launch_bounds__(64, (lw_waves<R, B>())) k_lw(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
+__global__ void __launch_bounds__(64, lw64_waves<B>()) k_lw(const Tabs<R> *__restrict__ T, ColIn in_, RunPar par, int col0,
                                            int n, ColScal cs, RecPtrs rp, AccT<R> acc, Surr sg, char *__restrict__ pool)
 {
     const ColIn in = band_in<EXT>(in_);
@@ -831,13 +819,13 @@ template <typename R> __device__ __forceinline__ void lds_fill_lw(float4 *dst, c
 
 // k_lw (FP64, one lane per column) with the band's tables and the transmittance table in LDS (absb, the table
 // of the layers above laytrop, and the minor gases of bands 3 and 5 stay in global memory: the rest of every
-// band then fits).  Persistent workgroups of 4 x lw_waves waves, as many as the CUs hold; each copies the tables
+// band then fits).  Persistent workgroups of 4 x lw64_waves waves, as many as the CUs hold; each copies the tables
 // into LDS once and its waves then run 64-column blocks.  Same arithmetic as k_lw.  Bound by memory latency at two
 // waves per SIMD (0.3 to 0.4 of the issue slots): the LW kernels of a 954x835x60 call take 124 ms alone on the GPU, 144
 // with the optics evaluated in both sweeps and whole entries gathered from L2.
-template <typename R, int B> constexpr int lwl64_wpg() { return 4 * lw_waves<R, B>(); }
+template <int B> constexpr int lwl64_wpg() { return 4 * lw64_waves<B>(); }
 template <int B, bool SURR = false, bool EXT = true>
-__global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<double, B>()))
+__global__ void __launch_bounds__(64 * lwl64_wpg<B>(), lw64_waves<B>())
     k_lwl64(const Tabs<double> *__restrict__ T, ColIn in_, RunPar par, int col0, int n, ColScal cs, RecPtrs rp,
             AccT<double> acc, Surr sg, char *__restrict__ pool)
 {
@@ -846,7 +834,7 @@ __global__ void __launch_bounds__((64 * lwl64_wpg<double, B>()), (lw_waves<doubl
     const LwImg<double> &im = T->lw_img[B];
     lds_fill_lw<double>(lwl64_tab, im, T->exp_tbl);
     const auto Bl = lds_band<double, B>((const WR_L double *)lwl64_tab, im, T->lw[B], T->lw[B].absb);
-    constexpr int WPG = lwl64_wpg<double, B>();
+    constexpr int WPG = lwl64_wpg<B>();
     const int lane = threadIdx.x % 64, w = wave_slot();
     WR_G char *slot = (WR_G char *)(pool + (size_t)w * lw64_slot_bytes(LW_NG[B], in.nlay + 2));
     for (int blk = w; blk * 64 < n; blk += gridDim.x * WPG)

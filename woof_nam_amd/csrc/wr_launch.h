@@ -164,7 +164,7 @@ void launch_band(const BandJob<R> &j, int id, hipStream_t s, char *pool)
             }
         } else if constexpr (B < 16 && sizeof(R) == 8) {
             // k_lwl64: persistent workgroups, as many as the CUs hold at once
-            constexpr unsigned WPG = lwl64_wpg<R, B>();
+            constexpr unsigned WPG = lwl64_wpg<B>();
             const size_t lds = (size_t)j.c->host_d.lw_img[B].n * sizeof(double) + ETAB_LDS;
             static std::atomic<int> per_cu{-1};  // workgroups per CU, once per instance (one table set per process)
             if (per_cu < 0 && ((j.c->lw_lds64 >> B) & 1)) {
@@ -293,8 +293,8 @@ void launch_band_nam(const BandJob<R> &j, int id, hipStream_t s, char *pool)
     }
 }
 
-// True when the band kernels may leave stream s: the context has auxiliary streams (their pools are
-// allocated by wr_create).  Under graph capture the fork and join events bring the auxiliary streams
+// True when the band kernels may leave stream s: the context has auxiliary streams and a pool for each (wr_create; a
+// context of small tiles, which run in two launches, has one pool).  Under graph capture the fork and join events bring the auxiliary streams
 // into the graph, so a captured tile holds the same band concurrency as an eager one.
 inline bool spread_bands(wr_ctx *c, hipStream_t s)
 {

@@ -7,8 +7,8 @@
 // the other; the optics do not.  So the small tiles run
 //   k_lay    the optics of every (64-column block, band, layer): transmittances and sources (LW), layer
 //            R/T (SW) to the pool, one wave each, all of them independent;
-//   k_sweep  the sweeps of every (block, band) over those values, MANY_GW g-points per wave, with the loads of
-//            the layers ahead in flight; the level sums over the waves of a band meet in LDS in g order.
+//   k_sweep  the sweeps of every (block, band) over those values, MANY_GW g-points per wave; the level sums over
+//            the waves of a band meet in LDS in g order.
 // Both use the expressions of the per-band kernels, so the outputs are the same bits.
 //
 // Values that only clouds need are written and read only for the layers of a block that hold cloud.  The NAM

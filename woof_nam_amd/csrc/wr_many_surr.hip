@@ -1,4 +1,4 @@
-// wr_many_surr.hip -- the one-launch band kernel of small tiles (mixed precision, learned gas optics, McICA route).
+// wr_many_surr.hip -- the two launches of small tiles (mixed precision, learned gas optics, McICA route).
 #include "wr_many.h"
 
 namespace wr {

@@ -4,7 +4,7 @@
 // GEMM: C[M x N] = A[M x K] * B[K x N] with arbitrary element strides on A, B and C, operands
 // staged through LDS as BF16, gfx950's v_mfma_f32_16x16x32_bf16 tiles, FP32 accumulation.  A
 // 256-thread workgroup computes a 64 x 64 tile of C (4 waves, 2 x 2 MFMA tiles of 16 x 16 each); K
-// advances 32 per step.  Each thread stages a run of 8 elements of A and of B along whichever of
+// advances 64 per step.  Each thread stages two runs of 8 elements of A and of B along whichever of
 // their dimensions is contiguous in memory (one 16- or 32-byte load when aligned and whole), so the
 // staging reads are coalesced for row-major activations, transposed activations and weights alike.
 // Split-K writes deterministic partial sums, reduced by k_splitk_reduce.
@@ -112,7 +112,7 @@ __device__ __forceinline__ void stage_store(const Staged &s, bool rows_contig, _
 }
 
 // 64 x 64 tile per workgroup.  The loads of the next K step are in flight while the MFMAs of this one run; a step
-// is GK = 64 deep, so that a split of a weight gradient (1,024 samples) is 16 of them.  Bound by the latency of a
+// is GK = 64 deep, so that a weight gradient's split of 256 samples is 4 of them.  Bound by the latency of a
 // step where the grid is small (the weight gradients), by the operands' bytes otherwise.
 template <typename TA, typename TB, int EPI>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
@@ -184,8 +184,8 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
 
 // ---- fused inference: the three layers of the network in one kernel ----------------------------
 // H1 = SiLU(X W1^T + b1) and H2 = SiLU(H1 W2^T + b2) stay in LDS (BF16); Y = H2 W3^T + b3 is written
-// output-major in BF16, Y[n * ldy + m].  Same MFMA operands, K order, bias, SiLU and BF16 roundings as the three-GEMM chain,
-// so the outputs equal the chain's bit for bit; the weights ([n][k] rows, BF16) are read straight
+// output-major in BF16, Y[n * ldy + m].  Same MFMA operands, K order, bias, SiLU and BF16 roundings as the
+// three-GEMM chain, so the outputs equal the chain's bit for bit; the weights ([n][k] rows, BF16) are read straight
 // into MFMA operands (L2-resident).
 constexpr int FH = 128, FO = 504, FLD = FH + 8;
 

@@ -371,14 +371,4 @@ __device__ __forceinline__ void sw_cloud(const Tabs<R> *__restrict__ T, int B, d
     asy = asyliq + asyice + (R)asyran + (R)0;
 }
 
-// sw_cloud of radiation layer kin of column rc with the layer's radii and rain path (path form)
-template <typename R>
-__device__ __forceinline__ void sw_cloud_l(const Tabs<R> *__restrict__ T, int B, const SwLay<R> &L, const RadCol &rc, int kin,
-                                           const RunPar &par, R &tau, R &ssa, R &asy)
-{
-    double rl, ri, rp;
-    rc.props(kin, par.re_liq, par.re_ice, rl, ri, rp);
-    sw_cloud<R>(T, B, L.cwp, rl, L.cip, ri, tau, ssa, asy, rp);
-}
-
 }  // namespace wr
