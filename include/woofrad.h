@@ -137,8 +137,9 @@ void wr_default_params(wr_params *p);
 int wr_create(wr_ctx **out, const char *table_path, int device, int32_t max_cols);
 
 /* Device bytes wr_create allocates for a context of `max_cols` columns (tables, tile work space and
- * the band streams' level pools, under the same WR_POOL_GB / WR_BAND_STREAMS settings), computed on
- * the host without allocating: callers size max_cols from free device memory with it, as
+ * the level pools, under the same WR_POOL_GB / WR_BAND_STREAMS / WR_MANY_COLS settings; where the
+ * device has less free, wr_create makes do with smaller pools if it can), computed on the host
+ * without allocating: callers size max_cols from free device memory with it, as
  * namgpu/physics/rrtm/rrtm_call.py:183-203 (batch_count) sizes its batches.  0 for max_cols <= 0. */
 uint64_t wr_context_bytes(int32_t max_cols);
 

@@ -9,8 +9,8 @@ seeds) arrive at any time.  The server
   device; a tile is handed to the next free slot as soon as one frees up (requests that arrive
   while others run join the tile queue at once: continuous batching at tile granularity);
 * runs each tile as one replay of a HIP graph captured once per slot (the kernels of a tile:
-  column scalars, day list, 16 LW and 14 SW band kernels spread over the context's band streams,
-  post; with precision "surrogate" also the layer features and the network's inference kernel,
+  layer records, column scalars, day list, 16 LW and 14 SW band kernels spread over the context's band
+  streams, or two launches for all bands in tiles of up to 65,536 columns, post; with precision "surrogate" also the layer features and the network's inference kernel,
   with the table fallback of columns outside the training envelope) over the slot's staging buffers.
   The slots are the library's (wr_slot_*): a tile is one library call that gathers it into the
   staging buffers with the request's seed and the tile's column count (one kernel), replays the
