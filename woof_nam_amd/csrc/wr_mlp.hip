@@ -91,7 +91,7 @@ __device__ __forceinline__ Staged stage_load(const T *X, long long ld_row, long 
         } else {
             const int row = r0 + (tid >> 2);
             const unsigned k = kk + (tid & 3) * 8 + u * 32;
-            const int cnt = row < nrow && k < k_end ? (int)min(8u, k_end - k) : 0;
+            const int cnt = row < nrow ? max(0, min(8, (int)(k_end - k))) : 0;
             s.v[u] = run8(X + (cnt > 0 ? (size_t)row * ld_row + (size_t)k * ld_k : 0), ld_k, cnt);
         }
     }
