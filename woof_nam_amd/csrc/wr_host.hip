@@ -549,6 +549,7 @@ constexpr int MANY_COLS_DEFAULT = 65536;
 //   FP64 McICA  1,000 columns     968 /    778 /    739 /    735 /    737 /    734
 //               4,096           3,088 /  2,546 /  2,290 /  1,947 /  1,869 /  1,879
 //   FP64 NAM    4,096           6,583 /  4,458 /  3,269 /  2,832 /  2,564 /  2,424
+//               20,000         30,535 / 20,600 / 14,858 / 12,438 / 11,232 / 11,025
 //               40,000         60,348 / 40,766 / 30,000 / 24,545 / 22,018 / 21,759
 //   mixed McICA 4,096             947 /    920 /    888 /    885 /    895 /    886
 constexpr size_t MANY_POOL = (size_t)2e9;
